@@ -1,0 +1,667 @@
+// Prompt chunks of the two recurrences with a matrix state and one decay per head and token, on
+// the fp32 matrix instructions:
+//   selective scan   S <- a_t S + dt_t B_t x_t^T,  y_t = S^T C_t + d x_t     (a_t from dt_t)
+//   retention        S <- a S + k_t v_t^T,         o_t = S^T q_t, normed and gated per head
+// A sequence's rows go in chunks of 32.  With c_i the sum of the log2 decays from the chunk's
+// start through row i, S0 the state before it, k / q / v the rows (k times dt for the scan):
+//   o_i   = 2^(c_i) q_i S0 + sum_{j <= i} 2^(c_i - c_j) (q_i . k_j) v_j
+//   S_end = 2^(c_end) S0 + sum_j k_j (2^(c_end - c_j) v_j)^T
+// Everything is fp32 (v_mfma_f32_32x32x2_f32: the vector units' rate without packed
+// instructions, but four times the operations per LDS or register read), the decays' sums fp64:
+// differences of sums of the size of 30 in fp32 would lose two digits.
+//
+// chunk_frag_kernel prepares every (chunk, key head) side by side: q and k (rotated and scaled
+// for the retention) as operand fragments and the 32 x 32 products q_i . k_j; the scan's keys
+// belong to a group, so its heads share them.  chunk_scalar_kernel sums the scan's decays.
+// chunk_walk_kernel then walks the chunks of a (sequence, head): a wave owns 32 state columns in
+// accumulators.  An accumulator lane holds column l & 31 and rows 8 g + 4 (l >> 5) + r in
+// register 4 g + r: read as the B operand of the next product, step r of piece g contracts over
+// the rows 8 g + r and 8 g + 4 + r, so with A fragments stored in that order (lane (i, hh) of
+// piece g: 4 consecutive entries from 8 g + 4 hh on, one 16-byte load for four products) the
+// state, the values and the outputs feed each other without lane traffic.
+//
+// Bound by the fp32 matrix rate (144 products of 64 cycles per chunk, head and 32 columns of a
+// 128-row state; 140 TFLOP/s in a register loop): 16384 rows of 8 sequences, 64 heads x 128 x 64
+// states 452 us (276 us of products) where the row-by-row scan took 1420; 8 heads x 128 x 128
+// (segments) 264 us in all, by rows 790.
+//
+// A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
+// steps whose (sequence, head, 32 columns) triples leave SIMDs idle run in segments of rows:
+// the same walk without outputs leaves every segment's own state, chunk_join_kernel turns these
+// into the state before each segment, and the full walk starts from there.
+#include <type_traits>
+
+#include "../kernels/common.h"
+#include "stream.h"
+
+namespace akap_stream {
+
+using akap::bf16;
+using akap::f32x16;
+
+namespace {
+
+constexpr int kL = 32;      // rows of a chunk
+constexpr int kScal = 256;  // floats of the scan's scalars per (chunk, head): 5 x 32, and room
+
+__device__ __forceinline__ float ldv(const float* p) { return *p; }
+__device__ __forceinline__ float ldv(const bf16* p) { return (float)*p; }
+__device__ __forceinline__ void ld4(const float* p, float (&v)[4]) {
+  const float4 a = *(const float4*)p;
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void ld4(const bf16* p, float (&v)[4]) {
+  const akap::bf16x4 a = *(const akap::bf16x4*)p;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (float)a[i];
+}
+
+// Rows of a chunk through a buffer descriptor: reads past `bytes` give zeros.
+using Rsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ Rsrc rows_of(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ float rd(Rsrc r, uint32_t off, float) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+__device__ __forceinline__ bf16 rd(Rsrc r, uint32_t off, bf16) {
+  return __builtin_bit_cast(bf16, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+}
+__device__ __forceinline__ void st4(float* p, float a, float b, float c, float d) {
+  *(float4*)p = make_float4(a, b, c, d);
+}
+__device__ __forceinline__ void st4(bf16* p, float a, float b, float c, float d) {
+  const akap::bf16x4 o = {(bf16)a, (bf16)b, (bf16)c, (bf16)d};
+  *(akap::bf16x4*)p = o;
+}
+
+// the same value, as one the compiler knows nothing about: what is derived from it is formed anew
+// in every round of a loop instead of being kept in registers across it
+__device__ __forceinline__ uint32_t fresh(uint32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// 16 bytes per lane from global memory to LDS (a lane's place: the wave's address + 16 lane)
+__device__ __forceinline__ void dma16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                   (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+
+__device__ __forceinline__ f32x16 mfma(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// decay^k for a decay given by its log2 (-inf: a decay of zero)
+__device__ __forceinline__ float decay_pow(float l2, int k) {
+  return k == 0 ? 1.0f : exp2f(l2 * (float)k);
+}
+
+// entries of the per-chunk buffers: sequence b owns those from base(b) on
+__device__ __forceinline__ int base_of(const int32_t* q_start, int b, int rows) {
+  return q_start[b] / rows + b;
+}
+
+// the sequence that owns an entry, and the rows [r0, r1) of the entry (r1 <= r0: none)
+__device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int rows, int& r0, int& r1) {
+  int lo = 0, hi = p.B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (base_of(p.q_start, mid, rows) <= entry) lo = mid; else hi = mid - 1;
+  }
+  const int first = p.q_start[lo], end = p.q_start[lo + 1];
+  r0 = first + (entry - base_of(p.q_start, lo, rows)) * rows;
+  r1 = min(r0 + rows, end);
+  if (r0 < first) r1 = r0;
+  return lo;
+}
+
+__device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
+  return slot >= 0 && slot < p.num_slots;
+}
+
+// ------------------------------------------------------------------ fragments of q and k
+// One workgroup per (chunk, key head).  Buffer of an entry: [q: NT 4 fragments][k transposed:
+// the same][q . k: 4 fragments], 64 lanes x 4 floats each; rows past the chunk's end are zero.
+template <int MODE, int NT, typename TY>
+__global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
+  constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
+  __shared__ __align__(16) float qs[kL * LS > 4096 ? kL * LS : 4096];
+  __shared__ __align__(16) float ks[kL * LS];
+  float* red = qs;   // the waves' shares of the products, once every wave has read q
+  const int entry = blockIdx.x, kh = blockIdx.y;
+  int r0, r1;
+  const int b = locate(p, entry, kL, r0, r1);
+  if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
+  const int n = r1 - r0, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int half = p.rot_dims / 2;
+  // a thread keeps to four columns; its rows' loads are in flight together
+  const int d = (tid % (N / 4)) * 4, i0 = tid / (N / 4);
+  constexpr int RS = 256 / (N / 4), RN = kL / RS;   // rows per turn, turns
+  float q4[RN][4], k4[RN][4], q2[MODE == 1 ? RN : 1][4], k2[MODE == 1 ? RN : 1][4];
+  int64_t pos[MODE == 1 ? RN : 1];
+  const bool rot = MODE == 1 && d < p.rot_dims, low = d < half;
+#pragma unroll
+  for (int u = 0; u < RN; ++u) {
+    const int t = r0 + min(i0 + u * RS, n - 1);
+    if (MODE == 0) {
+      const float* row = p.xbc + (size_t)t * p.x_stride + p.H * p.V + kh * N + d;
+      ld4(row, k4[u]);
+      ld4(row + p.KH * N, q4[u]);
+    } else {
+      const TY* row = (const TY*)p.proj + (size_t)t * p.proj_stride + kh * N;
+      ld4(row + p.q_off + d, q4[u]);
+      ld4(row + p.k_off + d, k4[u]);
+      if (rot) {
+        const int d2 = low ? d + half : d - half;
+        pos[u] = p.positions[t];
+        ld4(row + p.q_off + d2, q2[u]);
+        ld4(row + p.k_off + d2, k2[u]);
+      }
+    }
+  }
+  if (rot) {
+    const int a = low ? d : d - half;
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const float* cs = p.cos_sin + (size_t)pos[u] * p.rot_dims + a;
+      float c4[4], s4[4];
+      ld4(cs, c4);
+      ld4(cs + half, s4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float sn = low ? -s4[j] : s4[j];
+        q4[u][j] = q4[u][j] * c4[j] + q2[u][j] * sn;
+        k4[u][j] = k4[u][j] * c4[j] + k2[u][j] * sn;
+      }
+    }
+  }
+  const float kscale = MODE == 1 ? 1.0f / sqrtf((float)N) : 1.0f;
+#pragma unroll
+  for (int u = 0; u < RN; ++u) {
+    const int i = i0 + u * RS;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b4 = a;
+    if (i < n) {
+      a = make_float4(q4[u][0], q4[u][1], q4[u][2], q4[u][3]);
+      b4 = make_float4(k4[u][0] * kscale, k4[u][1] * kscale, k4[u][2] * kscale, k4[u][3] * kscale);
+    }
+    *(float4*)(qs + i * LS + d) = a;
+    *(float4*)(ks + i * LS + d) = b4;
+  }
+  __syncthreads();
+  const int li = lane & 31, hh = lane >> 5;
+  float4* out = (float4*)(p.frag + ((size_t)entry * p.KH + kh) * p.frag_floats);
+  for (int f = wave; f < NT * 4; f += 4) {
+    out[f * 64 + lane] = *(const float4*)(qs + li * LS + 8 * f + 4 * hh);
+    const float* kk = ks + (8 * (f & 3) + 4 * hh) * LS + 32 * (f >> 2) + li;
+    out[(NT * 4 + f) * 64 + lane] = make_float4(kk[0], kk[LS], kk[2 * LS], kk[3 * LS]);
+  }
+  // q . k with the keys as rows: lane (i, hh) register 4 g + r is q_i . k_(8 g + 4 hh + r), the
+  // operand the walk needs; the waves contract a part of the entries each
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int f = wave; f < NT * 4; f += 4) {
+    const float4 a = *(const float4*)(ks + li * LS + 8 * f + 4 * hh);
+    const float4 c = *(const float4*)(qs + li * LS + 8 * f + 4 * hh);
+    acc = mfma(a.x, c.x, acc);
+    acc = mfma(a.y, c.y, acc);
+    acc = mfma(a.z, c.z, acc);
+    acc = mfma(a.w, c.w, acc);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *(float4*)(red + wave * 1024 + (g * 64 + lane) * 4) =
+        make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+  __syncthreads();
+  float4 s = *(const float4*)(red + tid * 4);
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    const float4 t = *(const float4*)(red + w * 1024 + tid * 4);
+    s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+  }
+  out[NT * 8 * 64 + tid] = s;
+}
+
+// ------------------------------------------------------------------ step sizes and decays
+// Half a wave per (chunk, head) of the selective scan, a lane per row.  With c the sums of the log2
+// decays (formed in fp64): [32] dt, [32] 2^c, [32] dt 2^(c_end - c), [32] c, [32] what c lost when
+// it was rounded.  Rows past the end: dt 0, decay 1.
+template <typename TY>
+__global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams p) {
+  const int entry = blockIdx.x, i = threadIdx.x & 31;
+  int r0, r1;
+  const int b = locate(p, entry, kL, r0, r1);
+  if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
+  const int n = r1 - r0;
+  const TY* src = (const TY*)p.proj + (size_t)(r0 + min(i, n - 1)) * p.proj_stride + p.dt_off;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int h = blockIdx.y * 32 + u * 8 + (threadIdx.x >> 5);
+    if (h >= p.H) return;   // (all lanes of a half wave share h)
+    const float v = ldv(src + h) + p.dt_bias[h];
+    const float dt = i < n ? (v > 20.f ? v : log1pf(expf(v))) : 0.f;
+    double l = i < n ? -(double)expf(p.a_log[h]) * 1.4426950408889634 * (double)dt : 0.0;
+    if (l < -4096.0) l = -4096.0;  // 2^l is zero long before; keeps the sums finite
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) {
+      const double up = __shfl_up(l, o, 32);
+      if (i >= o) l += up;
+    }
+    const double end = __shfl(l, 31, 32);
+    float* sc = p.scal + ((size_t)entry * p.H + h) * kScal;
+    const float hi = (float)l;
+    sc[i] = dt;
+    sc[kL + i] = exp2f(hi);
+    sc[2 * kL + i] = i < n ? dt * exp2f((float)(end - l)) : 0.f;
+    sc[3 * kL + i] = hi;
+    sc[4 * kL + i] = (float)(l - (double)hi);
+  }
+}
+
+// ------------------------------------------------------------------ the walk
+// HW heads (of one key head) of V / 32 waves each, a wave per 32 state columns; FULL: outputs,
+// from the state in the slot (or, SEGM, from the segment buffer); else the segment's own state
+// from zeros.  A chunk's fragments and scalars arrive by LDS-DMA while the chunk before is
+// computed (two buffers of 37 KB, so two workgroups share a CU), its values in registers: a wave
+// waits once per chunk, for loads issued some 10000 cycles earlier.
+template <int MODE, int NT, int V, int HW, typename TY, bool FULL, bool SEGM>
+__global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkScanParams p) {
+  constexpr int N = NT * 32, NF = NT * 4, VW = V / 32, NW = VW * HW;
+  constexpr bool kNorm = MODE == 1 && FULL;
+  // fragments of a buffer: [q (FULL)][k][q . k (FULL)][scalars of the heads (scan)]
+  constexpr int K0 = FULL ? NF : 0, G0 = K0 + NF, C0 = G0 + (FULL ? 4 : 0);
+  constexpr int NB = C0 + (MODE == 0 ? HW : 0);
+  __shared__ __align__(16) float4 buf[2][NB * 64];
+  __shared__ __align__(16) float tab[MODE == 1 ? NW * 3 * kL : 4];   // per wave, see below
+  __shared__ __align__(16) float pd[kNorm ? 1024 : 4];       // retention: 2^(c_i - c_j), by lane
+  __shared__ __align__(16) float ssq[kNorm ? 2 * NW * kL : 4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h0 = blockIdx.y * HW, hw = wave / VW, h = h0 + hw;
+  const int li = lane & 31, hh = lane >> 5;
+  int b = blockIdx.x, r0, r1;
+  if (SEGM) {
+    b = locate(p, blockIdx.x, p.SEG, r0, r1);
+  } else {
+    r0 = p.q_start[b];
+    r1 = p.q_start[b + 1];
+  }
+  if (r1 <= r0) return;
+  const int first = p.q_start[b];
+  const int slot = p.seq_slot[first];
+  if (!live_slot(p, slot)) return;
+  const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
+  const int col = (wave % VW) * 32 + li;
+  const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
+  // retention: decay^k, decay^(k + 1), and the weights of a cut chunk's values in the new state
+  float* tb = tab + (MODE == 1 ? wave * 3 * kL : 0);
+  if (MODE == 1) {
+    if (lane < kL) {
+      tb[lane] = decay_pow(l2, lane);
+      tb[kL + lane] = decay_pow(l2, lane + 1);
+      tb[2 * kL + lane] = decay_pow(l2, kL - 1 - lane);
+    }
+    if (kNorm) {
+      for (int e = tid; e < 1024; e += 64 * NW) {
+        const int ln = (e >> 2) & 63, j = 8 * (e >> 8) + 4 * (ln >> 5) + (e & 3), i = ln & 31;
+        pd[e] = j <= i ? decay_pow(l2, i - j) : 0.f;
+      }
+    }
+  }
+  // entry (row, column) of the state: the scan keeps [N, V], the retention [V, N]
+  float* sp = (SEGM ? p.seg + ((size_t)blockIdx.x * p.H + h) * N * V
+                    : p.state + ((size_t)slot * p.H + h) * N * V);
+  f32x16 S[NT];
+  const bool load = FULL && (SEGM || p.positions[first] != 0);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 32 * t + 8 * g + 4 * hh;
+      if (!load) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = 0.f;
+      } else if (MODE == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = sp[(size_t)(row + r) * V + col];
+      } else {
+        const float4 v = *(const float4*)(sp + (size_t)col * N + row);
+        S[t][4 * g] = v.x; S[t][4 * g + 1] = v.y; S[t][4 * g + 2] = v.z; S[t][4 * g + 3] = v.w;
+      }
+    }
+  const int c0 = (r0 - first) / kL, chunks = (r1 - r0 + kL - 1) / kL;
+  const size_t cb = (size_t)base_of(p.q_start, b, kL) + c0;
+  const uint32_t l16 = lane * 16;
+  auto stage = [&](int c, float4* to) {
+    const char* src = (const char*)p.frag + ((cb + c) * p.KH + kh) * p.frag_floats * 4 +
+                      (FULL ? 0 : NF * 1024) + wave * 1024;
+#pragma unroll
+    for (int u = 0; u < (C0 + NW - 1) / NW; ++u)
+      if ((u + 1) * NW <= C0 || u * NW + wave < C0)
+        dma16(src + u * NW * 1024 + l16, to + (u * NW + wave) * 64);
+    if (MODE == 0 && wave < HW)
+      dma16((const char*)(p.scal + ((cb + c) * p.H + h0 + wave) * kScal) + l16,
+            to + (C0 + wave) * 64);
+  };
+  // values of a chunk's rows 8 g + 4 hh + r at a lane's column
+  const int ld = MODE == 0 ? p.x_stride : p.proj_stride;
+  constexpr int es = MODE == 0 ? 4 : sizeof(TY);
+  using TX = typename std::conditional<MODE == 0, float, TY>::type;
+  const uint32_t lx = (uint32_t)(4 * hh * ld + (MODE == 0 ? 0 : p.v_off) + h * V + col) * es;
+  TX xn[16];
+  auto values = [&](int c) {
+    const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+    const Rsrc rs = rows_of((MODE == 0 ? (const char*)p.xbc : (const char*)p.proj) + (size_t)t0 * ld * es,
+                            (uint32_t)(n * ld * es));
+    const uint32_t step = (uint32_t)ld * es;
+    uint32_t o = fresh(lx);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      xn[s] = rd(rs, o, TX{});
+      o += (s & 3) == 3 ? 5 * step : step;
+    }
+  };
+  const float dsk = MODE == 0 ? p.d_skip[h] : 0.f;
+  float total = 0.f;   // log2 decay of the segment
+  stage(0, buf[0]);
+  values(0);
+  // outputs transposed: row 8 g + 4 hh + r of the accumulator is a column of the state, lane li the
+  // token.  They are written after the next chunk's wait, which would otherwise wait for them.
+  f32x16 O;
+  auto write = [&](int c) {
+    const int t = r0 + c * kL + li;
+    if (t >= r1) return;
+    const int at = h * V + (wave % VW) * 32 + 4 * hh;
+    if (MODE == 0) {
+      float* o = p.y + (size_t)t * p.H * V + at;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        st4(o + 8 * g, O[4 * g], O[4 * g + 1], O[4 * g + 2], O[4 * g + 3]);
+    } else {
+      TY* o = (TY*)p.out + (size_t)t * p.out_stride + at;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        st4(o + 8 * g, O[4 * g], O[4 * g + 1], O[4 * g + 2], O[4 * g + 3]);
+    }
+  };
+  // (now and next are restrict so that the reads of one buffer are known not to touch the other:
+  // else every read would wait for the DMA under way)
+  auto step = [&](int c, const float4* __restrict__ now, float4* __restrict__ next) {
+    const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+    // (vmcnt 0, lgkmcnt 0, as a builtin: the compiler then knows that the values have arrived)
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();   // this chunk has landed; the other buffer is free
+    asm volatile("" ::: "memory");
+    float x[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) x[s] = (float)xn[s];
+    if (c + 1 < chunks) {
+      stage(c + 1, next);
+      values(c + 1);
+    }
+    if (FULL && c > 0) write(c - 1);
+    const float4* cur = now + lane;
+    const float* sc = MODE == 0 ? (const float*)(now + (C0 + hw) * 64) : nullptr;
+    const float* we = MODE == 0 ? sc + 2 * kL : tb + 2 * kL;
+    const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
+    if (MODE == 0 && !FULL) total += sc[4 * kL - 1];
+    if (MODE == 1 && n < kL && lane < kL)
+      tb[2 * kL + lane] = lane < n ? tb[n - 1 - lane] : 0.f;   // (the last chunk)
+    akap::bf16x4 zb[kNorm ? 4 : 1];
+    float4 zf[kNorm ? 4 : 1];
+    if (FULL) {
+      if (kNorm) {
+        const TY* zr = (const TY*)p.proj + (size_t)(t0 + min(li, n - 1)) * p.proj_stride + p.g_off +
+                       h * V + (wave % VW) * 32 + 4 * hh;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if (sizeof(TY) == 2) zb[g] = *(const akap::bf16x4*)(zr + 8 * g);
+          else zf[g] = *(const float4*)(zr + 8 * g);
+        }
+      }
+      // two chains: independent products in flight, and shorter sums
+      f32x16 O2;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) O[i] = O2[i] = 0.f;
+#pragma unroll
+      for (int f = 0; f < NF; f += 2) {
+        const int t = f >> 2, g = f & 3;
+        const float4 a = cur[f * 64], d = cur[(f + 1) * 64];
+        O = mfma(S[t][4 * g], a.x, O);
+        O2 = mfma(S[t][4 * g + 4], d.x, O2);
+        O = mfma(S[t][4 * g + 1], a.y, O);
+        O2 = mfma(S[t][4 * g + 5], d.y, O2);
+        O = mfma(S[t][4 * g + 2], a.z, O);
+        O2 = mfma(S[t][4 * g + 6], d.z, O2);
+        O = mfma(S[t][4 * g + 3], a.w, O);
+        O2 = mfma(S[t][4 * g + 7], d.w, O2);
+      }
+      float P[16];
+      const float ch_i = MODE == 0 ? sc[3 * kL + li] : 0.f, cl_i = MODE == 0 ? sc[4 * kL + li] : 0.f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 g4 = cur[(G0 + g) * 64];
+        const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
+        if (MODE == 0) {
+          // the sums as float pairs: a difference of sums then has the error of its own size
+          const float4 d4 = *(const float4*)(sc + 8 * g + 4 * hh);
+          const float4 h4 = *(const float4*)(sc + 3 * kL + 8 * g + 4 * hh);
+          const float4 l4 = *(const float4*)(sc + 4 * kL + 8 * g + 4 * hh);
+          const float dt[4] = {d4.x, d4.y, d4.z, d4.w};
+          const float ch[4] = {h4.x, h4.y, h4.z, h4.w}, cl[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = 8 * g + 4 * hh + r;
+            const float d = (ch_i - ch[r]) + (cl_i - cl[r]);
+            float f = gv[r] * (dt[r] * __builtin_amdgcn_exp2f(d));
+            // (d_skip x is the diagonal's share of the same product)
+            f += j == li ? dsk : 0.f;
+            asm("" : "+v"(f));     // a select, no branch
+            P[4 * g + r] = j <= li ? f : 0.f;
+          }
+        } else {
+          const float4 d4 = *(const float4*)(pd + (g * 64 + lane) * 4);
+          const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float f = gv[r] * dd[r];
+            asm("" : "+v"(f));
+            P[4 * g + r] = 8 * g + 4 * hh + r <= li ? f : 0.f;
+          }
+        }
+      }
+      const float e = MODE == 0 ? sc[kL + li] : tb[kL + li];
+#pragma unroll
+      for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
+      // a value that is not finite must not reach the rows before its own (0 x inf)
+      float fin = 0.f;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) fin = fmaf(x[s], 0.f, fin);
+      if (__builtin_expect(__any(fin != 0.f), 0)) {
+#pragma unroll 1
+        for (int i = 0; i < kL; ++i) {
+          f32x16 one = O;
+#pragma unroll
+          for (int s = 0; s < 16; ++s)
+            one = mfma(8 * (s >> 2) + 4 * hh + (s & 3) <= i ? x[s] : 0.f, P[s], one);
+#pragma unroll
+          for (int s = 0; s < 16; ++s) O[s] = li == i ? one[s] : O[s];
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) O = mfma(x[s], P[s], O);
+      }
+    }
+    // the state after the chunk
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S[t][i] *= dend;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 w4 = *(const float4*)(we + 8 * g + 4 * hh);
+      const float xw[4] = {x[4 * g] * w4.x, x[4 * g + 1] * w4.y, x[4 * g + 2] * w4.z,
+                           x[4 * g + 3] * w4.w};
+      float4 k4[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) k4[t] = cur[(K0 + t * 4 + g) * 64];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].x, xw[0], S[t]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].y, xw[1], S[t]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].z, xw[2], S[t]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].w, xw[3], S[t]);
+    }
+    if (FULL) {
+      float inv = 1.f;
+      if (kNorm) {
+        // the head's root mean square: a lane's columns, the other half's, the other waves'
+        float ss = 0.f;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) ss = fmaf(O[s], O[s], ss);
+        ss += __shfl_xor(ss, 32, 64);
+        float* sq = ssq + (c & 1) * NW * kL;
+        if (hh == 0) sq[wave * kL + li] = ss;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        ss = 0.f;
+#pragma unroll
+        for (int w = 0; w < VW; ++w) ss += sq[(hw * VW + w) * kL + li];
+        inv = 1.0f / sqrtf(ss / (float)V + p.eps);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float zv[4];
+          if (sizeof(TY) == 2) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) zv[r] = (float)zb[g][r];
+          } else {
+            zv[0] = zf[g].x; zv[1] = zf[g].y; zv[2] = zf[g].z; zv[3] = zf[g].w;
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            O[4 * g + r] = O[4 * g + r] * inv * zv[r] * (1.0f / (1.0f + __expf(-zv[r])));
+        }
+      }
+    }
+  };
+#pragma unroll 1
+  for (int c = 0; c < chunks; ++c) step(c, buf[c & 1], buf[(c + 1) & 1]);
+  if (FULL) write(chunks - 1);
+  if (FULL && SEGM) return;  // the slots were written when the segments were joined
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 32 * t + 8 * g + 4 * hh;
+      if (MODE == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sp[(size_t)(row + r) * V + col] = S[t][4 * g + r];
+      } else {
+        *(float4*)(sp + (size_t)col * N + row) = make_float4(S[t][4 * g], S[t][4 * g + 1],
+                                                             S[t][4 * g + 2], S[t][4 * g + 3]);
+      }
+    }
+  if (SEGM && lane == 0 && wave % VW == 0)
+    p.seg_decay[(size_t)blockIdx.x * p.H + h] =
+        MODE == 0 ? exp2f(total) : decay_pow(l2, r1 - r0);
+}
+
+// the state before each segment from the segments' own states, and the sequence's final state
+// into its slot: a thread per four entries, the loads of eight segments in flight together
+__global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p) {
+  const int b = blockIdx.x, h = blockIdx.y;
+  const size_t hs = (size_t)p.V * p.N;
+  const size_t e = ((size_t)blockIdx.z * 256 + threadIdx.x) * 4;
+  const int r0 = p.q_start[b], r1 = p.q_start[b + 1];
+  if (r1 <= r0 || e >= hs) return;
+  const int slot = p.seq_slot[r0];
+  if (!live_slot(p, slot)) return;
+  const int nseg = (r1 - r0 + p.SEG - 1) / p.SEG;
+  const size_t sb = base_of(p.q_start, b, p.SEG);
+  float4* st = (float4*)(p.state + ((size_t)slot * p.H + h) * hs + e);
+  float4 prev = p.positions[r0] != 0 ? *st : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int s0 = 0; s0 < nseg; s0 += 8) {
+    float4 own[8];
+    float dec[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const size_t at = (sb + min(s0 + u, nseg - 1)) * p.H + h;
+      own[u] = *(const float4*)(p.seg + at * hs + e);
+      dec[u] = p.seg_decay[at];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (s0 + u >= nseg) break;
+      *(float4*)(p.seg + ((sb + s0 + u) * p.H + h) * hs + e) = prev;
+      prev.x = fmaf(dec[u], prev.x, own[u].x);
+      prev.y = fmaf(dec[u], prev.y, own[u].y);
+      prev.z = fmaf(dec[u], prev.z, own[u].z);
+      prev.w = fmaf(dec[u], prev.w, own[u].w);
+    }
+  }
+  *st = prev;
+}
+
+template <int MODE, int NT, int V, int HW, typename TY>
+void run(const ChunkScanParams& p, hipStream_t s) {
+  const int chunks = p.T / kL + p.B;
+  chunk_frag_kernel<MODE, NT, TY><<<dim3(chunks, p.KH), 256, 0, s>>>(p);
+  if (MODE == 0)
+    chunk_scalar_kernel<TY><<<dim3(chunks, (p.H + 31) / 32), 256, 0, s>>>(p);
+  constexpr int nt = 2 * V * HW;
+  if (p.SEG == 0) {
+    chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<dim3(p.B, p.H / HW), nt, 0, s>>>(p);
+    return;
+  }
+  const int segs = p.T / p.SEG + p.B;
+  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<dim3(segs, p.H / HW), nt, 0, s>>>(p);
+  chunk_join_kernel<<<dim3(p.B, p.H, (p.V * p.N + 1023) / 1024), 256, 0, s>>>(p);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<dim3(segs, p.H / HW), nt, 0, s>>>(p);
+}
+
+// two heads of 64 columns that share their keys go through one workgroup: the keys' fragments
+// are staged once for both
+template <int MODE, int NT, typename TY>
+void pick_v(const ChunkScanParams& p, hipStream_t s) {
+  if (p.V == 128) run<MODE, NT, 128, 1, TY>(p, s);
+  else if (MODE == 0 && (p.H / p.KH) % 2 == 0) run<MODE, NT, 64, MODE == 0 ? 2 : 1, TY>(p, s);
+  else run<MODE, NT, 64, 1, TY>(p, s);
+}
+
+template <int MODE, typename TY>
+void pick(const ChunkScanParams& p, hipStream_t s) {
+  if (p.N == 128) pick_v<MODE, 4, TY>(p, s);
+  else pick_v<MODE, 2, TY>(p, s);
+}
+
+}  // namespace
+
+bool chunk_scan_sizes(int V, int N) {
+  return (V == 64 || V == 128) && (N == 64 || N == 128);
+}
+
+int chunk_scan_segment(int T, int B, int H, int V) {
+  // A step with fewer (sequence, head, 32 columns) triples than most SIMDs of the chip is cut into
+  // segments, if a sequence of it may be longer than one (only the rows of all are known here):
+  // the second pass over the keys costs less than idle SIMDs.  8 x 2048 rows, 8 heads x 128 x 128
+  // (256 waves otherwise): 285 us in segments; 64 heads x 128 x 64 (1024 waves): 475 us whole.
+  if ((int64_t)B * H * (V / 32) >= 768) return 0;
+  return T >= 1024 || T >= 384 * (int64_t)B ? 256 : 0;
+}
+
+void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s) {
+  if (p.T <= 0 || p.B <= 0) return;
+  if (p.mode == 0) {
+    if (f32) pick<0, float>(p, s); else pick<0, bf16>(p, s);
+  } else {
+    if (f32) pick<1, float>(p, s); else pick<1, bf16>(p, s);
+  }
+}
+
+}  // namespace akap_stream

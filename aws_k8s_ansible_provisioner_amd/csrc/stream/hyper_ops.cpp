@@ -192,8 +192,43 @@ void selective_scan(Tensor y, Tensor xbc, Tensor proj, int64_t dt_off, Tensor dt
               "selective_scan: state [slots, H, N, V]");
   const SeqArgs sa = seq_args(T, seq_slot, positions, q_start);
   const c10::DeviceGuard g(xbc.device());
+  const bool f32 = is_f32(proj, "proj");
+  // Prompt chunks in matrix form.  A chunk costs the same for one row as for 32, so steps of short
+  // portions stay with the scan: with convolution and norm, 64 heads x 64 x 128, 4 portions of 8
+  // rows take 43 us in the scan and 47 here, of 16 rows 48 and 47, of 32 rows 58 and 46 (64
+  // portions: 87 / 101, 118 / 104, 189 / 119).
+  if (sa.q_start != nullptr && sa.B > 0 && T >= 16 * (int64_t)sa.B &&
+      akap_stream::chunk_scan_sizes((int)V, (int)N) && (uintptr_t)xbc.data_ptr() % 16 == 0 &&
+      (uintptr_t)y.data_ptr() % 16 == 0) {
+    akap_stream::ChunkScanParams p{};
+    p.mode = 0;
+    p.q_start = sa.q_start; p.seq_slot = sa.slot; p.positions = sa.pos;
+    p.T = sa.T; p.B = sa.B; p.H = (int)H; p.KH = (int)G; p.V = (int)V; p.N = (int)N;
+    p.num_slots = (int)state.size(0);
+    p.state = state.data_ptr<float>();
+    const int64_t chunks = p.T / 32 + p.B;
+    p.frag_floats = 64 * p.N + 1024;
+    const auto opt = xbc.options();
+    const Tensor frag = at::empty({chunks * p.KH * p.frag_floats}, opt);
+    const Tensor scal = at::empty({chunks * p.H * 256}, opt);
+    p.frag = frag.data_ptr<float>(); p.scal = scal.data_ptr<float>();
+    p.SEG = akap_stream::chunk_scan_segment(p.T, p.B, p.H, p.V);
+    Tensor seg, dec;
+    if (p.SEG > 0) {
+      const int64_t segs = p.T / p.SEG + p.B;
+      seg = at::empty({segs * p.H * p.N * p.V}, opt);
+      dec = at::empty({segs * p.H}, opt);
+      p.seg = seg.data_ptr<float>(); p.seg_decay = dec.data_ptr<float>();
+    }
+    p.proj = proj.data_ptr(); p.proj_stride = (int)proj.stride(0); p.dt_off = (int)dt_off;
+    p.y = y.data_ptr<float>(); p.xbc = xbc.data_ptr<float>(); p.x_stride = (int)xbc.size(1);
+    p.dt_bias = f32_vec(dt_bias, H, "dt_bias"); p.a_log = f32_vec(a_log, H, "a_log");
+    p.d_skip = f32_vec(d_skip, H, "d_skip");
+    akap_stream::launch_chunk_scan(p, f32, cur_stream());
+    return;
+  }
   akap_stream::launch_selective_scan(y.data_ptr<float>(), xbc.data_ptr<float>(), proj.data_ptr(),
-                                     (int)proj.stride(0), (int)dt_off, is_f32(proj, "proj"),
+                                     (int)proj.stride(0), (int)dt_off, f32,
                                      f32_vec(dt_bias, H, "dt_bias"), f32_vec(a_log, H, "a_log"),
                                      f32_vec(d_skip, H, "d_skip"), state.data_ptr<float>(), sa.slot,
                                      sa.pos, sa.q_start, sa.T, sa.B, (int)H, (int)V, (int)N, (int)G,

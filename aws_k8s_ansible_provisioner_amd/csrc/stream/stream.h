@@ -219,6 +219,45 @@ struct RetentionParams {
 int retention_dreg(int D, int V);
 void launch_retention(RetentionParams p, bool f32, hipStream_t s);
 
+// ---- prompt chunks of the selective scan and the retention in fp32 matrix form (chunk_scan.hip) ----
+struct ChunkScanParams {
+  int mode;                   // 0: selective scan, 1: retention
+  const int32_t* q_start;     // [B + 1]
+  const int32_t* seq_slot;    // [T]
+  const int64_t* positions;   // [T]
+  int T, B, H, KH, V, N;      // KH: key heads (groups of the scan, heads of the retention)
+  int num_slots;
+  float* state;               // scan [slots, H, N, V], retention [slots, H, V, N]
+  // workspaces for T / 32 + B chunks: fragments [chunks, KH, frag_floats = 64 N + 1024], and for
+  // the scan scalars [chunks, H, 256]
+  float* frag;
+  int frag_floats;
+  float* scal;
+  // segments of SEG rows (0: none), T / SEG + B of them: states [segs, H, N V], decays [segs, H]
+  float* seg;
+  float* seg_decay;
+  int SEG;
+  const void* proj;           // scan: step sizes at column dt_off; retention: q, k, v and gate
+  int proj_stride;
+  // selective scan
+  float* y;                   // [T, H V]
+  const float* xbc;           // rows of x_stride floats: [x | B | C]
+  int x_stride, dt_off;
+  const float* dt_bias;
+  const float* a_log;
+  const float* d_skip;
+  // retention
+  void* out;
+  int out_stride, q_off, k_off, v_off, g_off, rot_dims;
+  const float* cos_sin;
+  const float* log2_decay;
+  float eps;
+};
+bool chunk_scan_sizes(int V, int N);
+// rows per segment of a step, 0: the sequences are walked whole
+int chunk_scan_segment(int T, int B, int H, int V);
+void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s);
+
 struct TalkParams {
   void* out;            // rows of out_stride elements; head h at columns [h Dv, (h + 1) Dv)
   int out_stride;

@@ -1,0 +1,153 @@
+"""Prompt chunks of the selective scan and the retention in fp32 matrix form (GPU) against the same
+ops on CPU tensors: sequences around the chunk size of 32 rows and the segment size of 256, several
+sequences per step (some continued from their slots, one a padding sequence), every head size of
+the matrix form, projections that are column slices of wider rows, and values that are not finite.
+
+Tolerance: both sides sum at most N + 32 products per entry in fp32 in different orders; the
+relative 2-norm error of such sums is a few times 2^-24, 2e-6 leaves a factor of ten."""
+import math
+
+import pytest
+import torch
+
+from aws_k8s_ansible_provisioner_amd.ops import stream as sops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rel(a, b):
+    return float((a.double().cpu() - b.double()).norm() / b.double().norm().clamp_min(1e-30))
+
+
+def _step(lens, starts, seed=0):
+    q_start = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    pos = torch.cat([torch.arange(s, s + n) for n, s in zip(lens, starts)]).to(torch.int64)
+    slot = torch.cat([torch.full((n,), b if s >= 0 else -1, dtype=torch.int32)
+                      for b, (n, s) in enumerate(zip(lens, starts))])
+    return q_start, pos.clamp_min(0), slot
+
+
+# (rows per sequence, first position; -1: a padding sequence without a slot)
+STEPS = [([5], [0]), ([32], [7]), ([33, 31, 64], [0, 3, 0]), ([1, 65, 40, 90], [9, 0, -1, 11]),
+         ([300, 257, 256, 40], [0, 5, 0, 2]), ([1100], [0])]
+
+
+def _scan_inputs(T, B, H, V, N, G, dt, wide, seed):
+    g = torch.Generator().manual_seed(seed)
+    C = H * V + 2 * G * N
+    xbc = torch.randn(T, C, generator=g)
+    proj = torch.randn(T, H + wide, generator=g).to(dt)[:, wide // 2:]
+    state = torch.randn(B, H, N, V, generator=g)
+    return (xbc, proj, torch.randn(H, generator=g) * 0.5 - 1.0, torch.randn(H, generator=g) * 0.5,
+            torch.randn(H, generator=g) * 0.2 + 1.0, state)
+
+
+def _run_scan(inp, step, H, V, N, G, dev):
+    xbc, proj, bias, a_log, d_skip, state = inp
+    wide = proj.stride(0)
+    full = torch.zeros(proj.shape[0], wide, dtype=proj.dtype, device=dev)
+    off = wide - proj.shape[1] if wide > proj.shape[1] else 0
+    full[:, off:off + proj.shape[1]] = proj.to(dev)
+    q_start, pos, slot = (t.to(dev) for t in step)
+    st = state.clone().to(dev)
+    y = torch.zeros(xbc.shape[0], H * V, device=dev)
+    sops.selective_scan(y, xbc.to(dev), full[:, off:], 0, bias.to(dev), a_log.to(dev),
+                        d_skip.to(dev), st, slot, pos, q_start, H, V, N, G)
+    return y, st
+
+
+@pytest.mark.parametrize("H,V,N,G,dt", [(4, 64, 128, 1, torch.bfloat16), (6, 64, 64, 2, torch.float32),
+                                        (2, 128, 128, 2, torch.bfloat16),
+                                        (3, 128, 64, 1, torch.float32), (3, 64, 128, 1, torch.float32)])
+@pytest.mark.parametrize("lens,starts", STEPS)
+def test_selective_scan_chunks(lens, starts, H, V, N, G, dt):
+    step = _step(lens, starts)
+    inp = _scan_inputs(sum(lens), len(lens), H, V, N, G, dt, 6, seed=sum(lens) + V)
+    want = _run_scan(inp, step, H, V, N, G, "cpu")
+    got = _run_scan(inp, step, H, V, N, G, DEV)
+    live = (step[2] >= 0)
+    assert _rel(got[0][live.to(DEV)], want[0][live]) < 2e-6
+    assert _rel(got[1], want[1]) < 2e-6
+    assert torch.equal(got[1].cpu()[[b for b, s in enumerate(starts) if s < 0]],
+                       inp[5][[b for b, s in enumerate(starts) if s < 0]])
+
+
+def _run_retention(inp, step, H, D, V, offs, cs, l2, dev):
+    proj, state = inp
+    q_start, pos, slot = (t.to(dev) for t in step)
+    st = state.clone().to(dev)
+    buf = torch.zeros(proj.shape[0], H * V + 8, dtype=proj.dtype, device=dev)
+    sops.retention(buf[:, :H * V], proj.to(dev), *offs, st, slot, pos, q_start,
+                   None if cs is None else cs.to(dev), l2.to(dev), H, D, V, 1e-5)
+    return buf[:, :H * V], st
+
+
+@pytest.mark.parametrize("H,D,V,rot,dt", [(2, 128, 128, 64, torch.float32), (3, 64, 128, 0, torch.float32),
+                                          (2, 128, 64, 128, torch.bfloat16),
+                                          (4, 64, 64, 16, torch.bfloat16)])
+@pytest.mark.parametrize("lens,starts", STEPS)
+def test_retention_chunks(lens, starts, H, D, V, rot, dt):
+    step = _step(lens, starts)
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(T + D)
+    # gate first, then q, k, v behind a few unused columns
+    offs = (H * V + 8, H * V + 8 + H * D, H * V + 8 + 2 * H * D, 0)
+    proj = torch.randn(T, 2 * H * V + 2 * H * D + 12, generator=g).to(dt)
+    state = torch.randn(B, H, V, D, generator=g)
+    l2 = torch.log2(torch.tensor([1.0, 0.97, 0.5, 0.999][:H]))
+    ang = torch.arange(2048)[:, None] * (0.5 ** torch.arange(max(1, rot // 2)))[None, :]
+    cs = torch.cat([torch.cos(ang), torch.sin(ang)], 1) if rot else None
+    args = (step, H, D, V, (offs[0], offs[1], offs[2], offs[3]), cs, l2)
+    want = _run_retention((proj, state), *args, "cpu")
+    got = _run_retention((proj, state), *args, DEV)
+    live = (step[2] >= 0)
+    # bf16 outputs: one rounding to 8 bits (2^-9 relative) on either side
+    assert _rel(got[0][live.to(DEV)].float(), want[0][live].float()) < (6e-3 if dt == torch.bfloat16
+                                                                        else 4e-6)
+    assert _rel(got[1], want[1]) < 2e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_chunks_values_not_finite(bad):
+    """A value that is not finite reaches the rows from its own on and no row before it, in its
+    column of its head alone."""
+    H, V, N, G = 2, 64, 64, 1
+    lens, starts = [70, 40], [0, 0]
+    step = _step(lens, starts)
+    inp = _scan_inputs(110, 2, H, V, N, G, torch.float32, 0, seed=3)
+    inp[0][45, 10] = bad
+    want = _run_scan(inp, step, H, V, N, G, "cpu")[0]
+    got = _run_scan(inp, step, H, V, N, G, DEV)[0].cpu()
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    ok = torch.isfinite(want)
+    assert _rel(got[ok], want[ok]) < 2e-6
+    proj = torch.randn(110, 4 * H * V, generator=torch.Generator().manual_seed(4))
+    proj[45, 2 * H * V + 10] = bad
+    args = (step, H, V, V, (0, H * V, 2 * H * V, 3 * H * V), None, torch.log2(torch.tensor([0.9, 0.5])))
+    st = torch.zeros(2, H, V, V)
+    want = _run_retention((proj, st), *args, "cpu")[0]
+    got = _run_retention((proj, st), *args, DEV)[0].cpu()
+    # (the head's norm spreads it over the head's row, as zeros or as NaN: which of the two hangs on
+    # whether the product of the row with itself is formed before or after the state's)
+    ok = torch.ones(110, H * V, dtype=torch.bool)
+    ok[45:70, :V] = False
+    assert bool(torch.isfinite(got[ok]).all()) and not bool(torch.isfinite(got[45:70, 10]).any())
+    assert _rel(got[ok], want[ok]) < 4e-6
+
+
+def test_scan_decays_to_zero():
+    """Step sizes that take a decay to zero inside a chunk (its logarithm far below fp32's range)."""
+    H, V, N, G = 2, 64, 64, 1
+    step = _step([96], [4])
+    inp = list(_scan_inputs(96, 1, H, V, N, G, torch.float32, 0, seed=8))
+    inp[1] = inp[1].clone()
+    inp[1][40] = 3000.0
+    inp[1][41] = 3.0e4
+    inp[3] = torch.tensor([3.0, math.log(1e5)])
+    want = _run_scan(tuple(inp), step, H, V, N, G, "cpu")
+    got = _run_scan(tuple(inp), step, H, V, N, G, DEV)
+    # (outputs grow by the step sizes: compared row by row, the largest relative to its row)
+    d = (got[0].cpu() - want[0]).norm(dim=1) / want[0].norm(dim=1)
+    assert float(d.max()) < 5e-6
+    assert _rel(got[1], want[1]) < 5e-6
