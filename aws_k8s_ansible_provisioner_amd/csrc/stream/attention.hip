@@ -23,7 +23,6 @@
 //   from accumulator to B operand without any lane movement, and the V^T operand is one
 //   16-byte load from the grouped V cache.  K / V fragments come straight from global memory
 //   (L1 / L2 hits across the workgroup's four waves and the heads of a GQA group).
-#include <cstdlib>
 
 #include "../kernels/common.h"
 #include "stream.h"
@@ -619,29 +618,30 @@ static bool mfma_ok(const AttnParams& p, bool f32) {
 
 void launch_sink_attention_prefill(const AttnParams& p, bool f32, hipStream_t s) {
   if (p.num_tiles <= 0) return;
+  if (!f32 && flash_prefill_sizes(p.H, p.G, p.D, p.D, p.BS, p.tile_rows, p.scale)) {
+    FlashParams f{};
+    f.out = p.out; f.out_stride = p.out_stride;
+    f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
+    f.block_tables = p.block_tables; f.max_blocks = p.max_blocks;
+    f.q_start = p.q_start; f.seq_lens = p.seq_lens;
+    f.tile_seq = p.tile_seq; f.tile_row = p.tile_row;
+    f.num_tiles = p.num_tiles; f.tile_rows = p.tile_rows;
+    f.gate = p.gate; f.gate_stride = p.gate_stride; f.sink = p.sink;
+    f.scale = p.scale; f.chunk = p.chunk; f.window = p.window;
+    f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS;
+    launch_flash_prefill(f, s);
+    return;
+  }
   const dim3 grid((unsigned)p.num_tiles * p.H);
   if (mfma_ok(p, f32) && (p.tile_rows == 128 || p.tile_rows == 256)) {
     // (tile, K/V head) units padded to a multiple of the 8 XCDs, rep workgroups each
     const dim3 grid((unsigned)((p.num_tiles * p.G + 7) / 8 * 8) * (p.H / p.G));
     const int tr = p.tile_rows;
-    static const int nq = [] {  // AKAP_STREAM_NQ=1|2: column tiles per wave (A/B knob)
-      const char* e = getenv("AKAP_STREAM_NQ");
-      return e ? atoi(e) : 2;
-    }();
-    if (nq == 1 || p.D == 256) {
-      switch (p.D) {
-        case 32: sink_attn_prefill_mfma_kernel<1, 1><<<grid, 2 * tr, 0, s>>>(p); break;
-        case 64: sink_attn_prefill_mfma_kernel<2, 1><<<grid, 2 * tr, 0, s>>>(p); break;
-        case 128: sink_attn_prefill_mfma_kernel<4, 1><<<grid, 2 * tr, 0, s>>>(p); break;
-        default: sink_attn_prefill_mfma_kernel<8, 1><<<grid, 2 * tr, 0, s>>>(p); break;
-      }
-    } else {
-      switch (p.D) {
-        case 32: sink_attn_prefill_mfma_kernel<1, 2><<<grid, tr, 0, s>>>(p); break;
-        case 64: sink_attn_prefill_mfma_kernel<2, 2><<<grid, tr, 0, s>>>(p); break;
-        default: sink_attn_prefill_mfma_kernel<4, 2><<<grid, tr, 0, s>>>(p); break;
-      }
-    }
+    // (sizes 64 and 128 went to the LDS-staged kernel above)
+    if (p.D == 32)
+      sink_attn_prefill_mfma_kernel<1, 2><<<grid, tr, 0, s>>>(p);
+    else
+      sink_attn_prefill_mfma_kernel<8, 1><<<grid, 2 * tr, 0, s>>>(p);
     return;
   }
   const size_t sm = 4 * (p.D + 64) * sizeof(float);

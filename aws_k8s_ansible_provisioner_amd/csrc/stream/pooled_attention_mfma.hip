@@ -307,6 +307,22 @@ bool pooled_mfma_supported(int H, int G, int D, int Dv, int BS) {
 void launch_pooled_window_prefill_mfma(const PoolAttnParams& p, const int32_t* tile_seq,
                                        const int32_t* tile_row, int num_tiles, hipStream_t s) {
   if (num_tiles <= 0) return;
+  if (flash_prefill_sizes(p.H, p.G, p.D, p.Dv, p.BS, 128, p.scale)) {
+    FlashParams f{};
+    f.out = p.out; f.out_stride = p.out_stride;
+    f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
+    f.block_tables = p.block_tables; f.max_blocks = p.max_blocks;
+    f.q_start = p.q_start; f.positions = p.positions;
+    f.tile_seq = tile_seq; f.tile_row = tile_row;
+    f.num_tiles = num_tiles; f.tile_rows = 128;
+    f.unit_sink = p.unit_sink; f.scale = p.scale; f.window = p.window;
+    f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS;
+    if (p.pool > 0 && p.window > 0 && p.k_pool) {
+      f.k_pool = p.k_pool; f.v_pool = p.v_pool; f.pool = p.pool; f.PS = p.PS;
+    }
+    launch_flash_prefill(f, s);
+    return;
+  }
   const dim3 grid(num_tiles, p.H);
   const size_t lds = (size_t)4 * (p.D >> 4) * 64 * sizeof(bf16x8);
 #define AKAP_PWM(N) \

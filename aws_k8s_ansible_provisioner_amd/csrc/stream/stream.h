@@ -68,6 +68,37 @@ struct AttnParams {
 void launch_sink_attention_prefill(const AttnParams& p, bool f32, hipStream_t s);
 void launch_sink_attention_decode(const AttnParams& p, bool f32, hipStream_t s);
 
+// ---- attention of prompt chunks through LDS (flash_prefill.hip) -----------------------------------
+// bf16, key and value size 64 or 128, pages of whole 32-token pieces, tiles of whole 128 tokens
+struct FlashParams {
+  void* out;                    // rows of out_stride elements; head h at columns [h D, (h + 1) D)
+  int out_stride;
+  const void* q;                // [T, H, D]
+  const void* k_cache;          // [NB, G, BS, D]
+  const void* v_cache;          // [NB, G, BS / 8, D, 8]
+  const int32_t* block_tables;  // [B, max_blocks]
+  int max_blocks;
+  const int32_t* q_start;
+  const int32_t* seq_lens;      // a chunk's tokens are the last of seq_lens[b] positions, or
+  const int64_t* positions;     // (given) start at the position of its first row
+  const int32_t* tile_seq;
+  const int32_t* tile_row;
+  int num_tiles, tile_rows;
+  const void* gate;             // [T, H] logits with row stride gate_stride, or null
+  int gate_stride;
+  const float* sink;            // [H] or null
+  int unit_sink;                // a sink of score 0
+  float scale;
+  int chunk, window;            // 0: off
+  int H, G, D, BS;
+  // pooled entries of `pool` tokens before the window (0: none), fp32 [NB, G, PS, D]
+  const float* k_pool;
+  const float* v_pool;
+  int pool, PS;
+};
+bool flash_prefill_sizes(int H, int G, int D, int Dv, int BS, int tile_rows, float scale);
+void launch_flash_prefill(const FlashParams& p, hipStream_t s);
+
 // ---- grouped norms, token shift, latent attention, routed experts (latent.hip) ----------------
 // x (fp32 rows of d) += y + bias + y2 (each may be null; y / bias of the activation type, y2
 // fp32), then out1 = gnorm(x) * w1 and out2 = gnorm(x) * w2 (out2 / w2 may be null), the norm

@@ -1,0 +1,99 @@
+"""Attention of prompt chunks with keys and values staged through LDS (GPU) against the same ops on
+CPU tensors: both head sizes, every split of the query heads over the waves (1, 2, 3, 4, 8 heads to a
+key/value head), chunks that end inside 32-token pieces and 128-token tiles, cached tokens before them,
+chunk and window edges, sinks, gates, pooled entries past one step of 64, rows that are not 16-byte
+aligned, and pages of 32 and 64 tokens.
+
+Tolerance: weights and outputs are rounded to bf16 (relative 2^-9 each, on either side for the
+outputs): the 2-norm of the difference stays under 3 * 2^-9 of the result's."""
+import pytest
+import torch
+
+from aws_k8s_ansible_provisioner_amd.ops import stream as sops
+
+pytestmark = pytest.mark.gpu
+DEV, TOL = "cuda", 3 * 2.0 ** -9
+
+
+def _step(shape, G, D, BS, rows, seed):
+    """(cached, new) per sequence -> staged arrays and random caches (CPU)."""
+    g = torch.Generator().manual_seed(seed)
+    pages = [-(-(p + n) // BS) for p, n in shape]
+    perm = torch.randperm(sum(pages) + 2, generator=g)
+    bt = torch.zeros(len(shape), max(pages) + 1, dtype=torch.int32)
+    at, tiles, start, pos = 0, [], [0], []
+    for b, (p, n) in enumerate(shape):
+        bt[b, :pages[b]] = perm[at:at + pages[b]].to(torch.int32)
+        at += pages[b]
+        start.append(start[-1] + n)
+        pos.append(torch.arange(p, p + n))
+        tiles += [(p + min(n, r + rows), b, r) for r in range(0, n, rows)]
+    tiles.sort(key=lambda t: t[0])
+    pos = torch.cat(pos)
+    seq = torch.repeat_interleave(torch.arange(len(shape)), torch.tensor([n for _, n in shape]))
+    slots = bt[seq, pos // BS].long() * BS + pos % BS
+    NB = len(perm)
+    return dict(bt=bt, q_start=torch.tensor(start, dtype=torch.int32), pos=pos, slots=slots,
+                lens=torch.tensor([p + n for p, n in shape], dtype=torch.int32),
+                ts=torch.tensor([t[1] for t in tiles], dtype=torch.int32),
+                tr=torch.tensor([t[2] for t in tiles], dtype=torch.int32), rows=rows,
+                k=torch.randn(NB, G, BS, D, generator=g).bfloat16(),
+                v=torch.randn(NB, G, BS // 8, D, 8, generator=g).bfloat16(), gen=g)
+
+
+def _close(got, want):
+    got, want = got.cpu().double(), want.double()
+    assert float((got - want).norm() / want.norm()) < TOL
+    assert float((got - want).abs().max()) < 16 * 2.0 ** -9 * float(want.abs().max())
+
+
+SHAPES = [[(0, 1), (0, 33), (70, 64)], [(0, 300), (5, 129), (190, 31)], [(130, 257), (0, 128)]]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("H,G,D,BS,rows", [(4, 4, 128, 32, 128), (4, 2, 64, 64, 128), (6, 2, 128, 32, 128),
+                                           (8, 2, 128, 64, 256), (8, 1, 64, 32, 128),
+                                           (3, 1, 64, 32, 256)])
+@pytest.mark.parametrize("chunk,window", [(0, 0), (64, 0), (0, 45), (100, 70)])
+def test_sink_prefill_staged(shape, H, G, D, BS, rows, chunk, window):
+    s = _step(shape, G, D, BS, rows, seed=H * D + chunk)
+    T = int(s["q_start"][-1])
+    q = torch.randn(T, H, D, generator=s["gen"]).bfloat16()
+    odd = window > 0                      # rows that start at odd elements / 16-byte pieces
+    proj = torch.randn(T, H + 3, generator=s["gen"]).bfloat16()
+    gate = proj[:, 2:2 + H] if chunk else None
+    sink = torch.randn(H, generator=s["gen"]) * 3 if chunk or window else None
+    args = (s["bt"], s["lens"], s["q_start"], s["ts"], s["tr"])
+    outs = []
+    for dev in ("cpu", DEV):
+        wide = torch.zeros(T, H * D + (5 if odd else 8), dtype=torch.bfloat16, device=dev)
+        out = wide[:, 1 if odd else 0:][:, :H * D]
+        sops.sink_attention_prefill(out, q.to(dev), s["k"].to(dev), s["v"].to(dev),
+                                    *(a.to(dev) for a in args), rows,
+                                    proj.to(dev)[:, 2:2 + H] if gate is not None else None,
+                                    sink.to(dev) if sink is not None else None, D ** -0.5, chunk,
+                                    window)
+        outs.append(out)
+    _close(outs[1], outs[0])
+
+
+@pytest.mark.parametrize("H,G,D,window,pool", [(4, 2, 128, 40, 4), (8, 2, 64, 70, 1), (3, 1, 64, 64, 16),
+                                               (2, 2, 128, 33, 40)])
+@pytest.mark.parametrize("shape", [[(0, 150), (260, 70)], [(500, 33), (0, 40), (37, 129)]])
+def test_pooled_prefill_staged(shape, H, G, D, window, pool):
+    BS = 32
+    s = _step(shape, G, D, BS, 128, seed=H + D + window)
+    T = int(s["q_start"][-1])
+    q = torch.randn(T, H, D, generator=s["gen"]).bfloat16()
+    n = sops.pool_slots(BS, pool)
+    NB = s["k"].shape[0]
+    kp, vp = (torch.randn(NB, G, n, D, generator=s["gen"]) for _ in range(2))
+    outs = []
+    for dev in ("cpu", DEV):
+        out = torch.zeros(T, H * D, dtype=torch.bfloat16, device=dev)
+        sops.pooled_window_attention_prefill(
+            out, q.to(dev), s["k"].to(dev), s["v"].to(dev), kp.to(dev), vp.to(dev), s["bt"].to(dev),
+            s["q_start"].to(dev), s["pos"].to(dev), s["slots"].to(dev), s["ts"].to(dev),
+            s["tr"].to(dev), 128, D ** -0.5, window, pool, True)
+        outs.append(out)
+    _close(outs[1], outs[0])
