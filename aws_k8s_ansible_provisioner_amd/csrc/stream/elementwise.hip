@@ -5,6 +5,7 @@
 // the residual sum are fp32 whatever the storage type.
 #include "../kernels/common.h"
 #include "stream.h"
+#include "value_groups.h"
 
 namespace akap_stream {
 
@@ -362,9 +363,20 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_kernel(ProjParams p)
 // The same with 8 elements (four rotation pairs) per thread and access, the token's q (up to
 // 2048 NQ elements) and k (up to 2048) held in registers between the two passes.  Needs D, the
 // slice offsets and the row stride to be multiples of 8 elements and 16-byte aligned pointers.
+// Workgroups past the rows' write the values (write_values; vrows 0: none do, a row's own workgroup
+// writes its values), as large steps do.  Bound by memory and by a chain of latencies per workgroup
+// (row, sums, weights and angles, store): at 16384 rows of 16 / 4 heads of 128 79 us with values
+// element by element and a barrier pair per sum, 91 with the values taken out alone, 69.5 with both
+// sums behind one barrier and weights, angles and slot requested ahead of it.
 template <typename T, int NQ>
-__global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParams p) {
-  __shared__ float scratch[16];
+__global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParams p, int vrows) {
+  __shared__ float scratch[32];
+  if ((int)blockIdx.x >= p.T) {
+    write_values<T>({(const T*)p.proj + p.k_off, p.proj_stride, (T*)p.v_cache, p.slots, p.num_slots,
+                     p.T, p.G, p.D, p.BS, vrows, 0.f, false, nullptr, (const T*)p.k_b},
+                    (int64_t)(blockIdx.x - p.T) * 256 + threadIdx.x);
+    return;
+  }
   const int t = blockIdx.x;
   const T* row = (const T*)p.proj + (size_t)t * p.proj_stride;
   const T* qr = row + p.q_off;
@@ -399,26 +411,51 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParam
 #pragma unroll
     for (int e = 0; e < 8; ++e) sk += k[e] * k[e];
   }
-  sq = block_sum(sq, scratch);
-  sk = block_sum(sk, scratch);
-  const float iq = 1.0f / sqrtf(sq / (float)HD + p.eps);
-  const float ik = 1.0f / sqrtf(sk / (float)GD + p.eps);
   int64_t pos = p.positions[t];
   if (pos < 0) pos = 0;
   if (pos >= p.max_pos) pos = p.max_pos - 1;
+  // weights and angles requested ahead of the sums
   const float* cs = p.cos_sin ? p.cos_sin + (size_t)pos * p.rot_dims : nullptr;
   const int rh = p.rot_dims >> 1;
-  // norm weight, then rotation of the pairs (2i, 2i+1) with i < rot_dims / 2
-  auto finish = [&](float (&v)[8], const float* w, float inv, int c) {
-    float ww[8];
+  const bool tab = cs != nullptr && (rh & 3) == 0 && ((uintptr_t)p.cos_sin & 15) == 0;
+  float wq[NQ][8], wk[8], cq[NQ][4], zq[NQ][4], ck4[4], zk4[4];
+  auto ahead = [&](const float* w, int c, float (&ww)[8], float (&co)[4], float (&si)[4]) {
     ldv(ww, w + c);
+    const int i0 = (c % p.D) >> 1;
+    if (tab && i0 < rh) {
+      ldv(co, cs + i0);
+      ldv(si, cs + rh + i0);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int c = (i * 256 + threadIdx.x) * 8;
+    if (c < HD) ahead(p.q_w, c, wq[i], cq[i], zq[i]);
+  }
+  if (ck < GD) ahead(p.k_w, ck, wk, ck4, zk4);
+  const int64_t slot = p.slots[t];
+  // both sums meet behind one barrier
+  sq = akap::wave_sum_dpp(sq);
+  sk = akap::wave_sum_dpp(sk);
+  if ((threadIdx.x & 63) == 0) {
+    scratch[threadIdx.x >> 6] = sq;
+    scratch[4 + (threadIdx.x >> 6)] = sk;
+  }
+  __syncthreads();
+  sq = (scratch[0] + scratch[1]) + (scratch[2] + scratch[3]);
+  sk = (scratch[4] + scratch[5]) + (scratch[6] + scratch[7]);
+  const float iq = 1.0f / sqrtf(sq / (float)HD + p.eps);
+  const float ik = 1.0f / sqrtf(sk / (float)GD + p.eps);
+  // norm weight, then rotation of the pairs (2i, 2i+1) with i < rot_dims / 2
+  auto finish = [&](float (&v)[8], const float (&ww)[8], float inv, int c, const float (&co4)[4],
+                    const float (&si4)[4]) {
     const int i0 = (c % p.D) >> 1;
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
       float u = v[e] * inv * ww[e], z = v[e + 1] * inv * ww[e + 1];
       const int i = i0 + (e >> 1);
       if (cs && i < rh) {
-        const float co = cs[i], si = cs[rh + i];
+        const float co = tab ? co4[e >> 1] : cs[i], si = tab ? si4[e >> 1] : cs[rh + i];
         const float ru = u * co - z * si;
         z = z * co + u * si;
         u = ru;
@@ -432,25 +469,24 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParam
   for (int i = 0; i < NQ; ++i) {
     const int c = (i * 256 + threadIdx.x) * 8;
     if (c < HD) {
-      finish(q[i], p.q_w, iq, c);
+      finish(q[i], wq[i], iq, c, cq[i], zq[i]);
       stv(qo + c, q[i]);
     }
   }
-  const int64_t slot = p.slots[t];
   if (slot < 0 || slot >= p.num_slots) return;
   const int64_t blk = slot / p.BS;
   const int off = (int)(slot % p.BS);
   // raw k -> V cache [NB, G, BS/8, D, 8]: the token's element of every (dimension) group.
   // Adjacent lanes take adjacent dimensions (16 bytes apart), so a wave's store covers whole
   // cache lines; the row is re-read from the projection (an L1 / L2 hit).
-  for (int c = threadIdx.x; c < GD; c += 256) {
+  for (int c = vrows ? GD : threadIdx.x; c < GD; c += 256) {
     const int g = c / p.D, d = c - g * p.D;
     ((T*)p.v_cache)[((((size_t)blk * p.G + g) * (p.BS >> 3) + (off >> 3)) * p.D + d) * 8 +
                     (off & 7)] = (T)(ldf(kr + c) + (p.k_b ? ldf((const T*)p.k_b + c) : 0.f));
   }
   if (ck >= GD) return;
   const int g = ck / p.D, d0 = ck % p.D;
-  finish(k, p.k_w, ik, ck);
+  finish(k, wk, ik, ck, ck4, zk4);
   stv((T*)p.k_cache + (((size_t)blk * p.G + g) * p.BS + off) * p.D + d0, k);
 }
 
@@ -467,10 +503,13 @@ void launch_proj_norm_rope_cache(const ProjParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
   if (f32 ? proj_vec_ok<float>(p) : proj_vec_ok<bf16>(p)) {
     const bool two = p.H * p.D > 2048;
-    if (f32 && two) proj_norm_rope_cache_vec_kernel<float, 2><<<p.T, 256, 0, s>>>(p);
-    else if (f32) proj_norm_rope_cache_vec_kernel<float, 1><<<p.T, 256, 0, s>>>(p);
-    else if (two) proj_norm_rope_cache_vec_kernel<bf16, 2><<<p.T, 256, 0, s>>>(p);
-    else proj_norm_rope_cache_vec_kernel<bf16, 1><<<p.T, 256, 0, s>>>(p);
+    const int vrows = p.T >= 512 && p.BS % 8 == 0 && aligned(p.v_cache, 16) ? 8 : 0;
+    const int64_t vt = vrows ? value_group_threads(p.T, p.G, p.D, vrows) : 0;
+    const int n = p.T + (int)((vt + 255) / 256);
+    if (f32 && two) proj_norm_rope_cache_vec_kernel<float, 2><<<n, 256, 0, s>>>(p, vrows);
+    else if (f32) proj_norm_rope_cache_vec_kernel<float, 1><<<n, 256, 0, s>>>(p, vrows);
+    else if (two) proj_norm_rope_cache_vec_kernel<bf16, 2><<<n, 256, 0, s>>>(p, vrows);
+    else proj_norm_rope_cache_vec_kernel<bf16, 1><<<n, 256, 0, s>>>(p, vrows);
     return;
   }
   if (f32)

@@ -156,6 +156,74 @@ __global__ __launch_bounds__(128) void pool_cache_blocks_kernel(const PoolParams
   }
 }
 
+// The same in 16-byte pieces (bf16; pool, D and Dv multiples of 8, D / 8 a power of two up to 256,
+// aligned caches): a workgroup takes 256 rows x one key/value head, lists the rows that end a block
+// and does them in turn; keys by (token, 8 dimensions), values by (dimension, 8-token group), all of
+// a thread's loads in flight, the partial sums meet in LDS.  Bound by the latency of one round of
+// loads: the row-by-row form chained `pool` of them (43 us at 12800 rows and blocks of 64).
+__global__ __launch_bounds__(256) void pool_cache_blocks_vec_kernel(const PoolParams p) {
+  __shared__ int ends[256];
+  __shared__ int count;
+  __shared__ float part[256 * 8];
+  const int g = blockIdx.y, tid = threadIdx.x, t0 = blockIdx.x * 256;
+  if (tid == 0) count = 0;
+  __syncthreads();
+  const int t = t0 + tid;
+  if (t < p.T && p.slots[t] >= 0 && ((int)p.positions[t] + 1) % p.pool == 0)
+    ends[atomicAdd(&count, 1)] = t;
+  __syncthreads();
+  const int n = count, lk = p.D >> 3, tk = 256 / lk;   // lanes of a key row, rows per turn
+  const float inv = 1.0f / (float)p.pool;
+  for (int u = 0; u < n; ++u) {
+    const int row = ends[u], pos = (int)p.positions[row], first = pos + 1 - p.pool;
+    const int b = p.q_start ? seq_of_row(p.q_start, p.B, row) : row;
+    const int32_t* bt = p.block_tables + (size_t)b * p.max_blocks;
+    const size_t out = ((size_t)bt[first / p.BS] * p.G + g) * p.PS + (first % p.BS) / p.pool;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int j = tid / lk; j < p.pool; j += tk) {
+      const int q = first + j;
+      const akap::bf16x8 k = *(const akap::bf16x8*)((const bf16*)p.k_cache +
+          (((size_t)bt[q / p.BS] * p.G + g) * p.BS + q % p.BS) * p.D + (tid % lk) * 8);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] += (float)k[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[tid * 8 + i] = acc[i];
+    __syncthreads();
+    for (int d = tid; d < p.D; d += 256) {
+      float s = 0.f;
+      for (int w = 0; w < tk; ++w) s += part[w * p.D + d];
+      p.k_pool[out * p.D + d] = s * inv;
+    }
+    // a dimension's groups lie Dv 16-byte entries apart; a thread takes every 2nd, 4th ... of them
+    const int ng = p.pool >> 3, split = p.Dv >= 256 ? 1 : 256 / p.Dv;
+    const int dv = tid % p.Dv, gp = tid / p.Dv;
+    for (int d0 = 0; d0 < p.Dv; d0 += 256) {
+      const int d = d0 + dv;
+      float s = 0.f;
+      if (d < p.Dv && gp < split) {
+#pragma unroll 4
+        for (int j = gp; j < ng; j += split) {
+          const int q = first + 8 * j;
+          const akap::bf16x8 v = *(const akap::bf16x8*)((const bf16*)p.v_cache +
+              ((((size_t)bt[q / p.BS] * p.G + g) * (p.BS >> 3) + (q % p.BS >> 3)) * p.Dv + d) * 8);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s += (float)v[i];
+        }
+      }
+      __syncthreads();
+      part[tid] = s;
+      __syncthreads();
+      if (gp == 0 && d < p.Dv) {
+        for (int w = 1; w < split; ++w) s += part[w * p.Dv + dv];
+        p.v_pool[out * p.Dv + d] = s * inv;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------------------ attention
 // One workgroup per (row, key/value head, up to 16 query heads of the group), one wave per query
 // head.  The visible
@@ -247,12 +315,30 @@ __global__ void pooled_window_attention_kernel(const PoolAttnParams p, const int
 
 void launch_bias_rope_cache(const RopeCacheParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
+  HeadNormParams h{};
+  h.proj = p.proj; h.proj_stride = p.proj_stride;
+  h.q_out = p.q_out; h.k_cache = p.k_cache; h.v_cache = p.v_cache;
+  h.slots = p.slots; h.positions = p.positions;
+  h.T = p.T; h.H = p.H; h.G = p.G; h.D = p.D; h.Dv = p.Dv; h.BS = p.BS;
+  h.q_off = p.q_off; h.k_off = p.k_off; h.v_off = p.v_off;
+  h.num_slots = p.num_slots;
+  h.cos_sin = p.cos_sin; h.max_pos = p.max_pos; h.rot_dims = p.cos_sin ? p.rot_dims : 0;
+  h.bias = p.bias;
+  if (launch_head_cache_vec(h, f32, s)) return;
   if (f32) bias_rope_cache_kernel<float><<<p.T, 256, 0, s>>>(p);
   else bias_rope_cache_kernel<bf16><<<p.T, 256, 0, s>>>(p);
 }
 
 void launch_pool_cache_blocks(const PoolParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
+  const int lk = p.D >> 3;
+  // (from 512 rows on: 256 rows to a workgroup; fewer rows, as in decode steps, a workgroup each)
+  if (!f32 && p.T >= 512 && ((p.pool | p.D | p.Dv | p.BS) & 7) == 0 && lk <= 256 &&
+      (lk & (lk - 1)) == 0 && p.Dv <= 256 && 256 % p.Dv == 0 &&
+      (((uintptr_t)p.k_cache | (uintptr_t)p.v_cache) & 15) == 0) {
+    pool_cache_blocks_vec_kernel<<<dim3((p.T + 255) / 256, p.G), 256, 0, s>>>(p);
+    return;
+  }
   const int RB = p.T >= 1024 ? kPoolRows : 1;
   const dim3 grid((p.T + RB - 1) / RB, p.G);
   if (f32) pool_cache_blocks_kernel<float><<<grid, 128, 0, s>>>(p, RB);

@@ -221,8 +221,11 @@ struct HeadNormParams {
   const float* cos_sin;       // [max_pos, rot_dims] = [cos | sin], rotate-half pairs, or null
   const int64_t* positions;   // [T] (with cos_sin)
   int max_pos, rot_dims;
+  const float* bias;          // [N] laid out like proj's columns, added first, or null
 };
 void launch_head_norm_cache(const HeadNormParams& p, bool f32, hipStream_t s);
+// the form in 16-byte pieces alone; false where sizes or alignment do not allow it
+bool launch_head_cache_vec(const HeadNormParams& p, bool f32, hipStream_t s);
 
 struct RetentionParams {
   void* out;            // rows of out_stride elements; head h at columns [h V, (h + 1) V)

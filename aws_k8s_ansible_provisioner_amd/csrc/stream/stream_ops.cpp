@@ -759,7 +759,7 @@ void head_norm_cache(Tensor proj, Tensor q_out, Tensor k_cache, Tensor v_cache, 
   p.q_off = q_off; p.k_off = k_off; p.v_off = v_off;
   p.num_slots = k_cache.size(0) * k_cache.size(2);
   p.eps = (float)eps; p.norm_qk = norm_qk; p.norm_v = norm_v;
-  p.q_w = p.k_w = p.cos_sin = nullptr;
+  p.q_w = p.k_w = p.cos_sin = p.bias = nullptr;
   p.positions = nullptr;
   p.max_pos = p.rot_dims = 0;
   for (const auto* w : {&q_w, &k_w})
