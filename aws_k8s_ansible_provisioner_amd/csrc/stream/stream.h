@@ -317,6 +317,9 @@ struct TalkParams {
 size_t talking_attention_lds(int H, int D);
 void launch_talking_attention(const TalkParams& p, bool f32, hipStream_t s);
 void launch_talking_merge(const TalkParams& p, bool f32, hipStream_t s);
+// prompt chunks with keys staged through LDS, heads mixed and gated as well; false: not these sizes
+bool launch_talk_staged(const TalkParams& p, const int32_t* tile_seq, const int32_t* tile_row,
+                        int num_tiles, int tile_rows, hipStream_t s);
 // matrix-core form for prompt chunks (bf16): fills the workspace of a one-partition split for
 // the rows of the tile map (tile_seq / tile_row: sequence and first chunk row of a tile of
 // tile_rows tokens, a multiple of 32); launch_talking_merge finishes

@@ -1004,6 +1004,9 @@ void talking_attention_prefill_mfma(Tensor out, Tensor q, Tensor k_cache, Tensor
   TORCH_CHECK(first_row >= 0 && first_row <= p.T, "talking_attention_prefill_mfma: first_row");
   p.row0 = first_row;
   const c10::DeviceGuard g(q.device());
+  if (akap_stream::launch_talk_staged(p, tile_seq.data_ptr<int32_t>(), tile_row.data_ptr<int32_t>(),
+                                      (int)tile_seq.numel(), (int)tile_rows, cur_stream()))
+    return;
   akap_stream::launch_talking_prefill_mfma(p, tile_seq.data_ptr<int32_t>(),
                                            tile_row.data_ptr<int32_t>(), (int)tile_seq.numel(),
                                            (int)tile_rows, cur_stream());

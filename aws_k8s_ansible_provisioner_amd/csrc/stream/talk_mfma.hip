@@ -1,4 +1,6 @@
-// Head-mixed attention of prompt chunks on the matrix cores (bf16 cache).
+// Head-mixed attention on the matrix cores (bf16 cache): prompt chunks at the sizes that
+// talk_prefill.hip does not take (head sizes other than 64 and 128, pages that are not whole 32-token
+// pieces, tiles that are not whole 128 queries), and decode rows.
 //
 // One workgroup of four waves per (tile of 32 queries of one sequence, query head g).  Keys go
 // by steps of 128: wave w scores keys [32 w, 32 w + 32) of the step (S^T = K Q^T on

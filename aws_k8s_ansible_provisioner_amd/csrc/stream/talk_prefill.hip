@@ -1,0 +1,382 @@
+// Head-mixed attention of prompt chunks on the matrix cores, 128 queries of one query head against
+// all value heads at a time (bf16 caches K [NB, G, BS, D], V [NB, G, BS / 8, Dv, 8], D = 64 or 128,
+// pages of whole 32-token pieces), and the launch that mixes the heads and gates.
+#include "../kernels/common.h"
+#include "stream.h"
+
+namespace akap_stream {
+
+using akap::bf16;
+using akap::bf16x4;
+using akap::bf16x8;
+using akap::f32x16;
+
+namespace {
+
+constexpr int kKeys = 64;              // keys per step
+constexpr int kQ = 128;                // queries of a workgroup
+constexpr float kLog2e = 1.44269504088896f;
+
+__device__ __forceinline__ void dma16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                   (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+__device__ __forceinline__ float both_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float both_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// key of row r of a 32-key tile: a lane's weights then are whole 8-key value groups
+__device__ __forceinline__ int row_key(int r) {
+  return 16 * (r >> 4) + 8 * ((r >> 2) & 1) + 4 * ((r >> 3) & 1) + (r & 3);
+}
+template <int D>
+__device__ __forceinline__ int swz(int key, int c) {
+  return D == 128 ? c ^ (key & 15) : c ^ ((key >> 1) & 7);
+}
+
+__device__ __forceinline__ int sequence_of(const int32_t* q_start, int B, int t) {
+  int lo = 0, hi = B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (q_start[mid] <= t) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+// The sums of a 32-token block of the step in the workspace: [H][G Dv / 4][tokens of the block][4],
+// so that a wave's lanes (a token each) store and read neighbouring 16-byte pieces.
+__device__ __forceinline__ size_t ws_at(const TalkParams& p, int t, int g, int e4) {
+  const int blk = t >> 5, nr = min(32, p.T - 32 * blk), GV = p.G * p.Dv;
+  return (size_t)blk * 32 * p.H * GV + ((size_t)(g * (GV >> 2) + e4) * nr + (t & 31)) * 4;
+}
+
+// Eight waves; a step takes 64 keys.  Wave w scores the 32 queries w & 3 against the 32 keys w >> 2
+// (S^T = K Q^T; a query is a lane column), agrees on the maximum with the wave of the other keys and
+// puts its weights into LDS as operands; then every wave multiplies the weights of all 128 queries
+// with ITS 32 TPW value entries (O^T = V^T P^T), whose fragments it takes straight from the cache: a
+// value is read once per 128 queries.  Keys arrive in LDS by DMA, two buffers.  The scores of step
+// i + 1 are formed beside the first half of step i's products, its weights beside the second half,
+// so a step has two barriers and the softmax runs under products.
+template <int D, int TPW>
+__global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const int32_t* tile_seq,
+                                                             const int32_t* tile_row, int num_tiles,
+                                                             int tile_rows) {
+  constexpr int KS = D / 16;
+  constexpr int PW = kKeys * D * 2 / 1024 / 8;          // 1-KB pieces of the keys per wave
+  constexpr int kK = kKeys * D * 2, kP = kQ * kKeys * 2;   // bytes of a buffer of keys, of weights
+  __shared__ __align__(16) unsigned char lds[3 * kK + 2 * kP + 3 * kQ * 4];
+  bf16* kl0 = (bf16*)lds;
+  bf16x8* ps0 = (bf16x8*)(lds + 3 * kK);
+  float* m_loc = (float*)(lds + 3 * kK + 2 * kP);       // [2][kQ]
+  float* alpha_s = m_loc + 2 * kQ;                      // [kQ]
+
+  // the heads of a tile run side by side on one XCD (they read the same values), longest tiles first
+  const int subs = tile_rows / kQ, units = num_tiles * subs;
+  const int per = (int)blockIdx.x >> 3, g = per % p.H;
+  const int unit = units - 1 - (per / p.H * 8 + ((int)blockIdx.x & 7));
+  if (unit < 0) return;
+  const int tile = unit / subs;
+  const int b = __builtin_amdgcn_readfirstlane(tile_seq[tile]);
+  const int r_first = tile_row[tile] + kQ * (unit - tile * subs);
+  const int q0 = p.q_start[b], chunk = p.q_start[b + 1] - q0;
+  if (r_first >= chunk) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, hf = lane >> 5, qt = w & 3, kb = w >> 2;
+  const int ctx = (int)p.positions[q0];
+  const int last = ctx + min(r_first + kQ, chunk) - 1;  // last key that any query sees
+  const int steps = last / kKeys + 1;
+  const int kvh = g / (p.H / p.G), BS = p.BS, G = p.G, Dv = p.Dv;
+  const __attribute__((address_space(4))) int* bt =
+      (const __attribute__((address_space(4))) int*)(p.block_tables + (size_t)b * p.max_blocks);
+  const int last_piece = last >> 5;
+
+  int koff[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int s = (w * PW + i) * 64 + lane, key = s / (D / 8), c = swz<D>(key, s % (D / 8));
+    koff[i] = (key & 31) * D + c * 8;
+  }
+  // page and row in it of the 32-key piece a walk stands at; past the last piece it stays there
+  struct Walk {
+    int piece, idx, row;
+  };
+  auto advance = [&](Walk& c) {
+    if (c.piece >= last_piece) return;
+    ++c.piece;
+    c.row += 32;
+    if (c.row == BS) { c.row = 0; ++c.idx; }
+  };
+  Walk kw = {0, 0, 0}, vw = {0, 0, 0};
+  if (w >> 2) advance(kw);
+  auto stage = [&](int buf) {                            // the keys of the next step
+    const bf16* kc = (const bf16*)p.k_cache +
+                     (((size_t)bt[kw.idx] * G + kvh) * BS + kw.row) * D;
+    bf16* kl = kl0 + buf * (kK / 2);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) dma16(kc + koff[i], kl + (w * PW + i) * 512);
+    advance(kw);
+    advance(kw);
+  };
+  // value fragments of the next half step (32 keys); 8-key groups past the last key repeat the last
+  const int NT = G * (Dv >> 5), DVT = Dv >> 5;
+  const int ti0 = ((int)blockIdx.y * 8 + w) * TPW;
+  bf16x8 vf[2][TPW][2];
+  int cvk[TPW], dvk[TPW];
+#pragma unroll
+  for (int k = 0; k < TPW; ++k) {
+    const int ti = min(ti0 + k, NT - 1);
+    cvk[k] = ti / DVT;
+    dvk[k] = (ti - cvk[k] * DVT) * 256;
+  }
+  auto values = [&](int half) {
+    const size_t page = (size_t)bt[vw.idx] * G;
+    const int lim = (last >> 3) - 4 * vw.piece;
+    const unsigned off0 = (unsigned)((min(hf, lim) * Dv + r) * 8);
+    const unsigned off1 = (unsigned)((min(2 + hf, lim) * Dv + r) * 8);
+#pragma unroll
+    for (int k = 0; k < TPW; ++k) {
+      const bf16* vc = (const bf16*)p.v_cache +
+                       ((page + cvk[k]) * (BS >> 3) + (vw.row >> 3)) * Dv * 8 + dvk[k];
+      vf[half][k][0] = *(const bf16x8*)(vc + off0);
+      vf[half][k][1] = *(const bf16x8*)(vc + off1);
+    }
+    advance(vw);
+  };
+
+  stage(0);
+  stage(1);
+  stage(2);
+  bf16x8 qf[KS];
+  const int tok = r_first + 32 * qt + r;
+  {
+    const bool valid = tok < chunk;
+    const bf16* q = (const bf16*)p.q + ((size_t)(q0 + (valid ? tok : 0)) * p.H + g) * D + 8 * hf;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+      const bf16x8 v = *(const bf16x8*)(q + 16 * s);
+      qf[s] = valid ? v : z;
+    }
+  }
+  const int limit = tok < chunk ? ctx + tok : -1;
+  const int w_first = r_first + 32 * qt + 31 < chunk ? ctx + r_first + 32 * qt : -1;
+  const float sc2 = p.scale * kLog2e;
+  float m_run = -1e30f, l_run = 0.f, mx = -INFINITY;
+  f32x16 acc[TPW][4], s;
+#pragma unroll
+  for (int k = 0; k < TPW; ++k)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[k][q][i] = 0.f;
+
+  auto scores = [&](int buf) {
+    const bf16* kl = kl0 + buf * (kK / 2);
+    const int key = 32 * kb + row_key(r);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < KS; ++c) {
+      const bf16x8 kf = *(const bf16x8*)(kl + key * D + swz<D>(key, 2 * c + hf) * 8);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s, 0, 0, 0);
+    }
+  };
+  auto maximum = [&](int t) {
+    const int first = t * kKeys + 32 * kb;
+    if (first + 31 > w_first) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (first + 16 * (i >> 3) + 8 * hf + (i & 7) > limit) s[i] = -INFINITY;
+    }
+    mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = both_max(mx) * sc2;
+    m_loc[kb * kQ + 32 * qt + r] = mx;      // (both halves' lanes hold the same)
+  };
+  auto weights = [&](int t) {
+    const float m_new = fmaxf(fmaxf(m_run, mx), m_loc[(kb ^ 1) * kQ + 32 * qt + r]);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], sc2, -m_new));
+      sum[i & 1] += s[i];
+    }
+    l_run = l_run * alpha + (sum[0] + sum[1]);
+    m_run = m_new;
+    bf16x8* ps = ps0 + (t & 1) * (kP / 16);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      bf16x8 pb;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) pb[j] = (bf16)s[8 * e + j];
+      ps[(4 * qt + 2 * kb + e) * 64 + lane] = pb;
+    }
+    alpha_s[32 * qt + r] = alpha;           // (as both key halves' waves do)
+  };
+  auto products = [&](int t, int half) {
+    const bf16x8* ps = ps0 + (t & 1) * (kP / 16);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const bf16x8 pf = ps[(4 * q + 2 * half + e) * 64 + lane];
+#pragma unroll
+        for (int k = 0; k < TPW; ++k)
+          acc[k][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[half][k][e], pf, acc[k][q], 0, 0, 0);
+      }
+  };
+
+  values(0);
+  values(1);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  scores(0);
+  maximum(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  weights(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // (the last step forms the scores and weights of one step more, all of them masked, rather than
+  // branch around them)
+  for (int t = 0, b1 = 1, b0 = 0; t < steps; ++t) {
+    {
+      float a[4];
+      bool moved = false;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        a[q] = alpha_s[32 * q + r];
+        moved |= a[q] != 1.0f;
+      }
+      if (__any(moved)) {
+#pragma unroll
+        for (int k = 0; k < TPW; ++k)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[k][q][i] *= a[q];
+      }
+    }
+    scores(b1);
+    products(t, 0);
+    maximum(t + 1);
+    // the keys of step t + 2 have landed, those of step t were last read before the barrier before
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    values(0);
+    stage(b0);
+    weights(t + 1);
+    products(t, 1);
+    values(1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    b0 = b0 == 2 ? 0 : b0 + 1;
+    b1 = b1 == 2 ? 0 : b1 + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (nothing may land after the end)
+  // both key halves' sums; the normalised sums of the wave's value entries
+  l_run = both_sum(l_run);
+  if (hf == 0) m_loc[kb * kQ + 32 * qt + r] = l_run;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int tq = r_first + 32 * q + r;
+    if (tq >= chunk) continue;
+    const float inv = 1.0f / (m_loc[32 * q + r] + m_loc[kQ + 32 * q + r]);
+#pragma unroll
+    for (int k = 0; k < TPW; ++k)
+      if (ti0 + k < NT) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *(float4*)(p.ws_o + ws_at(p, q0 + tq, g, 8 * (ti0 + k) + 2 * j + hf)) =
+              make_float4(acc[k][q][4 * j] * inv, acc[k][q][4 * j + 1] * inv,
+                          acc[k][q][4 * j + 2] * inv, acc[k][q][4 * j + 3] * inv);
+      }
+  }
+}
+
+// out = talk x the heads' normalised sums, times the gate.  A lane takes 4 value entries of a token,
+// all heads' sums of them in flight together.  Bound by reading
+// the sums: 90 us for 8000 rows of 16 x 512 fp32 (262 MB) and their gates and outputs; a workgroup per
+// token with 4-byte loads took 174.
+template <int HM>
+__global__ __launch_bounds__(256) void talk_mix_kernel(TalkParams p) {
+  const int t = ((p.row0 >> 5) + blockIdx.x) * 32 + (threadIdx.x & 31);
+  const int e4 = blockIdx.y * 8 + (threadIdx.x >> 5), GV = p.G * p.Dv;
+  if (e4 * 4 >= GV || t < p.row0 || t >= p.T) return;
+  if (p.seq_lens[sequence_of(p.q_start, p.B, t)] <= 0) return;
+  const int c = __builtin_amdgcn_readfirstlane(e4 * 4 / p.Dv);   // (a wave's: Dv is whole 32s)
+  const int dv = e4 * 4 - c * p.Dv, rep = p.H / p.G;
+  float4 o[HM];
+#pragma unroll
+  for (int g = 0; g < HM; ++g)
+    if (g < p.H) o[g] = *(const float4*)(p.ws_o + ws_at(p, t, g, e4));
+  const bool wide = ((p.gate_stride & 3) | ((uintptr_t)p.gate & 7) | (p.out_stride & 3) |
+                     ((uintptr_t)p.out & 7)) == 0;
+  for (int i = 0; i < rep; ++i) {
+    const int h = c * rep + i;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < HM; ++g)
+      if (g < p.H && (p.talk || g == h)) {
+        const float f = p.talk ? p.talk[(size_t)h * p.H + g] : 1.f;
+        v[0] = fmaf(f, o[g].x, v[0]); v[1] = fmaf(f, o[g].y, v[1]);
+        v[2] = fmaf(f, o[g].z, v[2]); v[3] = fmaf(f, o[g].w, v[3]);
+      }
+    const int col = h * p.Dv + dv;
+    if (p.gate) {
+      const bf16* gp = (const bf16*)p.gate + (size_t)t * p.gate_stride + col;
+      bf16x4 z;
+      if (wide) {
+        z = *(const bf16x4*)gp;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[e] = gp[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= 1.0f / (1.0f + __expf(-(float)z[e]));
+    }
+    bf16* at = (bf16*)p.out + (size_t)t * p.out_stride + col;
+    const bf16x4 ob = {(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+    if (wide) {
+      *(bf16x4*)at = ob;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) at[e] = ob[e];
+    }
+  }
+}
+
+}  // namespace
+
+bool launch_talk_staged(const TalkParams& p, const int32_t* tile_seq, const int32_t* tile_row,
+                        int num_tiles, int tile_rows, hipStream_t s) {
+  if ((p.D != 64 && p.D != 128) || p.Dv % 32 || p.BS % 32 || tile_rows % kQ || !(p.scale > 0.f) ||
+      p.H > 32 || ((uintptr_t)p.ws_o & 15))
+    return false;
+  const int NT = p.G * (p.Dv / 32), units = num_tiles * (tile_rows / kQ);
+  if (units > 0) {
+    // 8 value tiles of 32 per grid row with one per wave, 16 with two
+    const int tpw = NT <= 8 ? 1 : 2;
+    const dim3 grid((units + 7) / 8 * 8 * p.H, (NT + 8 * tpw - 1) / (8 * tpw));
+#define AKAP_TS(DD, TP) \
+  talk_staged_kernel<DD, TP><<<grid, 512, 0, s>>>(p, tile_seq, tile_row, num_tiles, tile_rows)
+    if (p.D == 64) {
+      if (tpw == 1) AKAP_TS(64, 1); else AKAP_TS(64, 2);
+    } else {
+      if (tpw == 1) AKAP_TS(128, 1); else AKAP_TS(128, 2);
+    }
+#undef AKAP_TS
+  }
+  if (p.T > p.row0) {
+    const dim3 grid((p.T + 31) / 32 - (p.row0 >> 5), (p.G * p.Dv / 4 + 7) / 8);
+    if (p.H <= 8) talk_mix_kernel<8><<<grid, 256, 0, s>>>(p);
+    else if (p.H <= 16) talk_mix_kernel<16><<<grid, 256, 0, s>>>(p);
+    else talk_mix_kernel<32><<<grid, 256, 0, s>>>(p);
+  }
+  return true;
+}
+
+}  // namespace akap_stream

@@ -1,0 +1,63 @@
+"""Head-mixed attention of prompt chunks with keys staged through LDS (GPU) against the same op on CPU
+tensors: both head sizes, value sizes that fill one, several and two grid rows of 32-entry tiles (also
+with a last wave that has none), chunks that end inside 32-key pieces, 64-key steps and 128-query
+tiles, cached tokens before them, pages of 32, 64 and 96 tokens, single rows that lead the step, rows
+that are not 16-byte aligned, no mixing and no gate.
+
+Tolerance: weights and outputs are rounded to bf16 (relative 2^-9 each, on either side for the
+outputs): the 2-norm of the difference stays under 3 * 2^-9 of the result's; mixing sums up to H heads'
+rounded weights, whose errors are independent."""
+import pytest
+import torch
+
+from aws_k8s_ansible_provisioner_amd.ops import stream as sops
+
+pytestmark = pytest.mark.gpu
+DEV, TOL = "cuda", 3 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("H,G,D,Dv,BS,shape,nd,extra", [
+    (4, 2, 64, 64, 32, [(0, 33)], 0, "gate talk"),
+    (2, 1, 128, 32, 64, [(0, 128), (5, 1), (64, 129)], 0, "talk"),
+    (16, 4, 128, 128, 64, [(70, 131), (0, 64), (191, 300)], 0, "gate talk"),
+    (32, 8, 128, 128, 64, [(3, 200), (0, 61)], 0, "gate talk"),
+    (6, 3, 64, 96, 96, [(95, 97), (0, 31), (1, 96)], 0, "gate"),
+    (9, 3, 64, 160, 32, [(0, 127), (31, 66)], 0, ""),
+    (8, 4, 128, 64, 64, [(200, 1), (17, 1), (9, 150)], 2, "gate talk odd"),
+])
+def test_chunks(H, G, D, Dv, BS, shape, nd, extra):
+    g = torch.Generator().manual_seed(H * D + Dv)
+    pages = [-(-(p + n) // BS) for p, n in shape]
+    NB = sum(pages) + 1
+    perm, at = torch.randperm(NB, generator=g), 0
+    bt = torch.zeros(len(shape), max(pages), dtype=torch.int32)
+    tiles, start = [], [0]
+    for b, (p, n) in enumerate(shape):
+        bt[b, :pages[b]] = perm[at:at + pages[b]].to(torch.int32)
+        at += pages[b]
+        start.append(start[-1] + n)
+        if b >= nd:
+            tiles += [(p + min(n, r + 256), b, r) for r in range(0, n, 256)]
+    tiles.sort()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)
+    T, pad = start[-1], 3 if "odd" in extra else 0
+    pos = torch.cat([torch.arange(p, p + n) for p, n in shape])
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v = rnd(T, H, D), rnd(NB, G, BS, D), rnd(NB, G, BS // 8, Dv, 8)
+    gate = rnd(T, H * Dv + pad) if "gate" in extra else None
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g) if "talk" in extra else None
+    lens, qs = i32([p + n for p, n in shape]), i32(start)
+    ts, tr = i32([t[1] for t in tiles]), i32([t[2] for t in tiles])
+
+    def run(dev):
+        m = lambda x: None if x is None else x.to(dev)
+        out = torch.zeros(T, H * Dv + pad, dtype=torch.bfloat16, device=dev)
+        w = (lambda x: x[:, pad:]) if pad else (lambda x: x)
+        sops.talking_attention_prefill(w(out), m(q), m(k), m(v), m(bt), m(lens), m(qs), m(pos),
+                                       m(ts), m(tr), 256, m(talk),
+                                       w(m(gate)) if gate is not None else None, D ** -0.5, nd)
+        return out.float().cpu()
+
+    a, b = run(DEV), run("cpu")
+    assert float((a - b).norm() / b.norm()) <= TOL
+    assert float((a - b).abs().max()) <= 8 * TOL * float(b.abs().max())
