@@ -161,6 +161,8 @@ struct PGemmArgs {
   void* Y;          // bf16 [M, N] (row stride ldy), or [M, N/2] with the SwiGLU epilogue
   const int* offs;  // grouped: [groups] cumulative row ends (device)
   int groups;       // 0 = dense
+  const int* rows;  // grouped, or null: row r's X row is rows[r] / top (device)
+  int top, x_rows;  // x_rows: rows of X (M where rows is null)
   int M, N, K, ldx, ldy;
   int stagger;      // unit body: workgroups start their K loops at decorrelated offsets
   int gm;           // raster: M tiles per block of the tile map (0 = 8)

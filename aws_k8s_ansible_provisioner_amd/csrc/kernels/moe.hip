@@ -263,6 +263,117 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
   }
 }
 
+// The same for up to 32 experts without atomics, over 16 workgroups that need no word from each
+// other: every one counts all ids by segments, each wave one segment, and places its own.  A wave counts by ballots into its own row of counters; a second walk puts every id at its
+// cursor plus its rank among the lanes with the same id -- a stable sort.  Bound by latencies: 32768
+// ids of 8 experts 19 us; in one workgroup 26 us with an LDS atomic per id, 29 us with ballots.
+constexpr int kAlignE = 32;
+
+__global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __restrict__ ids, int n,
+                                                             int E, int block,
+                                                             int32_t* __restrict__ sorted_ids,
+                                                             int32_t* __restrict__ offsets,
+                                                             int32_t* __restrict__ num_padded,
+                                                             int32_t* __restrict__ inv,
+                                                             int32_t* __restrict__ tile_expert,
+                                                             int max_tiles) {
+  __shared__ int seg[16][kAlignE], run[16][kAlignE];   // ids per segment, per wave of my segment
+  __shared__ int total[kAlignE], mine[kAlignE], offs[kAlignE + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x;
+  int bits = 0;
+  while ((1 << bits) < E) ++bits;
+  // lanes that hold the same id as this one (none: not an expert), by a ballot per bit of it
+  auto peers = [&](int id) {
+    const bool ok = (unsigned)id < (unsigned)E;
+    uint64_t same = __ballot(ok);
+    for (int k = 0; k < bits; ++k) {
+      const uint64_t m = __ballot((id >> k) & 1);
+      same &= (id >> k) & 1 ? m : ~m;
+    }
+    return ok ? same : 0;
+  };
+  auto walk = [&](int lo, int hi, auto use) {
+    for (int i0 = lo; i0 < hi; i0 += 1024) {
+      int id[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int i = i0 + 64 * u + lane;
+        id[u] = i < hi ? ids[i] : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (i0 + 64 * u < hi) use(id[u], i0 + 64 * u + lane);
+    }
+  };
+  const uint64_t below = (1ull << lane) - 1;
+  auto count = [&](int* row, int lo, int hi) {
+    if (lane < E) row[lane] = 0;
+    walk(lo, hi, [&](int id, int) {
+      const uint64_t same = peers(id);
+      if (same && !(same & below)) row[id] += __popcll(same);   // the first of them
+    });
+  };
+  // segments and, in mine, runs of whole 64s
+  const int sper = (((n + 15) >> 4) + 63) & ~63;
+  const int s0 = min(b * sper, n), s1 = min(s0 + sper, n);
+  const int rper = (((s1 - s0 + 15) >> 4) + 63) & ~63;
+  const int r0 = min(s0 + wave * rper, s1), r1 = min(r0 + rper, s1);
+  count(seg[wave], min(wave * sper, n), min(wave * sper + sper, n));
+  count(run[wave], r0, r1);
+  __syncthreads();
+  if (tid < E) {
+    int sum = 0;
+    for (int w = 0; w < 16; ++w) {                       // runs -> ids of my segment before the run
+      const int c = run[w][tid];
+      run[w][tid] = sum;
+      sum += c;
+    }
+    int before = 0;
+    sum = 0;
+    for (int s = 0; s < 16; ++s) {
+      if (s == b) before = sum;
+      sum += seg[s][tid];
+    }
+    total[tid] = sum;
+    mine[tid] = before;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int acc = 0;
+    for (int e = 0; e < E; ++e) {
+      offs[e] = acc;
+      acc += (total[e] + block - 1) / block * block;
+    }
+    offs[E] = acc;
+    if (b == 0) *num_padded = acc;
+  }
+  __syncthreads();
+  if (b == 0) {
+    if (tid <= E) offsets[tid] = offs[tid];
+    for (int e = wave; e < E; e += 16)
+      for (int i = offs[e] + total[e] + lane; i < offs[e + 1]; i += 64) sorted_ids[i] = n;
+    if (tile_expert != nullptr)
+      for (int t = tid; t < max_tiles; t += 1024) {
+        int e = -1;
+        if (t * block < offs[E])
+          for (e = 0; offs[e + 1] <= t * block;) ++e;
+        tile_expert[t] = e;
+      }
+  }
+  if (lane < E) run[wave][lane] += offs[lane] + mine[lane];
+  walk(r0, r1, [&](int id, int i) {
+    const uint64_t same = peers(id);
+    int pos = -1;
+    if (same) {
+      pos = run[wave][id] + __popcll(same & below);
+      if (!(same & below)) run[wave][id] = pos + __popcll(same);
+      sorted_ids[pos] = i;
+    }
+    if (inv != nullptr && i < r1) inv[i] = pos;
+  });
+}
+
 // Grouped GEMM over expert-sorted rows:  Y[r] = A[row(r)] . W[e(tile)]^T
 // A_GATHER: row(r) = sorted_ids[r] / topk (token rows of the hidden state; padding rows
 // read as zeros); else row(r) = r (the previous grouped GEMM's output).  Same 64x64x64
@@ -419,6 +530,12 @@ void launch_moe_combine(const void* Y, const float* wts, const int32_t* inv, voi
 void launch_moe_align(const int32_t* topk_ids, int n, int E, int block, int32_t* sorted_ids,
                       int32_t* expert_offsets, int32_t* num_padded, int32_t* inv,
                       int32_t* tile_expert, int max_tiles, hipStream_t s) {
+  // (4096 ids 5.7 -> 6.9 us, 32768 ids 26 -> 19: below 8192 one workgroup is done sooner)
+  if (E <= kAlignE && n >= 8192) {
+    moe_align_few_kernel<<<16, 1024, 0, s>>>(topk_ids, n, E, block, sorted_ids, expert_offsets,
+                                            num_padded, inv, tile_expert, max_tiles);
+    return;
+  }
   moe_align_kernel<<<1, 1024, (3 * E + 1) * sizeof(int), s>>>(topk_ids, n, E, block, sorted_ids,
                                                         expert_offsets, num_padded, inv,
                                                         tile_expert, max_tiles);

@@ -49,6 +49,9 @@
 // Grouped (MoE): group g owns rows [offs[g-1], offs[g]) of X and weight W + g*N*K; the same
 // raster runs over the concatenated list of every group's M tiles; the grid is an upper bound
 // (sum of ceil(rows_g / 256) <= ceil(M / 256) + G) and surplus WGs exit.
+// With PGemmArgs.rows a tile's X rows are gathered by the DMA's per-lane offsets (a row's 128 bytes of
+// a K tile are one line wherever it lies): 16384 tokens of 2048, 2 of 8 experts of 1408 383 us up and
+// 238 us down; the 64 x 128 tiles of moe_dgemm.hip 626 and 290.
 // SwiGLU epilogue (EPI_SILU): W rows are the [gate; up] halves of a [2F, K] weight; tile column
 // v reads weight row ((v >> 4) & 1) * F + (v >> 5) * 16 + (v & 15) (the gdgemm.hip mapping), so
 // gate and up of one output column land in the same lane of adjacent fragments and the kernel
@@ -168,6 +171,16 @@ __device__ __forceinline__ bool pg_tile(const PGemmArgs& p, int& tm, int& tn, in
 // descriptor's range read as 0), W rows of tile columns n0.. (SILU_ROWS: the [gate; up] row
 // interleave of the SwiGLU epilogue, `nhalf` = F).  Leaves the tile in acc (lane: rows
 // wm*128 + i*16 + fr, 4 consecutive columns wn*64 + j*16 + fg*4 per fragment).
+// Where output row r's X row lies: r itself, or (expert rows gathered from their tokens) row
+// ids[r] / top; rows past the group's end repeat its last row (their outputs are never stored).
+struct PgRows {
+  const int32_t* ids = nullptr;
+  int top = 1, hi = 0;
+  __device__ __forceinline__ int operator()(int r) const {
+    return ids ? ids[min(r, hi - 1)] / top : r;
+  }
+};
+
 // a wave's accumulator fragments: rows i (8 x 16), columns j (2 NJ x 16)
 template <int NJ2>
 struct PgAcc {
@@ -178,7 +191,7 @@ template <int NB, bool SILU_ROWS, int WAVES, typename ACC, int SCHED = 1>
 __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_rsrc_t rx,
                                             const __amdgpu_buffer_rsrc_t rw, int ldx, int K,
                                             int nhalf, int m0, int n0, int kt0, int nk,
-                                            ACC& accs) {
+                                            ACC& accs, const PgRows rows = {}) {
   using G = PgGeo<WAVES>;
   constexpr int P = G::P, NJ = G::NJ;
   auto& acc = accs.v;
@@ -208,7 +221,7 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
       const int row = r0 + (lane >> 3);
       const int chunk = (lane & 7) ^ ((row >> 1) & 7);
       if (h == 0 || h == 3) {
-        voff[h][e] = (uint32_t)(((m0 + row) * ldx + chunk * 8) * 2);
+        voff[h][e] = (uint32_t)((rows(m0 + row) * ldx + chunk * 8) * 2);
         dst[h][e] = r0 * 8;
       } else {
         const int v = n0 + row;
@@ -457,7 +470,7 @@ template <bool SILU_ROWS, typename ACC>
 __device__ __forceinline__ void pg_mainloop_u(bf16x8* lds, const __amdgpu_buffer_rsrc_t rx,
                                               const __amdgpu_buffer_rsrc_t rw, int ldx, int K,
                                               int nhalf, int m0, int n0, int ku0, int nu,
-                                              int st0, ACC& accs) {
+                                              int st0, ACC& accs, const PgRows rows) {
   auto& acc = accs.v;  // [8][8]
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -471,7 +484,7 @@ __device__ __forceinline__ void pg_mainloop_u(bf16x8* lds, const __amdgpu_buffer
     const int row = r16 * 16 + (lane >> 2);
     const int c = pu_swz(row, lane & 3);  // logical chunk held by this lane's LDS slot
     if (e < 4) {
-      voff[e] = (uint32_t)(((m0 + row) * ldx + c * 8) * 2);
+      voff[e] = (uint32_t)((rows(m0 + row) * ldx + c * 8) * 2);
     } else {
       const int v = n0 + row;
       int wr = v;
@@ -589,9 +602,11 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   const bf16* X = static_cast<const bf16*>(p.X);
   const bf16* W = static_cast<const bf16*>(p.W) + (GROUPED ? (size_t)group * p.N * p.K : 0);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)X, (short)0, (int)((size_t)p.M * p.ldx * 2), 0x00020000);
+      (void*)X, (short)0, (int)((size_t)p.x_rows * p.ldx * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
       (void*)W, (short)0, (int)((size_t)p.N * p.K * 2), 0x00020000);
+  PgRows rows;
+  if (GROUPED) rows = {p.rows, p.top, row_hi};
   PgAcc<2 * PgGeo<WAVES>::NJ> accs;
   auto& acc = accs.v;
   if constexpr (SCHED == 3) {
@@ -601,11 +616,11 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
     const int h = (id ^ (id >> 3)) & 7;  // those that share a W panel (consecutive ids)
     const int st0 = p.stagger ? (h * nu) / 8 : 0;
     pg_mainloop_u<EPI == EPI_SILU>(lds, rx, rw, p.ldx, p.K, p.N >> 1, m0, n0, 0, nu, st0,
-                                   accs);
+                                   accs, rows);
   } else {
     pg_mainloop<NB, EPI == EPI_SILU, WAVES, decltype(accs), SCHED>(lds, rx, rw, p.ldx, p.K,
                                                                    p.N >> 1, m0, n0, 0,
-                                                                   p.K / PG_BK, accs);
+                                                                   p.K / PG_BK, accs, rows);
   }
 
   // ---- epilogue: lane holds rows wm*128 + i*16 + fr, 4 consecutive cols per fragment ---------

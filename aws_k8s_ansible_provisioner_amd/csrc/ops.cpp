@@ -830,13 +830,24 @@ void kv_pull(Tensor src_planes, Tensor dst_planes, int64_t block_elems, Tensor p
 // Prefill / large-M GEMM (pgemm.hip): out = x . w^T (epi 0) or silu(gate) * up over the
 // [gate; up] halves of w (epi 2, out [M, N/2]).  offs (int32 [G], device) -> expert-grouped:
 // rows of x sorted by group, w [G, N, K].
-void pgemm(Tensor out, Tensor x, Tensor w, int64_t epi, std::optional<Tensor> offs) {
+// rows (int32, grouped only): output row r takes x row rows[r] / top.
+void pgemm(Tensor out, Tensor x, Tensor w, int64_t epi, std::optional<Tensor> offs,
+           std::optional<Tensor> rows, int64_t top) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(out);
   CHECK_LAST_CONTIG(x); CHECK_CONTIG(w); CHECK_LAST_CONTIG(out);
   TORCH_CHECK(x.dim() == 2 && out.dim() == 2, "x, out must be 2-D");
   TORCH_CHECK(epi == akap::EPI_STORE || epi == akap::EPI_SILU, "pgemm epilogue: store | silu");
   akap::PGemmArgs a{};
-  a.M = x.size(0);
+  a.M = a.x_rows = x.size(0);
+  a.top = 1;
+  if (rows) {
+    CHECK_GPU(*rows); CHECK_CONTIG(*rows);
+    TORCH_CHECK(offs && rows->scalar_type() == at::kInt && top >= 1,
+                "pgemm rows: grouped, int32, top >= 1");
+    a.M = rows->numel();
+    a.rows = rows->data_ptr<int>();
+    a.top = (int)top;
+  }
   a.K = x.size(1);
   a.N = w.size(-2);
   TORCH_CHECK(w.size(-1) == a.K, "w [.., N, K] must match x [M, K]");
@@ -859,7 +870,7 @@ void pgemm(Tensor out, Tensor x, Tensor w, int64_t epi, std::optional<Tensor> of
   a.ldy = out.stride(0);
   TORCH_CHECK(a.ldx % 8 == 0 && a.ldy % 4 == 0, "row strides must keep 16-B / 8-B alignment");
   // the DMA addresses X and one group's W through buffer descriptors with 32-bit offsets
-  TORCH_CHECK((int64_t)a.M * a.ldx * 2 < (int64_t(1) << 31) &&
+  TORCH_CHECK((int64_t)a.x_rows * a.ldx * 2 < (int64_t(1) << 31) &&
                   (int64_t)a.N * a.K * 2 < (int64_t(1) << 31),
               "pgemm: X and each weight matrix must stay below 2 GiB");
   const c10::DeviceGuard g(x.device());
@@ -1330,7 +1341,9 @@ TORCH_LIBRARY(akap, m) {
       "Tensor? ss_in=None, Tensor(d!)? ss_out=None, Tensor(e!)? aout=None, "
       "Tensor? ln_out=None, int bn=0, int ns=0, Tensor(f!)? counters=None, int bm=64) -> ()");
   m.def("wgemm(Tensor(a!) out, Tensor x, Tensor w) -> ()");
-  m.def("pgemm(Tensor(a!) out, Tensor x, Tensor w, int epi=0, Tensor? offs=None) -> ()");
+  m.def(
+      "pgemm(Tensor(a!) out, Tensor x, Tensor w, int epi=0, Tensor? offs=None, Tensor? rows=None, "
+      "int top=1) -> ()");
   m.def("kgemm(Tensor(a!) out, Tensor x, Tensor w, int bm, int epi, float eps, Tensor? ss_in, "
         "Tensor(b!)? ss_out, Tensor(c!)? aout, Tensor? ln_out) -> ()");
   m.def("dgemm_ok(int M, int N, int K, int splitk, int pf) -> bool");

@@ -769,10 +769,20 @@ def fused_moe(h, w13, w2, topk_w, topk_ids, out=None, clamp=None):
     if clamp is not None:
         units = (1, topk_w.contiguous(), float(clamp[0]), float(clamp[1]))
         topk_w = torch.ones_like(topk_w)
+    dev = h.device
+    if clamp is None and _moe_large(n, E, h, w13, w2):
+        # rows sorted by expert without padding, tiles of 256 x 256
+        inv = torch.empty(n, dtype=torch.int32, device=dev)
+        sorted_ids, offsets, _ = moe_align(topk_ids, E, 1, inv=inv)
+        act = torch.empty(n, F, dtype=h.dtype, device=dev)
+        torch.ops.akap.pgemm(act, h, w13, EPI_SILU, offsets[1:], sorted_ids, K)
+        y2 = torch.empty(n, d, dtype=h.dtype, device=dev)
+        torch.ops.akap.pgemm(y2, act, w2, EPI_STORE, offsets[1:])
+        torch.ops.akap.moe_combine(y2, topk_w.contiguous(), inv, out)
+        return out
     bm = moe_tile_rows(n, E)
     cap = moe_capacity(n, E, bm)
     tiles = cap // bm
-    dev = h.device
     inv = torch.empty(n, dtype=torch.int32, device=dev)
     tile_expert = torch.empty(tiles, dtype=torch.int32, device=dev)
     sorted_ids, _, _ = moe_align(topk_ids, E, bm, inv=inv, tile_expert=tile_expert)
@@ -792,6 +802,19 @@ def fused_moe(h, w13, w2, topk_w, topk_ids, out=None, clamp=None):
                              _moe_pf(F), bm)
     torch.ops.akap.moe_combine(y2, topk_w.contiguous(), inv, out)
     return out
+
+
+def _moe_large(n: int, num_experts: int, h, w13, w2) -> bool:
+    """fused_moe on 256 x 256 tiles (pgemm, rows sorted without padding)?  From 208 rows per expert
+    on, or from 128 where the up projection's tiles alone fill the chip (MI355X, 8 experts, top 2,
+    small tiles -> these: d = 2048, F = 1408, T = 768 96 -> 100 us, T = 896 113 -> 103, T = 2048
+    207 -> 157, T = 16384 1014 -> 650; d = 4096, F = 3584, T = 448 279 -> 301, T = 512 323 -> 307,
+    T = 4096 1703 -> 826)."""
+    d, F = h.shape[1], w2.shape[2]
+    rows = 128 if num_experts * (2 * F // 256) >= 192 else 208
+    return (n >= rows * num_experts and h.stride(-1) == 1 and h.stride(0) % 8 == 0
+            and h.shape[0] * h.stride(0) * 2 < 2 ** 31 and w13.is_contiguous()
+            and w2.is_contiguous() and pgemm_supported(n, 2 * F, d) and pgemm_supported(n, d, F))
 
 
 def moe_down_splitk(n: int, num_experts: int, bm: int, F: int) -> int:
