@@ -264,7 +264,8 @@ __global__ __launch_bounds__(64) void latent_decode_mfma_kernel(LatentAttnParams
 }
 
 
-// ---- wide latents (R >= 256): four waves share one tile of 32 query columns -------------------
+// ---- wide latents (R >= 256): four waves share one tile of 32 query columns
+// (Prompt chunks at R = 512, r = 64: latent_prefill.hip.)
 // At R = 512 a single wave's output accumulators alone are 256 registers.  Four waves split the
 // work of a 128-key step instead: wave w scores keys [32 w, 32 w + 32) of the step against the
 // whole query tile (S^T = K Q^T over all R + r dimensions), the waves agree on the running
@@ -615,7 +616,9 @@ void launch_prefill(const LatentAttnParams& p, hipStream_t s) {
   constexpr int DK = 32 * NV + 16 * NKR;
   const int units = p.num_tiles * (p.tile_rows / 32);
   const unsigned padded = (unsigned)((units + 7) / 8 * 8);
-  if constexpr (NV >= 8) {
+  if constexpr (NV == 16 && NKR == 4) {
+    launch_latent_prefill_wide(p, s);
+  } else if constexpr (NV >= 8) {
     latent_prefill_coop_kernel<NV, NKR><<<padded * p.H, 256, CoopSmem<NV, NKR>::bytes(p), s>>>(p);
   } else {
     // narrow latents: one wave per tile and head, 4 heads per workgroup

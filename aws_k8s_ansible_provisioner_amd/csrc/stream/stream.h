@@ -174,6 +174,7 @@ void launch_latent_attention(const LatentAttnParams& p, bool f32, hipStream_t s)
 // bf16, R / r among the built sizes (latent_mfma_sizes), BS % 32 == 0, 16-byte aligned rows
 bool latent_mfma_sizes(int R, int r);
 void launch_latent_prefill_mfma(const LatentAttnParams& p, hipStream_t s);
+void launch_latent_prefill_wide(const LatentAttnParams& p, hipStream_t s);   // R = 512, r = 64
 void launch_latent_decode_mfma(const LatentAttnParams& p, hipStream_t s);
 
 // out [H, T, N] (strides o_hs / o_ts) = a [H, T, K] (strides a_hs / a_ts, unit in k) x
