@@ -230,17 +230,20 @@ __global__ __launch_bounds__(512, 2) void latent_prefill_wide_kernel(LatentAttnP
     }
     scores(0, false);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    stage(1, 0, 2 * KI);
-    next();
+    if (steps > 1) {
+      stage(1, 0, 2 * KI);
+      next();
+    }
     weights();
     for (int st = 0; st < steps; ++st) {
       // rows of step st + 1 have landed, weights are written
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      // (the last step scores one step more, all of it masked)
-      scores(st + 1, true);
+      if (st + 1 < steps) scores(st + 1, true);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      next();
-      if (st + 1 < steps) weights();
+      if (st + 1 < steps) {
+        next();
+        weights();
+      }
     }
     l_run = both_sum(l_run);
     m_loc[kb * 64 + 32 * head + r] = l_run;
