@@ -241,8 +241,6 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   weights(0);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  // (the last step forms the scores and weights of one step more, all of them masked, rather than
-  // branch around them)
   for (int t = 0, b1 = 1, b0 = 0; t < steps; ++t) {
     {
       float a[4];
@@ -261,16 +259,19 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
             for (int i = 0; i < 16; ++i) acc[k][q][i] *= a[q];
       }
     }
-    scores(b1);
+    const bool ahead = t + 1 < steps;
+    if (ahead) scores(b1);
     products(t, 0);
-    maximum(t + 1);
+    if (ahead) maximum(t + 1);
     // the keys of step t + 2 have landed, those of step t were last read before the barrier before
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    values(0);
-    stage(b0);
-    weights(t + 1);
+    if (ahead) {
+      values(0);
+      stage(b0);
+      weights(t + 1);
+    }
     products(t, 1);
-    values(1);
+    if (ahead) values(1);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     b0 = b0 == 2 ? 0 : b0 + 1;
     b1 = b1 == 2 ? 0 : b1 + 1;
