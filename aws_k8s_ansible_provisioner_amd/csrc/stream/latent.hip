@@ -13,6 +13,7 @@
 namespace akap_stream {
 
 using akap::bf16;
+using akap::bf16x8;
 using akap::block_sum;
 using akap::wave_max;
 using akap::wave_sum;
@@ -194,6 +195,119 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepParams p) {
     const float c = cs[i], s = cs[half + i];
     stf(dst + p.kv_rank + a, u * c - v * s);
     stf(dst + p.kv_rank + b, v * c + u * s);
+  }
+}
+
+// The same for large steps (bf16, ranks and offsets of whole 16-byte pieces, q_rank up to 512 NQ,
+// kv_rank up to 512): 32 rows per workgroup, a wave for 4 of them with all their loads in flight.  The
+// normed latents pass through LDS, where 8 rows that fill one group are transposed and leave as whole
+// 16-byte entries; rows of a group that lies across workgroups or sequences are written element by
+// element.  Bound by memory: 7600 rows of 768 + 512 + 64 25 us; 46 with a workgroup per row, whose
+// every 2-byte group entry is a store of its own.
+template <int NQ>
+__global__ __launch_bounds__(512) void latent_prep_rows_kernel(LatentPrepParams p) {
+  constexpr int RW = 32;
+  __shared__ bf16x8 vals[RW][64];
+  __shared__ int64_t slot_of[RW];
+  __shared__ int lead[RW];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t0 = blockIdx.x * RW;
+  const int qc = p.q_rank >> 3, kc = p.kv_rank >> 3;
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8 q[4][NQ], kv[4];
+  int64_t slot[4], pos[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = min(t0 + 4 * w + i, p.T - 1);
+    const bf16* row = (const bf16*)p.proj + (size_t)t * p.proj_stride;
+#pragma unroll
+    for (int c = 0; c < NQ; ++c)
+      q[i][c] = lane + 64 * c < qc ? *(const bf16x8*)(row + p.q_off + (lane + 64 * c) * 8) : zero;
+    kv[i] = p.cache && lane < kc ? *(const bf16x8*)(row + p.kv_off + lane * 8) : zero;
+    slot[i] = p.cache ? p.slots[t] : -1;
+    pos[i] = p.cache ? p.positions[t] : 0;
+    if (t0 + 4 * w + i >= p.T || slot[i] >= p.num_slots) slot[i] = -1;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = t0 + 4 * w + i;
+    float ss = 0.f, sk = 0.f;
+#pragma unroll
+    for (int c = 0; c < NQ; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += (float)q[i][c][e] * (float)q[i][c][e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sk += (float)kv[i][e] * (float)kv[i][e];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      ss += __shfl_xor(ss, o, 64);
+      sk += __shfl_xor(sk, o, 64);
+    }
+    const float inv = 1.0f / sqrtf(ss / (float)p.q_rank + p.eps);
+    const float invk = 1.0f / sqrtf(sk / (float)p.kv_rank + p.eps);
+    if (t < p.T) {
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) {
+        const int at = (lane + 64 * c) * 8;
+        if (lane + 64 * c < qc) {
+          bf16x8 o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)q[i][c][e] * inv * p.q_w[at + e]);
+          *(bf16x8*)((bf16*)p.cq_out + (size_t)t * p.q_rank + at) = o;
+        }
+      }
+    }
+    if (lane == 0) slot_of[4 * w + i] = slot[i];
+    if (slot[i] < 0) continue;                       // (the wave's)
+    bf16* dst = (bf16*)p.cache + (size_t)slot[i] * (p.kv_rank + p.rot_dim);
+    if (lane < kc) {
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)kv[i][e] * invk * p.kv_w[lane * 8 + e]);
+      *(bf16x8*)(dst + lane * 8) = o;
+      vals[4 * w + i][lane] = o;
+    }
+    const int64_t at = pos[i] < 0 ? 0 : (pos[i] >= p.max_pos ? p.max_pos - 1 : pos[i]);
+    const float* cs = p.cos_sin + (size_t)at * p.rot_dim;
+    const int half = p.rot_dim / 2;
+    const bf16* kr = (const bf16*)p.proj + (size_t)t * p.proj_stride + p.kv_off + p.kv_rank;
+    for (int j = lane; j < half; j += 64) {
+      const int a = p.half_pairs ? j : 2 * j, b = p.half_pairs ? j + half : 2 * j + 1;
+      const float u = (float)kr[a], v = (float)kr[b], c = cs[j], s = cs[half + j];
+      dst[p.kv_rank + a] = (bf16)(u * c - v * s);
+      dst[p.kv_rank + b] = (bf16)(v * c + u * s);
+    }
+  }
+  if (!p.cache || !p.vgroups) return;
+  __syncthreads();
+  if (tid < RW) {                                    // first row of a whole group?
+    bool l = slot_of[tid] >= 0 && (slot_of[tid] & 7) == 0 && tid + 7 < RW;
+    for (int k = 1; k < 8 && l; ++k) l = slot_of[tid + k] == slot_of[tid] + k;
+    lead[tid] = l;
+  }
+  __syncthreads();
+  if (lane >= kc) return;
+#pragma unroll
+  for (int u = 0; u < RW / 8; ++u) {
+    const int r = 8 * u + w;
+    const int64_t s = slot_of[r];
+    if (s < 0) continue;
+    bf16* grp = (bf16*)p.vgroups + (size_t)(s >> 3) * p.kv_rank * 8 + lane * 64 + (s & 7);
+    if (lead[r]) {
+      bf16x8 v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = vals[r + k][lane];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bf16x8 o = {v[0][e], v[1][e], v[2][e], v[3][e], v[4][e], v[5][e], v[6][e], v[7][e]};
+        *(bf16x8*)(grp + 8 * e) = o;
+      }
+    } else {
+      const int first = r - (int)(s & 7);
+      if (first >= 0 && lead[first]) continue;       // its first row's wave writes it
+      const bf16x8 v = vals[r][lane];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) grp[8 * e] = v[e];
+    }
   }
 }
 
@@ -758,6 +872,16 @@ void launch_token_shift(void* out, const void* h, const float* mu, void* state,
 
 void launch_latent_prep(const LatentPrepParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
+  // (fewer rows leave most CUs without one of these workgroups)
+  if (!f32 && p.T >= 2048 && ((p.q_rank | p.q_off | p.proj_stride) & 7) == 0 && p.q_rank <= 2048 &&
+      (((uintptr_t)p.proj | (uintptr_t)p.cq_out) & 15) == 0 &&
+      (!p.cache || (((p.kv_rank | p.kv_off | p.rot_dim) & 7) == 0 && p.kv_rank <= 512 &&
+                    (((uintptr_t)p.cache | (uintptr_t)p.vgroups) & 15) == 0))) {
+    const int n = (p.T + 31) / 32;
+    if (p.q_rank <= 1024) latent_prep_rows_kernel<2><<<n, 512, 0, s>>>(p);
+    else latent_prep_rows_kernel<4><<<n, 512, 0, s>>>(p);
+    return;
+  }
   if (f32) latent_prep_kernel<float><<<p.T, 256, 0, s>>>(p);
   else latent_prep_kernel<bf16><<<p.T, 256, 0, s>>>(p);
 }

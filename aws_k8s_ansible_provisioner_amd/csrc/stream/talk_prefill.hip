@@ -58,9 +58,14 @@ __device__ __forceinline__ size_t ws_at(const TalkParams& p, int t, int g, int e
 // (S^T = K Q^T; a query is a lane column), agrees on the maximum with the wave of the other keys and
 // puts its weights into LDS as operands; then every wave multiplies the weights of all 128 queries
 // with ITS 32 TPW value entries (O^T = V^T P^T), whose fragments it takes straight from the cache: a
-// value is read once per 128 queries.  Keys arrive in LDS by DMA, two buffers.  The scores of step
-// i + 1 are formed beside the first half of step i's products, its weights beside the second half,
-// so a step has two barriers and the softmax runs under products.
+// value is read once per 128 queries.  Keys arrive in LDS by DMA, two steps ahead (three buffers).  The
+// scores of step i + 1 are formed beside the first half of step i's products, its weights beside the
+// second half.  The running maximum is exact, so the largest weight is 1 and not rounded.
+//
+// Bound by the chain of a step (score products, maximum, barrier, exponentials, barrier: alone 186 of
+// 357 us) beside the products (116 us of the matrix units' time): 8 chunks of 1000 tokens behind 1000
+// cached, 16 / 4 heads of 128 357 us; 64 queries per workgroup with every fragment from the caches
+// took 919.  Opposite order of matrix and vector work in a SIMD's two waves gained nothing (381).
 template <int D, int TPW>
 __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const int32_t* tile_seq,
                                                              const int32_t* tile_row, int num_tiles,
@@ -299,9 +304,8 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
 }
 
 // out = talk x the heads' normalised sums, times the gate.  A lane takes 4 value entries of a token,
-// all heads' sums of them in flight together.  Bound by reading
-// the sums: 90 us for 8000 rows of 16 x 512 fp32 (262 MB) and their gates and outputs; a workgroup per
-// token with 4-byte loads took 174.
+// all heads' sums of them in flight together.  Bound by reading the sums: 90 us for 8000 rows of
+// 16 x 512 fp32 (262 MB), their gates and outputs; a workgroup per token with 4-byte loads took 174.
 template <int HM>
 __global__ __launch_bounds__(256) void talk_mix_kernel(TalkParams p) {
   const int t = ((p.row0 >> 5) + blockIdx.x) * 32 + (threadIdx.x & 31);

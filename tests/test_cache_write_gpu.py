@@ -75,6 +75,33 @@ def test_head_caches(form, n, dt):
         _same(a.cpu(), b, dt)
 
 
+@pytest.mark.parametrize("n,q_rank,kv_rank,rot,form", [
+    (2047, 768, 512, 64, ""), (2048, 768, 512, 64, ""), (2077, 1536, 512, 64, "half"),
+    (2050, 1032, 96, 16, ""), (2049, 64, 256, 32, "rows"), (2051, 768, 512, 64, "queries")])
+def test_latent_rows(n, q_rank, kv_rank, rot, form):
+    """Both sides of 2048 rows (32 to a workgroup); rows without the grouped copy, and without any."""
+    g = torch.Generator().manual_seed(n)
+    BS, dt = 64, torch.bfloat16
+    slots, pos, NB = _step(n, BS, n)
+    proj = torch.randn(n, 8 + q_rank + kv_rank + rot, generator=g).to(dt)
+    cs = sops.rotary_table(4 * BS + 200, rot, 1e4, None, "cpu")
+    qw, kw = torch.rand(q_rank, generator=g) + 0.5, torch.rand(kv_rank, generator=g) + 0.5
+
+    def run(dev):
+        c = lambda t: t.clone().to(dev)
+        cq = torch.zeros(n, q_rank, dtype=dt, device=dev)
+        rows = torch.zeros(NB, BS, kv_rank + rot, dtype=dt, device=dev)
+        groups = torch.zeros(NB, BS // 8, kv_rank, 8, dtype=dt, device=dev)
+        sops.latent_prep(c(proj), cq, None if form == "queries" else rows, c(pos), c(slots), c(cs),
+                         c(qw), c(kw), q_rank, kv_rank, rot, 8, 8 + q_rank, 1e-5,
+                         vgroups=None if form in ("rows", "queries") else groups,
+                         half=form == "half")
+        return cq, rows, groups
+
+    for a, b in zip(run(DEV), run("cpu")):
+        _same(a.cpu(), b, dt)
+
+
 @pytest.mark.parametrize("D,Dv,pool,BS", [(64, 128, 64, 64), (128, 64, 32, 64), (64, 32, 16, 16),
                                           (256, 256, 64, 64), (72, 64, 64, 64)])
 def test_pooled_blocks(D, Dv, pool, BS):
