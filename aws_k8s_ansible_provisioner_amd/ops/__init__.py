@@ -750,8 +750,9 @@ def fused_moe(h, w13, w2, topk_w, topk_ids, out=None, clamp=None):
 
     GPU: moe_align (device-side sort + tile->expert map, 32-row tiles) -> grouped k-pipelined
     MFMA GEMM gathering token rows with the SwiGLU in its epilogue (csrc/kernels/
-    moe_dgemm.hip) -> grouped GEMM -> deterministic gather-combine.  All buffer shapes depend
-    only on (T, top_k, E), so the whole block captures in a hipGraph.
+    moe_dgemm.hip) -> grouped GEMM -> deterministic gather-combine.  Large steps (_moe_large): rows
+    sorted without padding, both GEMMs on the 256 x 256 tiles of csrc/kernels/pgemm.hip.  All buffer
+    shapes depend only on (T, top_k, E), so the whole block captures in a hipGraph.
     w13 [E, 2F, d], w2 [E, d, F].  clamp = (limit, alpha): clamped gated units instead of SwiGLU,
     with the routing weight on the expert's input -- g = min(w[t,k] gate, limit), u =
     clamp(w[t,k] up, -limit, limit), g sigmoid(alpha g) (u + 1) -- and a plain sum over k."""
