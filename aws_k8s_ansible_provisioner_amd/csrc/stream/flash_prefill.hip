@@ -12,14 +12,14 @@
 // without lane traffic.  The K rows are XOR-swizzled by the DMA's source address, the fragment
 // reads are free of bank conflicts.
 //
-// The running maximum is exact, so the largest weight is 1 and not rounded (letting it lag by up to
-// 8 log2 units saved 14 of 199 us and cost 1 to 7 % more error); a sink is where maximum and sum
-// start.
+// The running maximum is exact and moves by 32 keys, so every weight that is the largest so far is 1
+// and not rounded: letting it lag by up to 8 log2 units cost 1 to 7 % more error, one maximum per 64
+// keys 0.25 % (and took 196 and 149 us); a sink is where maximum and sum start.
 //
-// Bound by the vector work of the softmax beside the products (about 3200 cycles of exponentials,
-// maxima and roundings per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4 heads
-// of 128, causal: 199 us (0.69 PFLOP/s; fragments straight from the caches took 331), 5 prompts of
-// up to 3001 tokens through a window of 1024 and pooled blocks of 64: 153 us (553).
+// Bound by the vector work of the softmax beside the products (about 3400 cycles of exponentials,
+// maxima, roundings and rescaling per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4
+// heads of 128, causal: 211 us (0.65 PFLOP/s; fragments straight from the caches took 331), 5 prompts
+// of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 164 us (553).
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const float sc2 = p.scale * kLog2e;
   const bool sunk = p.sink != nullptr || p.unit_sink;
   float m_run = p.sink ? fmaxf(p.sink[h] * kLog2e, -1e30f) : p.unit_sink ? 0.f : -1e30f;
-  float l_run = sunk ? 1.f : 0.f;
+  float l_run = sunk && hf == 0 ? 1.f : 0.f;       // (a lane's own keys; the halves meet at the end)
   f32x16 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -186,43 +186,39 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 #pragma unroll
         for (int d = 0; d < DT; ++d)
           vf[k][e][d] = *(const bf16x8*)(vl + ((4 * k + 2 * e + hf) * D + 32 * d + r) * 8);
-    float mx = -INFINITY;
-    if (masked) {
+    // maximum, weights and products of 32 keys at a time
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 2; ++k) {
+      float mx = -INFINITY;
+      if (masked) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           if (!seen(32 * k + 16 * (i >> 3) + 8 * hf + (i & 7))) s[k][i] = -INFINITY;
           mx = fmaxf(mx, s[k][i]);
         }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
+      } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[k][i]);
-    }
-    mx = both_max(mx);
-    const float m_new = fmaxf(m_run, mx * sc2);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float sum[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
+      }
+      mx = both_max(mx);
+      const float m_new = fmaxf(m_run, mx * sc2);
+      float sum[2] = {0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float e = __builtin_amdgcn_exp2f(fmaf(s[k][i], sc2, -m_new));
         s[k][i] = e;
-        sum[i & 3] += e;
+        sum[i & 1] += e;
       }
-    l_run = l_run * alpha + both_sum((sum[0] + sum[1]) + (sum[2] + sum[3]));
-    if (__any(m_new != m_run)) {
+      if (__any(m_new != m_run)) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
 #pragma unroll
-      for (int d = 0; d < DT; ++d)
+        for (int d = 0; d < DT; ++d)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
-    }
-    m_run = m_new;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
+          for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
+      }
+      m_run = m_new;
+      l_run += sum[0] + sum[1];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         bf16x8 pb;
@@ -232,6 +228,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
         for (int d = 0; d < DT; ++d)
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k][e][d], pb, o[d], 0, 0, 0);
       }
+    }
   };
 
   if (POOL) {
@@ -291,6 +288,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   }
 
   if (!active) return;
+  l_run = both_sum(l_run);
   float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   const int t_out = q0 + (valid ? tok : 0);
   if (p.gate) {
