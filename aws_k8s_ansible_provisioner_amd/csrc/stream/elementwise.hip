@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_kernel(ProjParams p)
 // Workgroups past the rows' write the values (write_values; vrows 0: none do, a row's own workgroup
 // writes its values), as large steps do.  Bound by memory and by a chain of latencies per workgroup
 // (row, sums, weights and angles, store): at 16384 rows of 16 / 4 heads of 128 79 us with values
-// element by element and a barrier pair per sum, 91 with the values taken out alone, 69.5 with both
+// element by element and a barrier pair per sum, 91 with the values taken out alone, 63 with both
 // sums behind one barrier and weights, angles and slot requested ahead of it.
 template <typename T, int NQ>
 __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParams p, int vrows) {

@@ -280,8 +280,9 @@ __global__ __launch_bounds__(256) void head_norm_cache_kernel(HeadNormParams p) 
 // their loads in flight together, weights and biases read once; D / 8 lanes per query / key head.
 // The first nqk workgroups take the (rows, head) pairs of q and k, the others the values
 // (write_values).  Bound by memory and by the loads' latency: 13600 rows of 16 / 4 / 4 heads of 128
-// with normed values 83 us with values one by one, 57 with R = 1, 47.5 with 4; 12800 rows with biases
-// and rotation 89 us element by element, 79.5 with R = 1, 73 with 4.
+// with normed values 44 us (83 with values one by one, 57 with R = 1, 47.5 with only the groups whole
+// that begin at a multiple of 8 rows); 12800 rows with biases and rotation 57 us (89 element by
+// element, 79.5 and 73).
 template <typename T, int R>
 __global__ __launch_bounds__(256) void head_norm_cache_vec_kernel(HeadNormParams p, int nqk,
                                                                   int vrows) {

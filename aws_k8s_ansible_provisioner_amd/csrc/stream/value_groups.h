@@ -4,7 +4,8 @@
 // write every entry in eight parts from eight workgroups, on eight XCDs with an L2 each.  Here a
 // thread takes 8 dimensions of `vrows` neighbouring rows (8; 1 for small steps, whose rows are mostly
 // sequences of their own): 8 rows that fill one group are transposed in registers and leave as whole
-// entries.
+// entries, wherever among the rows the group begins (sequences of ragged steps begin at any row);
+// rows of a group that is not whole are written element by element.
 #pragma once
 
 #include "../kernels/common.h"
@@ -62,18 +63,21 @@ __device__ __forceinline__ void write_values(const ValueGroups<T>& a, int64_t it
   const int e = (int)(item % per), g = e / lph, c = (e - g * lph) * 8;
   const int n = live ? min(a.vrows, a.T_ - t0) : 0;
   const int64_t s0 = live ? a.slots[t0] : -1;
-  bool whole = n == 8 && s0 >= 0 && (s0 & 7) == 0 && s0 + 7 < a.num_slots;
-  if (a.vrows == 8) {
+  // the 8 rows that fill the first group which begins at or after row t (its slot s)
+  auto group = [&](int t, int64_t s, int& first) {
+    first = t + (int)((8 - (s & 7)) & 7);
+    const int64_t f = (s + 7) & ~(int64_t)7;
+    bool whole = s >= 0 && first + 8 <= a.T_ && f + 7 < a.num_slots;
 #pragma unroll
-    for (int i = 1; i < 8; ++i)     // (all eight requested together)
-      whole &= a.slots[min(live ? t0 + i : 0, a.T_ - 1)] == s0 + i;
-  }
-  const T* src = a.src + (size_t)(live ? t0 : 0) * a.stride + g * a.Dv + c;
+    for (int i = 0; i < 8; ++i)     // (all eight requested together)
+      whole &= a.slots[min(first + i, a.T_ - 1)] == f + i;
+    return whole;
+  };
   float add[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (a.bias) vg::ld8(a.bias + g * a.Dv + c, add);
   if (a.bias_t) vg::ld8(a.bias_t + g * a.Dv + c, add);
-  auto row = [&](int i, float (&v)[8]) {      // (every lane of a wave, rows clamped)
-    vg::ld8(src + (size_t)i * a.stride, v);
+  auto row = [&](int t, float (&v)[8]) {      // (every lane of a head, rows clamped)
+    vg::ld8(a.src + (size_t)t * a.stride + g * a.Dv + c, v);
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] += add[k];
     if (a.norm) {
@@ -91,31 +95,36 @@ __device__ __forceinline__ void write_values(const ValueGroups<T>& a, int64_t it
                       c) * 8 + (slot & 7);
   };
   if (a.vrows == 8) {
-    float v[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) row(min(i, n > 0 ? n - 1 : 0), v[i]);
+    if (!live) return;
+    // the group that begins among my rows, and the one that began among the 8 before and may end here
+    int mine, prev = 0;
+    const bool whole = group(t0, s0, mine);
+    const bool before = t0 > 0 && group(t0 - 8, a.slots[t0 - 8], prev);
     if (whole) {
-      T* o = dst(s0);
+      float v[8][8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) row(mine + i, v[i]);
+      T* o = dst(a.slots[mine]);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const float r[8] = {v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k], v[6][k], v[7][k]};
         vg::st8(o + k * 8, r);
       }
-      return;
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i >= n) continue;
-      const int64_t slot = a.slots[t0 + i];
+    for (int t = t0; t < t0 + n; ++t) {       // what is in neither
+      if ((whole && t >= mine) || (before && t >= prev && t < prev + 8)) continue;
+      float v[8];
+      row(t, v);
+      const int64_t slot = a.slots[t];
       if (slot < 0 || slot >= a.num_slots) continue;
       T* o = dst(slot);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o[k * 8] = (T)v[i][k];
+      for (int k = 0; k < 8; ++k) o[k * 8] = (T)v[k];
     }
     return;
   }
   float v[8];
-  row(0, v);
+  row(live ? t0 : 0, v);
   if (s0 < 0 || s0 >= a.num_slots) return;
   T* o = dst(s0);
 #pragma unroll
