@@ -628,7 +628,7 @@ void launch_sink_attention_prefill(const AttnParams& p, bool f32, hipStream_t s)
     f.num_tiles = p.num_tiles; f.tile_rows = p.tile_rows;
     f.gate = p.gate; f.gate_stride = p.gate_stride; f.sink = p.sink;
     f.scale = p.scale; f.chunk = p.chunk; f.window = p.window;
-    f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS;
+    f.B = p.B; f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS; f.NB = p.NB;
     launch_flash_prefill(f, s);
     return;
   }

@@ -81,9 +81,11 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, hf = lane >> 5;
   const int b = __builtin_amdgcn_readfirstlane(p.tile_seq[tile]);
+  if (b < 0 || b >= p.B) return;                        // (every exit here is the workgroup's)
   const int q0 = p.q_start[b], q_len = p.q_start[b + 1] - q0;
   if (q_len <= 0) return;
   const int ctx = p.positions ? (int)p.positions[q0] : p.seq_lens[b] - q_len;
+  if (ctx < 0 && !p.positions) return;                  // fewer keys than rows
   const int kv_len = ctx + q_len;
   const int unit = part * NW + w, sub = unit / rep, h = g * rep + unit - sub * rep;
   const int tok0 = p.tile_row[tile] + 32 * sub;        // the wave's first token of the chunk
@@ -104,10 +106,10 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int g_last = ctx + min(g_tok1, q_len - 1);
   const int key_first = lower(ctx + g_tok0) & ~31;      // staging starts at a 32-key piece
   const int w_lo0 = lower(w_first), w_lo1 = lower(w_last);
-  const int steps = (g_last - key_first) / kKeys + 1;
+  const int steps = max((g_last - key_first) / kKeys + 1, 1);
   const int32_t* bt = p.block_tables + (size_t)b * p.max_blocks;
   const int BS = p.BS, G = p.G;
-  const int last_piece = (kv_len - 1) >> 5;
+  const int last_piece = max(kv_len - 1, 0) >> 5;
 
   // staging of step t: a wave's pieces lie in one 32-key piece of it, so page and row are uniform
   int koff[PW], voff[PW];
@@ -122,7 +124,10 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
         min((key_first >> 5) + t * 2 + (w * PW) / (PIECES / 2), last_piece));
   };
   const __attribute__((address_space(4))) int* btc = (const __attribute__((address_space(4))) int*)bt;
-  auto page_of = [&](int t) { return btc[piece_of(t) * 32 / BS]; };
+  auto page_of = [&](int t) {       // entries outside the cache or the table: page 0
+    const int idx = piece_of(t) * 32 / BS, page = idx < p.max_blocks ? btc[idx] : 0;
+    return page >= 0 && page < p.NB ? page : 0;
+  };
   auto stage = [&](int t, int buf, int page) {
     bf16* kl = lds + buf * kBuf;
     bf16* vl = kl + kKeys * D;

@@ -368,6 +368,7 @@ akap_stream::PoolAttnParams attn_params(Tensor& out, Tensor& q, Tensor& k_cache,
   }
   TORCH_CHECK(p.B >= 1 && p.B <= block_tables.size(0), "attention: a block-table row per sequence");
   p.H = (int)H; p.G = (int)G; p.D = (int)D; p.Dv = (int)Dv; p.BS = (int)k_cache.size(2);
+  p.NB = (int)k_cache.size(0);
   p.PS = (int)PS; p.window = (int)window; p.pool = (int)pool; p.unit_sink = unit_sink ? 1 : 0;
   return p;
 }

@@ -316,7 +316,7 @@ void launch_pooled_window_prefill_mfma(const PoolAttnParams& p, const int32_t* t
     f.tile_seq = tile_seq; f.tile_row = tile_row;
     f.num_tiles = num_tiles; f.tile_rows = 128;
     f.unit_sink = p.unit_sink; f.scale = p.scale; f.window = p.window;
-    f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS;
+    f.B = p.B; f.H = p.H; f.G = p.G; f.D = p.D; f.BS = p.BS; f.NB = p.NB;
     if (p.pool > 0 && p.window > 0 && p.k_pool) {
       f.k_pool = p.k_pool; f.v_pool = p.v_pool; f.pool = p.pool; f.PS = p.PS;
     }

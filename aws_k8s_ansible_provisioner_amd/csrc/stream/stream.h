@@ -90,7 +90,7 @@ struct FlashParams {
   int unit_sink;                // a sink of score 0
   float scale;
   int chunk, window;            // 0: off
-  int H, G, D, BS;
+  int B, H, G, D, BS, NB;
   // pooled entries of `pool` tokens before the window (0: none), fp32 [NB, G, PS, D]
   const float* k_pool;
   const float* v_pool;
@@ -485,7 +485,7 @@ struct PoolAttnParams {
   const int64_t* positions;
   const int64_t* slots;
   float scale;
-  int max_blocks, T, B, H, G, D, Dv, BS, PS, window, pool, unit_sink;
+  int max_blocks, T, B, H, G, D, Dv, BS, NB, PS, window, pool, unit_sink;
 };
 void launch_pooled_window_attention(const PoolAttnParams& p, bool f32, hipStream_t s);
 // matrix-core form for prompt chunks (bf16): the rows of the tile map (tile_seq / tile_row:

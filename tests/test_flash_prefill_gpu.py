@@ -97,3 +97,38 @@ def test_pooled_prefill_staged(shape, H, G, D, window, pool):
             s["tr"].to(dev), 128, D ** -0.5, window, pool, True)
         outs.append(out)
     _close(outs[1], outs[0])
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_sink_prefill_ranges(D):
+    """Tiles that name no sequence and sequences with fewer keys than rows are passed over; block-table
+    entries outside the cache or past the table's end are page 0.  The same at every head size."""
+    H, G, BS, rows = 8, 2, 32, 128
+    s = _step([(0, 150), (40, 90), (0, 70)], G, D, BS, rows, seed=D)
+    q = torch.randn(310, H, D, generator=s["gen"]).bfloat16()
+
+    def run(bt, lens, ts):
+        out = torch.full((310, H * D), 7.0, dtype=torch.bfloat16, device=DEV)
+        sops.sink_attention_prefill(out, *(t.to(DEV) for t in (q, s["k"], s["v"], bt, lens, s["q_start"],
+                                                              ts, s["tr"])), rows, None, None,
+                                    D ** -0.5)
+        torch.cuda.synchronize()
+        return out.cpu()
+
+    whole = run(s["bt"], s["lens"], s["ts"])
+    lens = s["lens"].clone()
+    lens[1] = 0
+    got = run(s["bt"], lens, s["ts"])
+    assert (got[150:240] == 7).all()
+    assert torch.equal(got[:150], whole[:150]) and torch.equal(got[240:], whole[240:])
+    for bad in (-1, 3):
+        got = run(s["bt"], s["lens"], torch.where(s["ts"] == 2, bad, s["ts"]).to(torch.int32))
+        assert (got[240:] == 7).all() and torch.equal(got[:240], whole[:240])
+    zero, out_of_range = s["bt"].clone(), s["bt"].clone()
+    zero[0, 2], out_of_range[0, 2] = 0, -1
+    zero[1, 1], out_of_range[1, 1] = 0, s["k"].shape[0]
+    assert torch.equal(run(out_of_range, s["lens"], s["ts"]), run(zero, s["lens"], s["ts"]))
+    cut = s["bt"].clone()
+    cut[:, 3:] = 0
+    assert torch.equal(run(s["bt"][:, :3].contiguous(), s["lens"], s["ts"]),
+                       run(cut, s["lens"], s["ts"]))
