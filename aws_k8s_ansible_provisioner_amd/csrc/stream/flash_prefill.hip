@@ -14,7 +14,9 @@
 //
 // The running maximum is exact and moves by 32 keys, so every weight that is the largest so far is 1
 // and not rounded: letting it lag by up to 8 log2 units cost 1 to 7 % more error, one maximum per 64
-// keys 0.25 % (and took 196 and 149 us); a sink is where maximum and sum start.
+// keys 0.25 % (and took 196 and 149 us).  It is a maximum over keys alone: a head's sink enters the
+// finished sums in fp32 (as the start of the maximum, a sink above the scores would have every weight
+// rounded: 1.1 to 1.4 times the error); only the sink of score 0 starts maximum and sum.
 //
 // Bound by the vector work of the softmax beside the products (about 3400 cycles of exponentials,
 // maxima, roundings and rescaling per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4
@@ -153,9 +155,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     }
   }
   const float sc2 = p.scale * kLog2e;
-  const bool sunk = p.sink != nullptr || p.unit_sink;
-  float m_run = p.sink ? fmaxf(p.sink[h] * kLog2e, -1e30f) : p.unit_sink ? 0.f : -1e30f;
-  float l_run = sunk && hf == 0 ? 1.f : 0.f;       // (a lane's own keys; the halves meet at the end)
+  float m_run = p.unit_sink ? 0.f : -1e30f;
+  float l_run = p.unit_sink && hf == 0 ? 1.f : 0.f;   // (a lane's own keys; the halves meet at the end)
   f32x16 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -294,7 +295,14 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 
   if (!active) return;
   l_run = both_sum(l_run);
-  float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  float corr = 1.f;
+  if (p.sink) {
+    const float sk = p.sink[h], mk = m_run * 0.693147180559945f;   // back from log2 units
+    const float m = fmaxf(mk, sk);
+    corr = expf(mk - m);
+    l_run = l_run * corr + expf(sk - m);
+  }
+  float inv = l_run > 0.f ? corr / l_run : 0.f;
   const int t_out = q0 + (valid ? tok : 0);
   if (p.gate) {
     const float z = (float)((const bf16*)p.gate)[(size_t)t_out * p.gate_stride + h];
