@@ -306,7 +306,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int t_out = q0 + (valid ? tok : 0);
   if (p.gate) {
     const float z = (float)((const bf16*)p.gate)[(size_t)t_out * p.gate_stride + h];
-    inv *= 1.0f / (1.0f + __expf(-z));
+    inv *= 1.0f / (1.0f + expf(-z));
   }
   // a lane holds entries 32 d + 8 j + 4 hf + (0..3) of its token; the halves exchange, so that each
   // stores 8 neighbouring entries

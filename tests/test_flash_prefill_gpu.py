@@ -161,3 +161,23 @@ def test_sink_prefill_error_does_not_grow_with_the_sink(sink):
         got = out.cpu().double().view(T, H, D)
         errs.append(float(((got - want).norm(dim=2) / want.norm(dim=2))[32:].mean()))
     assert errs[1] < 1.03 * errs[0], errs
+
+
+def test_sink_prefill_gate_is_exact_to_fp32():
+    """Gates far below zero: a row that sees one key has its value times sigmoid(z) as the result, which
+    must round to the bf16 that the exact product rounds to but for fp32 errors.  An error of e times the
+    value turns a share e / 2^-7.5 of the roundings over.  Exponential, sum, division and product err by
+    1.5 * 2^-24 on average: 1.6e-5; an exponential whose argument z log2(e) is rounded to fp32 first errs
+    by some 20 * 2^-24: 2e-4.  The line is at five times the former."""
+    H, G, D, T = 16, 16, 128, 512
+    s = _step([(0, T)], G, D, 32, 128, seed=9)
+    z = (-60 - 25 * torch.rand(T, H, generator=s["gen"])).bfloat16()
+    out = torch.empty(T, H * D, dtype=torch.bfloat16, device=DEV)
+    q = torch.randn(T, H, D, generator=s["gen"]).bfloat16()
+    sops.sink_attention_prefill(
+        out, q.to(DEV), *(s[n].to(DEV) for n in ("k", "v", "bt", "lens", "q_start", "ts", "tr")), 128,
+        z.to(DEV), None, D ** -0.5, 1)                  # chunks of one position: a row sees its own key
+    v = s["v"][s["bt"][0, :16].long()].transpose(3, 4).transpose(1, 2).reshape(16 * 4, G, 8, D)
+    v = v.transpose(1, 2).reshape(T, G, D).double()
+    want = (v * torch.sigmoid(z.double())[:, :, None]).view(T, H * D)
+    assert float((out.cpu() != want.bfloat16()).float().mean()) < 8e-5
