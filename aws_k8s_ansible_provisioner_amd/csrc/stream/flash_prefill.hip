@@ -37,6 +37,7 @@ namespace {
 
 constexpr int kKeys = 64;              // keys per step
 constexpr float kLog2e = 1.44269504088896f;
+constexpr float kLowest = -3.402823466e38f;   // a running maximum over no keys
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -63,6 +64,7 @@ __device__ __forceinline__ int swz(int key, int c) {
   return D == 128 ? c ^ (key & 15) : c ^ ((key >> 1) & 7);
 }
 
+// POOL: the pooled form (positions given, pooled entries before the window if there are any)
 template <int D, int NW, bool POOL>
 __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashParams p) {
   constexpr int KS = D / 16, DT = D / 32;       // contraction steps of a score, tiles of an output
@@ -155,8 +157,11 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     }
   }
   const float sc2 = p.scale * kLog2e;
-  float m_run = p.unit_sink ? 0.f : -1e30f;
-  float l_run = p.unit_sink && hf == 0 ? 1.f : 0.f;   // (a lane's own keys; the halves meet at the end)
+  // The maximum in log2 units of the scaled scores; POOL: of the scores themselves, so that the
+  // difference is exact however large they are, with all weights (the sink's too) times 2^8, so that
+  // what the exponential gives (nothing below 2^-126) holds every weight that a bf16 can hold
+  float m_run = p.unit_sink ? 0.f : kLowest;
+  float l_run = p.unit_sink && hf == 0 ? (POOL ? 256.f : 1.f) : 0.f;   // (a lane's own keys; the halves meet at the end)
   f32x16 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -207,16 +212,17 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[k][i]);
       }
       mx = both_max(mx);
-      const float m_new = fmaxf(m_run, mx * sc2);
+      const float m_new = fmaxf(m_run, POOL ? mx : mx * sc2);
       float sum[2] = {0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[k][i], sc2, -m_new));
+        const float e = __builtin_amdgcn_exp2f(POOL ? fmaf(s[k][i] - m_new, sc2, 8.f)
+                                                    : fmaf(s[k][i], sc2, -m_new));
         s[k][i] = e;
         sum[i & 1] += e;
       }
       if (__any(m_new != m_run)) {
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        const float alpha = __builtin_amdgcn_exp2f(POOL ? (m_run - m_new) * sc2 : m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int d = 0; d < DT; ++d)
@@ -241,10 +247,9 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     // pooled entries 0 .. nb - 1 (what the workgroup's last token sees), 64 at a time through the
     // second buffer: fp32 rows, rounded to bf16 operands on the way
     const int W = p.window, P = p.pool;
-    const int nb = g_last - W + 1 > 0 ? (g_last - W + 1) / P : 0;
-    const int w_nb = w_last - W + 1 > 0 ? (w_last - W + 1) / P : 0;      // the wave's last token
-    const int w_all = w_first - W + 1 > 0 ? (w_first - W + 1) / P : 0;   // its first token
-    const int mine = valid && pos - W + 1 > 0 ? (pos - W + 1) / P : 0;
+    auto before = [&](int i) { return P > 0 && i - W + 1 > 0 ? (i - W + 1) / P : 0; };
+    const int nb = before(g_last), w_nb = before(w_last), w_all = before(w_first);
+    const int mine = valid ? before(pos) : 0;          // (the wave's last and first token above)
     bf16* kl = lds + kBuf;
     bf16* vl = kl + kKeys * D;
     for (int c0 = 0; c0 < nb; c0 += kKeys) {
@@ -358,7 +363,7 @@ void launch_flash_prefill(const FlashParams& p, hipStream_t s) {
     if (units % 8 == 0) AKAP_FP(DD, 8, PL); \
     else AKAP_FP(DD, 4, PL);              \
   } while (0)
-  if (p.pool > 0) {
+  if (p.positions) {
     if (p.D == 64) AKAP_FP_D(64, true); else AKAP_FP_D(128, true);
   } else {
     if (p.D == 64) AKAP_FP_D(64, false); else AKAP_FP_D(128, false);

@@ -6,6 +6,8 @@ aligned, and pages of 32 and 64 tokens.
 
 Tolerance: weights and outputs are rounded to bf16 (relative 2^-9 each, on either side for the
 outputs): the 2-norm of the difference stays under 3 * 2^-9 of the result's."""
+import math
+
 import pytest
 import torch
 
@@ -181,3 +183,53 @@ def test_sink_prefill_gate_is_exact_to_fp32():
     v = v.transpose(1, 2).reshape(T, G, D).double()
     want = (v * torch.sigmoid(z.double())[:, :, None]).view(T, H * D)
     assert float((out.cpu() != want.bfloat16()).float().mean()) < 8e-5
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_pooled_prefill_small_weights(D):
+    """Weights that only a denormal bf16 holds: keys `e` log2 units below the sink of score 0, with values
+    of 2^126, add up to i + 1 times 2^(126 - e) at row i (all powers of two but the count: exact but for the
+    rounding of the result)."""
+    H, G, T = 4, 2, 64
+    s = _step([(0, T)], G, D, 32, 128, seed=1)
+    q, k = torch.zeros(T, H, D, dtype=torch.bfloat16), torch.zeros_like(s["k"])
+    q[..., 0] = 1.0
+    v = torch.full_like(s["v"], 2.0 ** 126)
+    for e in (100, 126, 128, 133):
+        k[..., 0] = -float(e)
+        out = torch.empty(T, H * D, dtype=torch.bfloat16, device=DEV)
+        sops.pooled_window_attention_prefill(
+            out, *(t.to(DEV) for t in (q, k, v)), None, None,
+            *(s[n].to(DEV) for n in ("bt", "q_start", "pos", "slots", "ts", "tr")), 128,
+            math.log(2.0), 0, 0, True)
+        want = torch.arange(1, T + 1).double()[:, None] * 2.0 ** (126 - e)
+        # (log2(e) ln 2 in fp32 is 1 to 2^-24, times the score)
+        assert float((out.cpu().double() / want - 1).abs().max()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("unit_sink", [True, False])
+@pytest.mark.parametrize("size,shift", [(2.0 ** 17, 0.0), (2.0 ** 55, 0.0), (2.0 ** 17, -2.0 ** 103)])
+def test_pooled_prefill_scores_of_any_size(unit_sink, size, shift):
+    """Finite scores of any size: far apart (one weight is 1, the others 0), or all far below zero."""
+    H, G, D, T, window, pool = 4, 2, 128, 200, 70, 16
+    s = _step([(0, T)], G, D, 32, 128, seed=2)
+    q = (torch.randn(T, H, D, generator=s["gen"]) * size).bfloat16()
+    k = (s["k"].float() * size).bfloat16()
+    n = sops.pool_slots(32, pool)
+    kp = (torch.randn(len(k), G, n, D, generator=s["gen"]) * size).bfloat16().float()   # (as operands)
+    vp = torch.randn(len(k), G, n, D, generator=s["gen"])
+    if shift:                               # every key at the same place, far below
+        q[:], k[:], kp[:] = 2.0 ** 10, shift, shift
+    outs = []
+    for dev in ("cpu", DEV):
+        out = torch.zeros(T, H * D, dtype=torch.bfloat16, device=dev)
+        sops.pooled_window_attention_prefill(
+            out, *(t.to(dev) for t in (q, k, s["v"], kp, vp)),
+            *(s[a].to(dev) for a in ("bt", "q_start", "pos", "slots", "ts", "tr")), 128, D ** -0.5,
+            window, pool, unit_sink)
+        outs.append(out.cpu())
+    assert outs[0].isfinite().all() and outs[1].isfinite().all()
+    if outs[0].any():
+        _close(outs[1], outs[0])
+    else:
+        assert not outs[1].any()
