@@ -16,6 +16,7 @@ namespace {
 constexpr int kKeys = 64;              // keys per step
 constexpr int kQ = 128;                // queries of a workgroup
 constexpr float kLog2e = 1.44269504088896f;
+constexpr float kLowest = -3.402823466e38f;   // a running maximum over no keys
 
 __device__ __forceinline__ void dma16(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
@@ -171,7 +172,8 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
   const int limit = tok < chunk ? ctx + tok : -1;
   const int w_first = r_first + 32 * qt + 31 < chunk ? ctx + r_first + 32 * qt : -1;
   const float sc2 = p.scale * kLog2e;
-  float m_run = -1e30f, l_run = 0.f, mx = -INFINITY;
+  // (the maximum of the scores themselves: differences to it are exact however large they are)
+  float m_run = kLowest, l_run = 0.f, mx = -INFINITY;
   f32x16 acc[TPW][4], s;
 #pragma unroll
   for (int k = 0; k < TPW; ++k)
@@ -201,16 +203,16 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
     mx = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx = both_max(mx) * sc2;
+    mx = both_max(mx);
     m_loc[kb * kQ + 32 * qt + r] = mx;      // (both halves' lanes hold the same)
   };
   auto weights = [&](int t) {
     const float m_new = fmaxf(fmaxf(m_run, mx), m_loc[(kb ^ 1) * kQ + 32 * qt + r]);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * sc2);
     float sum[2] = {0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], sc2, -m_new));
+      s[i] = __builtin_amdgcn_exp2f((s[i] - m_new) * sc2);
       sum[i & 1] += s[i];
     }
     l_run = l_run * alpha + (sum[0] + sum[1]);

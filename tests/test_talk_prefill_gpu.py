@@ -61,3 +61,37 @@ def test_chunks(H, G, D, Dv, BS, shape, nd, extra):
     a, b = run(DEV), run("cpu")
     assert float((a - b).norm() / b.norm()) <= TOL
     assert float((a - b).abs().max()) <= 8 * TOL * float(b.abs().max())
+
+
+def _two_prompts(g, H=8, G=4, D=128, Dv=64, BS=32):
+    """Two sequences, the second continued at an odd position: (arguments, run)."""
+    shape = [(0, 200), (77, 150)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    a = dict(q=rnd(350, H, D), k=rnd(16, G, BS, D), v=rnd(16, G, BS // 8, Dv, 8),
+             bt=torch.randperm(16, generator=g).view(2, 8).to(torch.int32), lens=i32([200, 227]),
+             qs=i32([0, 200, 350]), pos=torch.cat([torch.arange(p, p + n) for p, n in shape]),
+             ts=i32([0, 0, 1, 1]), tr=i32([0, 128, 0, 128]))
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+
+    def run(dev):
+        out = torch.zeros(350, H * Dv, dtype=torch.bfloat16, device=dev)
+        sops.talking_attention_prefill(
+            out, *(a[n].to(dev) for n in ("q", "k", "v", "bt", "lens", "qs", "pos", "ts", "tr")), 128,
+            talk.to(dev), None, D ** -0.5, 0)
+        return out.float().cpu()
+
+    return a, run
+
+
+@pytest.mark.parametrize("size,place", [(2.0 ** 17, 0.0), (2.0 ** 55, 0.0), (1.0, -2.0 ** 103)])
+def test_scores_of_any_size(size, place):
+    """Finite scores of any size: far apart (one weight is 1, the others 0), or all at one place far below
+    zero (equal weights)."""
+    a, run = _two_prompts(torch.Generator().manual_seed(5))
+    a["q"], a["k"] = (a["q"].float() * size).bfloat16(), (a["k"].float() * size).bfloat16()
+    if place:
+        a["q"][:], a["k"][:] = 2.0 ** 10, place
+    got, want = run(DEV), run("cpu")
+    assert want.isfinite().all() and got.isfinite().all()
+    assert float((got - want).norm() / want.norm()) <= TOL
