@@ -30,6 +30,7 @@ namespace {
 
 constexpr int kKeys = 64;
 constexpr float kLog2e = 1.44269504088896f;
+constexpr float kLowest = -3.402823466e38f;   // a running maximum over no keys
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ void dma16(const void* g, void* l) {
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(512, 2) void latent_prefill_wide_kernel(LatentAttnP
     bf16x8 qf[KS];
     const int pos = valid ? ctx + r0 + r : -1, pos_first = r0 + 31 < rend ? ctx + r0 : -1;
     const float sc2 = p.scale * kLog2e;
-    float m_run = -1e30f, l_run = 0.f, mx;
+    float m_run = kLowest, l_run = 0.f, mx;
     f32x16 s;
     // a lane's fragments: four row addresses, the rest are immediate offsets
     const bf16* kp[4];

@@ -233,3 +233,19 @@ def test_pooled_prefill_scores_of_any_size(unit_sink, size, shift):
         _close(outs[1], outs[0])
     else:
         assert not outs[1].any()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_sink_prefill_scores_far_below_zero(D):
+    """Equal scores below -1e30 (a power of two: exact in fp32) are equal weights."""
+    H, G, T = 8, 2, 200
+    s = _step([(0, T)], G, D, 32, 128, seed=6)
+    q, k = torch.full((T, H, D), 2.0 ** 10).bfloat16(), torch.full_like(s["k"], -2.0 ** 103)
+    outs = []
+    for dev in ("cpu", DEV):
+        out = torch.zeros(T, H * D, dtype=torch.bfloat16, device=dev)
+        sops.sink_attention_prefill(out, *(t.to(dev) for t in (q, k, s["v"])),
+                                    *(s[n].to(dev) for n in ("bt", "lens", "q_start", "ts", "tr")), 128,
+                                    None, None, D ** -0.5)
+        outs.append(out)
+    _close(outs[1], outs[0])

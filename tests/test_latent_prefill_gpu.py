@@ -57,3 +57,19 @@ def test_chunks(H, BS, shape, lead, tile_rows):
     a, b = a[:, start[lead]:], b[:, start[lead]:]
     assert float((a - b).norm() / b.norm()) <= TOL
     assert float((a - b).abs().max()) <= 8 * TOL * float(b.abs().max())
+
+
+def test_scores_far_below_zero():
+    """All keys at one place whose scores lie below -1e30 (a power of two: exact): equal weights, so every row is
+    that place again."""
+    H, T = 3, 70
+    q_lat, q = torch.full((H, T, R), 2.0 ** 10), torch.zeros(T, H, 128 + ROT)
+    cache = torch.full((4, 32, R + ROT), -2.0 ** 103)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    out = torch.zeros(H, T, R, dtype=torch.bfloat16, device=DEV)
+    bf = lambda x: x.bfloat16().to(DEV)
+    sops.latent_attention_prefill(out, bf(q_lat), bf(q), 128, bf(cache),
+                                  bf(cache[..., :R].reshape(4, 4, R, 8)), i32([[2, 0, 3]]), i32([T]),
+                                  i32([0, T]), torch.arange(T, device=DEV), i32([0]), i32([0]), 128,
+                                  (R + ROT) ** -0.5)
+    assert float((out.double().cpu() / -2.0 ** 103 - 1).abs().max()) <= 2.0 ** -8
