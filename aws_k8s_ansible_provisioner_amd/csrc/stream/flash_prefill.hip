@@ -22,6 +22,8 @@
 // maxima, roundings and rescaling per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4
 // heads of 128, causal: 211 us (0.65 PFLOP/s; fragments straight from the caches took 331), 5 prompts
 // of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 164 us (553).
+#include <type_traits>
+
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -168,8 +170,13 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
 
-  // one step of 64 keys: scores against the staged keys, weights of those that `seen` admits
-  auto compute = [&](const bf16* kl, const bf16* vl, bool masked, auto seen) {
+  // one step of 64 keys: scores against the staged keys, weights of those that `seen` admits.  Keys
+  // before klo or past khi are seen by no query of the wave (later tokens, and what a page's last owner
+  // left behind the sequence's end); a weight of 0 would not hide values that are not finite, so their
+  // groups are read as the nearest that the wave sees, and pooled entries, which every wave's queries
+  // see to another end, are cleared one by one.
+  auto compute = [&](const bf16* kl, const bf16* vl, bool masked, int klo, int khi, auto pooled,
+                     auto seen) {
     f32x16 s[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -193,10 +200,11 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int e = 0; e < 2; ++e)
+      for (int e = 0; e < 2; ++e) {
+        const int n = min(max(4 * k + 2 * e + hf, klo >> 3), khi >> 3);
 #pragma unroll
-        for (int d = 0; d < DT; ++d)
-          vf[k][e][d] = *(const bf16x8*)(vl + ((4 * k + 2 * e + hf) * D + 32 * d + r) * 8);
+        for (int d = 0; d < DT; ++d) vf[k][e][d] = *(const bf16x8*)(vl + (n * D + 32 * d + r) * 8);
+      }
     // maximum, weights and products of 32 keys at a time
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -236,6 +244,13 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
         bf16x8 pb;
 #pragma unroll
         for (int j = 0; j < 8; ++j) pb[j] = (bf16)s[k][8 * e + j];
+        if (pooled() && masked) {
+#pragma unroll
+          for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (32 * k + 16 * e + 8 * hf + j > khi) vf[k][e][d][j] = (bf16)0.f;
+        }
 #pragma unroll
         for (int d = 0; d < DT; ++d)
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k][e][d], pb, o[d], 0, 0, 0);
@@ -276,7 +291,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
       }
       __syncthreads();
       if (active && c0 < w_nb)
-        compute(kl, vl, c0 + kKeys > w_all, [&](int key) { return c0 + key < mine; });
+        compute(kl, vl, c0 + kKeys > w_all, 0, min(w_nb - 1 - c0, kKeys - 1), std::true_type{}, [&](int key) { return c0 + key < mine; });
     }
   }
 
@@ -292,9 +307,9 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     const int key0 = key_first + t * kKeys;
     if (active && key0 <= w_last && key0 + kKeys > w_lo0) {
       const bf16* kl = lds + (t & 1) * kBuf;
-      compute(kl, kl + kKeys * D, key0 + kKeys - 1 > w_first || key0 < w_lo1, [&](int key) {
-        return key0 + key <= limit && key0 + key >= lo_l;
-      });
+      compute(kl, kl + kKeys * D, key0 + kKeys - 1 > w_first || key0 < w_lo1, max(w_lo0 - key0, 0),
+              min(w_last - key0, kKeys - 1), std::false_type{},
+              [&](int key) { return key0 + key <= limit && key0 + key >= lo_l; });
     }
   }
 

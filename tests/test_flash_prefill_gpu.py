@@ -249,3 +249,62 @@ def test_sink_prefill_scores_far_below_zero(D):
                                     None, None, D ** -0.5)
         outs.append(out)
     _close(outs[1], outs[0])
+
+
+@pytest.mark.parametrize("pooled", [False, True])
+@pytest.mark.parametrize("D,window", [(64, 45), (128, 70), (128, 0)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_values_that_are_not_finite_stay_where_they_are_seen(pooled, D, window, bad):
+    """A value that is not finite reaches the rows that see it and at most the others of their 32-token
+    piece (and 8-token group); what lies behind a sequence's last group in its page reaches none."""
+    H, G, BS, pool = 8, 2, 32, 8
+    shape = [(0, 150), (37, 171)]
+    s = _step(shape, G, D, BS, 128, seed=D + window)
+    q = torch.randn(321, H, D, generator=s["gen"]).bfloat16()
+    n = sops.pool_slots(BS, pool)
+    kp, vp = (torch.randn(len(s["k"]), G, n, D, generator=s["gen"]) for _ in range(2))
+
+    def run(k, v, vp):
+        out = torch.zeros(321, H * D, dtype=torch.bfloat16, device=DEV)
+        m = lambda *names: [s[a].to(DEV) for a in names]
+        if pooled:
+            sops.pooled_window_attention_prefill(
+                out, q.to(DEV), k.to(DEV), v.to(DEV), kp.to(DEV), vp.to(DEV),
+                *m("bt", "q_start", "pos", "slots", "ts", "tr"), 128, D ** -0.5, window, pool, True)
+        else:
+            sops.sink_attention_prefill(out, q.to(DEV), k.to(DEV), v.to(DEV),
+                                        *m("bt", "lens", "q_start", "ts", "tr"), 128, None, None,
+                                        D ** -0.5, 0, window)
+        return out.cpu()
+
+    clean = run(s["k"], s["v"], vp)
+    # behind the sequences' last groups
+    k, v = s["k"].clone(), s["v"].clone()
+    for b, (p, c) in enumerate(shape):
+        end = -(-(p + c) // 8) * 8
+        k[s["bt"][b, end // BS], :, end % BS:] = bad
+        v[s["bt"][b, end // BS], :, end % BS // 8:] = bad
+    assert torch.equal(run(k, v, vp), clean)
+    # one value of the second sequence
+    i = torch.arange(37, 208)
+    piece = (i - 37) // 32 * 32 + 37
+    last = (piece + 31).clamp_max(207)
+    lo = (lambda x: (x - window + 1).clamp_min(0)) if window else torch.zeros_like
+    for j in (3, 39, 100, 166, 200):
+        v = s["v"].clone()
+        v[s["bt"][1, j // BS], 1, j % BS // 8, 5, j % 8] = bad
+        got = run(s["k"], v, vp)
+        assert torch.equal(got[:150], clean[:150])
+        got, want = (x[150:].view(171, H, D) for x in (got, clean))
+        out_of_reach = ((last | 7) < j) | ((lo(piece) & ~7) > j)
+        assert torch.equal(got[out_of_reach], want[out_of_reach])
+        assert not got[(i >= j) & (lo(i) <= j)][:, H // 2:, 5].isfinite().any()
+    # one pooled entry
+    if pooled and window:
+        for c in (0, 7, 13):
+            bad_vp = vp.clone()
+            bad_vp[s["bt"][1, c * pool // BS], 1, c * pool % BS // pool, 5] = bad
+            got = run(s["k"], s["v"], bad_vp)[150:].view(171, H, D)
+            unseen = c * pool + pool - 1 > last - window
+            assert torch.equal(got[unseen], clean[150:].view(171, H, D)[unseen])
+            assert not got[c * pool + pool - 1 <= i - window][:, H // 2:, 5].isfinite().any()
