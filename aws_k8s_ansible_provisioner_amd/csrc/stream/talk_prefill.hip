@@ -96,6 +96,7 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
   const int ctx = (int)p.positions[q0];
   const int last = ctx + min(r_first + kQ, chunk) - 1;  // last key that any query sees
   const int steps = last / kKeys + 1;
+  auto last_of = [&](int q) { return ctx + min(r_first + 32 * q + 32, chunk) - 1; };   // of a query tile
   const int kvh = g / (p.H / p.G), BS = p.BS, G = p.G, Dv = p.Dv;
   const __attribute__((address_space(4))) int* bt =
       (const __attribute__((address_space(4))) int*)(p.block_tables + (size_t)b * p.max_blocks);
@@ -230,7 +231,10 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
   auto products = [&](int t, int half) {
     const bf16x8* ps = ps0 + (t & 1) * (kP / 16);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 4; ++q) {
+      // keys past a query tile's last take no part: a weight of 0 would not hide a value that is not
+      // finite
+      if (t * kKeys + 32 * half > last_of(q)) continue;
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const bf16x8 pf = ps[(4 * q + 2 * half + e) * 64 + lane];
@@ -238,6 +242,7 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
         for (int k = 0; k < TPW; ++k)
           acc[k][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[half][k][e], pf, acc[k][q], 0, 0, 0);
       }
+    }
   };
 
   values(0);

@@ -95,3 +95,26 @@ def test_scores_of_any_size(size, place):
     got, want = run(DEV), run("cpu")
     assert want.isfinite().all() and got.isfinite().all()
     assert float((got - want).norm() / want.norm()) <= TOL
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("Dv", [64, 128])
+def test_values_that_are_not_finite_stay_where_they_are_seen(Dv, bad):
+    """A value that is not finite reaches the rows that see it and at most those of their 32-row piece that
+    share its 32-key piece; what lies behind a sequence's last 8-token group in its page reaches none."""
+    a, run = _two_prompts(torch.Generator().manual_seed(7), Dv=Dv)
+    clean, v = run(DEV), a["v"].clone()
+    for b, end in ((0, 200), (1, 232)):
+        a["k"][a["bt"][b, end // 32], :, end % 32:] = bad
+        a["v"][a["bt"][b, end // 32], :, end % 32 // 8:] = bad
+    assert torch.equal(run(DEV), clean)
+    row = torch.arange(150)
+    last = 77 + (row | 31).clamp_max(149)
+    for j in (3, 80, 110, 141, 200, 226):
+        a["v"] = v.clone()
+        a["v"][a["bt"][1, j // 32], 1, j % 32 // 8, 5, j % 8] = bad
+        got = run(DEV)
+        assert torch.equal(got[:200], clean[:200])
+        out_of_reach = last < (j & ~31)
+        assert torch.equal(got[200:][out_of_reach], clean[200:][out_of_reach])
+        assert not got[200:][row + 77 >= j].view(-1, 8, Dv)[:, 2:4, 5].isfinite().any()
