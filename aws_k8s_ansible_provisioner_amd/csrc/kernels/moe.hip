@@ -264,9 +264,10 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
 }
 
 // The same for up to 32 experts without atomics, over 16 workgroups that need no word from each
-// other: every one counts all ids by segments, each wave one segment, and places its own.  A wave counts by ballots into its own row of counters; a second walk puts every id at its
-// cursor plus its rank among the lanes with the same id -- a stable sort.  Bound by latencies: 32768
-// ids of 8 experts 19 us; in one workgroup 26 us with an LDS atomic per id, 29 us with ballots.
+// other: every one counts all ids by segments, each wave one segment, and places its own.  A wave counts
+// by ballots into its own row of counters; a second walk puts every id at its cursor plus its rank among
+// the lanes with the same id -- a stable sort.  Bound by latencies: 32768 ids of 8 experts 19 us; in one
+// workgroup 26 us with an LDS atomic per id, 29 us with ballots.
 constexpr int kAlignE = 32;
 
 __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __restrict__ ids, int n,
@@ -307,11 +308,18 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
     }
   };
   const uint64_t below = (1ull << lane) - 1;
+  // a lane's counters are read and written by the other lanes of its wave
+  auto wave_sync = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   auto count = [&](int* row, int lo, int hi) {
     if (lane < E) row[lane] = 0;
+    wave_sync();
     walk(lo, hi, [&](int id, int) {
       const uint64_t same = peers(id);
       if (same && !(same & below)) row[id] += __popcll(same);   // the first of them
+      wave_sync();
     });
   };
   // segments and, in mine, runs of whole 64s
@@ -362,14 +370,17 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
       }
   }
   if (lane < E) run[wave][lane] += offs[lane] + mine[lane];
+  wave_sync();
   walk(r0, r1, [&](int id, int i) {
     const uint64_t same = peers(id);
     int pos = -1;
+    if (same) pos = run[wave][id] + __popcll(same & below);
+    wave_sync();
     if (same) {
-      pos = run[wave][id] + __popcll(same & below);
       if (!(same & below)) run[wave][id] = pos + __popcll(same);
       sorted_ids[pos] = i;
     }
+    wave_sync();
     if (inv != nullptr && i < r1) inv[i] = pos;
   });
 }

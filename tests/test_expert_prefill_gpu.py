@@ -75,3 +75,16 @@ def test_routing(T, d, n, top, dt):
     assert float((w - torch.softmax(val, -1)).abs().max()) <= 4 * tol + 1e-6
     few = sops.route_topk(h[:100].to(DEV), r.to(DEV), b.to(DEV), top)      # a row at a time: same sums
     assert torch.equal(few[0].cpu().long(), ids[:100]) and torch.equal(few[1].cpu(), w[:100])
+
+
+@pytest.mark.parametrize("n,E,run", [(8192, 32, 1), (9000, 8, 64), (16500, 3, 4000)])
+def test_align_runs(n, E, run):
+    """Ids by turns in runs: a counter goes from lane to lane of a wave, or stays with one for long."""
+    ids = (torch.arange(n) // run % E).to(torch.int32)
+    inv = torch.empty(n, dtype=torch.int32, device=DEV)
+    s, offs, total = ops.moe_align(ids.to(DEV), E, 1, inv=inv)
+    order = ids.sort(stable=True).indices.to(torch.int32)
+    assert int(total) == n and torch.equal(s.cpu()[:n], order)
+    assert torch.equal(inv.cpu()[order.long()], torch.arange(n, dtype=torch.int32))
+    assert torch.equal(offs.cpu(), torch.tensor([0] + torch.bincount(ids, minlength=E).cumsum(0).tolist(),
+                                                dtype=torch.int32))
