@@ -26,9 +26,10 @@
 // (segments) 264 us in all, by rows 790.
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
-// steps whose (sequence, head, 32 columns) triples leave SIMDs idle run in segments of rows:
-// the same walk without outputs leaves every segment's own state, chunk_join_kernel turns these
-// into the state before each segment, and the full walk starts from there.
+// where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
+// segments of rows: the same walk without outputs leaves every segment's own state,
+// chunk_join_kernel turns these into the state before each segment, and the full walk starts
+// from there.  Only the device knows the sequences' lengths: each workgroup counts the long ones.
 #include <type_traits>
 
 #include "../kernels/common.h"
@@ -114,6 +115,34 @@ __device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int r
   r1 = min(r0 + rows, end);
   if (r0 < first) r1 = r0;
   return lo;
+}
+
+// Is a sequence of n rows walked whole?  Cut are those longer than a segment, unless they are so many
+// that whole they fill the chip: from 768 waves on the second pass over the keys costs more than
+// idle SIMDs (8 x 2048 rows, 8 heads x 128 x 128, 256 waves otherwise: 264 us in segments; 64 heads x
+// 128 x 64, 1024 waves: 452 us whole).
+constexpr int kFill = 768;
+
+__device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
+  if (n <= p.SEG) return true;
+  const int per = p.H * (p.V / 32);
+  if (p.B * per < kFill) return false;
+  int count = 0;
+  for (int b0 = 0; b0 < p.B; b0 += 64) {
+    const int b = b0 + (int)(threadIdx.x & 63);
+    count += __popcll(__ballot(b < p.B && p.q_start[b + 1] - p.q_start[b] > p.SEG));
+  }
+  return count * per >= kFill;
+}
+
+// first segment of sequence b in the buffers (long sequences alone have any): counted like the
+// entries, or, where most sequences are short, from 2 q_start[b] / SEG on (a long one of n rows has
+// at most 2 n / SEG of them)
+__host__ __device__ __forceinline__ bool few_long(int T, int B, int SEG) { return B > T / SEG + 2; }
+
+__device__ __forceinline__ size_t seg_base(const ChunkScanParams& p, int b) {
+  return few_long(p.T, p.B, p.SEG) ? (size_t)(2 * (int64_t)p.q_start[b] / p.SEG)
+                                   : (size_t)base_of(p.q_start, b, p.SEG);
 }
 
 __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
@@ -262,8 +291,8 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
 
 // ------------------------------------------------------------------ the walk
 // HW heads (of one key head) of V / 32 waves each, a wave per 32 state columns; FULL: outputs,
-// from the state in the slot (or, SEGM, from the segment buffer); else the segment's own state
-// from zeros.  A chunk's fragments and scalars arrive by LDS-DMA while the chunk before is
+// from the state in the slot (or, SEGM and the sequence is cut, from the segment buffer); else the
+// segment's own state from zeros.  A chunk's fragments and scalars arrive by LDS-DMA while the chunk before is
 // computed (two buffers of 37 KB, so two workgroups share a CU), its values in registers: a wave
 // waits once per chunk, for loads issued some 10000 cycles earlier.
 template <int MODE, int NT, int V, int HW, typename TY, bool FULL, bool SEGM>
@@ -279,17 +308,25 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   __shared__ __align__(16) float ssq[kNorm ? 2 * NW * kL : 4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h0 = blockIdx.y * HW, hw = wave / VW, h = h0 + hw;
   const int li = lane & 31, hh = lane >> 5;
-  int b = blockIdx.x, r0, r1;
-  if (SEGM) {
-    b = locate(p, blockIdx.x, p.SEG, r0, r1);
+  // SEGM: a workgroup per segment of a cut sequence and head, FULL ahead of all of them one per sequence
+  // and head for those that are not cut (side by side, so that they spread over the CUs as without
+  // SEGM: between workgroups that only leave, 24 sequences of 600 rows took 275 us and not 187)
+  const int whole = SEGM && !FULL ? 0 : p.B * (p.H / HW);
+  const bool cut = SEGM && (int)blockIdx.x >= whole;
+  const int entry = blockIdx.x - (cut ? whole : 0), entries = cut ? p.T / p.SEG + p.B : p.B;
+  const int h0 = entry / entries * HW, hw = wave / VW, h = h0 + hw;
+  int b = entry % entries, r0, r1;
+  if (cut) {
+    b = locate(p, b, p.SEG, r0, r1);
   } else {
     r0 = p.q_start[b];
     r1 = p.q_start[b + 1];
   }
   if (r1 <= r0) return;
   const int first = p.q_start[b];
+  if (SEGM && walked_whole(p, p.q_start[b + 1] - first) == cut) return;
+  const size_t seg = cut ? seg_base(p, b) + (r0 - first) / p.SEG : 0;
   const int slot = p.seq_slot[first];
   if (!live_slot(p, slot)) return;
   const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
@@ -311,10 +348,10 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     }
   }
   // entry (row, column) of the state: the scan keeps [N, V], the retention [V, N]
-  float* sp = (SEGM ? p.seg + ((size_t)blockIdx.x * p.H + h) * N * V
-                    : p.state + ((size_t)slot * p.H + h) * N * V);
+  float* sp = cut ? p.seg + (seg * p.H + h) * N * V
+                  : p.state + ((size_t)slot * p.H + h) * N * V;
   f32x16 S[NT];
-  const bool load = FULL && (SEGM || p.positions[first] != 0);
+  const bool load = FULL && (cut || p.positions[first] != 0);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -553,7 +590,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll 1
   for (int c = 0; c < chunks; ++c) step(c, buf[c & 1], buf[(c + 1) & 1]);
   if (FULL) write(chunks - 1);
-  if (FULL && SEGM) return;  // the slots were written when the segments were joined
+  if (FULL && cut) return;   // the slots were written when the segments were joined
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -567,9 +604,8 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
                                                              S[t][4 * g + 2], S[t][4 * g + 3]);
       }
     }
-  if (SEGM && lane == 0 && wave % VW == 0)
-    p.seg_decay[(size_t)blockIdx.x * p.H + h] =
-        MODE == 0 ? exp2f(total) : decay_pow(l2, r1 - r0);
+  if (SEGM && !FULL && lane == 0 && wave % VW == 0)
+    p.seg_decay[seg * p.H + h] = MODE == 0 ? exp2f(total) : decay_pow(l2, r1 - r0);
 }
 
 // the state before each segment from the segments' own states, and the sequence's final state
@@ -579,11 +615,11 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
   const size_t hs = (size_t)p.V * p.N;
   const size_t e = ((size_t)blockIdx.z * 256 + threadIdx.x) * 4;
   const int r0 = p.q_start[b], r1 = p.q_start[b + 1];
-  if (r1 <= r0 || e >= hs) return;
+  if (r1 <= r0 || walked_whole(p, r1 - r0) || e >= hs) return;
   const int slot = p.seq_slot[r0];
   if (!live_slot(p, slot)) return;
   const int nseg = (r1 - r0 + p.SEG - 1) / p.SEG;
-  const size_t sb = base_of(p.q_start, b, p.SEG);
+  const size_t sb = seg_base(p, b);
   float4* st = (float4*)(p.state + ((size_t)slot * p.H + h) * hs + e);
   float4 prev = p.positions[r0] != 0 ? *st : make_float4(0.f, 0.f, 0.f, 0.f);
   for (int s0 = 0; s0 < nseg; s0 += 8) {
@@ -616,13 +652,13 @@ void run(const ChunkScanParams& p, hipStream_t s) {
     chunk_scalar_kernel<TY><<<dim3(chunks, (p.H + 31) / 32), 256, 0, s>>>(p);
   constexpr int nt = 2 * V * HW;
   if (p.SEG == 0) {
-    chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<dim3(p.B, p.H / HW), nt, 0, s>>>(p);
+    chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
     return;
   }
   const int segs = p.T / p.SEG + p.B;
-  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<dim3(segs, p.H / HW), nt, 0, s>>>(p);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<segs * (p.H / HW), nt, 0, s>>>(p);
   chunk_join_kernel<<<dim3(p.B, p.H, (p.V * p.N + 1023) / 1024), 256, 0, s>>>(p);
-  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<dim3(segs, p.H / HW), nt, 0, s>>>(p);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<(p.B + segs) * (p.H / HW), nt, 0, s>>>(p);
 }
 
 // two heads of 64 columns that share their keys go through one workgroup: the keys' fragments
@@ -646,13 +682,22 @@ bool chunk_scan_sizes(int V, int N) {
   return (V == 64 || V == 128) && (N == 64 || N == 128);
 }
 
-int chunk_scan_segment(int T, int B, int H, int V) {
-  // A step with fewer (sequence, head, 32 columns) triples than most SIMDs of the chip is cut into
-  // segments, if a sequence of it may be longer than one (only the rows of all are known here):
-  // the second pass over the keys costs less than idle SIMDs.  8 x 2048 rows, 8 heads x 128 x 128
-  // (256 waves otherwise): 285 us in segments; 64 heads x 128 x 64 (1024 waves): 475 us whole.
-  if ((int64_t)B * H * (V / 32) >= 768) return 0;
-  return T >= 1024 || T >= 384 * (int64_t)B ? 256 : 0;
+int chunk_scan_segment(int mode, int T, int B, int H, int V) {
+  // Only the rows of all sequences are known here; which are long enough to be cut, and whether they
+  // are, walked_whole() says.  Below kFill waves in all, long ones are cut.  Above, a step may be one
+  // long prompt beside many short sequences or running rows (8 heads x 128 x 128: 64 rows and a prompt
+  // of 2048 178 us in segments, 433 whole; 23 prompts of 100 and one of 5000 186, 998); where nothing
+  // is cut, the two launches more take 5 us (24 prompts of 600: 187 -> 193; 40 of 900: 467 -> 476).  The
+  // scan, whose many heads fill the chip with a few prompts, takes them only where the mean length
+  // says that most sequences are short (64 heads x 128 x 64, 64 rows and a prompt of 2048: 263 us, 441
+  // whole).
+  const bool full = (int64_t)B * H * (V / 32) >= kFill;
+  if (!full) return T >= 1024 || T >= 384 * (int64_t)B ? 256 : 0;
+  return T - B >= 1024 && (mode == 1 || T < 256 * (int64_t)B) ? 256 : 0;
+}
+
+int64_t chunk_scan_segments(int T, int B, int SEG) {
+  return few_long(T, B, SEG) ? 2 * (int64_t)T / SEG + 2 : (int64_t)T / SEG + B;
 }
 
 void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s) {

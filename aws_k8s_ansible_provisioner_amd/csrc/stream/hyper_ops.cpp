@@ -196,7 +196,8 @@ void selective_scan(Tensor y, Tensor xbc, Tensor proj, int64_t dt_off, Tensor dt
   // Prompt chunks in matrix form.  A chunk costs the same for one row as for 32, so steps of short
   // portions stay with the scan: with convolution and norm, 64 heads x 64 x 128, 4 portions of 8
   // rows take 43 us in the scan and 47 here, of 16 rows 48 and 47, of 32 rows 58 and 46 (64
-  // portions: 87 / 101, 118 / 104, 189 / 119).
+  // portions: 87 / 101, 118 / 104, 189 / 119).  The mean length decides: a prompt beside more running
+  // rows than a sixteenth of the step stays with the scan too.
   if (sa.q_start != nullptr && sa.B > 0 && T >= 16 * (int64_t)sa.B &&
       akap_stream::chunk_scan_sizes((int)V, (int)N) && (uintptr_t)xbc.data_ptr() % 16 == 0 &&
       (uintptr_t)y.data_ptr() % 16 == 0) {
@@ -212,10 +213,10 @@ void selective_scan(Tensor y, Tensor xbc, Tensor proj, int64_t dt_off, Tensor dt
     const Tensor frag = at::empty({chunks * p.KH * p.frag_floats}, opt);
     const Tensor scal = at::empty({chunks * p.H * 256}, opt);
     p.frag = frag.data_ptr<float>(); p.scal = scal.data_ptr<float>();
-    p.SEG = akap_stream::chunk_scan_segment(p.T, p.B, p.H, p.V);
+    p.SEG = akap_stream::chunk_scan_segment(p.mode, p.T, p.B, p.H, p.V);
     Tensor seg, dec;
     if (p.SEG > 0) {
-      const int64_t segs = p.T / p.SEG + p.B;
+      const int64_t segs = akap_stream::chunk_scan_segments(p.T, p.B, p.SEG);
       seg = at::empty({segs * p.H * p.N * p.V}, opt);
       dec = at::empty({segs * p.H}, opt);
       p.seg = seg.data_ptr<float>(); p.seg_decay = dec.data_ptr<float>();
@@ -434,6 +435,11 @@ void pooled_window_attention_prefill_mfma(Tensor out, Tensor q, Tensor k_cache, 
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(akap_stream, m) {
+  // rows per segment of a step of the selective scan (mode 0) or the retention (1), 0: none
+  m.def("chunk_scan_segment(int mode, int T, int B, int H, int V) -> int",
+        [](int64_t mode, int64_t T, int64_t B, int64_t H, int64_t V) -> int64_t {
+          return akap_stream::chunk_scan_segment((int)mode, (int)T, (int)B, (int)H, (int)V);
+        });
   m.def("hyper_step(Tensor(a!) out, Tensor(b!) xs, Tensor? ya, Tensor? yb, Tensor? bias, "
         "Tensor? mix, Tensor? w_out, Tensor w_in, Tensor norm_w, float eps, Tensor? fresh=None) "
         "-> ()");

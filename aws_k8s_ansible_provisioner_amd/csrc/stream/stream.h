@@ -268,7 +268,8 @@ struct ChunkScanParams {
   float* frag;
   int frag_floats;
   float* scal;
-  // segments of SEG rows (0: none), T / SEG + B of them: states [segs, H, N V], decays [segs, H]
+  // sequences of more than SEG rows (0: none) in segments: chunk_scan_segments() states [H, N V] and
+  // decays [H]
   float* seg;
   float* seg_decay;
   int SEG;
@@ -289,8 +290,10 @@ struct ChunkScanParams {
   float eps;
 };
 bool chunk_scan_sizes(int V, int N);
-// rows per segment of a step, 0: the sequences are walked whole
-int chunk_scan_segment(int T, int B, int H, int V);
+// rows per segment of a step, 0: every sequence is walked whole
+int chunk_scan_segment(int mode, int T, int B, int H, int V);
+// segments that the long sequences of a step can have
+int64_t chunk_scan_segments(int T, int B, int SEG);
 void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s);
 
 struct TalkParams {

@@ -835,7 +835,8 @@ void retention(Tensor out, Tensor proj, int64_t q_off, int64_t k_off, int64_t v_
   const c10::DeviceGuard g(proj.device());
   // Prompt chunks in matrix form; steps of short portions stay with the row form, as a chunk costs
   // the same for one row as for 32: 8 heads x 128 x 128, 4 portions of 8 rows take 14 us by rows
-  // and 16 here, of 16 rows 21 and 16, of 32 rows 38 and 17.  Rows are read four entries at a time.
+  // and 16 here, of 16 rows 21 and 16, of 32 rows 38 and 17.  (The mean length decides, as only that
+  // is known here.)  Rows are read four entries at a time.
   if (p.q_start != nullptr && p.num_seqs > 0 && T >= 16 * (int64_t)p.num_seqs &&
       akap_stream::chunk_scan_sizes((int)V, (int)D) && p.rot_dims % 8 == 0 &&
       ((p.proj_stride | p.q_off | p.k_off | p.g_off | p.out_stride) & 3) == 0 &&
@@ -851,10 +852,10 @@ void retention(Tensor out, Tensor proj, int64_t q_off, int64_t k_off, int64_t v_
     const auto opt = state.options();
     const Tensor frag = at::empty({(T / 32 + c.B) * H * c.frag_floats}, opt);
     c.frag = frag.data_ptr<float>();
-    c.SEG = akap_stream::chunk_scan_segment(c.T, c.B, c.H, c.V);
+    c.SEG = akap_stream::chunk_scan_segment(c.mode, c.T, c.B, c.H, c.V);
     Tensor sg, dec;
     if (c.SEG > 0) {
-      const int64_t segs = T / c.SEG + c.B;
+      const int64_t segs = akap_stream::chunk_scan_segments(c.T, c.B, c.SEG);
       sg = at::empty({segs * H * V * D}, opt);
       dec = at::empty({segs * H}, opt);
       c.seg = sg.data_ptr<float>(); c.seg_decay = dec.data_ptr<float>();

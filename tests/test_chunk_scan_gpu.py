@@ -1,7 +1,7 @@
 """Prompt chunks of the selective scan and the retention in fp32 matrix form (GPU) against the same
 ops on CPU tensors: sequences around the chunk size of 32 rows and the segment size of 256, several
-sequences per step (some continued from their slots, one a padding sequence), every head size of
-the matrix form, projections that are column slices of wider rows, and values that are not finite.
+sequences per step (some continued from their slots, one a padding sequence), steps whose long
+sequences are cut into segments and such that are walked whole, every head size of the matrix form, projections that are column slices of wider rows, and values that are not finite.
 
 Tolerance: both sides sum at most N + 32 products per entry in fp32 in different orders; the
 relative 2-norm error of such sums is a few times 2^-24, 2e-6 leaves a factor of ten."""
@@ -73,6 +73,33 @@ def test_selective_scan_chunks(lens, starts, H, V, N, G, dt):
                        inp[5][[b for b, s in enumerate(starts) if s < 0]])
 
 
+# lens, starts, heads of the scan and of the retention (V 64): two cut sequences of five, one continued, a
+# padding sequence; one long continued one; a prompt among rows of one token (whose number alone would
+# fill the chip); as many long sequences as fill it, so that none is cut
+CUT = [([700, 600, 1, 3, 257], [0, 10, 0, -1, 4], 4, 4), ([1100], [9], 4, 4),
+       ([1] * 50 + [1100] + [1] * 10 + [300], [7] * 50 + [0] + [5] * 10 + [40], 8, 8),
+       ([300] * 24 + [1] * 10, [0, 3] * 12 + [9] * 10, 16, 16)]
+
+
+@pytest.mark.parametrize("lens,starts,H,_", CUT)
+def test_selective_scan_segments(lens, starts, H, _):
+    V, N, G = 64, 64, 2
+    T, B = sum(lens), len(lens)
+    assert torch.ops.akap_stream.chunk_scan_segment(0, T, B, H, V) == 256
+    step = _step(lens, starts)
+    inp = _scan_inputs(T, B, H, V, N, G, torch.bfloat16, 0, seed=T)
+    want = _run_scan(inp, step, H, V, N, G, "cpu")
+    got = _run_scan(inp, step, H, V, N, G, DEV)
+    live = step[2] >= 0
+    assert _rel(got[0][live.to(DEV)], want[0][live]) < 2e-6
+    assert _rel(got[1], want[1]) < 2e-6
+    for b in range(B):                     # (each sequence for itself: a lost one is small beside the rest)
+        if starts[b] >= 0:
+            assert _rel(got[1][b], want[1][b]) < 1e-5
+        else:
+            assert torch.equal(got[1][b].cpu(), inp[5][b])
+
+
 def _run_retention(inp, step, H, D, V, offs, cs, l2, dev):
     proj, state = inp
     q_start, pos, slot = (t.to(dev) for t in step)
@@ -106,6 +133,27 @@ def test_retention_chunks(lens, starts, H, D, V, rot, dt):
     assert _rel(got[0][live.to(DEV)].float(), want[0][live].float()) < (6e-3 if dt == torch.bfloat16
                                                                         else 4e-6)
     assert _rel(got[1], want[1]) < 2e-6
+
+
+@pytest.mark.parametrize("lens,starts,_,H", CUT)
+def test_retention_segments(lens, starts, _, H):
+    D = V = 64
+    T, B = sum(lens), len(lens)
+    assert torch.ops.akap_stream.chunk_scan_segment(1, T, B, H, V) == 256
+    step = _step(lens, starts)
+    g = torch.Generator().manual_seed(T)
+    proj, state = torch.randn(T, 4 * H * V, generator=g), torch.randn(B, H, V, D, generator=g)
+    args = (step, H, D, V, (0, H * D, 2 * H * D, 3 * H * D), None,
+            torch.log2(torch.linspace(0.9, 0.999, H)))
+    want = _run_retention((proj, state), *args, "cpu")
+    got = _run_retention((proj, state), *args, DEV)
+    live = step[2] >= 0
+    assert _rel(got[0][live.to(DEV)], want[0][live]) < 4e-6
+    for b in range(B):
+        if starts[b] >= 0:
+            assert _rel(got[1][b], want[1][b]) < 1e-5
+        else:
+            assert torch.equal(got[1][b].cpu(), state[b])
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
