@@ -155,9 +155,12 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 template <int MODE, int NT, typename TY>
 __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
-  __shared__ __align__(16) float qs[kL * LS > 4096 ? kL * LS : 4096];
-  __shared__ __align__(16) float ks[kL * LS];
-  float* red = qs;   // the waves' shares of the products, once every wave has read q
+  // q and k, then (once every wave has read them) the waves' shares of the products
+  using TR = typename std::conditional<MODE == 0, double, float>::type;
+  constexpr int kRed = 4096 * sizeof(TR) / 4;
+  __shared__ __align__(16) float rows[2 * kL * LS > kRed ? 2 * kL * LS : kRed];
+  float *qs = rows, *ks = rows + kL * LS;
+  TR* red = (TR*)rows;
   const int entry = blockIdx.x, kh = blockIdx.y;
   int r0, r1;
   const int b = locate(p, entry, kL, r0, r1);
@@ -226,31 +229,40 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
     out[(NT * 4 + f) * 64 + lane] = make_float4(kk[0], kk[LS], kk[2 * LS], kk[3 * LS]);
   }
   // q . k with the keys as rows: lane (i, hh) register 4 g + r is q_i . k_(8 g + 4 hh + r), the
-  // operand the walk needs; the waves contract a part of the entries each
-  f32x16 acc;
+  // operand the walk needs; the waves contract a part of the entries each.  The scan's in four chains
+  // that meet in fp64: the products have mostly one sign, and the error of one long fp32 sum of them
+  // was most of the outputs' (8.7e-8 against 64 bits, row by row 7.4e-8, so 7.0e-8)
+  constexpr int NC = MODE == 0 ? 4 : 1;
+  f32x16 acc[NC];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[n][i] = 0.f;
   for (int f = wave; f < NT * 4; f += 4) {
     const float4 a = *(const float4*)(ks + li * LS + 8 * f + 4 * hh);
     const float4 c = *(const float4*)(qs + li * LS + 8 * f + 4 * hh);
-    acc = mfma(a.x, c.x, acc);
-    acc = mfma(a.y, c.y, acc);
-    acc = mfma(a.z, c.z, acc);
-    acc = mfma(a.w, c.w, acc);
+    acc[0] = mfma(a.x, c.x, acc[0]);
+    acc[1 % NC] = mfma(a.y, c.y, acc[1 % NC]);
+    acc[2 % NC] = mfma(a.z, c.z, acc[2 % NC]);
+    acc[3 % NC] = mfma(a.w, c.w, acc[3 % NC]);
   }
   __syncthreads();
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
-    *(float4*)(red + wave * 1024 + (g * 64 + lane) * 4) =
-        make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
-  __syncthreads();
-  float4 s = *(const float4*)(red + tid * 4);
+  for (int i = 0; i < 16; ++i) {
+    TR sum = acc[0][i];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) {
-    const float4 t = *(const float4*)(red + w * 1024 + tid * 4);
-    s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+    for (int n = 1; n < NC; ++n) sum += acc[n][i];
+    red[wave * 1024 + ((i >> 2) * 64 + lane) * 4 + (i & 3)] = sum;
   }
-  out[NT * 8 * 64 + tid] = s;
+  __syncthreads();
+  TR s[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s[r] = red[tid * 4 + r];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) s[r] += red[w * 1024 + tid * 4 + r];
+  }
+  out[NT * 8 * 64 + tid] = make_float4((float)s[0], (float)s[1], (float)s[2], (float)s[3]);
 }
 
 // ------------------------------------------------------------------ step sizes and decays
