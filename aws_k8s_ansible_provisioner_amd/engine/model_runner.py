@@ -220,6 +220,8 @@ class ModelRunner:
         d = self.mcfg.hidden_size
         width = d * 4 + (self.model.hq + 2 * self.model.hkv) * self.model.D + 3 * self.model.ffn
         act = self.cap_tokens * width * 2 * 3 + self.max_seqs * self.mcfg.vocab_size * 12
+        if hasattr(self.model, "step_scratch_bytes"):   # buffers that grow with the step's rows
+            act += self.model.step_scratch_bytes(self.cap_tokens, self.max_seqs)
         reserve = act + 3 * 2**30
         budget = min(total * self.ecfg.gpu_memory_utilization - used, free) - reserve
         n = int(budget // per_block)

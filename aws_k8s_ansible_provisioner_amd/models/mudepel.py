@@ -343,6 +343,12 @@ class MudepelLM:
             vs.append(segs[j + 1] if j is not None else None)
         return ks, vs
 
+    def step_scratch_bytes(self, rows: int, seqs: int) -> int:
+        """Most that a state-space layer's scan allocates for itself in a step of that size."""
+        ms = [s.mixer for s in self.cfg.layer_specs if isinstance(s.mixer, StateSpaceSpec)]
+        return max((sops.recurrence_scratch_bytes(rows, seqs, m.heads, m.groups, m.vdim, m.state, True)
+                    for m in ms), default=0)
+
     def allocate_state(self, num_slots: int) -> None:
         """Per state-space layer run and sequence slot: the last taps - 1 convolution inputs
         [slots, taps - 1, C] (activation type) and the states [slots, H, N, V] (fp32)."""

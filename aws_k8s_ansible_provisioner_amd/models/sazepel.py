@@ -322,6 +322,12 @@ class SazepelLM:
             self.state.append(torch.zeros(max(1, num_slots), r.heads, r.vdim, r.dim,
                                           dtype=torch.float32, device=self.device))
 
+    def step_scratch_bytes(self, rows: int, seqs: int) -> int:
+        """Most that a layer's recurrence allocates for itself in a step of that size."""
+        specs = [self._parts(s)[1] for s in self.cfg.layer_specs]
+        return max(sops.recurrence_scratch_bytes(rows, seqs, r.heads, r.heads, r.vdim, r.dim, False)
+                   for r in specs)
+
     def state_bytes_per_slot(self) -> int:
         return sum(4 * self._parts(self.cfg.layer_specs[i])[1].state_floats for i in self.runs)
 

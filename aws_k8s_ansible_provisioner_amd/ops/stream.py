@@ -868,6 +868,24 @@ RETENTION_SEGMENTED_ROWS = 1024
 RETENTION_SEGMENT = 256
 
 
+def recurrence_scratch_bytes(rows: int, seqs: int, heads: int, key_heads: int, value: int, key: int,
+                             scan: bool) -> int:
+    """Upper bound of what one call of retention (or, scan, selective_scan) with up to `rows` rows of
+    up to `seqs` sequences allocates beside its arguments: the buffers of the matrix form
+    (csrc/stream/chunk_scan.hip: operand fragments and scalars per chunk of 32 rows, which take
+    steps of 16 rows a sequence and more, and states per segment of 256), and of the retention's
+    row form in segments."""
+    n = 0
+    if value in (64, 128) and key in (64, 128):
+        s = max(1, min(seqs, rows // 16))
+        n = (rows // 32 + s) * (key_heads * (64 * key + 1024) + (heads * 256 if scan else 0))
+        n += max(2 * rows // 256 + 2, rows // 256 + min(s, 768 * 32 // (heads * value) + 1)) \
+            * heads * (value * key + 1)
+    if not scan and rows >= RETENTION_SEGMENTED_ROWS:
+        n = max(n, (rows // RETENTION_SEGMENT + seqs) * heads * value * key)
+    return 4 * n
+
+
 def retention(out: torch.Tensor, proj: torch.Tensor, q_off: int, k_off: int, v_off: int,
               g_off: int, state: torch.Tensor, seq_slot: torch.Tensor, positions: torch.Tensor,
               q_start: Optional[torch.Tensor], cos_sin: Optional[torch.Tensor],

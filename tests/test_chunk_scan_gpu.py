@@ -222,3 +222,31 @@ def test_scan_output_error():
         want.append((q[t] @ S).view(-1))
     assert _rel(y, torch.stack(want)) < 1.02e-7
     assert _rel(state[0], S) < 1e-7
+
+
+@pytest.mark.parametrize("lens", [[700], [64] * 8, [2100], [300] * 5, [1] * 60 + [1500], [1] * 150 + [1600],
+                                  [16] * 40])
+@pytest.mark.parametrize("H,KH", [(8, 1), (64, 8)])
+def test_scratch_stays_below_what_the_cache_leaves(lens, H, KH):
+    """What a call asks the allocator for is within the bound that the cache's size leaves room for, and a
+    matrix-form step takes more than an eighth of that (segments or not)."""
+    V, N, T, B = 64, 64, sum(lens), len(lens)
+    q_start, pos, slot = (t.to(DEV) for t in _step(lens, [0] * B))
+    xbc, proj = torch.zeros(T, H * V + 2 * KH * N, device=DEV), torch.zeros(T, 4 * H * V, device=DEV)
+    state, one, y = torch.zeros(B, H, V, N, device=DEV), torch.ones(H, device=DEV), torch.empty(T, H * V, device=DEV)
+
+    def took(f):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_stats()["requested_bytes.all.current"]
+        f()
+        return torch.cuda.memory_stats()["requested_bytes.all.peak"] - before
+
+    n = took(lambda: sops.selective_scan(y, xbc, proj, 0, one, one, one, state, slot, pos, q_start, H, V,
+                                         N, KH))
+    most = sops.recurrence_scratch_bytes(T, B, H, KH, V, N, True)
+    assert n <= most and (T < 16 * B or n > most / 8)
+    n = took(lambda: sops.retention(y, proj, 0, H * V, 2 * H * V, 3 * H * V, state, slot, pos, q_start,
+                                    None, -one, H, N, V, 1e-5))
+    most = sops.recurrence_scratch_bytes(T, B, H, H, V, N, False)
+    assert n <= most and (T < 16 * B or n > most / 8)
