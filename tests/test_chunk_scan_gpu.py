@@ -246,7 +246,8 @@ def test_scratch_stays_below_what_the_cache_leaves(lens, H, KH):
                                          N, KH))
     most = sops.recurrence_scratch_bytes(T, B, H, KH, V, N, True)
     assert n <= most and (T < 16 * B or n > most / 8)
+    decay = -one
     n = took(lambda: sops.retention(y, proj, 0, H * V, 2 * H * V, 3 * H * V, state, slot, pos, q_start,
-                                    None, -one, H, N, V, 1e-5))
+                                    None, decay, H, N, V, 1e-5))
     most = sops.recurrence_scratch_bytes(T, B, H, H, V, N, False)
     assert n <= most and (T < 16 * B or n > most / 8)
