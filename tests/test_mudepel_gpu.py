@@ -79,7 +79,9 @@ def test_softcap_and_gated_act_kernels(dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("n,groups", [(48, 3), (512, 1), (640, 5), (4096, 8)])
+# (up to 2048, 4096 and 8192 entries of a part in registers, the last pieces partly filled; then element by element)
+@pytest.mark.parametrize("n,groups", [(48, 3), (512, 1), (640, 5), (4096, 8), (4096, 1), (5128, 1), (8192, 1),
+                                      (8200, 1)])
 def test_gate_group_norm_kernel(dtype, n, groups):
     g, dt = gen(n), DT[dtype]
     T = 6
