@@ -4,8 +4,9 @@
 // write every entry in eight parts from eight workgroups, on eight XCDs with an L2 each.  Here a
 // thread takes 8 dimensions of `vrows` neighbouring rows (8; 1 for small steps, whose rows are mostly
 // sequences of their own): 8 rows that fill one group are transposed in registers and leave as whole
-// entries, wherever among the rows the group begins (sequences of ragged steps begin at any row);
-// rows of a group that is not whole are written element by element.
+// entries, at whichever of a thread's rows the group begins.  Where it begins is told by the slot of the
+// first of the 8 rows, so the first group of a sequence that begins among them is written element by
+// element, by two threads (its later groups leave whole), as are rows of a group that is not whole.
 #pragma once
 
 #include "../kernels/common.h"
