@@ -23,7 +23,7 @@
 // heads of 128, causal: 200 us (0.69 PFLOP/s; fragments straight from the caches took 331), 5 prompts
 // of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 165 us (553).  Tried for the
 // pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
-// more, the step's body twice 170 us more (spills).
+// more, the step's body twice 170 us more (spills); roots and squares cost 4.
 #include <type_traits>
 
 #include "../kernels/common.h"
@@ -162,10 +162,14 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   }
   const float sc2 = p.scale * kLog2e;
   // The maximum in log2 units of the scaled scores; POOL: of the scores themselves, so that the
-  // difference is exact however large they are, with all weights (the sink's too) times 2^8, so that
-  // what the exponential gives (nothing below 2^-126) holds every weight that a bf16 can hold
+  // difference is exact however large they are, and a weight is the square of its root, as the
+  // exponential gives nothing below 2^-126 where a bf16 holds weights down to 2^-133
+  auto weight = [&](float below) {
+    const float root = __builtin_amdgcn_exp2f(below * (0.5f * sc2));
+    return root * root;
+  };
   float m_run = p.unit_sink ? 0.f : kLowest;
-  float l_run = p.unit_sink && hf == 0 ? (POOL ? 256.f : 1.f) : 0.f;   // (a lane's own keys; the halves meet at the end)
+  float l_run = p.unit_sink && hf == 0 ? 1.f : 0.f;   // (a lane's own keys; the halves meet at the end)
   f32x16 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -226,13 +230,13 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
       float sum[2] = {0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const float e = __builtin_amdgcn_exp2f(POOL ? fmaf(s[k][i] - m_new, sc2, 8.f)
-                                                    : fmaf(s[k][i], sc2, -m_new));
+        const float e = POOL ? weight(s[k][i] - m_new)
+                             : __builtin_amdgcn_exp2f(fmaf(s[k][i], sc2, -m_new));
         s[k][i] = e;
         sum[i & 1] += e;
       }
       if (__any(m_new != m_run)) {
-        const float alpha = __builtin_amdgcn_exp2f(POOL ? (m_run - m_new) * sc2 : m_run - m_new);
+        const float alpha = POOL ? weight(m_run - m_new) : __builtin_amdgcn_exp2f(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int d = 0; d < DT; ++d)
