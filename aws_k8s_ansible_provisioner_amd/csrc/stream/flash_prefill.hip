@@ -21,7 +21,7 @@
 // Bound by the vector work of the softmax beside the products (about 3400 cycles of exponentials,
 // maxima, roundings and rescaling per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4
 // heads of 128, causal: 200 us (0.69 PFLOP/s; fragments straight from the caches took 331), 5 prompts
-// of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 165 us (553).  Tried for the
+// of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 172 us (553).  Tried for the
 // pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
 // more, the step's body twice 170 us more (spills); roots and squares cost 4.
 #include <type_traits>

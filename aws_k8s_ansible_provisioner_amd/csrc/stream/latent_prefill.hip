@@ -11,7 +11,7 @@
 //
 // Bound by what a wave issues in order: a step's rows and groups are 138 KB, 2200 cycles of a CU's
 // load path, its products 2176 cycles of a SIMD; the step takes about 3600, and a workgroup 5 us to
-// start.  5 prompts of up to 2047 tokens (odd lengths), 16 heads: 298 us, 0.78 PFLOP/s; four waves on
+// start.  5 prompts of up to 2047 tokens (odd lengths), 16 heads: 296 us, 0.78 PFLOP/s; four waves on
 // one head's 32 queries with every fragment from the caches took 650.  One wave per head's whole
 // output (512 registers) spilled (1509 us); workgroups that take several units in turn lost more to
 // their imbalance than they gained at their start (388); either role at a higher wave priority 350.

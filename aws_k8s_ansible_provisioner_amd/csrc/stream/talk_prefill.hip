@@ -65,7 +65,7 @@ __device__ __forceinline__ size_t ws_at(const TalkParams& p, int t, int g, int e
 //
 // Bound by the chain of a step (score products, maximum, barrier, exponentials, barrier: half of the time
 // alone) beside the products (116 us of the matrix units' time): 8 chunks of 1000 tokens behind 1000
-// cached, 16 / 4 heads of 128 360 us; 64 queries per workgroup with every fragment from the caches
+// cached, 16 / 4 heads of 128 352 us; 64 queries per workgroup with every fragment from the caches
 // took 919.  Opposite order of matrix and vector work in a SIMD's two waves gained nothing (24 us
 // more).  A query tile's own end costs 8 us of them (a branch per tile; by pairs of tiles or by 16 keys
 // the same; a second body without branches spills).
