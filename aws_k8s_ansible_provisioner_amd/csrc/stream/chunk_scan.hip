@@ -145,6 +145,13 @@ __device__ __forceinline__ size_t seg_base(const ChunkScanParams& p, int b) {
                                    : (size_t)base_of(p.q_start, b, p.SEG);
 }
 
+// does a sequence whose first row is t go on from its slot's state?  (The scan's row form starts anew
+// at positions below 0 too.)
+__device__ __forceinline__ bool goes_on(const ChunkScanParams& p, int t) {
+  const int64_t pos = p.positions[t];
+  return p.mode == 0 ? pos > 0 : pos != 0;
+}
+
 __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
   return slot >= 0 && slot < p.num_slots;
 }
@@ -363,7 +370,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   float* sp = cut ? p.seg + (seg * p.H + h) * N * V
                   : p.state + ((size_t)slot * p.H + h) * N * V;
   f32x16 S[NT];
-  const bool load = FULL && (cut || p.positions[first] != 0);
+  const bool load = FULL && (cut || goes_on(p, first));
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -633,7 +640,7 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
   const int nseg = (r1 - r0 + p.SEG - 1) / p.SEG;
   const size_t sb = seg_base(p, b);
   float4* st = (float4*)(p.state + ((size_t)slot * p.H + h) * hs + e);
-  float4 prev = p.positions[r0] != 0 ? *st : make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 prev = goes_on(p, r0) ? *st : make_float4(0.f, 0.f, 0.f, 0.f);
   for (int s0 = 0; s0 < nseg; s0 += 8) {
     float4 own[8];
     float dec[8];

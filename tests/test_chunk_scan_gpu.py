@@ -100,6 +100,19 @@ def test_selective_scan_segments(lens, starts, H, _):
             assert torch.equal(got[1][b].cpu(), inp[5][b])
 
 
+@pytest.mark.parametrize("lens", [[40, 33], [1100]])
+def test_selective_scan_before_position_zero(lens):
+    """A live sequence whose rows' positions are below 0 starts anew, whole and in segments, as in the
+    row form (steps of fewer than 16 rows a sequence)."""
+    H, V, N, G, B = 4, 64, 64, 2, len(lens)
+    inp = _scan_inputs(sum(lens), B, H, V, N, G, torch.bfloat16, 0, seed=sum(lens))
+    q_start, pos, slot = _step(lens, [0] * B)
+    step = (q_start, pos - 5, slot)
+    want = _run_scan(inp, step, H, V, N, G, "cpu")
+    got = _run_scan(inp, step, H, V, N, G, DEV)
+    assert _rel(got[0], want[0]) < 2e-6 and _rel(got[1], want[1]) < 2e-6
+
+
 def _run_retention(inp, step, H, D, V, offs, cs, l2, dev):
     proj, state = inp
     q_start, pos, slot = (t.to(dev) for t in step)
