@@ -2,7 +2,7 @@
 host C++ runtime (block manager, scheduler core, tokenizer) -> ``_runtime.so``.
 
 Drives ``hipcc --offload-arch=gfx950`` directly (no hipify, no torch JIT cache), so the
-built objects live next to the sources and travel with the repo snapshot to a GPU box.
+built objects live next to the sources and travel with a copy of the tree.
 
 Content-addressed, not mtime-based: every object records the SHA-256 of what it was built
 from (its source, every header, the compile command, the torch version it compiles against)

@@ -46,7 +46,7 @@ __device__ __forceinline__ float silu_bf(float g) { return bf2f(f2bf(g / (1.f + 
 // SPL: 0 whole K, 1 fp32 partial slabs for the separate reduce pass, 2 in-launch combine of
 // the S slices (plain prologue only): fragment-native sc1 slabs + a per-tile last-arriver ticket,
 // as gdgemm.hip SPL 2 -- the reduce launch (5.0 us at Qwen3 down, M = 256) and its kernel
-// boundary go away (VERDICT r5 "Step A")
+// boundary go away
 template <int PRO, int EPI, int PF, int SPL, int S = 1>
 __global__ __launch_bounds__(256, 2) void dgemm_kernel(DGemmArgs p) {
   static_assert(SPL != 2 || PRO == PRO_PLAIN, "in-launch combine: plain prologue");

@@ -10,7 +10,7 @@
 // "half-tile" is 128 rows x 64 k (16 KB: two 1-KiB DMA instructions per wave), issued in the
 // order the phases consume them, so every wait is a counted `s_waitcnt vmcnt` (never 0 in
 // steady state: cdna_hip_programming.md "Pipelining across barriers", T3+T4).
-// DEFAULT K loop (SCHED 4, "stream-first", round 6): one counted wait + one barrier per K tile,
+// DEFAULT K loop (SCHED 4, "stream-first"): one counted wait + one barrier per K tile,
 // then the whole next K tile (four half-tiles, 64 KiB) is requested at once and streams into the
 // other buffer under this tile's 64 MFMAs per wave.  A no-math probe of exactly this operand
 // stream runs as fast as hipBLASLt's whole GEMM, and the phase pipeline below measured ~stream +

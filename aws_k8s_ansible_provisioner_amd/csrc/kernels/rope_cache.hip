@@ -156,7 +156,7 @@ constexpr int V_ROWS = V_SPAN + 7;  // a run starting in the span may end 7 toke
 // (5 unconditional, index-clamped 16-byte loads per thread) and its slots (slots[t0 - 1 ..
 // t0 + V_ROWS), one per thread) land in registers, then in LDS, and the run scan reads the
 // slots from LDS.  A strided fill loop and a scan of slots[] in global memory made the role a
-// chain of ~5 + 8 dependent round trips per workgroup (round 6: 44 us per 16k-token prefill
+// chain of ~5 + 8 dependent round trips per workgroup (44 us per 16k-token prefill
 // layer in the serving trace, ~3 TB/s of K/V traffic).
 template <bool F8>
 __device__ __forceinline__ void v_span(const bf16* __restrict__ qkv, int qkv_stride,

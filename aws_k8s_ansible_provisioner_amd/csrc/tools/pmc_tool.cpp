@@ -9,7 +9,7 @@
 // kernel dispatches, so it can stay on in production, including inside hipGraph replays.
 //
 // The counter set stays inside one pass of the hardware's per-block limits (<= 8 SQ, <= 4 TCC,
-// <= 2 GRBM counters; MI355X_MICROARCH / the gpurun notes): GRBM_COUNT + GRBM_GUI_ACTIVE
+// <= 2 GRBM counters): GRBM_COUNT + GRBM_GUI_ACTIVE
 // (GPU busy), SQ_WAVES, SQ_BUSY_CYCLES, SQ_WAVE_CYCLES, SQ_VALU_MFMA_BUSY_CYCLES (matrix-core
 // busy), SQ_LDS_BANK_CONFLICT, SQ_INSTS_VALU, TCC_EA0_RDREQ_sum + TCC_EA0_WRREQ_sum (memory-side
 // read / write requests: HBM + Infinity-Cache traffic).  Counters an agent does not offer are

@@ -91,7 +91,7 @@ class ModelRunner:
         self.cap_tokens = ecfg.max_num_batched_tokens + self.max_seqs
         # prefill tile map granularity (flattened q rows per workgroup of the flash-style GPU
         # kernel; the CPU reference attention ignores the map): with the longest-first flat
-        # grid (round 6) the 8-wave 256-row tile wins on long chunks (Qwen3 4 x 4096: 284.5 vs
+        # grid the 8-wave 256-row tile wins on long chunks (Qwen3 4 x 4096: 284.5 vs
         # 301.6 us, Llama-3-8B 32 x 512: 149.2 vs 154.5, 4 x 4096: 566.3 vs 578.8, q prep in
         # the kernel), the 128-row tile on chunks whose every prompt has <= 1024 rows (Qwen3
         # 32 x 512: 83.8 vs 87.9 us) -- profiles/r6_prefill_tile_order.md.  The 256-row kernel

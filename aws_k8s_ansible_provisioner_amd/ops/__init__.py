@@ -2,7 +2,7 @@
 
 Every op dispatches on the device of its inputs:
   * GPU tensors  -> the hand-written HIP kernel in ``_C.so`` (``torch.ops.akap.*``).
-    If the extension is missing on a GPU box this RAISES -- there is no silent
+    If the extension is missing where there is a GPU this RAISES -- there is no silent
     eager fallback on the GPU path.
   * CPU tensors  -> a plain PyTorch reference of the same op (used by the CPU test
     suite, the CPU mock engine and as the numerics oracle of the GPU tests).

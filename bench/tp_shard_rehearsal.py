@@ -34,7 +34,7 @@ def stub_collectives(tp: int) -> None:
     kernels (csrc/kernels/custom_allreduce.hip) on a one-rank communicator: the same launch,
     staging, flag protocol and fused residual + next-norm epilogue, minus the peer reads over
     xGMI -- so the per-rank step includes the all-reduce kernels' own cost, not a chain of
-    Python elementwise stand-ins (which inflated round 2's number by ~6 ms at B=256)."""
+    Python elementwise stand-ins (which inflated an earlier number by ~6 ms at B=256)."""
     h = torch.ops.akap.car_create(torch.cuda.current_device(), 0, 1, 1 << 23)
     torch.ops.akap.car_link_local(h, [h])
 
