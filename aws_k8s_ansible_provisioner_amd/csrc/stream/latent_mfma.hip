@@ -226,6 +226,7 @@ __global__ __launch_bounds__(64) void latent_decode_mfma_kernel(LatentAttnParams
   per = (per + 31) & ~31;
   const int jb = part * per;
   const int je = min(pos1, jb + per - 1);
+  if (jb > je && p.num_parts > 1) return;        // (the merge reads partitions with keys alone)
   bf16* qs = reinterpret_cast<bf16*>(smem);
   LatentState<NV> st;
   init(st);
@@ -550,6 +551,7 @@ __global__ __launch_bounds__(256) void latent_decode_coop_kernel(LatentAttnParam
   per = (per + 127) & ~127;
   const int jb = part * per;
   const int je = min(pos1, jb + per - 1);
+  if (jb > je && p.num_parts > 1) return;            // (the merge reads partitions with keys alone)
   CoopState<NVW> st;
   coop_init(st);
   if (jb <= je) {                                    // (workgroup-uniform)
@@ -584,30 +586,68 @@ __global__ __launch_bounds__(256) void latent_decode_coop_kernel(LatentAttnParam
     for (int i = 0; i < 16; ++i) wo[32 * dt + 8 * (i >> 2) + 4 * hf + (i & 3)] = st.o[dt][i];
 }
 
-// grid (B, H), 128 threads: merge the partitions of one (token, head)
-__global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentAttnParams p) {
-  extern __shared__ float wts[];                     // [parts] weights of the partitions
-  const int b = blockIdx.x, h = blockIdx.y;
-  if (p.seq_lens[b] <= 0) return;                    // (workgroup-uniform)
+// grid (B, H), R / 4 threads: merge the partitions of one (token, head).  Only the partitions with keys
+// were written (whole pieces of `piece` keys).  A lane keeps a partition's weight, 16 bytes of the sums
+// of eight are in flight together: bound by the latency of those reads.  2 rows of 16 heads, 17 of 32
+// partitions with keys: 29 us with a weight and a sum at a time, now 5.
+__global__ __launch_bounds__(128) void latent_decode_merge_kernel(LatentAttnParams p, int piece) {
+  constexpr int U = 8;
+  const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int kv = p.seq_lens[b];
+  if (kv <= 0) return;                               // (workgroup-uniform)
+  int per = (kv + p.num_parts - 1) / p.num_parts;
+  per = (per + piece - 1) / piece * piece;
+  const int live = (kv + per - 1) / per;
   const size_t base = ((size_t)b * p.H + h) * p.num_parts;
+  const float* ml = p.ws_ml + base * 2;
+  const int d = threadIdx.x * 4;
+  const float* wo = p.ws_o + base * p.R + min(d, p.R - 4);
+  const bool wide = (((uintptr_t)p.ws_o & 15) | ((uintptr_t)p.out & 7)) == 0;
   float m = -INFINITY;
-  for (int i = 0; i < p.num_parts; ++i)
-    if (p.ws_ml[(base + i) * 2 + 1] > 0.f) m = fmaxf(m, p.ws_ml[(base + i) * 2]);
-  float l = 0.f;
-  for (int i = 0; i < p.num_parts; ++i) {
-    const float li = p.ws_ml[(base + i) * 2 + 1];
-    const float w = li > 0.f ? __builtin_amdgcn_exp2f(p.ws_ml[(base + i) * 2] - m) : 0.f;
-    l += li * w;
-    if (threadIdx.x == 0) wts[i] = w;
+  for (int i = lane; i < live; i += 64)
+    if (ml[i * 2 + 1] > 0.f) m = fmaxf(m, ml[i * 2]);
+  m = akap::wave_max(m);
+  float l = 0.f, a[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0; c0 < live; c0 += 64) {
+    float w = 0.f;
+    if (c0 + lane < live) {
+      const float li = ml[(c0 + lane) * 2 + 1];
+      w = li > 0.f ? __builtin_amdgcn_exp2f(ml[(c0 + lane) * 2] - m) : 0.f;
+      l += li * w;
+    }
+    const int n = min(64, live - c0);
+    for (int i = 0; i < n; i += U) {
+      float4 o[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float* src = wo + (size_t)(c0 + min(i + u, n - 1)) * p.R;
+        if (wide) o[u] = *(const float4*)src;
+        else o[u] = make_float4(src[0], src[1], src[2], src[3]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float wi = __uint_as_float(
+            __builtin_amdgcn_readlane(__float_as_uint(w), min(i + u, n - 1)));
+        if (i + u < n && wi > 0.f) {
+          a[0] = fmaf(o[u].x, wi, a[0]);
+          a[1] = fmaf(o[u].y, wi, a[1]);
+          a[2] = fmaf(o[u].z, wi, a[2]);
+          a[3] = fmaf(o[u].w, wi, a[3]);
+        }
+      }
+    }
   }
-  __syncthreads();
+  l = akap::wave_sum(l);
   const float f = l > 0.f ? 1.0f / l : 0.f;
-  bf16* o = (bf16*)p.out + ((size_t)h * p.T + b) * p.R;
-  for (int d = threadIdx.x; d < p.R; d += 128) {
-    float a = 0.f;
-    for (int i = 0; i < p.num_parts; ++i)
-      if (wts[i] > 0.f) a += p.ws_o[(base + i) * p.R + d] * wts[i];
-    o[d] = (bf16)(a * f);
+  if (d < p.R) {
+    const akap::bf16x4 v = {(bf16)(a[0] * f), (bf16)(a[1] * f), (bf16)(a[2] * f), (bf16)(a[3] * f)};
+    bf16* to = (bf16*)p.out + ((size_t)h * p.T + b) * p.R + d;
+    if (wide) {
+      *reinterpret_cast<akap::bf16x4*>(to) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[e] = v[e];
+    }
   }
 }
 
@@ -637,7 +677,7 @@ void launch_decode(const LatentAttnParams& p, hipStream_t s) {
   else
     latent_decode_mfma_kernel<NV, NKR><<<grid, 64, (size_t)32 * q_pitch(DK) * sizeof(bf16), s>>>(p);
   if (p.num_parts > 1)
-    latent_decode_merge_kernel<<<dim3(p.B, p.H), 128, p.num_parts * sizeof(float), s>>>(p);
+    latent_decode_merge_kernel<<<dim3(p.B, p.H), NV > 8 ? 128 : 64, 0, s>>>(p, NV >= 8 ? 128 : 32);
 }
 
 // ---- per-head products of small batches ------------------------------------------------------

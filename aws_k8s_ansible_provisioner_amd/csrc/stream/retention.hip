@@ -711,6 +711,7 @@ __global__ __launch_bounds__(1024) void talking_attention_kernel(TalkParams p) {
   const int per = (pieces + p.num_parts - 1) / p.num_parts;
   const int lo = part * per * TA_PIECE;
   const int hi = min(nkeys, lo + per * TA_PIECE);
+  if (lo >= hi && p.num_parts > 1) return;         // (the merge reads partitions with keys alone)
   const int rep = p.H / p.G;
   const int GV = p.G * p.Dv;
   const bool owner = tid < GV;
@@ -829,46 +830,92 @@ __global__ __launch_bounds__(1024) void talking_attention_kernel(TalkParams p) {
   }
 }
 
+// The merge: a workgroup per (row, 64 columns of the value heads' sums), a wave per quarter of the
+// heads, so that a row's partitions are read by GV / 64 workgroups with four partitions' loads in flight
+// (one workgroup per row over all columns: 140 us for 11 rows of 32 heads and 32 partitions of which
+// one holds keys, now 5).  Only partitions with keys were written, the first live_parts of them.
+__device__ __forceinline__ int live_parts(const TalkParams& p, int t) {
+  if (p.num_parts == 1) return 1;
+  const int pieces = ((int)p.positions[t] + p.piece) / p.piece;
+  const int per = (pieces + p.num_parts - 1) / p.num_parts;
+  return pieces > 0 ? (pieces + per - 1) / per : 0;
+}
+
 template <typename T, int HMAX>
-__global__ __launch_bounds__(1024) void talking_merge_kernel(TalkParams p) {
-  extern __shared__ float lds[];
-  float* wgt = lds;                  // [parts][H] weight of a partition's sums
-  float* inv_l = wgt + p.num_parts * p.H;
+__global__ __launch_bounds__(256) void talking_merge_kernel(TalkParams p) {
+  constexpr int HQ = HMAX / 4, U = 4;
+  __shared__ float sums[HMAX * 64];      // the heads' normalised sums of the columns
+  __shared__ float talk[HMAX * HMAX];
   const int t = blockIdx.x + p.row0;
   const int b = p.q_start ? find_seq(p.q_start, p.B, t) : t;
   if (p.seq_lens[b] <= 0) return;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int GV = p.G * p.Dv;
-  for (int g = tid; g < p.H; g += nt) {
-    float mx = -INFINITY;
-    for (int q = 0; q < p.num_parts; ++q)
-      mx = fmaxf(mx, p.ws_ml[(((size_t)t * p.num_parts + q) * p.H + g) * 2]);
-    float tot = 0.f;
-    for (int q = 0; q < p.num_parts; ++q) {
-      const float* ml = p.ws_ml + (((size_t)t * p.num_parts + q) * p.H + g) * 2;
-      const float w = ml[0] == -INFINITY ? 0.f : __expf(ml[0] - mx);
-      wgt[q * p.H + g] = w;
-      tot += ml[1] * w;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int GV = p.G * p.Dv, H = p.H, P = p.num_parts, live = live_parts(p, t);
+  const int col = blockIdx.y * 64 + lane, colc = min(col, GV - 1);
+  if (p.talk)
+    for (int e = tid; e < H * H; e += 256) talk[e] = p.talk[e];
+  const int g0 = wave * HQ;
+  const float* ml = p.ws_ml + ((size_t)t * P * H + g0) * 2;
+  const float* o = p.ws_o + ((size_t)t * P * H + g0) * GV + colc;
+  float mx[HQ], tot[HQ], acc[HQ];
+#pragma unroll
+  for (int i = 0; i < HQ; ++i) mx[i] = -INFINITY, tot[i] = 0.f, acc[i] = 0.f;
+  for (int q = lane; q < live; q += 64)
+#pragma unroll
+    for (int i = 0; i < HQ; ++i)
+      if (g0 + i < H) mx[i] = fmaxf(mx[i], ml[((size_t)q * H + i) * 2]);
+#pragma unroll
+  for (int i = 0; i < HQ; ++i) mx[i] = wave_max(mx[i]);
+  for (int c0 = 0; c0 < live; c0 += 64) {
+    float w[HQ];                         // a partition per lane
+#pragma unroll
+    for (int i = 0; i < HQ; ++i) {
+      w[i] = 0.f;
+      if (g0 + i < H && c0 + lane < live) {
+        const float* c = ml + ((size_t)(c0 + lane) * H + i) * 2;
+        w[i] = c[0] == -INFINITY ? 0.f : __expf(c[0] - mx[i]);
+        tot[i] += c[1] * w[i];
+      }
     }
-    inv_l[g] = 1.0f / tot;
+    const int n = min(64, live - c0);
+    for (int q0 = 0; q0 < n; q0 += U) {
+      float part[U][HQ];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < HQ; ++i)
+          part[u][i] = q0 + u < n && g0 + i < H ? o[((size_t)(c0 + q0 + u) * H + i) * GV] : 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < HQ; ++i) {
+          const float wq = __uint_as_float(
+              __builtin_amdgcn_readlane(__float_as_uint(w[i]), min(q0 + u, n - 1)));
+          acc[i] = fmaf(wq, part[u][i], acc[i]);
+        }
+    }
   }
+#pragma unroll
+  for (int i = 0; i < HQ; ++i)
+    sums[(g0 + i) * 64 + lane] = acc[i] * (1.0f / wave_sum(tot[i]));
   __syncthreads();
-  if (tid >= GV) return;
-  float acc[HMAX];
+  if (col >= GV) return;
+  const int rep = H / p.G, c = col / p.Dv, dv = col - c * p.Dv;
+  for (int i = wave; i < rep; i += 4) {
+    const int h = c * rep + i;
+    float v = 0.f;
+    if (p.talk) {
 #pragma unroll
-  for (int g = 0; g < HMAX; ++g) acc[g] = 0.f;
-  for (int q = 0; q < p.num_parts; ++q) {
-    // every partition wrote its sums (zeros when it had no keys): the loads of a partition go
-    // out together, unconditionally
-    const float* o = p.ws_o + ((size_t)t * p.num_parts + q) * p.H * GV + tid;
-    float part[HMAX];
-#pragma unroll
-    for (int g = 0; g < HMAX; ++g) part[g] = g < p.H ? o[(size_t)g * GV] : 0.f;
-#pragma unroll
-    for (int g = 0; g < HMAX; ++g)
-      if (g < p.H) acc[g] = fmaf(wgt[q * p.H + g], part[g], acc[g]);
+      for (int g = 0; g < HMAX; ++g)
+        if (g < H) v = fmaf(talk[h * H + g], sums[g * 64 + lane], v);
+    } else {
+      v = sums[h * 64 + lane];
+    }
+    const int at = h * p.Dv + dv;
+    if (p.gate) v *= sigmoidf(ldf((const T*)p.gate + (size_t)t * p.gate_stride + at));
+    stf((T*)p.out + (size_t)t * p.out_stride + at, v);
   }
-  talk_finish<T, HMAX>(p, t, tid / p.Dv, tid % p.Dv, acc, inv_l);
 }
 
 // ------------------------------------------------------------------ routing by the largest logits
@@ -1166,17 +1213,17 @@ size_t talking_attention_lds(int H, int D) {
   return (size_t)(H * D + H * TA_PIECE + 3 * H + TA_PIECE) * sizeof(float);
 }
 
-void launch_talking_attention(const TalkParams& p, bool f32, hipStream_t s) {
+void launch_talking_attention(TalkParams p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
+  p.piece = TA_PIECE;
   const int nt = ((p.G * p.Dv + 63) / 64) * 64;
   const size_t lds = talking_attention_lds(p.H, p.D);
   const int rows = p.T;
-  const dim3 grid(rows, p.num_parts);
-  const size_t mlds = (size_t)(p.num_parts + 1) * p.H * sizeof(float);
-#define AKAP_TA(TY, HM)                                                          \
-  do {                                                                           \
-    talking_attention_kernel<TY, HM><<<grid, nt, lds, s>>>(p);                   \
-    if (p.num_parts > 1) talking_merge_kernel<TY, HM><<<rows, nt, mlds, s>>>(p); \
+  const dim3 grid(rows, p.num_parts), mgrid(rows, (p.G * p.Dv + 63) / 64);
+#define AKAP_TA(TY, HM)                                                         \
+  do {                                                                          \
+    talking_attention_kernel<TY, HM><<<grid, nt, lds, s>>>(p);                  \
+    if (p.num_parts > 1) talking_merge_kernel<TY, HM><<<mgrid, 256, 0, s>>>(p); \
   } while (0)
   if (f32) {
     if (p.H <= 8) AKAP_TA(float, 8); else if (p.H <= 16) AKAP_TA(float, 16); else AKAP_TA(float, 32);
@@ -1191,9 +1238,8 @@ void launch_talking_attention(const TalkParams& p, bool f32, hipStream_t s) {
 void launch_talking_merge(const TalkParams& p, bool f32, hipStream_t s) {
   const int rows = p.T - p.row0;
   if (rows <= 0) return;
-  const int nt = ((p.G * p.Dv + 63) / 64) * 64;
-  const size_t mlds = (size_t)(p.num_parts + 1) * p.H * sizeof(float);
-#define AKAP_TM(TY, HM) talking_merge_kernel<TY, HM><<<rows, nt, mlds, s>>>(p)
+  const dim3 grid(rows, (p.G * p.Dv + 63) / 64);
+#define AKAP_TM(TY, HM) talking_merge_kernel<TY, HM><<<grid, 256, 0, s>>>(p)
   if (f32) {
     if (p.H <= 8) AKAP_TM(float, 8); else if (p.H <= 16) AKAP_TM(float, 16); else AKAP_TM(float, 32);
   } else {

@@ -312,14 +312,15 @@ struct TalkParams {
   int gate_stride;
   float scale;
   int T, B, H, G, D, Dv, BS;
-  // split form: (max, sum) [T, parts, H, 2] and unnormalised sums [T, parts, H, G Dv]
+  // split form: (max, sum) [T, parts, H, 2] and unnormalised sums [T, parts, H, G Dv] of the
+  // partitions that hold keys (whole pieces of `piece` keys, as even as they go)
   float* ws_ml;
   float* ws_o;
-  int num_parts;
+  int num_parts, piece;
   int row0;             // first row of a merge-only launch
 };
 size_t talking_attention_lds(int H, int D);
-void launch_talking_attention(const TalkParams& p, bool f32, hipStream_t s);
+void launch_talking_attention(TalkParams p, bool f32, hipStream_t s);
 void launch_talking_merge(const TalkParams& p, bool f32, hipStream_t s);
 // prompt chunks with keys staged through LDS, heads mixed and gated as well; false: not these sizes
 bool launch_talk_staged(const TalkParams& p, const int32_t* tile_seq, const int32_t* tile_row,

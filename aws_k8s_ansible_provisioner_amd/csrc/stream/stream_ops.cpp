@@ -938,7 +938,7 @@ akap_stream::TalkParams talk_params(const Tensor& out, const Tensor& q, const Te
   }
   p.scale = (float)scale;
   p.T = T; p.H = H; p.G = G; p.D = D; p.Dv = Dv; p.BS = BS;
-  p.ws_ml = nullptr; p.ws_o = nullptr; p.num_parts = 1; p.row0 = 0;
+  p.ws_ml = nullptr; p.ws_o = nullptr; p.num_parts = 1; p.piece = 128; p.row0 = 0;
   TORCH_CHECK(akap_stream::talking_attention_lds(H, D) <= 65536,
               "talking_attention: heads x head size too large for the query row in LDS");
   return p;

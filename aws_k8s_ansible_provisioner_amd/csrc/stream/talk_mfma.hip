@@ -258,6 +258,7 @@ __global__ __launch_bounds__(256) void talk_decode_mfma_kernel(TalkParams p) {
   const int per = (steps + p.num_parts - 1) / p.num_parts;
   const int lo = part * per * 128;
   const int hi = min(last + 1, lo + per * 128);    // keys [lo, hi)
+  if (lo >= hi) return;                            // (the merge reads partitions with keys alone)
   const int32_t* bt = p.block_tables + (size_t)t * p.max_blocks;
   const float sc2 = p.scale * 1.44269504088896f;
   const int DVT = p.Dv >> 5, NT = p.G * DVT;

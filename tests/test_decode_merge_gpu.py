@@ -1,0 +1,102 @@
+"""Split decode attention: partitions without keys are neither written nor read, at few and many
+partitions (past a wave's 64 lanes), whole and ragged pieces, heads and columns that do not fill a
+workgroup."""
+import pytest
+import torch
+
+from aws_k8s_ansible_provisioner_amd.ops import stream as sops
+
+pytestmark = pytest.mark.gpu
+BS = 32
+LENS = [1, 2250, 0, 333, 128, 40]
+
+
+def _table(g):
+    pages = [-(-n // BS) for n in LENS]
+    bt = torch.zeros(len(LENS), max(pages), dtype=torch.int32)
+    order, at = torch.randperm(sum(pages), generator=g).int(), 0
+    for b, n in enumerate(pages):
+        bt[b, :n] = order[at:at + n]
+        at += n
+    return bt, torch.tensor(LENS, dtype=torch.int32), sum(pages)
+
+
+def _close(got, want, dtype):
+    """bf16: weights and outputs are rounded once each, 2^-9 of a value at most; the roundings of the
+    keys are independent, so a row's error stays below 2^-8 of its norm, with half as much again for
+    the reference's own rounding."""
+    bound = 6e-3 if dtype == torch.bfloat16 else 2e-5
+    for b, n in enumerate(LENS):
+        if n:
+            err = (got[b].float().cpu() - want[b].float()).norm() / want[b].float().norm()
+            assert err < bound, (b, n, float(err))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("parts", [2, 5, 70])
+@pytest.mark.parametrize("H,G,D", [(6, 2, 64), (4, 4, 128), (3, 1, 32)])
+def test_sink_attention(dtype, parts, H, G, D):
+    g = torch.Generator().manual_seed(parts * D)
+    bt, sl, NB = _table(g)
+    q = torch.randn(len(LENS), H, D, generator=g).to(dtype)
+    kc = torch.randn(NB, G, BS, D, generator=g).to(dtype)
+    vc = torch.randn(NB, G, BS // 8, D, 8, generator=g).to(dtype)
+    gate, sink = torch.randn(len(LENS), H, generator=g).to(dtype), torch.randn(H, generator=g)
+    want = torch.zeros(len(LENS), H * D, dtype=dtype)
+    for window in (0, 600):
+        sops.sink_attention_decode(want, q, kc, vc, bt, sl, gate, sink, D ** -0.5, 0, window)
+        ws = sops.decode_workspace(len(LENS), H, D, parts, "cuda")
+        for t in ws:
+            t.fill_(float("nan"))
+        got = torch.zeros_like(want, device="cuda")
+        sops.sink_attention_decode(got, *(t.cuda() for t in (q, kc, vc, bt, sl, gate, sink)), D ** -0.5,
+                                   0, window, ws, parts)
+        _close(got, want, dtype)
+
+
+@pytest.mark.parametrize("parts", [2, 5, 70])
+@pytest.mark.parametrize("H,R,r", [(5, 512, 64), (16, 256, 32), (3, 96, 16)])
+def test_latent_attention(parts, H, R, r):
+    g = torch.Generator().manual_seed(parts * R)
+    bt, sl, NB = _table(g)
+    T, bf = len(LENS), torch.bfloat16
+    cache = torch.randn(NB, BS, R + r, generator=g).to(bf)
+    vg = cache[:, :, :R].reshape(-1, BS // 8, 8, R).transpose(2, 3).contiguous()
+    ql = (0.3 * torch.randn(H, T, R, generator=g)).to(bf)
+    q = torch.randn(T, H, r, generator=g).to(bf)
+    pos = (sl - 1).clamp(min=0).long()
+    want = torch.zeros(H, T, R, dtype=bf)
+    sops.latent_attention(want, ql, q, 0, cache, bt, sl, None, pos, (R + r) ** -0.5)
+    ws = sops.latent_decode_workspace(T, H, R, parts, "cuda")
+    for t in ws:
+        t.fill_(float("nan"))
+    got = torch.zeros_like(want, device="cuda")
+    ql, q, cache, vg, bt, sl, pos = (t.cuda() for t in (ql, q, cache, vg, bt, sl, pos))
+    sops.latent_attention_decode(got, ql, q, 0, cache, vg, bt, sl, pos, (R + r) ** -0.5, ws, parts)
+    _close(got.transpose(0, 1), want.transpose(0, 1), bf)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("parts", [2, 5, 70])
+@pytest.mark.parametrize("H,G,D,Dv", [(16, 4, 64, 128), (32, 8, 32, 64), (6, 2, 32, 96), (3, 3, 16, 32)])
+def test_talking_attention(dtype, parts, H, G, D, Dv):
+    g = torch.Generator().manual_seed(parts * Dv + H)
+    bt, sl, NB = _table(g)
+    T = len(LENS)
+    q = torch.randn(T, H, D, generator=g).to(dtype)
+    kc = torch.randn(NB, G, BS, D, generator=g).to(dtype)
+    vc = torch.randn(NB, G, BS // 8, Dv, 8, generator=g).to(dtype)
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    gate = torch.randn(T, H * Dv, generator=g).to(dtype)
+    pos = (sl - 1).clamp(min=0).long()
+    for mix in (talk, None):
+        want = torch.zeros(T, H * Dv, dtype=dtype)
+        sops.talking_attention(want, q, kc, vc, bt, sl, None, pos, mix, gate, D ** -0.5)
+        ws = sops.talking_attention_workspace(T, H, G, Dv, parts, "cuda")
+        for t in ws:
+            t.fill_(float("nan"))
+        got = torch.zeros_like(want, device="cuda")
+        dev = [t.cuda() for t in (q, kc, vc, bt, sl, pos)]
+        sops.talking_attention_decode(got, *dev, mix.cuda() if mix is not None else None, gate.cuda(),
+                                      D ** -0.5, ws, parts)
+        _close(got, want, dtype)
