@@ -157,19 +157,20 @@ __global__ __launch_bounds__(128) void pool_cache_blocks_kernel(const PoolParams
 }
 
 // The same in 16-byte pieces (bf16; pool, D and Dv multiples of 8, D / 8 a power of two up to 256,
-// aligned caches): a workgroup takes 256 rows x one key/value head, lists the rows that end a block
+// aligned caches): a workgroup takes `rows` rows (256 at most) x one key/value head, lists the rows that end a block
 // and does them in turn; keys by (token, 8 dimensions), values by (dimension, 8-token group), all of
 // a thread's loads in flight, the partial sums meet in LDS.  Bound by the latency of one round of
 // loads: the row-by-row form chained `pool` of them (43 us at 12800 rows and blocks of 64).
-__global__ __launch_bounds__(256) void pool_cache_blocks_vec_kernel(const PoolParams p) {
+__global__ __launch_bounds__(256) void pool_cache_blocks_vec_kernel(const PoolParams p,
+                                                                    const int rows) {
   __shared__ int ends[256];
   __shared__ int count;
   __shared__ float part[256 * 8];
-  const int g = blockIdx.y, tid = threadIdx.x, t0 = blockIdx.x * 256;
+  const int g = blockIdx.y, tid = threadIdx.x, t0 = blockIdx.x * rows;
   if (tid == 0) count = 0;
   __syncthreads();
   const int t = t0 + tid;
-  if (t < p.T && p.slots[t] >= 0 && ((int)p.positions[t] + 1) % p.pool == 0)
+  if (tid < rows && t < p.T && p.slots[t] >= 0 && ((int)p.positions[t] + 1) % p.pool == 0)
     ends[atomicAdd(&count, 1)] = t;
   __syncthreads();
   const int n = count, lk = p.D >> 3, tk = 256 / lk;   // lanes of a key row, rows per turn
@@ -332,11 +333,13 @@ void launch_bias_rope_cache(const RopeCacheParams& p, bool f32, hipStream_t s) {
 void launch_pool_cache_blocks(const PoolParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
   const int lk = p.D >> 3;
-  // (from 512 rows on: 256 rows to a workgroup; fewer rows, as in decode steps, a workgroup each)
-  if (!f32 && p.T >= 512 && ((p.pool | p.D | p.Dv | p.BS) & 7) == 0 && lk <= 256 &&
+  if (!f32 && ((p.pool | p.D | p.Dv | p.BS) & 7) == 0 && lk <= 256 &&
       (lk & (lk - 1)) == 0 && p.Dv <= 256 && 256 % p.Dv == 0 &&
       (((uintptr_t)p.k_cache | (uintptr_t)p.v_cache) & 15) == 0) {
-    pool_cache_blocks_vec_kernel<<<dim3((p.T + 255) / 256, p.G), 256, 0, s>>>(p);
+    // One block's end to a workgroup, mostly: in turn by 256 rows' workgroups they took 15 us at any
+    // size.  In small steps every row may end a block of its own sequence: a workgroup each.
+    const int rows = p.T < 512 ? 1 : p.pool < 64 ? 64 : p.pool < 256 ? p.pool : 256;
+    pool_cache_blocks_vec_kernel<<<dim3((p.T + rows - 1) / rows, p.G), 256, 0, s>>>(p, rows);
     return;
   }
   const int RB = p.T >= 1024 ? kPoolRows : 1;
