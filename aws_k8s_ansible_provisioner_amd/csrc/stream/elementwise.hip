@@ -365,16 +365,15 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_kernel(ProjParams p)
 // slice offsets and the row stride to be multiples of 8 elements and 16-byte aligned pointers.
 // Workgroups past the rows' write the values (write_values; vrows 0: none do, a row's own workgroup
 // writes its values), as large steps do.  Bound by memory and by a chain of latencies per workgroup
-// (row, sums, weights and angles, store): at 16384 rows of 16 / 4 heads of 128 79 us with values
-// element by element and a barrier pair per sum, 91 with the values taken out alone, 63 with both
-// sums behind one barrier and weights, angles and slot requested ahead of it.
+// (row, sums, weights and angles, store), so both sums meet behind one barrier and weights, angles and
+// slot are requested ahead of it: 232 rows of 32 / 8 heads of 128 7.8 us.
 template <typename T, int NQ>
 __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParams p, int vrows) {
   __shared__ float scratch[32];
   if ((int)blockIdx.x >= p.T) {
     write_values<T>({(const T*)p.proj + p.k_off, p.proj_stride, (T*)p.v_cache, p.slots, p.num_slots,
                      p.T, p.G, p.D, p.BS, vrows, 0.f, false, nullptr, (const T*)p.k_b},
-                    (int64_t)(blockIdx.x - p.T) * 256 + threadIdx.x);
+                    (blockIdx.x - p.T) * 256u + threadIdx.x);
     return;
   }
   const int t = blockIdx.x;
@@ -474,8 +473,9 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParam
     }
   }
   if (slot < 0 || slot >= p.num_slots) return;
-  const int64_t blk = slot / p.BS;
-  const int off = (int)(slot % p.BS);
+  size_t blk;
+  int off;
+  slot_at(slot, p.num_slots, p.BS, blk, off);
   // raw k -> V cache [NB, G, BS/8, D, 8]: the token's element of every (dimension) group.
   // Adjacent lanes take adjacent dimensions (16 bytes apart), so a wave's store covers whole
   // cache lines; the row is re-read from the projection (an L1 / L2 hit).
@@ -488,6 +488,108 @@ __global__ __launch_bounds__(256) void proj_norm_rope_cache_vec_kernel(ProjParam
   const int g = ck / p.D, d0 = ck % p.D;
   finish(k, wk, ik, ck, ck4, zk4);
   stv((T*)p.k_cache + (((size_t)blk * p.G + g) * p.BS + off) * p.D + d0, k);
+}
+
+// The same for large steps of bf16 rows whose heads divide 512 elements: a wave per token instead of a
+// workgroup, q (512 NC elements at most) and k (512 NK) of it in registers, sums and angles without
+// LDS or a barrier.  The first nv workgroups write the values (write_values).
+//
+// Bound by memory and, before, by its instructions (317 per wave and 8 elements a lane, most of them
+// divisions of indices and slots): 16384 rows of 16 / 4 heads of 128 61 us with a workgroup per token,
+// now 40 (184 MB); 5000 rows of 32 / 8 heads 33 -> 29, 1000 rows of 16 / 4 heads 11.9 -> 10.7.  Two
+// tokens to a wave 42 to 46.
+template <int NC, int NK>
+__global__ __launch_bounds__(256, 4) void proj_norm_rope_cache_wave_kernel(ProjParams p, int nv) {
+  if ((int)blockIdx.x < nv) {
+    write_values<bf16>({(const bf16*)p.proj + p.k_off, p.proj_stride, (bf16*)p.v_cache, p.slots,
+                        p.num_slots, p.T, p.G, p.D, p.BS, 8, 0.f, false, nullptr, (const bf16*)p.k_b},
+                       blockIdx.x * 256u + threadIdx.x);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int t = __builtin_amdgcn_readfirstlane((int)((blockIdx.x - nv) * 4 + (threadIdx.x >> 6)));
+  if (t >= p.T) return;
+  const int HD = p.H * p.D, GD = p.G * p.D, c0 = lane * 8;
+  const bf16* row = (const bf16*)p.proj + (size_t)t * p.proj_stride;
+  akap::bf16x8 q[NC], k[NK];
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if (512 * i + c0 < HD) q[i] = *(const akap::bf16x8*)(row + p.q_off + 512 * i + c0);
+#pragma unroll
+  for (int i = 0; i < NK; ++i)
+    if (512 * i + c0 < GD) k[i] = *(const akap::bf16x8*)(row + p.k_off + 512 * i + c0);
+  const int64_t pos = p.positions[t], slot = p.slots[t];
+  // angles of the lane's four pairs: the same in every head
+  const int rh = p.rot_dims >> 1, i0 = (c0 & (p.D - 1)) >> 1;
+  const bool rot = p.cos_sin && i0 < rh;
+  float co[4], si[4];
+  if (rot) {
+    const int64_t at = pos < 0 ? 0 : pos < p.max_pos ? pos : p.max_pos - 1;
+    ldv(co, p.cos_sin + (size_t)at * p.rot_dims + i0);
+    ldv(si, p.cos_sin + (size_t)at * p.rot_dims + rh + i0);
+  }
+  auto biased = [&](const akap::bf16x8& x, const void* bias, int c, float (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
+    if (bias) {
+      float bb[8];
+      ldv(bb, (const bf16*)bias + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += bb[e];
+    }
+  };
+  auto squares = [&](const akap::bf16x8& x, const void* bias, int c) {
+    float v[8], s = 0.f;
+    biased(x, bias, c, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += v[e] * v[e];
+    return s;
+  };
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if (512 * i + c0 < HD) sq += squares(q[i], p.q_b, 512 * i + c0);
+#pragma unroll
+  for (int i = 0; i < NK; ++i)
+    if (512 * i + c0 < GD) sk += squares(k[i], p.k_b, 512 * i + c0);
+  const float iq = 1.0f / sqrtf(akap::wave_sum_dpp(sq) / (float)HD + p.eps);
+  const float ik = 1.0f / sqrtf(akap::wave_sum_dpp(sk) / (float)GD + p.eps);
+  auto finish = [&](const akap::bf16x8& x, const void* bias, const float* weights, int c, float inv,
+                    float (&v)[8]) {
+    float w[8];
+    ldv(w, weights + c);
+    biased(x, bias, c, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = v[e] * inv * w[e];
+    if (rot) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float u = v[e] * co[e >> 1] - v[e + 1] * si[e >> 1];
+        v[e + 1] = v[e + 1] * co[e >> 1] + v[e] * si[e >> 1];
+        v[e] = u;
+      }
+    }
+  };
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = 512 * i + c0;
+    if (c >= HD) continue;
+    finish(q[i], p.q_b, p.q_w, c, iq, v);
+    stv((bf16*)p.q_out + (size_t)t * HD + c, v);
+  }
+  if (slot < 0 || slot >= p.num_slots) return;
+  size_t page;
+  int off;
+  slot_at(slot, p.num_slots, p.BS, page, off);
+#pragma unroll
+  for (int i = 0; i < NK; ++i) {
+    const int c = 512 * i + c0;
+    if (c >= GD) continue;
+    const int g = c >> (31 - __clz(p.D));
+    finish(k[i], p.k_b, p.k_w, c, ik, v);
+    stv((bf16*)p.k_cache + ((page * p.G + g) * p.BS + off) * p.D + (c & (p.D - 1)), v);
+  }
 }
 
 template <typename T>
@@ -505,6 +607,17 @@ void launch_proj_norm_rope_cache(const ProjParams& p, bool f32, hipStream_t s) {
     const bool two = p.H * p.D > 2048;
     const int vrows = p.T >= 512 && p.BS % 8 == 0 && aligned(p.v_cache, 16) ? 8 : 0;
     const int64_t vt = vrows ? value_group_threads(p.T, p.G, p.D, vrows) : 0;
+    // (from some waves per CU on: 512 rows of 32 heads 8.5 us by workgroups, 10.4 by waves; 1000 rows of 16
+    // heads 11.9 and 10.7)
+    if (!f32 && vrows && p.T >= 768 && (p.D & (p.D - 1)) == 0 && p.D <= 512 && p.G * p.D <= 1024 &&
+        (!p.cos_sin || ((p.rot_dims & 7) == 0 && aligned(p.cos_sin, 16)))) {
+      const int nv = (int)((vt + 255) / 256), nb = nv + (p.T + 3) / 4;
+      if (p.H * p.D > 2048 || p.G * p.D > 512)
+        proj_norm_rope_cache_wave_kernel<8, 2><<<nb, 256, 0, s>>>(p, nv);
+      else
+        proj_norm_rope_cache_wave_kernel<4, 1><<<nb, 256, 0, s>>>(p, nv);
+      return;
+    }
     const int n = p.T + (int)((vt + 255) / 256);
     if (f32 && two) proj_norm_rope_cache_vec_kernel<float, 2><<<n, 256, 0, s>>>(p, vrows);
     else if (f32) proj_norm_rope_cache_vec_kernel<float, 1><<<n, 256, 0, s>>>(p, vrows);

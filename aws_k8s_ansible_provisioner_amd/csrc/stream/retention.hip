@@ -276,99 +276,124 @@ __global__ __launch_bounds__(256) void head_norm_cache_kernel(HeadNormParams p) 
 }
 
 // The same in 16-byte pieces (D a multiple of 8 with D / 8 a power of two up to 64, Dv a multiple
-// of 8, for normed values a power of two of pieces as well): 8 dimensions of R rows per thread, all
-// their loads in flight together, weights and biases read once; D / 8 lanes per query / key head.
-// The first nqk workgroups take the (rows, head) pairs of q and k, the others the values
-// (write_values).  Bound by memory and by the loads' latency: 13600 rows of 16 / 4 / 4 heads of 128
-// with normed values 44 us (83 with values one by one, 57 with R = 1, 47.5 with only the groups whole
-// that begin at a multiple of 8 rows); 12800 rows with biases and rotation 57 us (89 element by
-// element, 79.5 and 73).
-template <typename T, int R>
-__global__ __launch_bounds__(256) void head_norm_cache_vec_kernel(HeadNormParams p, int nqk,
-                                                                  int vrows) {
-  const int lph = p.D >> 3;
-  if ((int)blockIdx.x < nqk) {
-    const int item = (blockIdx.x * 256 + threadIdx.x) / lph, j = threadIdx.x & (lph - 1);
-    const int heads = p.H + p.G;
-    const int t0 = item / heads * R, u = item % heads;   // the shuffles need every lane
+// of 8, for normed values a power of two of pieces as well).  D / 8 lanes per query / key head; a
+// thread takes 8 dimensions of R rows and of every S-th head, U at most, all rows in flight
+// together, the rows' angles read once for the heads and the heads' weights and biases once for the
+// rows.  A rotated entry's partner comes from its lane.  The first nv workgroups write the
+// values, whose chain of loads is the longest (write_values).
+//
+// Bound by the loads' latency and by instructions: 7200 rows of 16 / 4 / 4 heads of 128 with normed
+// values 43 us with 4 rows of a head to a thread (184 registers, five waves on a CU at a time, 64-bit
+// divisions of slots, the partners loaded again), now 29; 12800 rows with biases and rotation 57 -> 35
+// (160 MB), 1640 rows of 32 / 8 / 8 heads 18 -> 13.  With the values' workgroups last 37 and 38.
+template <typename T, int R, int U>
+__global__ __launch_bounds__(256, 4) void head_norm_cache_vec_kernel(HeadNormParams p, int nv,
+                                                                     int vrows, int S) {
+  typedef T Piece __attribute__((ext_vector_type(8)));
+  if ((int)blockIdx.x < nv) {
+    write_values<T>({(const T*)p.proj + p.v_off, p.proj_stride, (T*)p.v_cache, p.slots, p.num_slots, p.T,
+                     p.G, p.Dv, p.BS, vrows, p.eps, p.norm_v, p.bias ? p.bias + p.v_off : nullptr,
+                     nullptr},
+                    blockIdx.x * 256u + threadIdx.x);
+    return;
+  }
+  const int lph = p.D >> 3, lane = threadIdx.x & 63;
+  const uint32_t item = ((blockIdx.x - nv) * 256u + threadIdx.x) >> (31 - __clz(lph));
+  const uint32_t rb = item / (uint32_t)S;
+  const int s = (int)(item - rb * S), t0 = (int)rb * R, heads = p.H + p.G;
+  const int d = (threadIdx.x & (lph - 1)) * 8, half = p.rot_dims >> 1;
+  const bool rot = p.cos_sin && d < p.rot_dims, low = d < half;
+  auto off_of = [&](int u) { return u < p.H ? p.q_off + u * p.D : p.k_off + (u - p.H) * p.D; };
+  Piece x[R][U];
+  bool cached[R];
+  size_t krow[R];                                       // row of key head 0 in the cache
+#pragma unroll
+  for (int r = 0; r < R; ++r) {                         // (rows and heads clamped: shuffles need all)
+    const int t = min(t0 + r, p.T - 1);
+    const T* row = (const T*)p.proj + (size_t)t * p.proj_stride + d;
+#pragma unroll
+    for (int i = 0; i < U; ++i) x[r][i] = *(const Piece*)(row + off_of(min(s + S * i, heads - 1)));
+    const int64_t slot = p.slots[t];
+    cached[r] = slot >= 0 && slot < p.num_slots;
+    size_t page;
+    int off;
+    slot_at(cached[r] ? slot : 0, p.num_slots, p.BS, page, off);
+    krow[r] = page * p.G * p.BS + off;
+  }
+  float c8[R][8], s8[R][8];
+  if (rot) {
+    const int i0 = low ? d : d - half;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t pos = p.positions[min(t0 + r, p.T - 1)];
+      const float* cs = p.cos_sin + (size_t)(pos < p.max_pos ? pos : p.max_pos - 1) * p.rot_dims;
+      ld8(cs + i0, c8[r]);
+      ld8(cs + half + i0, s8[r]);
+    }
+  }
+  const int partner = rot ? (low ? lane + (half >> 3) : lane - (half >> 3)) : lane;
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    const int u = min(s + S * i, heads - 1);
     const bool isq = u < p.H;
-    const int off = isq ? p.q_off + u * p.D : p.k_off + (u - p.H) * p.D;
     const float* w = isq ? p.q_w : p.k_w;
-    const int d = j * 8, half = p.rot_dims >> 1;
-    const bool rot = p.cos_sin && d < p.rot_dims, low = d < half;
-    const int d2 = low ? d + half : d - half;
-    float v[R][8], v2[R][8], c8[R][8], s8[R][8];
-    int64_t slot[R], pos[R];
+    float b8[8], w8[8];
+    if (p.bias) ld8(p.bias + off_of(u) + d, b8);
+    if (w) ld8(w + d, w8);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int t = min(t0 + r, p.T - 1);
-      const T* src = (const T*)p.proj + (size_t)t * p.proj_stride + off;
-      ld8(src + d, v[r]);
-      slot[r] = isq ? 0 : p.slots[t];
-      if (rot) {
-        pos[r] = p.positions[t];
-        ld8(src + d2, v2[r]);
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = (float)x[r][i][k];
+      if (p.bias) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] += b8[k];
       }
-    }
-    float b1[8], b2[8], w1[8], w2[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      b1[i] = b2[i] = 0.f;
-      w1[i] = w2[i] = 1.f;
-    }
-    if (p.bias) {
-      ld8(p.bias + off + d, b1);
-      if (rot) ld8(p.bias + off + d2, b2);
-    }
-    if (w) {
-      ld8(w + d, w1);
-      if (rot) ld8(w + d2, w2);
-    }
-    if (rot) {
-      const int i0 = low ? d : d - half;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float* cs = p.cos_sin + (size_t)(pos[r] < p.max_pos ? pos[r] : p.max_pos - 1) *
-                                          p.rot_dims;
-        ld8(cs + i0, c8[r]);
-        ld8(cs + half + i0, s8[r]);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[r][i] += b1[i];
       float inv = 1.0f;
       if (p.norm_qk) {
         float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) ss += v[r][i] * v[r][i];
-        for (int o = lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        for (int k = 0; k < 8; ++k) ss += v[k] * v[k];
+        if (lph == 16) {                                // (a DPP row)
+          ss += akap::dpp_mov<0x128>(ss);
+          ss += akap::dpp_mov<0x124>(ss);
+          ss += akap::dpp_mov<0x122>(ss);
+          ss += akap::dpp_mov<0x121>(ss);
+        } else {
+          for (int o = lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        }
         inv = 1.0f / sqrtf(ss / (float)p.D + p.eps);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] *= inv;
       }
+      if (p.q_w || p.k_w) {                             // (lanes of a wave may differ in w)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[r][i] *= inv * w1[i];
-      if (rot) {
+        for (int k = 0; k < 8; ++k) v[k] *= w ? w8[k] : 1.f;
+      }
+      if (p.cos_sin) {
+        float v2[8];
+        if (half == 64) {                               // 8 lanes away: the DPP row turned by half
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          v[r][i] = v[r][i] * c8[r][i] +
-                    (v2[r][i] + b2[i]) * inv * w2[i] * (low ? -s8[r][i] : s8[r][i]);
+          for (int k = 0; k < 8; ++k) v2[k] = akap::dpp_mov<0x128>(v[k]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) v2[k] = __shfl(v[k], partner, 64);
+        }
+        if (rot) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            v[k] = v[k] * c8[r][k] + v2[k] * (low ? -s8[r][k] : s8[r][k]);
+        }
       }
       const int t = t0 + r;
-      if (t >= p.T) continue;
+      if (t >= p.T || s + S * i >= heads) continue;
       if (isq) {
-        st8((T*)p.q_out + ((size_t)t * p.H + u) * p.D + d, v[r]);
-      } else if (slot[r] >= 0 && slot[r] < p.num_slots) {
-        st8((T*)p.k_cache + ((size_t)(slot[r] / p.BS * p.G + u - p.H) * p.BS + slot[r] % p.BS) * p.D +
-                d, v[r]);
+        st8((T*)p.q_out + ((size_t)t * p.H + u) * p.D + d, v);
+      } else if (cached[r]) {
+        st8((T*)p.k_cache + (krow[r] + (size_t)(u - p.H) * p.BS) * p.D + d, v);
       }
     }
-    return;
   }
-  write_values<T>({(const T*)p.proj + p.v_off, p.proj_stride, (T*)p.v_cache, p.slots, p.num_slots, p.T,
-                   p.G, p.Dv, p.BS, vrows, p.eps, p.norm_v, p.bias ? p.bias + p.v_off : nullptr,
-                   nullptr},
-                  (int64_t)(blockIdx.x - nqk) * 256 + threadIdx.x);
 }
 
 // ------------------------------------------------------------------ retention
@@ -1132,20 +1157,28 @@ bool launch_head_cache_vec(const HeadNormParams& p, bool f32, hipStream_t s) {
       (((uintptr_t)p.proj | (uintptr_t)p.q_out | (uintptr_t)p.k_cache | (uintptr_t)p.v_cache |
         (uintptr_t)p.q_w | (uintptr_t)p.k_w | (uintptr_t)p.cos_sin | (uintptr_t)p.bias) & 15))
     return false;
-  // large steps: 4 rows per thread, values by groups of 8 rows; below mostly rows of sequences of
-  // their own, and too few for that
-  const bool large = p.T >= 512;
-  const int R = large ? 4 : 1, vrows = large ? 8 : 1;
-  const int64_t qk = (int64_t)((p.T + R - 1) / R) * (p.H + p.G) * lph;
-  const int64_t vt = value_group_threads(p.T, p.G, p.Dv, vrows);
-  const int nqk = (int)((qk + 255) / 256), n = nqk + (int)((vt + 255) / 256);
-  if (large) {
-    if (f32) head_norm_cache_vec_kernel<float, 4><<<n, 256, 0, s>>>(p, nqk, vrows);
-    else head_norm_cache_vec_kernel<bf16, 4><<<n, 256, 0, s>>>(p, nqk, vrows);
+  // large steps: values by groups of 8 rows; below mostly rows of sequences of their own, and too few
+  // for that
+  const int vrows = p.T >= 512 ? 8 : 1, heads = p.H + p.G;
+  const int nv = (int)((value_group_threads(p.T, p.G, p.Dv, vrows) + 255) / 256);
+#define AKAP_HN(TY, R, U)                                                                          \
+  do {                                                                                             \
+    const int S = (heads + U - 1) / U;                                                             \
+    const int nqk = (int)(((int64_t)((p.T + R - 1) / R) * S * lph + 255) / 256);                   \
+    head_norm_cache_vec_kernel<TY, R, U><<<nv + nqk, 256, 0, s>>>(p, nv, vrows, S);                \
+  } while (0)
+  // a thread takes more rows and heads while that leaves four waves for each SIMD
+  const int64_t waves = (int64_t)p.T * heads * lph / 64;
+  if (f32) {
+    AKAP_HN(float, 1, 1);
+  } else if (waves >= 32768) {
+    AKAP_HN(bf16, 2, 4);
+  } else if (waves >= 8192) {
+    AKAP_HN(bf16, 1, 2);
   } else {
-    if (f32) head_norm_cache_vec_kernel<float, 1><<<n, 256, 0, s>>>(p, nqk, vrows);
-    else head_norm_cache_vec_kernel<bf16, 1><<<n, 256, 0, s>>>(p, nqk, vrows);
+    AKAP_HN(bf16, 1, 1);
   }
+#undef AKAP_HN
   return true;
 }
 

@@ -31,6 +31,23 @@ __host__ __device__ __forceinline__ int64_t value_group_threads(int T, int G, in
   return (int64_t)((T + vrows - 1) / vrows) * G * (Dv >> 3);
 }
 
+// page of a slot and place in it, by a shift where the page is a power of two and by 32-bit division
+// otherwise: the 64-bit one of a few slots was a third of a cache write's instructions
+__device__ __forceinline__ void slot_at(int64_t slot, int64_t num_slots, int BS, size_t& page,
+                                        int& off) {
+  if (num_slots > 0x7fffffff) {
+    page = (size_t)(slot / BS);
+    off = (int)(slot - (int64_t)page * BS);
+  } else if ((BS & (BS - 1)) == 0) {
+    page = (uint32_t)slot >> (31 - __clz(BS));
+    off = (uint32_t)slot & (BS - 1);
+  } else {
+    const uint32_t pg = (uint32_t)slot / (uint32_t)BS;
+    page = pg;
+    off = (int)((uint32_t)slot - pg * BS);
+  }
+}
+
 namespace vg {
 __device__ __forceinline__ void ld8(const float* p, float (&v)[8]) {
   const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
@@ -57,79 +74,79 @@ __device__ __forceinline__ void st8(akap::bf16* p, const float (&v)[8]) {
 // `item` of value_group_threads(); with norm, Dv / 8 is a power of two up to 64 and the lanes of a
 // head are neighbours (whole waves call this, items in lane order)
 template <typename T>
-__device__ __forceinline__ void write_values(const ValueGroups<T>& a, int64_t item) {
-  const int lph = a.Dv >> 3, per = a.G * lph;
-  const int t0 = (int)(item / per) * a.vrows;
+__device__ __forceinline__ void write_values(const ValueGroups<T>& a, uint32_t item) {
+  typedef T Piece __attribute__((ext_vector_type(8)));
+  const uint32_t lph = a.Dv >> 3, per = a.G * lph, block = item / per;
+  const uint32_t e = item - block * per, g = e / lph, c = (e - g * lph) * 8;
+  const int t0 = (int)block * a.vrows;
   const bool live = t0 < a.T_;
-  const int e = (int)(item % per), g = e / lph, c = (e - g * lph) * 8;
-  const int n = live ? min(a.vrows, a.T_ - t0) : 0;
-  const int64_t s0 = live ? a.slots[t0] : -1;
-  // the 8 rows that fill the first group which begins at or after row t (its slot s)
-  auto group = [&](int t, int64_t s, int& first) {
-    first = t + (int)((8 - (s & 7)) & 7);
-    const int64_t f = (s + 7) & ~(int64_t)7;
-    bool whole = s >= 0 && first + 8 <= a.T_ && f + 7 < a.num_slots;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)     // (all eight requested together)
-      whole &= a.slots[min(first + i, a.T_ - 1)] == f + i;
-    return whole;
-  };
+  const T* src = a.src + g * a.Dv + c;
   float add[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (a.bias) vg::ld8(a.bias + g * a.Dv + c, add);
   if (a.bias_t) vg::ld8(a.bias_t + g * a.Dv + c, add);
-  auto row = [&](int t, float (&v)[8]) {      // (every lane of a head, rows clamped)
-    vg::ld8(a.src + (size_t)t * a.stride + g * a.Dv + c, v);
+  auto load = [&](int t) { return *(const Piece*)(src + (size_t)t * a.stride); };
+  auto row = [&](const Piece& x, float (&v)[8]) {      // (every lane of a head)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] += add[k];
+    for (int k = 0; k < 8; ++k) v[k] = (float)x[k] + add[k];
     if (a.norm) {
       float ss = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) ss += v[k] * v[k];
-      for (int o = lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      for (int o = (int)lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
       const float inv = 1.0f / sqrtf(ss / (float)a.Dv + a.eps);
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] *= inv;
     }
   };
   auto dst = [&](int64_t slot) {
-    return a.cache + (((size_t)(slot / a.BS * a.G + g) * (a.BS >> 3) + (slot % a.BS >> 3)) * a.Dv +
-                      c) * 8 + (slot & 7);
+    size_t page;
+    int off;
+    slot_at(slot, a.num_slots, a.BS, page, off);
+    return a.cache + (((page * a.G + g) * (a.BS >> 3) + (off >> 3)) * a.Dv + c) * 8 + (off & 7);
   };
-  if (a.vrows == 8) {
-    if (!live) return;
-    // the group that begins among my rows, and the one that began among the 8 before and may end here
-    int mine, prev = 0;
-    const bool whole = group(t0, s0, mine);
-    const bool before = t0 > 0 && group(t0 - 8, a.slots[t0 - 8], prev);
-    if (whole) {
-      float v[8][8];
+  auto single = [&](int t, int64_t slot) {
+    float v[8];
+    row(load(t), v);
+    if (slot < 0 || slot >= a.num_slots) return;
+    T* o = dst(slot);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) row(mine + i, v[i]);
-      T* o = dst(a.slots[mine]);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float r[8] = {v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k], v[6][k], v[7][k]};
-        vg::st8(o + k * 8, r);
-      }
-    }
-    for (int t = t0; t < t0 + n; ++t) {       // what is in neither
-      if ((whole && t >= mine) || (before && t >= prev && t < prev + 8)) continue;
-      float v[8];
-      row(t, v);
-      const int64_t slot = a.slots[t];
-      if (slot < 0 || slot >= a.num_slots) continue;
-      T* o = dst(slot);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o[k * 8] = (T)v[k];
-    }
+    for (int k = 0; k < 8; ++k) o[k * 8] = (T)v[k];
+  };
+  if (a.vrows != 8) {
+    single(live ? t0 : 0, live ? a.slots[t0] : -1);
     return;
   }
-  float v[8];
-  row(live ? t0 : 0, v);
-  if (s0 < 0 || s0 >= a.num_slots) return;
-  T* o = dst(s0);
+  if (!live) return;
+  // the group that begins among my rows (at the first multiple of 8 among the slots), and the one that
+  // began among the 8 before and may end here; the rows' loads are under way before either is known to
+  // be whole
+  const int n = min(8, a.T_ - t0), tb = max(t0 - 8, 0);
+  const int64_t s0 = a.slots[t0], sb = a.slots[tb];
+  const int mine = t0 + (int)((8 - (s0 & 7)) & 7), prev = tb + (int)((8 - (sb & 7)) & 7);
+  const int64_t fm = (s0 + 7) & ~(int64_t)7, fp = (sb + 7) & ~(int64_t)7;
+  Piece x[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) o[k * 8] = (T)v[k];
+  for (int i = 0; i < 8; ++i) x[i] = load(min(mine + i, a.T_ - 1));
+  bool whole = s0 >= 0 && mine + 8 <= a.T_ && fm + 7 < a.num_slots;
+  bool before = t0 > 0 && sb >= 0 && prev + 8 <= a.T_ && fp + 7 < a.num_slots;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    whole &= a.slots[min(mine + i, a.T_ - 1)] == fm + i;
+    before &= a.slots[min(prev + i, a.T_ - 1)] == fp + i;
+  }
+  if (whole) {
+    float v[8][8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) row(x[i], v[i]);
+    T* o = dst(fm);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float r[8] = {v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k], v[6][k], v[7][k]};
+      vg::st8(o + k * 8, r);
+    }
+  }
+  for (int t = t0; t < t0 + n; ++t)           // what is in neither
+    if (!(whole && t >= mine) && !(before && t >= prev && t < prev + 8)) single(t, a.slots[t]);
 }
 
 }  // namespace akap_stream

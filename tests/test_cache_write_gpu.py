@@ -75,6 +75,47 @@ def test_head_caches(form, n, dt):
         _same(a.cpu(), b, dt)
 
 
+@pytest.mark.parametrize("form,n,H,G,D,rot,BS", [
+    ("normed", 6601, 16, 4, 128, 128, 32),      # two rows and four heads to a thread
+    ("normed", 1703, 17, 3, 128, 64, 40),       # one row and two heads, the last ones missing
+    ("biased", 3301, 32, 8, 128, 128, 32), ("biased", 1650, 16, 5, 64, 64, 24),
+    ("biased", 700, 6, 2, 256, 128, 32),
+    ("whole", 767, 16, 4, 128, 128, 32), ("whole", 768, 16, 4, 128, 64, 32),   # a workgroup, a wave
+    ("whole", 771, 24, 8, 64, 64, 40), ("whole", 1027, 32, 8, 128, 128, 32),
+    ("whole", 800, 3, 1, 512, 16, 32), ("whole", 801, 5, 1, 96, 32, 32)])
+def test_large_steps(form, n, H, G, D, rot, BS):
+    """Both sides of the sizes from which a thread takes several rows and heads and a wave a whole
+    token; pages that are no power of two, heads and rows left over."""
+    g = torch.Generator().manual_seed(n)
+    dt = torch.bfloat16
+    slots, pos, NB = _step(n, BS, n)
+    N = (H + 2 * G) * D + 8
+    proj = torch.randn(n, N, generator=g).to(dt)
+    cs = sops.rotary_table(4 * BS + 200, rot, 1e4, None, "cpu")
+    bias = torch.randn(N, generator=g)
+    qw, kw = torch.rand(H * D, generator=g) + 0.5, torch.rand(G * D, generator=g) + 0.5
+    qb, kb = torch.randn(H * D, generator=g).to(dt), torch.randn(G * D, generator=g).to(dt)
+
+    def run(dev):
+        c = lambda t: t.clone().to(dev)
+        q = torch.zeros(n, H, D, dtype=dt, device=dev)
+        kc = torch.zeros(NB, G, BS, D, dtype=dt, device=dev)
+        vc = torch.zeros(NB, G, BS // 8, D, 8, dtype=dt, device=dev)
+        o = (8, 8 + H * D, 8 + (H + G) * D)
+        if form == "normed":
+            sops.head_norm_cache(c(proj), q, kc, vc, c(slots), H, G, D, D, *o, 1e-5, q_w=c(qw[:D]),
+                                 k_w=c(kw[:D]), cos_sin=c(cs), positions=c(pos))
+        elif form == "biased":
+            sops.bias_rope_cache(c(proj), q, kc, vc, c(pos), c(slots), c(cs), c(bias), H, G, D, D, *o)
+        else:
+            sops.proj_norm_rope_cache(c(proj), q, kc, vc, c(pos), c(slots), c(cs), c(qw), c(kw), H, G,
+                                      D, *o[:2], 1e-5, c(qb), c(kb))
+        return q, kc, vc
+
+    for a, b in zip(run(DEV), run("cpu")):
+        _same(a.cpu(), b, dt)
+
+
 @pytest.mark.parametrize("n,q_rank,kv_rank,rot,form", [
     (2047, 768, 512, 64, ""), (2048, 768, 512, 64, ""), (2077, 1536, 512, 64, "half"),
     (2050, 1032, 96, 16, ""), (2049, 64, 256, 32, "rows"), (2051, 768, 512, 64, "queries")])
