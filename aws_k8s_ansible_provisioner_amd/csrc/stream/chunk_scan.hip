@@ -1,29 +1,35 @@
 // Prompt chunks of the two recurrences with a matrix state and one decay per head and token, on
-// the fp32 matrix instructions:
+// the matrix instructions, with fp32 operands in three bf16 parts:
 //   selective scan   S <- a_t S + dt_t B_t x_t^T,  y_t = S^T C_t + d x_t     (a_t from dt_t)
 //   retention        S <- a S + k_t v_t^T,         o_t = S^T q_t, normed and gated per head
 // A sequence's rows go in chunks of 32.  With c_i the sum of the log2 decays from the chunk's
 // start through row i, S0 the state before it, k / q / v the rows (k times dt for the scan):
 //   o_i   = 2^(c_i) q_i S0 + sum_{j <= i} 2^(c_i - c_j) (q_i . k_j) v_j
 //   S_end = 2^(c_end) S0 + sum_j k_j (2^(c_end - c_j) v_j)^T
-// Everything is fp32 (v_mfma_f32_32x32x2_f32: the vector units' rate without packed
-// instructions, but four times the operations per LDS or register read), the decays' sums fp64:
-// differences of sums of the size of 30 in fp32 would lose two digits.
+// Values, states and sums are fp32, the decays' sums fp64: differences of sums of the size of 30 in fp32
+// would lose two digits.  The products with the state, which are most of the work, take their operands
+// apart, x = h + m + l with 8 bits each, and sum the six largest of the nine products in fp32 (h h, the
+// others' sums apart where there are registers for it): 2^-26 of a product is left out, and a sum of 16
+// products is rounded once per instruction, where v_mfma_f32_32x32x2_f32 rounds every two.  Against 64 bits,
+// 8 x 2048 rows: scan outputs 1.03e-7 and states 1.12e-7 (in fp32 products 1.04e-7 and 1.14e-7), retention
+// states 1.7e-7 (2.7e-7).  Operands that do not split (not finite, past bf16's range, or so small that
+// parts would be denormal, which the matrix units take as zero) go through the fp32 products.
 //
-// chunk_frag_kernel prepares every (chunk, key head) side by side: q and k (rotated and scaled
-// for the retention) as operand fragments and the 32 x 32 products q_i . k_j; the scan's keys
-// belong to a group, so its heads share them.  chunk_scalar_kernel sums the scan's decays.
+// chunk_frag_kernel prepares every (chunk, key head) side by side: the parts of q and k (rotated and
+// scaled for the retention) as operand fragments and the 32 x 32 products q_i . k_j in fp32; the scan's
+// keys belong to a group, so its heads share them.  chunk_scalar_kernel sums the scan's decays.
 // chunk_walk_kernel then walks the chunks of a (sequence, head): a wave owns 32 state columns in
 // accumulators.  An accumulator lane holds column l & 31 and rows 8 g + 4 (l >> 5) + r in
-// register 4 g + r: read as the B operand of the next product, step r of piece g contracts over
-// the rows 8 g + r and 8 g + 4 + r, so with A fragments stored in that order (lane (i, hh) of
-// piece g: 4 consecutive entries from 8 g + 4 hh on, one 16-byte load for four products) the
-// state, the values and the outputs feed each other without lane traffic.
+// register 4 g + r: with the fragments' entries in that order (lane (i, hh) of step j: entries
+// 16 j + 4 hh + 0..3 and 16 j + 8 + 4 hh + 0..3) eight neighbouring registers are an operand of the next
+// product, so the state, the values and the outputs feed each other without lane traffic.
 //
-// Bound by the fp32 matrix rate (144 products of 64 cycles per chunk, head and 32 columns of a
-// 128-row state; 140 TFLOP/s in a register loop): 16384 rows of 8 sequences, 64 heads x 128 x 64
-// states 452 us (276 us of products) where the row-by-row scan took 1420; 8 heads x 128 x 128
-// (segments) 264 us in all, by rows 790.
+// Bound by vector work (1000 instructions per chunk, half of them the state's parts) and products (4100
+// cycles per chunk) of a wave that has its SIMD alone or shares it with one other; the next step's
+// parts are formed between a step's products.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 347 us
+// where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
+// 128 x 128 (segments) 110 + 48 for the pass before it, of 136 + 66, while the fragments, half as large
+// again, take 66 of 52.
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
 // where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
@@ -38,6 +44,7 @@
 namespace akap_stream {
 
 using akap::bf16;
+using akap::bf16x8;
 using akap::f32x16;
 
 namespace {
@@ -76,6 +83,9 @@ __device__ __forceinline__ void st4(bf16* p, float a, float b, float c, float d)
   *(akap::bf16x4*)p = o;
 }
 
+// a value that all lanes hold, as a scalar
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // the same value, as one the compiler knows nothing about: what is derived from it is formed anew
 // in every round of a loop instead of being kept in registers across it
 __device__ __forceinline__ uint32_t fresh(uint32_t v) {
@@ -93,6 +103,52 @@ __device__ __forceinline__ f32x16 mfma(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+__device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// v = h + m + l exactly (8 bits each, rounded to nearest) unless v is too large for bf16 or not finite
+__device__ __forceinline__ void split8(const float (&v)[8], bf16x8& h, bf16x8& m, bf16x8& l) {
+  float r[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    h[i] = (bf16)v[i];
+    r[i] = v[i] - (float)h[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    m[i] = (bf16)r[i];
+    l[i] = (bf16)(r[i] - (float)m[i]);
+  }
+}
+// Magnitudes below this split.  The matrix units take a denormal part as zero, so the largest of the
+// values that meet in a lane has to be above the second limit: then what is lost is 2^-48 of it.
+constexpr float kSplits = 3.38e38f, kWhole = 0x1p-78f;
+__device__ __forceinline__ bool splits(float top) { return top < kSplits && !(top < kWhole && top > 0.f); }
+
+// Products of split operands: the largest go to `big`, the five next to `small`; what is left out is
+// 2^-26 of the product.
+__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x16& big,
+                                           f32x16& small) {
+  small = mfma16(a[2], b[0], small);
+  big = mfma16(a[0], b[0], big);
+  small = mfma16(a[0], b[2], small);
+  small = mfma16(a[1], b[1], small);
+  small = mfma16(a[1], b[0], small);
+  small = mfma16(a[0], b[1], small);
+}
+
+// N times one matrix product and V vector instructions, in this order: the next step's vector work runs
+// while a step's products do
+template <int N, int V>
+__device__ __forceinline__ void interleave() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+  }
+}
+
 // decay^k for a decay given by its log2 (-inf: a decay of zero)
 __device__ __forceinline__ float decay_pow(float l2, int k) {
   return k == 0 ? 1.0f : exp2f(l2 * (float)k);
@@ -103,15 +159,20 @@ __device__ __forceinline__ int base_of(const int32_t* q_start, int b, int rows) 
   return q_start[b] / rows + b;
 }
 
-// the sequence that owns an entry, and the rows [r0, r1) of the entry (r1 <= r0: none)
+// the sequence that owns an entry (the same in all lanes), and the rows [r0, r1) of the entry (r1 <= r0:
+// none): a chain of scalar loads
+typedef const __attribute__((address_space(4))) int32_t* ScalarInts;
+
 __device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int rows, int& r0, int& r1) {
+  const ScalarInts q_start = (ScalarInts)p.q_start;
+  entry = uniform(entry);
   int lo = 0, hi = p.B - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (base_of(p.q_start, mid, rows) <= entry) lo = mid; else hi = mid - 1;
+    if (q_start[mid] / rows + mid <= entry) lo = mid; else hi = mid - 1;
   }
-  const int first = p.q_start[lo], end = p.q_start[lo + 1];
-  r0 = first + (entry - base_of(p.q_start, lo, rows)) * rows;
+  const int first = q_start[lo], end = q_start[lo + 1];
+  r0 = first + (entry - (first / rows + lo)) * rows;
   r1 = min(r0 + rows, end);
   if (r0 < first) r1 = r0;
   return lo;
@@ -157,8 +218,10 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 }
 
 // ------------------------------------------------------------------ fragments of q and k
-// One workgroup per (chunk, key head).  Buffer of an entry: [q: NT 4 fragments][k transposed:
-// the same][q . k: 4 fragments], 64 lanes x 4 floats each; rows past the chunk's end are zero.
+// One workgroup per (chunk, key head).  Buffer of an entry, in pieces of 64 lanes x 16 bytes: [q: 3 parts
+// of N / 16 pieces][k transposed: the same, the retention's already times their weights in the new
+// state][q . k in fp32: 4][1 if a value does not split:
+// then the parts are the fp32 values' upper and lower halves]; rows past the chunk's end are zero.
 template <int MODE, int NT, typename TY>
 __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
@@ -166,6 +229,7 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
   using TR = typename std::conditional<MODE == 0, double, float>::type;
   constexpr int kRed = 4096 * sizeof(TR) / 4;
   __shared__ __align__(16) float rows[2 * kL * LS > kRed ? 2 * kL * LS : kRed];
+  __shared__ float wt[kL];     // retention: the rows' weights in the state after the chunk
   float *qs = rows, *ks = rows + kL * LS;
   TR* red = (TR*)rows;
   const int entry = blockIdx.x, kh = blockIdx.y;
@@ -227,14 +291,55 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
     *(float4*)(qs + i * LS + d) = a;
     *(float4*)(ks + i * LS + d) = b4;
   }
+  if (MODE == 1 && tid < kL) wt[tid] = tid < n ? decay_pow(p.log2_decay[kh], n - 1 - tid) : 0.f;
   __syncthreads();
   const int li = lane & 31, hh = lane >> 5;
-  float4* out = (float4*)(p.frag + ((size_t)entry * p.KH + kh) * p.frag_floats);
-  for (int f = wave; f < NT * 4; f += 4) {
-    out[f * 64 + lane] = *(const float4*)(qs + li * LS + 8 * f + 4 * hh);
-    const float* kk = ks + (8 * (f & 3) + 4 * hh) * LS + 32 * (f >> 2) + li;
-    out[(NT * 4 + f) * 64 + lane] = make_float4(kk[0], kk[LS], kk[2 * LS], kk[3 * LS]);
+  constexpr int NQ = N / 16;
+  float* buf = p.frag + ((size_t)entry * p.KH + kh) * p.frag_floats;
+  // piece f: contraction step f of q (entries 16 f + 4 hh + 0..3 and 8 on), rows 32 (f / 2) of the state
+  // and tokens 16 (f % 2) + 4 hh + 0..3 and 8 on of k
+  float v[2][NQ / 4][8];
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < NQ / 4; ++u) {
+    const int f = wave + 4 * u, j0 = 16 * (f & 1) + 4 * hh;
+    *(float4*)v[0][u] = *(const float4*)(qs + li * LS + 16 * f + 4 * hh);
+    *(float4*)(v[0][u] + 4) = *(const float4*)(qs + li * LS + 16 * f + 8 + 4 * hh);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j = j0 + (i & 3) + 8 * (i >> 2);
+      v[1][u][i] = ks[j * LS + 32 * (f >> 1) + li] * (MODE == 1 ? wt[j] : 1.f);
+    }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      float top = 0.f, zero = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        top = fmaxf(top, fabsf(v[w][u][i]));
+        zero = fmaf(v[w][u][i], 0.f, zero);
+      }
+      bad |= zero != 0.f || !splits(top);
+    }
   }
+  bad = __syncthreads_or(bad);
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int u = 0; u < NQ / 4; ++u) {
+      bf16x8 part[3];
+      split8(v[w][u], part[0], part[1], part[2]);
+      if (__builtin_expect(bad, 0)) {      // as they are, in two halves
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t bits = __float_as_uint(v[w][u][i]);
+          part[0][i] = __builtin_bit_cast(bf16, (uint16_t)(bits >> 16));
+          part[1][i] = __builtin_bit_cast(bf16, (uint16_t)bits);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        ((bf16x8*)buf)[(3 * NQ * w + wave + 4 * u + i * NQ) * 64 + lane] = part[i];
+    }
   // q . k with the keys as rows: lane (i, hh) register 4 g + r is q_i . k_(8 g + 4 hh + r), the
   // operand the walk needs; the waves contract a part of the entries each.  The scan's in four chains
   // that meet in fp64: the products have mostly one sign, and the error of one long fp32 sum of them
@@ -269,7 +374,8 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 #pragma unroll
     for (int w = 1; w < 4; ++w) s[r] += red[w * 1024 + tid * 4 + r];
   }
-  out[NT * 8 * 64 + tid] = make_float4((float)s[0], (float)s[1], (float)s[2], (float)s[3]);
+  ((float4*)buf)[6 * NQ * 64 + tid] = make_float4((float)s[0], (float)s[1], (float)s[2], (float)s[3]);
+  if (tid == 0) ((int*)buf)[6 * NQ * 256 + 1024] = bad;
 }
 
 // ------------------------------------------------------------------ step sizes and decays
@@ -311,18 +417,21 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
 // ------------------------------------------------------------------ the walk
 // HW heads (of one key head) of V / 32 waves each, a wave per 32 state columns; FULL: outputs,
 // from the state in the slot (or, SEGM and the sequence is cut, from the segment buffer); else the
-// segment's own state from zeros.  A chunk's fragments and scalars arrive by LDS-DMA while the chunk before is
-// computed (two buffers of 37 KB, so two workgroups share a CU), its values in registers: a wave
-// waits once per chunk, for loads issued some 10000 cycles earlier.
+// segment's own state from zeros.  Fragments and scalars arrive by LDS-DMA: those of q while the state
+// of the chunk before is formed, those of k (in time for the chunk's state) while its outputs are, so
+// that one buffer of each does and two workgroups share a CU; the values in registers a chunk ahead.
 template <int MODE, int NT, int V, int HW, typename TY, bool FULL, bool SEGM>
 __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkScanParams p) {
-  constexpr int N = NT * 32, NF = NT * 4, VW = V / 32, NW = VW * HW;
+  constexpr int N = NT * 32, NQ = NT * 2, VW = V / 32, NW = VW * HW;
   constexpr bool kNorm = MODE == 1 && FULL;
-  // fragments of a buffer: [q (FULL)][k][q . k (FULL)][scalars of the heads (scan)]
-  constexpr int K0 = FULL ? NF : 0, G0 = K0 + NF, C0 = G0 + (FULL ? 4 : 0);
-  constexpr int NB = C0 + (MODE == 0 ? HW : 0);
-  __shared__ __align__(16) float4 buf[2][NB * 64];
-  __shared__ __align__(16) float tab[MODE == 1 ? NW * 3 * kL : 4];   // per wave, see below
+  constexpr int XP = MODE == 1 && sizeof(TY) == 2 ? 1 : 3;   // parts of a value (of bf16 rows: itself)
+  // pieces of 1 KB: [q parts][q . k][scalars of the heads (scan)] and [k parts]; without outputs
+  // twice [k parts][scalars]
+  constexpr int KU = 3 * NQ, SU = MODE == 0 ? HW : 0, G0 = 3 * NQ, C0 = FULL ? G0 + 4 : KU;
+  constexpr int QB = C0 + SU;
+  __shared__ __align__(16) float4 qbuf[QB * 64];
+  __shared__ __align__(16) float4 kbuf[(FULL ? KU : QB) * 64];
+  __shared__ __align__(16) float tab[MODE == 1 ? NW * 2 * kL : 4];   // per wave, see below
   __shared__ __align__(16) float pd[kNorm ? 1024 : 4];       // retention: 2^(c_i - c_j), by lane
   __shared__ __align__(16) float ssq[kNorm ? 2 * NW * kL : 4];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -339,25 +448,25 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   if (cut) {
     b = locate(p, b, p.SEG, r0, r1);
   } else {
-    r0 = p.q_start[b];
-    r1 = p.q_start[b + 1];
+    b = uniform(b);
+    r0 = ((ScalarInts)p.q_start)[b];
+    r1 = ((ScalarInts)p.q_start)[b + 1];
   }
   if (r1 <= r0) return;
-  const int first = p.q_start[b];
-  if (SEGM && walked_whole(p, p.q_start[b + 1] - first) == cut) return;
-  const size_t seg = cut ? seg_base(p, b) + (r0 - first) / p.SEG : 0;
-  const int slot = p.seq_slot[first];
+  const int first = ((ScalarInts)p.q_start)[b];
+  if (SEGM && walked_whole(p, ((ScalarInts)p.q_start)[b + 1] - first) == cut) return;
+  const size_t seg = cut ? (size_t)uniform((int)seg_base(p, b) + (r0 - first) / p.SEG) : 0;
+  const int slot = uniform(p.seq_slot[first]);
   if (!live_slot(p, slot)) return;
   const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
   const int col = (wave % VW) * 32 + li;
   const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
-  // retention: decay^k, decay^(k + 1), and the weights of a cut chunk's values in the new state
-  float* tb = tab + (MODE == 1 ? wave * 3 * kL : 0);
+  // retention: decay^k and decay^(k + 1)
+  float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
   if (MODE == 1) {
     if (lane < kL) {
       tb[lane] = decay_pow(l2, lane);
       tb[kL + lane] = decay_pow(l2, lane + 1);
-      tb[2 * kL + lane] = decay_pow(l2, kL - 1 - lane);
     }
     if (kNorm) {
       for (int e = tid; e < 1024; e += 64 * NW) {
@@ -388,18 +497,27 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       }
     }
   const int c0 = (r0 - first) / kL, chunks = (r1 - r0 + kL - 1) / kL;
-  const size_t cb = (size_t)base_of(p.q_start, b, kL) + c0;
+  const size_t cb = (size_t)uniform(base_of(p.q_start, b, kL) + c0);
   const uint32_t l16 = lane * 16;
-  auto stage = [&](int c, float4* to) {
-    const char* src = (const char*)p.frag + ((cb + c) * p.KH + kh) * p.frag_floats * 4 +
-                      (FULL ? 0 : NF * 1024) + wave * 1024;
+  auto frag_of = [&](int c) { return (const char*)(p.frag + ((cb + c) * p.KH + kh) * p.frag_floats); };
+  auto pieces = [&](const char* src, float4* to, auto count) {
+    constexpr int n = decltype(count)::value;
 #pragma unroll
-    for (int u = 0; u < (C0 + NW - 1) / NW; ++u)
-      if ((u + 1) * NW <= C0 || u * NW + wave < C0)
-        dma16(src + u * NW * 1024 + l16, to + (u * NW + wave) * 64);
+    for (int u = 0; u < (n + NW - 1) / NW; ++u)
+      if ((u + 1) * NW <= n || u * NW + wave < n)
+        dma16(src + (u * NW + wave) * 1024 + l16, to + (u * NW + wave) * 64);
+  };
+  auto stage_scalars = [&](int c, float4* to) {
     if (MODE == 0 && wave < HW)
-      dma16((const char*)(p.scal + ((cb + c) * p.H + h0 + wave) * kScal) + l16,
-            to + (C0 + wave) * 64);
+      dma16((const char*)(p.scal + ((cb + c) * p.H + h0 + wave) * kScal) + l16, to + wave * 64);
+  };
+  auto stage_q = [&](int c) {
+    pieces(frag_of(c), qbuf, std::integral_constant<int, 3 * NQ>{});
+    pieces(frag_of(c) + 6 * NQ * 1024, qbuf + G0 * 64, std::integral_constant<int, 4>{});
+    stage_scalars(c, qbuf + C0 * 64);
+  };
+  auto stage_k = [&](int c, float4* to) {
+    pieces(frag_of(c) + 3 * NQ * 1024, to, std::integral_constant<int, KU>{});
   };
   // values of a chunk's rows 8 g + 4 hh + r at a lane's column
   const int ld = MODE == 0 ? p.x_stride : p.proj_stride;
@@ -407,7 +525,9 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   using TX = typename std::conditional<MODE == 0, float, TY>::type;
   const uint32_t lx = (uint32_t)(4 * hh * ld + (MODE == 0 ? 0 : p.v_off) + h * V + col) * es;
   TX xn[16];
+  int odd_n;          // does a key or query of the chunk not split?
   auto values = [&](int c) {
+    odd_n = *(const int*)(frag_of(c) + (6 * NQ + 4) * 1024);
     const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
     const Rsrc rs = rows_of((MODE == 0 ? (const char*)p.xbc : (const char*)p.proj) + (size_t)t0 * ld * es,
                             (uint32_t)(n * ld * es));
@@ -421,8 +541,6 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   };
   const float dsk = MODE == 0 ? p.d_skip[h] : 0.f;
   float total = 0.f;   // log2 decay of the segment
-  stage(0, buf[0]);
-  values(0);
   // outputs transposed: row 8 g + 4 hh + r of the accumulator is a column of the state, lane li the
   // token.  They are written after the next chunk's wait, which would otherwise wait for them.
   f32x16 O;
@@ -442,33 +560,297 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         st4(o + 8 * g, O[4 * g], O[4 * g + 1], O[4 * g + 2], O[4 * g + 3]);
     }
   };
-  // (now and next are restrict so that the reads of one buffer are known not to touch the other:
-  // else every read would wait for the DMA under way)
-  auto step = [&](int c, const float4* __restrict__ now, float4* __restrict__ next) {
-    const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+  float x[16];
+  bool odd, apart;    // the chunk's keys or queries, its weighted values do not split
+  auto arrive = [&] {                 // what this wave requested, then every wave
     // (vmcnt 0, lgkmcnt 0, as a builtin: the compiler then knows that the values have arrived)
     __builtin_amdgcn_s_waitcnt(0x0070);
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();   // this chunk has landed; the other buffer is free
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    float x[16];
+  };
+  auto take = [&](int c) {            // the chunk's values; the next one's are requested
 #pragma unroll
     for (int s = 0; s < 16; ++s) x[s] = (float)xn[s];
-    if (c + 1 < chunks) {
-      stage(c + 1, next);
-      values(c + 1);
+    odd = __builtin_amdgcn_readfirstlane(odd_n) != 0;
+    if (c + 1 < chunks) values(c + 1);
+  };
+  // the fp32 entries 4 (f & 1) .. + 3 of a piece's parts
+  auto joined = [&](const bf16x8* parts, int f) {
+    typedef uint32_t Words __attribute__((ext_vector_type(2)));   // two entries each
+    const Words* at = (const Words*)(parts + (f >> 1) * 64) + (f & 1);
+    const Words a = at[0], b = at[NQ * 128], d = at[NQ * 256];
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t top = 0xffff0000u;
+      const float lo = (__uint_as_float(a[i] << 16) + __uint_as_float(b[i] << 16)) +
+                       __uint_as_float(d[i] << 16);
+      const float hi = (__uint_as_float(a[i] & top) + __uint_as_float(b[i] & top)) +
+                       __uint_as_float(d[i] & top);
+      v[2 * i] = odd ? __uint_as_float(a[i] << 16 | (b[i] & ~top)) : lo;
+      v[2 * i + 1] = odd ? __uint_as_float((a[i] & top) | b[i] >> 16) : hi;
     }
-    if (FULL && c > 0) write(c - 1);
-    const float4* cur = now + lane;
-    const float* sc = MODE == 0 ? (const float*)(now + (C0 + hw) * 64) : nullptr;
-    const float* we = MODE == 0 ? sc + 2 * kL : tb + 2 * kL;
-    const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
-    if (MODE == 0 && !FULL) total += sc[4 * kL - 1];
-    if (MODE == 1 && n < kL && lane < kL)
-      tb[2 * kL + lane] = lane < n ? tb[n - 1 - lane] : 0.f;   // (the last chunk)
-    akap::bf16x4 zb[kNorm ? 4 : 1];
-    float4 zf[kNorm ? 4 : 1];
-    if (FULL) {
+    return make_float4(v[0], v[1], v[2], v[3]);
+  };
+  auto part8 = [&](const float* v, bf16x8 (&to)[3]) {
+    const float e[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+    split8(e, to[0], to[1], to[2]);
+  };
+  // the values times their weights in the state after the chunk (the retention's are in k), and their
+  // parts
+  float xw[16];
+  bf16x8 w[2][3];
+  float4 w4[MODE == 0 ? 4 : 1];
+  auto fetch_weights = [&](const float* sc) {
+    if (MODE == 0) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) w4[g] = *(const float4*)(sc + 2 * kL + 8 * g + 4 * hh);
+    }
+  };
+  auto weigh = [&] {
+    float zero = 0.f, top = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float f[4] = {w4[MODE == 0 ? g : 0].x, w4[MODE == 0 ? g : 0].y, w4[MODE == 0 ? g : 0].z,
+                          w4[MODE == 0 ? g : 0].w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = MODE == 0 ? x[4 * g + r] * f[r] : x[4 * g + r];
+        xw[4 * g + r] = v;
+        zero = fmaf(v, 0.f, zero);
+        if (XP == 3) top = fmaxf(top, fabsf(v));
+      }
+    }
+    if (XP == 3) {      // (both halves' tokens: the last of a chunk have weights of their step sizes)
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false,
+                                                         false);
+      top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+    }
+    apart = __any(zero != 0.f || !splits(top));
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      // (parts of the unrounded product)
+      float rest[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int g = 2 * m + (i >> 2);
+        const float f = MODE == 0 ? (&w4[MODE == 0 ? g : 0].x)[i & 3] : 1.f;
+        w[m][0][i] = (bf16)xw[8 * m + i];
+        rest[i] = fmaf(x[8 * m + i], f, -(float)w[m][0][i]);
+      }
+      if (XP == 3) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          w[m][1][i] = (bf16)rest[i];
+          w[m][2][i] = (bf16)(rest[i] - (float)w[m][1][i]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
+    }
+  };
+  // the state after the chunk: dend S + k^T xw
+  auto advance = [&](const float4* kb, float dend) {
+    const bf16x8* kp = (const bf16x8*)kb + fresh(lane);
+    if (__builtin_expect(odd || apart, 0)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) S[t][i] *= dend;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const float4 a = joined(kp, 4 * t + g);
+          S[t] = mfma(a.x, xw[4 * g], S[t]);
+          S[t] = mfma(a.y, xw[4 * g + 1], S[t]);
+          S[t] = mfma(a.z, xw[4 * g + 2], S[t]);
+          S[t] = mfma(a.w, xw[4 * g + 3], S[t]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      return;
+    }
+    // piece u: rows 32 (u / 2) of the state, tokens 16 (u % 2) on; the next one's fragments are on
+    // their way while a piece's products run, the smallest first
+    bf16x8 k[2][3];
+    auto fetch = [&](int u) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) k[u & 1][i] = kp[(u + i * NQ) * 64];
+    };
+    auto decay = [&](int t) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S[t][i] *= dend;
+    };
+    fetch(0);
+    decay(0);
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      const int t = u >> 1, m = u & 1;
+      if (u + 1 < NQ) fetch(u + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int ka[6] = {2, 0, 1, 1, 0, 0}, wa[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int i = 0; i < 6; ++i)
+        if (wa[i] < XP) S[t] = mfma16(k[m][ka[i]], w[m][wa[i]], S[t]);
+      if (m == 0 && t + 1 < NT) {
+        decay(t + 1);
+        interleave<XP == 3 ? 6 : 3, XP == 3 ? 3 : 6>();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto outputs = [&](int c) {
+    const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+    const int lane_ = (int)fresh(lane), li = lane_ & 31, hh = lane_ >> 5;
+    const bf16x8* qp = (const bf16x8*)qbuf + lane_;
+    const float* sc = MODE == 0 ? (const float*)(qbuf + (C0 + hw) * 64) : nullptr;
+    bf16x8 q[2][3];                   // (the next fragments are on their way while a step's products run)
+    auto fetch = [&](int j) {
+#pragma unroll
+      for (int u = 0; u < 3; ++u) q[j & 1][u] = qp[(j + u * NQ) * 64];
+    };
+    fetch(0);
+    float P[16];
+    const float ch_i = MODE == 0 ? sc[3 * kL + li] : 0.f, cl_i = MODE == 0 ? sc[4 * kL + li] : 0.f;
+    const float e = MODE == 0 ? sc[kL + li] : tb[kL + li];
+    // q_i . k_j times the decay between the tokens (the scan's: and dt_j), for j = 8 g + 4 hh + 0..3
+    float4 pl[4];
+    auto fetch_pairs = [&](int g) {
+      pl[0] = qbuf[(G0 + g) * 64 + lane_];
+      if (MODE == 0) {
+        pl[1] = *(const float4*)(sc + 8 * g + 4 * hh);
+        pl[2] = *(const float4*)(sc + 3 * kL + 8 * g + 4 * hh);
+        pl[3] = *(const float4*)(sc + 4 * kL + 8 * g + 4 * hh);
+      } else {
+        pl[1] = *(const float4*)(pd + (g * 64 + lane_) * 4);
+      }
+    };
+    auto pair_weights = [&](int g) {
+      const float gv[4] = {pl[0].x, pl[0].y, pl[0].z, pl[0].w};
+      const float dt[4] = {pl[1].x, pl[1].y, pl[1].z, pl[1].w};
+      if (MODE == 0) {
+        // the sums as float pairs: a difference of sums then has the error of its own size
+        const float ch[4] = {pl[2].x, pl[2].y, pl[2].z, pl[2].w};
+        const float cl[4] = {pl[3].x, pl[3].y, pl[3].z, pl[3].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 8 * g + 4 * hh + r;
+          const float d = (ch_i - ch[r]) + (cl_i - cl[r]);
+          float f = gv[r] * (dt[r] * __builtin_amdgcn_exp2f(d));
+          // (d_skip x is the diagonal's share of the same product)
+          f += j == li ? dsk : 0.f;
+          asm("" : "+v"(f));     // a select, no branch
+          P[4 * g + r] = j <= li ? f : 0.f;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float f = gv[r] * dt[r];
+          asm("" : "+v"(f));
+          P[4 * g + r] = 8 * g + 4 * hh + r <= li ? f : 0.f;
+        }
+      }
+    };
+    f32x16 O2;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) O[i] = O2[i] = 0.f;
+    bf16x8 a[2][3];
+    uint32_t seen = 0;                // bits of the lane's part of the state
+    auto state_parts = [&](int j) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = S[j >> 1][8 * (j & 1) + i];
+        seen |= __float_as_uint(v[i]);
+      }
+      split8(v, a[j & 1][0], a[j & 1][1], a[j & 1][2]);
+    };
+    constexpr int PG = NQ / 4;        // steps per group of pairs
+    fetch_pairs(0);
+    state_parts(0);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      if (j + 1 < NQ) fetch(j + 1);
+      if (PG == 1 ? j > 0 : j % PG == 1 && j + 1 < NQ) fetch_pairs(PG == 1 ? j : j / PG + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma_split(a[j & 1], q[j & 1], O, O2);
+      if (j + 1 < NQ) state_parts(j + 1);
+      if (j % PG == 0) {
+        pair_weights(j / PG);
+        interleave<6, MODE == 0 ? 18 : 12>();
+      } else {
+        interleave<6, 9>();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    fetch_weights(sc);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XP == 3) {
+      // (values and weights would take as long to split)
+#pragma unroll
+      for (int s = 0; s < 16; ++s) O = mfma(x[s], P[s], O);
+      weigh();
+      interleave<16, 9>();
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        bf16x8 v, b[3];
+        part8(P + 8 * m, b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (bf16)x[8 * m + i];
+#pragma unroll
+        for (int u = 2; u >= 0; --u) O = mfma16(v, b[u], O);
+      }
+      weigh();
+    }
+    float fin = 0.f;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) fin = fmaf(O[s], 0.f, fin);
+    seen &= 0x7fffffffu;
+    if (__builtin_expect(odd || __any(fin != 0.f || (seen != 0 && seen < __float_as_uint(kWhole))), 0)) {
+      // an operand that does not split, or is not finite: the fp32 products
+#pragma unroll
+      for (int i = 0; i < 16; ++i) O[i] = 0.f;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 a = joined(qp, 4 * t + g);
+          O = mfma(S[t][4 * g], a.x, O);
+          O = mfma(S[t][4 * g + 1], a.y, O);
+          O = mfma(S[t][4 * g + 2], a.z, O);
+          O = mfma(S[t][4 * g + 3], a.w, O);
+        }
+#pragma unroll
+      for (int s = 0; s < 16; ++s) O[s] *= e;
+      // a value that is not finite must not reach the rows before its own (0 x inf)
+#pragma unroll 1
+      for (int i = 0; i < kL; ++i) {
+        f32x16 one = O;
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+          one = mfma(8 * (s >> 2) + 4 * hh + (s & 3) <= i ? x[s] : 0.f, P[s], one);
+#pragma unroll
+        for (int s = 0; s < 16; ++s) O[s] = li == i ? one[s] : O[s];
+      }
+    }
+  };
+  values(0);
+  if constexpr (FULL) {
+    stage_q(0);
+#pragma unroll 1
+    for (int c = 0; c < chunks; ++c) {
+      const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+      arrive();                       // the queries are there, the keys before were used
+      take(c);
+      stage_k(c, kbuf);
+      if (c > 0) write(c - 1);
+      akap::bf16x4 zb[kNorm ? 4 : 1];
+      float4 zf[kNorm ? 4 : 1];
       if (kNorm) {
         const TY* zr = (const TY*)p.proj + (size_t)(t0 + min(li, n - 1)) * p.proj_stride + p.g_off +
                        h * V + (wave % VW) * 32 + 4 * hh;
@@ -478,118 +860,26 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
           else zf[g] = *(const float4*)(zr + 8 * g);
         }
       }
-      // two chains: independent products in flight, and shorter sums
-      f32x16 O2;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) O[i] = O2[i] = 0.f;
-#pragma unroll
-      for (int f = 0; f < NF; f += 2) {
-        const int t = f >> 2, g = f & 3;
-        const float4 a = cur[f * 64], d = cur[(f + 1) * 64];
-        O = mfma(S[t][4 * g], a.x, O);
-        O2 = mfma(S[t][4 * g + 4], d.x, O2);
-        O = mfma(S[t][4 * g + 1], a.y, O);
-        O2 = mfma(S[t][4 * g + 5], d.y, O2);
-        O = mfma(S[t][4 * g + 2], a.z, O);
-        O2 = mfma(S[t][4 * g + 6], d.z, O2);
-        O = mfma(S[t][4 * g + 3], a.w, O);
-        O2 = mfma(S[t][4 * g + 7], d.w, O2);
-      }
-      float P[16];
-      const float ch_i = MODE == 0 ? sc[3 * kL + li] : 0.f, cl_i = MODE == 0 ? sc[4 * kL + li] : 0.f;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 g4 = cur[(G0 + g) * 64];
-        const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
-        if (MODE == 0) {
-          // the sums as float pairs: a difference of sums then has the error of its own size
-          const float4 d4 = *(const float4*)(sc + 8 * g + 4 * hh);
-          const float4 h4 = *(const float4*)(sc + 3 * kL + 8 * g + 4 * hh);
-          const float4 l4 = *(const float4*)(sc + 4 * kL + 8 * g + 4 * hh);
-          const float dt[4] = {d4.x, d4.y, d4.z, d4.w};
-          const float ch[4] = {h4.x, h4.y, h4.z, h4.w}, cl[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int j = 8 * g + 4 * hh + r;
-            const float d = (ch_i - ch[r]) + (cl_i - cl[r]);
-            float f = gv[r] * (dt[r] * __builtin_amdgcn_exp2f(d));
-            // (d_skip x is the diagonal's share of the same product)
-            f += j == li ? dsk : 0.f;
-            asm("" : "+v"(f));     // a select, no branch
-            P[4 * g + r] = j <= li ? f : 0.f;
-          }
-        } else {
-          const float4 d4 = *(const float4*)(pd + (g * 64 + lane) * 4);
-          const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float f = gv[r] * dd[r];
-            asm("" : "+v"(f));
-            P[4 * g + r] = 8 * g + 4 * hh + r <= li ? f : 0.f;
-          }
-        }
-      }
-      const float e = MODE == 0 ? sc[kL + li] : tb[kL + li];
-#pragma unroll
-      for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
-      // a value that is not finite must not reach the rows before its own (0 x inf)
-      float fin = 0.f;
-#pragma unroll
-      for (int s = 0; s < 16; ++s) fin = fmaf(x[s], 0.f, fin);
-      if (__builtin_expect(__any(fin != 0.f), 0)) {
-#pragma unroll 1
-        for (int i = 0; i < kL; ++i) {
-          f32x16 one = O;
-#pragma unroll
-          for (int s = 0; s < 16; ++s)
-            one = mfma(8 * (s >> 2) + 4 * hh + (s & 3) <= i ? x[s] : 0.f, P[s], one);
-#pragma unroll
-          for (int s = 0; s < 16; ++s) O[s] = li == i ? one[s] : O[s];
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) O = mfma(x[s], P[s], O);
-      }
-    }
-    // the state after the chunk
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) S[t][i] *= dend;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float4 w4 = *(const float4*)(we + 8 * g + 4 * hh);
-      const float xw[4] = {x[4 * g] * w4.x, x[4 * g + 1] * w4.y, x[4 * g + 2] * w4.z,
-                           x[4 * g + 3] * w4.w};
-      float4 k4[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) k4[t] = cur[(K0 + t * 4 + g) * 64];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].x, xw[0], S[t]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].y, xw[1], S[t]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].z, xw[2], S[t]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) S[t] = mfma(k4[t].w, xw[3], S[t]);
-    }
-    if (FULL) {
-      float inv = 1.f;
+      outputs(c);
+      const float* sc = MODE == 0 ? (const float*)(qbuf + (C0 + hw) * 64) : nullptr;
+      const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
+      // the head's root mean square: a lane's columns, the other half's, the other waves'
+      float* sq = ssq + (c & 1) * NW * kL;
       if (kNorm) {
-        // the head's root mean square: a lane's columns, the other half's, the other waves'
         float ss = 0.f;
 #pragma unroll
         for (int s = 0; s < 16; ++s) ss = fmaf(O[s], O[s], ss);
         ss += __shfl_xor(ss, 32, 64);
-        float* sq = ssq + (c & 1) * NW * kL;
         if (hh == 0) sq[wave * kL + li] = ss;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        ss = 0.f;
+      }
+      arrive();                       // the keys are there, the queries were used
+      if (c + 1 < chunks) stage_q(c + 1);
+      advance(kbuf, dend);
+      if (kNorm) {
+        float ss = 0.f;
 #pragma unroll
         for (int w = 0; w < VW; ++w) ss += sq[(hw * VW + w) * kL + li];
-        inv = 1.0f / sqrtf(ss / (float)V + p.eps);
+        const float inv = 1.0f / sqrtf(ss / (float)V + p.eps);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           float zv[4];
@@ -605,21 +895,46 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         }
       }
     }
-  };
+  } else {
+    auto stage = [&](int c, float4* to) {
+      stage_k(c, to);
+      stage_scalars(c, to + C0 * 64);
+    };
+    // (now and next are restrict so that the reads of one buffer are known not to touch the other:
+    // else every read would wait for the DMA under way)
+    auto step = [&](int c, const float4* __restrict__ now, float4* __restrict__ next) {
+      const int n = min(kL, r1 - (r0 + c * kL));
+      arrive();
+      take(c);
+      if (c + 1 < chunks) stage(c + 1, next);
+      const float* sc = MODE == 0 ? (const float*)(now + (C0 + hw) * 64) : nullptr;
+      const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
+      if (MODE == 0) total += sc[4 * kL - 1];
+      fetch_weights(sc);
+      weigh();
+      advance(now, dend);
+    };
+    stage(0, qbuf);
 #pragma unroll 1
-  for (int c = 0; c < chunks; ++c) step(c, buf[c & 1], buf[(c + 1) & 1]);
+    for (int c = 0; c < chunks; c += 2) {
+      step(c, qbuf, kbuf);
+      if (c + 1 < chunks) step(c + 1, kbuf, qbuf);
+    }
+  }
   if (FULL) write(chunks - 1);
   if (FULL && cut) return;   // the slots were written when the segments were joined
+  // (addresses formed anew: kept since the state was read they would take the loop's registers)
+  const uint32_t first_at = fresh(MODE == 0 ? 4 * hh * V + col : col * N + 4 * hh);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int row = 32 * t + 8 * g + 4 * hh;
+      const int row = 32 * t + 8 * g;
       if (MODE == 0) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sp[(size_t)(row + r) * V + col] = S[t][4 * g + r];
+        for (int r = 0; r < 4; ++r) sp[first_at + (row + r) * V] = S[t][4 * g + r];
       } else {
-        *(float4*)(sp + (size_t)col * N + row) = make_float4(S[t][4 * g], S[t][4 * g + 1],
+        *(float4*)(sp + first_at + row) = make_float4(S[t][4 * g], S[t][4 * g + 1],
                                                              S[t][4 * g + 2], S[t][4 * g + 3]);
       }
     }

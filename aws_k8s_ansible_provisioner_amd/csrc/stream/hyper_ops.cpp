@@ -208,7 +208,7 @@ void selective_scan(Tensor y, Tensor xbc, Tensor proj, int64_t dt_off, Tensor dt
     p.num_slots = (int)state.size(0);
     p.state = state.data_ptr<float>();
     const int64_t chunks = p.T / 32 + p.B;
-    p.frag_floats = 64 * p.N + 1024;
+    p.frag_floats = 96 * p.N + 1028;
     const auto opt = xbc.options();
     const Tensor frag = at::empty({chunks * p.KH * p.frag_floats}, opt);
     const Tensor scal = at::empty({chunks * p.H * 256}, opt);

@@ -254,7 +254,7 @@ struct RetentionParams {
 int retention_dreg(int D, int V);
 void launch_retention(RetentionParams p, bool f32, hipStream_t s);
 
-// ---- prompt chunks of the selective scan and the retention in fp32 matrix form (chunk_scan.hip) ----
+// ---- prompt chunks of the selective scan and the retention in matrix form (chunk_scan.hip) ----
 struct ChunkScanParams {
   int mode;                   // 0: selective scan, 1: retention
   const int32_t* q_start;     // [B + 1]
@@ -263,7 +263,7 @@ struct ChunkScanParams {
   int T, B, H, KH, V, N;      // KH: key heads (groups of the scan, heads of the retention)
   int num_slots;
   float* state;               // scan [slots, H, N, V], retention [slots, H, V, N]
-  // workspaces for T / 32 + B chunks: fragments [chunks, KH, frag_floats = 64 N + 1024], and for
+  // workspaces for T / 32 + B chunks: fragments [chunks, KH, frag_floats = 96 N + 1028], and for
   // the scan scalars [chunks, H, 256]
   float* frag;
   int frag_floats;

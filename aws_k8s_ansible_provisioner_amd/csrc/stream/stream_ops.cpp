@@ -848,7 +848,7 @@ void retention(Tensor out, Tensor proj, int64_t q_off, int64_t k_off, int64_t v_
     c.T = (int)T; c.B = p.num_seqs; c.H = c.KH = (int)H; c.V = (int)V; c.N = (int)D;
     c.num_slots = p.num_slots;
     c.state = p.state;
-    c.frag_floats = 64 * c.N + 1024;
+    c.frag_floats = 96 * c.N + 1028;
     const auto opt = state.options();
     const Tensor frag = at::empty({(T / 32 + c.B) * H * c.frag_floats}, opt);
     c.frag = frag.data_ptr<float>();

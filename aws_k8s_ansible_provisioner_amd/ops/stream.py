@@ -878,7 +878,7 @@ def recurrence_scratch_bytes(rows: int, seqs: int, heads: int, key_heads: int, v
     n = 0
     if value in (64, 128) and key in (64, 128):
         s = max(1, min(seqs, rows // 16))
-        n = (rows // 32 + s) * (key_heads * (64 * key + 1024) + (heads * 256 if scan else 0))
+        n = (rows // 32 + s) * (key_heads * (96 * key + 1028) + (heads * 256 if scan else 0))
         n += max(2 * rows // 256 + 2, rows // 256 + min(s, 768 * 32 // (heads * value) + 1)) \
             * heads * (value * key + 1)
     if not scan and rows >= RETENTION_SEGMENTED_ROWS:

@@ -1,4 +1,4 @@
-"""Prompt chunks of the selective scan and the retention in fp32 matrix form (GPU) against the same
+"""Prompt chunks of the selective scan and the retention in matrix form (GPU) against the same
 ops on CPU tensors: sequences around the chunk size of 32 rows and the segment size of 256, several
 sequences per step (some continued from their slots, one a padding sequence), steps whose long
 sequences are cut into segments and such that are walked whole, every head size of the matrix form, projections that are column slices of wider rows, and values that are not finite.
@@ -264,3 +264,73 @@ def test_scratch_stays_below_what_the_cache_leaves(lens, H, KH):
                                     None, decay, H, N, V, 1e-5))
     most = sops.recurrence_scratch_bytes(T, B, H, H, V, N, False)
     assert n <= most and (T < 16 * B or n > most / 8)
+
+
+def _marked(rows, what):
+    """Scan inputs over `rows` rows, one operand with entries that do not split into three bf16 parts."""
+    H, V, N = 2, 64, 128
+    inp = list(_scan_inputs(rows, 1, H, V, N, 1, torch.float32, 0, seed=11))
+    xbc, state = inp[0].clone(), inp[5].clone()
+    inp[2] = inp[2] - 3.0                              # steps below 1: no product with one overflows
+    x, k, q = xbc.split([H * V, N, N], 1)
+    big = 3.395e38                                     # above bf16's largest, finite
+    if what == "keys":
+        k[:, 5], q[:, 5] = big, 1e-30
+        x *= 1e-30
+    elif what == "queries":
+        q[40, 7], k[:, 7] = big, 1e-36
+        state[:, :, 7] *= 1e-36
+    elif what == "values":
+        x[:, 9], k[:] = big, k * 1e-36
+    elif what == "state":
+        state[0, 0, 3, 8], q[:, 3] = big, 1e-36
+    elif what == "small":
+        x *= 1e-36
+        state *= 1e-36
+    else:                                              # an entry of that operand is not finite
+        name, v = what.split()
+        {"keys": k, "queries": q}.get(name, x)[40, 6] = float(v)
+        if name == "state":
+            x[40, 6] = 0.5
+            state[0, 1, 4, 9] = float(v)
+    inp[0], inp[5] = xbc, state
+    return tuple(inp), H, V, N
+
+
+@pytest.mark.parametrize("rows", [49, 300, 1100])
+@pytest.mark.parametrize("what", ["keys", "queries", "values", "state", "small", "keys inf", "keys nan",
+                                  "queries -inf", "state inf", "state nan"])
+def test_operands_that_do_not_split(what, rows):
+    """Magnitudes past bf16's, values that are not finite, and values whose parts are denormal: the same
+    numbers as row by row, and the same entries not finite.  Sums in another order over about 150 fp32
+    terms: 2e-6 of a head's row; of the small ones 1e-5, as their last bits are denormal."""
+    inp, H, V, N = _marked(rows, what)
+    step = _step([rows], [6])
+    want = _run_scan(inp, step, H, V, N, 1, "cpu")
+    got = _run_scan(inp, step, H, V, N, 1, DEV)
+    for a, b in zip(got[:2], want[:2]):
+        a, ok = a.cpu(), torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), ok)
+        scale = float(b[ok].abs().max())
+        assert _rel(a[ok].double() / scale, b[ok].double() / scale) < (1e-5 if what == "small" else 4e-6)
+
+
+@pytest.mark.parametrize("what", ["values inf", "values nan", "keys inf", "keys large"])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_retention_operands_that_do_not_split(what, dt):
+    """The state after the step, whose entries no norm mixes: a key that is not finite spoils its row of
+    the state, a value its column."""
+    H, V, T = 2, 128, 100
+    g = torch.Generator().manual_seed(5)
+    proj = torch.randn(T, 4 * H * V, generator=g).to(dt)
+    name, v = what.split()
+    proj[37, (2 if name == "values" else 1) * H * V + 11] = {"large": 3e38}.get(v) or float(v)
+    args = (_step([T], [3]), H, V, V, (0, H * V, 2 * H * V, 3 * H * V), None,
+            torch.log2(torch.tensor([0.97, 0.5])))
+    st = torch.randn(1, H, V, V, generator=g)
+    want = _run_retention((proj, st), *args, "cpu")[1]
+    got = _run_retention((proj, st), *args, DEV)[1].cpu()
+    ok = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), ok)
+    scale = float(want[ok].abs().max())
+    assert _rel(got[ok].double() / scale, want[ok].double() / scale) < 4e-6
