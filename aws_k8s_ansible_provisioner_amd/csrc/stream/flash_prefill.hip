@@ -3,11 +3,13 @@
 // pieces): causal, with a lower bound of visible keys from chunks counted from position 0 and / or a
 // window, pooled entries before the window, a sink in the softmax's denominator, a gate per head.
 //
-// A workgroup takes NW units of (32 tokens, query head) of one key/value head: the heads of a group
-// beside each other, so that 8 waves with 4 heads to a group cover 64 tokens.  64 keys and values at
-// a time arrive by LDS-DMA while the 64 before are computed (two buffers, one barrier per step);
-// each staged byte feeds NW waves, where fragments taken straight from the caches cost every wave
-// its own loads.  S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_32x32x16_bf16: the key rows in the
+// A workgroup takes 4 units of (32 tokens, query head) of one key/value head: with 4 heads to a group
+// the heads of 32 tokens.  64 keys and values at a time arrive by LDS-DMA while the 64 before are
+// computed (two buffers, one barrier per step); each staged byte feeds 4 waves, where fragments taken
+// straight from the caches cost every wave its own loads.  Two workgroups of 4 waves on a CU instead of
+// one of 8 stage twice the bytes, but one starts or ends under the other's steps and a tile's masked
+// steps are fewer: 64 prompts of 256 tokens 81 -> 64 us, 8 of 2048 196 -> 187, the pooled prompts below
+// 172 -> 165.  S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_32x32x16_bf16: the key rows in the
 // order that makes a lane's weights whole 8-key value groups, so they become the next operand
 // without lane traffic.  The K rows are XOR-swizzled by the DMA's source address, the fragment
 // reads are free of bank conflicts.
@@ -18,11 +20,14 @@
 // finished sums in fp32 (as the start of the maximum, a sink above the scores would have every weight
 // rounded: 1.1 to 1.4 times the error); only the sink of score 0 starts maximum and sum.
 //
-// Bound by the vector work of the softmax beside the products (about 3400 cycles of exponentials,
-// maxima, roundings and rescaling per SIMD and step against 2048 of products): 8 x 2048 tokens, 16 / 4
-// heads of 128, causal: 200 us (0.69 PFLOP/s; fragments straight from the caches took 331), 5 prompts
-// of up to 3001 tokens through a window of 1024 and pooled blocks of 64: 172 us (553).  Tried for the
-// pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
+// Bound by what a SIMD can issue: per 64 keys and wave about 280 vector instructions at 2.4 to 4
+// cycles, 32 exponentials at 8.5, 32 products that take 10 of issue each, 32 fragment reads at 8; two
+// waves together 5000 cycles where their products alone are 2112.  A wave's products interleaved by hand
+// with the weights of the step before, or the two halves of the waves in opposite phases between
+// barriers, cost 5 to 15 % instead of gaining; without the rescaling of the sums 8 % less, without the
+// exponentials 5 %.  8 x 2048 tokens, 16 / 4 heads of 128, causal: 187 us (0.73 PFLOP/s; fragments
+// straight from the caches took 331), 5 prompts of up to 3001 tokens through a window of 1024 and pooled
+// blocks of 64: 165 us (553).  Tried for the pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
 // more, the step's body twice 170 us more (spills); roots and squares cost 4.
 #include <type_traits>
 
@@ -40,6 +45,7 @@ using akap::u32x4;
 namespace {
 
 constexpr int kKeys = 64;              // keys per step
+constexpr int NW = 4;                  // waves of a workgroup
 constexpr float kLog2e = 1.44269504088896f;
 constexpr float kLowest = -3.402823466e38f;   // a running maximum over no keys
 
@@ -69,7 +75,7 @@ __device__ __forceinline__ int swz(int key, int c) {
 }
 
 // POOL: the pooled form (positions given, pooled entries before the window if there are any)
-template <int D, int NW, bool POOL>
+template <int D, bool POOL>
 __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashParams p) {
   constexpr int KS = D / 16, DT = D / 32;       // contraction steps of a score, tiles of an output
   constexpr int PIECES = kKeys * D * 2 / 1024;  // 1-KB pieces of the keys (and of the values)
@@ -374,22 +380,13 @@ bool flash_prefill_sizes(int H, int G, int D, int Dv, int BS, int tile_rows, flo
 
 void launch_flash_prefill(const FlashParams& p, hipStream_t s) {
   if (p.num_tiles <= 0) return;
-  const int units = p.tile_rows / 32 * (p.H / p.G);
-  // 8 waves share the staged keys where the units divide among them
-#define AKAP_FP(DD, NW, PL)                                                                  \
-  flash_prefill_kernel<DD, NW, PL><<<dim3((unsigned)p.num_tiles * p.G * (units / NW)), 64 * NW, 0, \
-                                     s>>>(p)
-#define AKAP_FP_D(DD, PL)                 \
-  do {                                    \
-    if (units % 8 == 0) AKAP_FP(DD, 8, PL); \
-    else AKAP_FP(DD, 4, PL);              \
-  } while (0)
+  const dim3 grid((unsigned)p.num_tiles * p.G * (p.tile_rows / 32 * (p.H / p.G) / NW));
+#define AKAP_FP(DD, PL) flash_prefill_kernel<DD, PL><<<grid, 64 * NW, 0, s>>>(p)
   if (p.positions) {
-    if (p.D == 64) AKAP_FP_D(64, true); else AKAP_FP_D(128, true);
+    if (p.D == 64) AKAP_FP(64, true); else AKAP_FP(128, true);
   } else {
-    if (p.D == 64) AKAP_FP_D(64, false); else AKAP_FP_D(128, false);
+    if (p.D == 64) AKAP_FP(64, false); else AKAP_FP(128, false);
   }
-#undef AKAP_FP_D
 #undef AKAP_FP
 }
 
