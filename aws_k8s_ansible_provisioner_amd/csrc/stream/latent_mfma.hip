@@ -266,7 +266,7 @@ __global__ __launch_bounds__(64) void latent_decode_mfma_kernel(LatentAttnParams
 
 
 // ---- wide latents (R >= 256): four waves share one tile of 32 query columns
-// (Prompt chunks at R = 512, r = 64: latent_prefill.hip.)
+// (R = 512, r = 64: latent_prefill.hip, latent_decode.hip.)
 // At R = 512 a single wave's output accumulators alone are 256 registers.  Four waves split the
 // work of a 128-key step instead: wave w scores keys [32 w, 32 w + 32) of the step against the
 // whole query tile (S^T = K Q^T over all R + r dimensions), the waves agree on the running
@@ -672,12 +672,16 @@ template <int NV, int NKR>
 void launch_decode(const LatentAttnParams& p, hipStream_t s) {
   constexpr int DK = 32 * NV + 16 * NKR;
   const dim3 grid(p.B, (p.H + 31) / 32, p.num_parts);
-  if constexpr (NV >= 8)
+  int piece = NV >= 8 ? 128 : 32;                    // a partition is whole pieces of so many keys
+  if constexpr (NV == 16 && NKR == 4) {
+    launch_latent_decode_rows(p, s);
+    piece = 32;
+  } else if constexpr (NV >= 8)
     latent_decode_coop_kernel<NV, NKR><<<grid, 256, CoopSmem<NV, NKR>::bytes(p), s>>>(p);
   else
     latent_decode_mfma_kernel<NV, NKR><<<grid, 64, (size_t)32 * q_pitch(DK) * sizeof(bf16), s>>>(p);
   if (p.num_parts > 1)
-    latent_decode_merge_kernel<<<dim3(p.B, p.H), NV > 8 ? 128 : 64, 0, s>>>(p, NV >= 8 ? 128 : 32);
+    latent_decode_merge_kernel<<<dim3(p.B, p.H), NV > 8 ? 128 : 64, 0, s>>>(p, piece);
 }
 
 // ---- per-head products of small batches ------------------------------------------------------

@@ -176,6 +176,7 @@ bool latent_mfma_sizes(int R, int r);
 void launch_latent_prefill_mfma(const LatentAttnParams& p, hipStream_t s);
 void launch_latent_prefill_wide(const LatentAttnParams& p, hipStream_t s);   // R = 512, r = 64
 void launch_latent_decode_mfma(const LatentAttnParams& p, hipStream_t s);
+void launch_latent_decode_rows(const LatentAttnParams& p, hipStream_t s);    // R = 512, r = 64
 
 // out [H, T, N] (strides o_hs / o_ts) = a [H, T, K] (strides a_hs / a_ts, unit in k) x
 // w [H, N, K]^T, bf16, K % 16 == 0, N % 32 == 0, 16-byte aligned rows; meant for a few rows (one
