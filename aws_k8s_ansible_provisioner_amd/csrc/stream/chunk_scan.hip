@@ -183,6 +183,7 @@ __device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int r
 // idle SIMDs (8 x 2048 rows, 8 heads x 128 x 128, 256 waves otherwise: 264 us in segments; 64 heads x
 // 128 x 64, 1024 waves: 452 us whole).
 constexpr int kFill = 768;
+constexpr int kScanWaves = 2048, kRetentionWaves = 1024;   // see chunk_scan_piece()
 
 __device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
   if (n <= p.SEG) return true;
@@ -197,13 +198,13 @@ __device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
 }
 
 // first segment of sequence b in the buffers (long sequences alone have any): counted like the
-// entries, or, where most sequences are short, from 2 q_start[b] / SEG on (a long one of n rows has
-// at most 2 n / SEG of them)
-__host__ __device__ __forceinline__ bool few_long(int T, int B, int SEG) { return B > T / SEG + 2; }
+// entries, or, where most sequences are short, from 2 q_start[b] / PIECE on (a long one of n rows has
+// at most 2 n / PIECE of them)
+__host__ __device__ __forceinline__ bool few_long(int T, int B, int PIECE) { return B > T / PIECE + 2; }
 
 __device__ __forceinline__ size_t seg_base(const ChunkScanParams& p, int b) {
-  return few_long(p.T, p.B, p.SEG) ? (size_t)(2 * (int64_t)p.q_start[b] / p.SEG)
-                                   : (size_t)base_of(p.q_start, b, p.SEG);
+  return few_long(p.T, p.B, p.PIECE) ? (size_t)(2 * (int64_t)p.q_start[b] / p.PIECE)
+                                     : (size_t)base_of(p.q_start, b, p.PIECE);
 }
 
 // does a sequence whose first row is t go on from its slot's state?  (The scan's row form starts anew
@@ -442,11 +443,11 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   // SEGM: between workgroups that only leave, 24 sequences of 600 rows took 275 us and not 187)
   const int whole = SEGM && !FULL ? 0 : p.B * (p.H / HW);
   const bool cut = SEGM && (int)blockIdx.x >= whole;
-  const int entry = blockIdx.x - (cut ? whole : 0), entries = cut ? p.T / p.SEG + p.B : p.B;
+  const int entry = blockIdx.x - (cut ? whole : 0), entries = cut ? p.T / p.PIECE + p.B : p.B;
   const int h0 = entry / entries * HW, hw = wave / VW, h = h0 + hw;
   int b = entry % entries, r0, r1;
   if (cut) {
-    b = locate(p, b, p.SEG, r0, r1);
+    b = locate(p, b, p.PIECE, r0, r1);
   } else {
     b = uniform(b);
     r0 = ((ScalarInts)p.q_start)[b];
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   if (r1 <= r0) return;
   const int first = ((ScalarInts)p.q_start)[b];
   if (SEGM && walked_whole(p, ((ScalarInts)p.q_start)[b + 1] - first) == cut) return;
-  const size_t seg = cut ? (size_t)uniform((int)seg_base(p, b) + (r0 - first) / p.SEG) : 0;
+  const size_t seg = cut ? (size_t)uniform((int)seg_base(p, b) + (r0 - first) / p.PIECE) : 0;
   const int slot = uniform(p.seq_slot[first]);
   if (!live_slot(p, slot)) return;
   const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
@@ -952,7 +953,7 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
   if (r1 <= r0 || walked_whole(p, r1 - r0) || e >= hs) return;
   const int slot = p.seq_slot[r0];
   if (!live_slot(p, slot)) return;
-  const int nseg = (r1 - r0 + p.SEG - 1) / p.SEG;
+  const int nseg = (r1 - r0 + p.PIECE - 1) / p.PIECE;
   const size_t sb = seg_base(p, b);
   float4* st = (float4*)(p.state + ((size_t)slot * p.H + h) * hs + e);
   float4 prev = goes_on(p, r0) ? *st : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -989,7 +990,7 @@ void run(const ChunkScanParams& p, hipStream_t s) {
     chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
     return;
   }
-  const int segs = p.T / p.SEG + p.B;
+  const int segs = p.T / p.PIECE + p.B;
   chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<segs * (p.H / HW), nt, 0, s>>>(p);
   chunk_join_kernel<<<dim3(p.B, p.H, (p.V * p.N + 1023) / 1024), 256, 0, s>>>(p);
   chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<(p.B + segs) * (p.H / HW), nt, 0, s>>>(p);
@@ -1030,8 +1031,20 @@ int chunk_scan_segment(int mode, int T, int B, int H, int V) {
   return T - B >= 1024 && (mode == 1 || T < 256 * (int64_t)B) ? 256 : 0;
 }
 
-int64_t chunk_scan_segments(int T, int B, int SEG) {
-  return few_long(T, B, SEG) ? 2 * (int64_t)T / SEG + 2 : (int64_t)T / SEG + B;
+int chunk_scan_piece(int mode, int T, int B, int H, int V) {
+  // A segment's chunks are a serial chain, 256 rows of them 40 us; where the step's segments would leave
+  // SIMDs idle they are shorter.  Up to 1024 waves of the retention, one per SIMD (8 heads x 128 x 128:
+  // a prompt of 400 rows 66 us in segments of 256, 36 of 64; of 2000 76 and 51 of 128; four of 1000 84
+  // and 64 of 128, 69 of 64), 2048 of the scan, whose many heads make the steps coarse (64 heads x 128 x
+  // 64: a prompt of 400 rows 74 and 47; two of 1000 113 and 87 of 128; one of 2000 86 and 90).
+  const int64_t most = mode == 0 ? kScanWaves : kRetentionWaves;
+  for (int piece = 64; piece < 256; piece *= 2)
+    if (chunk_scan_segments(T, B, piece) * H * (V / 32) <= most) return piece;
+  return 256;
+}
+
+int64_t chunk_scan_segments(int T, int B, int PIECE) {
+  return few_long(T, B, PIECE) ? 2 * (int64_t)T / PIECE + 2 : (int64_t)T / PIECE + B;
 }
 
 void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s) {

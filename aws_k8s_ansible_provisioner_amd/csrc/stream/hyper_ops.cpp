@@ -214,9 +214,10 @@ void selective_scan(Tensor y, Tensor xbc, Tensor proj, int64_t dt_off, Tensor dt
     const Tensor scal = at::empty({chunks * p.H * 256}, opt);
     p.frag = frag.data_ptr<float>(); p.scal = scal.data_ptr<float>();
     p.SEG = akap_stream::chunk_scan_segment(p.mode, p.T, p.B, p.H, p.V);
+    p.PIECE = akap_stream::chunk_scan_piece(p.mode, p.T, p.B, p.H, p.V);
     Tensor seg, dec;
     if (p.SEG > 0) {
-      const int64_t segs = akap_stream::chunk_scan_segments(p.T, p.B, p.SEG);
+      const int64_t segs = akap_stream::chunk_scan_segments(p.T, p.B, p.PIECE);
       seg = at::empty({segs * p.H * p.N * p.V}, opt);
       dec = at::empty({segs * p.H}, opt);
       p.seg = seg.data_ptr<float>(); p.seg_decay = dec.data_ptr<float>();
@@ -435,10 +436,15 @@ void pooled_window_attention_prefill_mfma(Tensor out, Tensor q, Tensor k_cache, 
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(akap_stream, m) {
-  // rows per segment of a step of the selective scan (mode 0) or the retention (1), 0: none
+  // rows above which a sequence of a step of the selective scan (mode 0) or the retention (1) is cut, 0:
+  // none; rows per segment of a cut one
   m.def("chunk_scan_segment(int mode, int T, int B, int H, int V) -> int",
         [](int64_t mode, int64_t T, int64_t B, int64_t H, int64_t V) -> int64_t {
           return akap_stream::chunk_scan_segment((int)mode, (int)T, (int)B, (int)H, (int)V);
+        });
+  m.def("chunk_scan_piece(int mode, int T, int B, int H, int V) -> int",
+        [](int64_t mode, int64_t T, int64_t B, int64_t H, int64_t V) -> int64_t {
+          return akap_stream::chunk_scan_piece((int)mode, (int)T, (int)B, (int)H, (int)V);
         });
   m.def("hyper_step(Tensor(a!) out, Tensor(b!) xs, Tensor? ya, Tensor? yb, Tensor? bias, "
         "Tensor? mix, Tensor? w_out, Tensor w_in, Tensor norm_w, float eps, Tensor? fresh=None) "

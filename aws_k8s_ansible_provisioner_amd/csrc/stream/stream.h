@@ -269,11 +269,11 @@ struct ChunkScanParams {
   float* frag;
   int frag_floats;
   float* scal;
-  // sequences of more than SEG rows (0: none) in segments: chunk_scan_segments() states [H, N V] and
-  // decays [H]
+  // sequences of more than SEG rows (0: none) in segments of PIECE: chunk_scan_segments() states
+  // [H, N V] and decays [H]
   float* seg;
   float* seg_decay;
-  int SEG;
+  int SEG, PIECE;
   const void* proj;           // scan: step sizes at column dt_off; retention: q, k, v and gate
   int proj_stride;
   // selective scan
@@ -291,10 +291,12 @@ struct ChunkScanParams {
   float eps;
 };
 bool chunk_scan_sizes(int V, int N);
-// rows per segment of a step, 0: every sequence is walked whole
+// rows above which a sequence of the step is cut, 0: every sequence is walked whole
 int chunk_scan_segment(int mode, int T, int B, int H, int V);
+// rows per segment of a cut one
+int chunk_scan_piece(int mode, int T, int B, int H, int V);
 // segments that the long sequences of a step can have
-int64_t chunk_scan_segments(int T, int B, int SEG);
+int64_t chunk_scan_segments(int T, int B, int PIECE);
 void launch_chunk_scan(const ChunkScanParams& p, bool f32, hipStream_t s);
 
 struct TalkParams {

@@ -853,9 +853,10 @@ void retention(Tensor out, Tensor proj, int64_t q_off, int64_t k_off, int64_t v_
     const Tensor frag = at::empty({(T / 32 + c.B) * H * c.frag_floats}, opt);
     c.frag = frag.data_ptr<float>();
     c.SEG = akap_stream::chunk_scan_segment(c.mode, c.T, c.B, c.H, c.V);
+    c.PIECE = akap_stream::chunk_scan_piece(c.mode, c.T, c.B, c.H, c.V);
     Tensor sg, dec;
     if (c.SEG > 0) {
-      const int64_t segs = akap_stream::chunk_scan_segments(c.T, c.B, c.SEG);
+      const int64_t segs = akap_stream::chunk_scan_segments(c.T, c.B, c.PIECE);
       sg = at::empty({segs * H * V * D}, opt);
       dec = at::empty({segs * H}, opt);
       c.seg = sg.data_ptr<float>(); c.seg_decay = dec.data_ptr<float>();

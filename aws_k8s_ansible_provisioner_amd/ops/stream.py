@@ -873,14 +873,16 @@ def recurrence_scratch_bytes(rows: int, seqs: int, heads: int, key_heads: int, v
     """Upper bound of what one call of retention (or, scan, selective_scan) with up to `rows` rows of
     up to `seqs` sequences allocates beside its arguments: the buffers of the matrix form
     (csrc/stream/chunk_scan.hip: operand fragments and scalars per chunk of 32 rows, which take
-    steps of 16 rows a sequence and more, and states per segment of 256), and of the retention's
-    row form in segments."""
+    steps of 16 rows a sequence and more, and states per segment: of 256 rows, or of 64 and more where
+    those of all heads take up to 1024 waves of 32 columns, 2048 of the scan), and of the retention's row
+    form in segments."""
     n = 0
     if value in (64, 128) and key in (64, 128):
         s = max(1, min(seqs, rows // 16))
         n = (rows // 32 + s) * (key_heads * (96 * key + 1028) + (heads * 256 if scan else 0))
-        n += max(2 * rows // 256 + 2, rows // 256 + min(s, 768 * 32 // (heads * value) + 1)) \
-            * heads * (value * key + 1)
+        short = (2048 if scan else 1024) * 32 // (heads * value)
+        n += max(2 * rows // 256 + 2, rows // 256 + min(s, 768 * 32 // (heads * value) + 1),
+                 min(2 * rows // 64 + 2, short)) * heads * (value * key + 1)
     if not scan and rows >= RETENTION_SEGMENTED_ROWS:
         n = max(n, (rows // RETENTION_SEGMENT + seqs) * heads * value * key)
     return 4 * n

@@ -334,3 +334,27 @@ def test_retention_operands_that_do_not_split(what, dt):
     assert torch.equal(torch.isfinite(got), ok)
     scale = float(want[ok].abs().max())
     assert _rel(got[ok].double() / scale, want[ok].double() / scale) < 4e-6
+
+
+# lengths at whole segments of 64 and 128 rows and one beside them, continued and not; heads that take each
+@pytest.mark.parametrize("lens,starts", [([384, 1, 257, 420], [3, 0, 0, 8]), ([1025, 512, 63], [0, 5, 2])])
+@pytest.mark.parametrize("mode,H,piece", [(0, 8, 64), (0, 56, 128), (1, 4, 64), (1, 28, 128), (1, 64, 256)])
+def test_shorter_segments(lens, starts, mode, H, piece):
+    V = N = 64
+    T, B = sum(lens), len(lens)
+    step = _step(lens, starts)
+    assert torch.ops.akap_stream.chunk_scan_piece(mode, T, B, H, V) == piece
+    g = torch.Generator().manual_seed(T + H)
+    if mode == 0:
+        inp = _scan_inputs(T, B, H, V, N, 2, torch.bfloat16, 0, seed=T)
+        want = _run_scan(inp, step, H, V, N, 2, "cpu")
+        got = _run_scan(inp, step, H, V, N, 2, DEV)
+    else:
+        proj, state = torch.randn(T, 4 * H * V, generator=g), torch.randn(B, H, V, N, generator=g)
+        args = (step, H, N, V, (0, H * V, 2 * H * V, 3 * H * V), None,
+                torch.log2(torch.linspace(0.9, 0.999, H)))
+        want = _run_retention((proj, state), *args, "cpu")
+        got = _run_retention((proj, state), *args, DEV)
+    assert _rel(got[0], want[0]) < (2e-6 if mode == 0 else 4e-6)
+    for b in range(B):
+        assert _rel(got[1][b], want[1][b]) < 1e-5
