@@ -517,16 +517,16 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const ConvArgs a, co
   }
 }
 
-// eight channels per thread (16-byte accesses of bf16), TAPS at compile time: a tile of RB rows
+// eight channels per thread (16-byte accesses of bf16), TAPS at compile time: a tile of rb rows
 // inside one sequence is fetched four rows at a time ahead of its products; tiles with a
 // sequence's start or end go row by row with the history from the tile or the slot
 constexpr int kConvRows8 = 32;
 
 template <typename TO, int TAPS>
-__global__ __launch_bounds__(128) void conv_silu_vec8_kernel(const ConvArgs a) {
+__global__ __launch_bounds__(128) void conv_silu_vec8_kernel(const ConvArgs a, int rb) {
   const int c = (blockIdx.y * 128 + threadIdx.x) * 8;
   if (c >= a.C) return;
-  const int tb = blockIdx.x * kConvRows8, te = min(a.T, tb + kConvRows8);
+  const int tb = blockIdx.x * rb, te = min(a.T, tb + rb);
   const bf16* in = (const bf16*)a.proj + a.off + c;
   TO* out = (TO*)a.out + c;
   float w[TAPS][8], hist[TAPS][8], bias[8];          // hist[j]: the input TAPS - 1 - j rows back
@@ -1088,12 +1088,18 @@ void launch_conv_silu(void* out, bool out_f32, const void* proj, int proj_stride
                     (uintptr_t)proj % 16 == 0 && (uintptr_t)state % 16 == 0 && taps >= 2 &&
                     taps <= 4;
   if (vec8) {
-    const dim3 g8((T + kConvRows8 - 1) / kConvRows8, (C / 8 + 127) / 128);
+    // rows of a workgroup, a serial chain: as many as leave 700 workgroups (4352 channels: 400 rows 21 us
+    // with 32, 14 with 16, 10.5 with 8, 10 with 4; 1850 rows 31, 22, 21, 23; 3700 33, 30, 30, 36; 16384
+    // 108, 110, 117, 139)
+    const unsigned cols = (C / 8 + 127) / 128;
+    int rb = kConvRows8;
+    while (rb > 8 && (unsigned)(T / rb) * cols < 700) rb /= 2;
+    const dim3 g8((T + rb - 1) / rb, cols);
 #define AKAP_CONV8(TO)                                                           \
   do {                                                                           \
-    if (taps == 2) conv_silu_vec8_kernel<TO, 2><<<g8, 128, 0, s>>>(a);           \
-    else if (taps == 3) conv_silu_vec8_kernel<TO, 3><<<g8, 128, 0, s>>>(a);      \
-    else conv_silu_vec8_kernel<TO, 4><<<g8, 128, 0, s>>>(a);                     \
+    if (taps == 2) conv_silu_vec8_kernel<TO, 2><<<g8, 128, 0, s>>>(a, rb);           \
+    else if (taps == 3) conv_silu_vec8_kernel<TO, 3><<<g8, 128, 0, s>>>(a, rb);      \
+    else conv_silu_vec8_kernel<TO, 4><<<g8, 128, 0, s>>>(a, rb);                     \
   } while (0)
     if (out_f32) AKAP_CONV8(float);
     else AKAP_CONV8(bf16);

@@ -358,3 +358,23 @@ def test_shorter_segments(lens, starts, mode, H, piece):
     assert _rel(got[0], want[0]) < (2e-6 if mode == 0 else 4e-6)
     for b in range(B):
         assert _rel(got[1][b], want[1][b]) < 1e-5
+
+
+@pytest.mark.parametrize("T", [5, 130, 1500, 3300])
+@pytest.mark.parametrize("C,taps", [(1040, 4), (6200, 2)])
+def test_convolution_rows(T, C, taps):
+    """Every number of rows that a workgroup of the convolution takes, over sequence ends."""
+    lens = [T - T // 3 - 1, 1, T // 3]
+    q_start, pos, slot = _step(lens, [3, 0, 4])
+    g = torch.Generator().manual_seed(T)
+    proj = torch.randn(T, C + 8, generator=g).to(torch.bfloat16)
+    w, b = torch.randn(C, taps, generator=g), torch.randn(C, generator=g)
+    state = torch.randn(3, taps - 1, C, generator=g).to(torch.bfloat16)
+    got = []
+    for dev in ("cpu", DEV):
+        st, out = state.clone().to(dev), torch.zeros(T, C, device=dev)
+        sops.conv_silu(out, proj.to(dev), 8, w.to(dev), b.to(dev), st, slot.to(dev), pos.to(dev),
+                       q_start.to(dev))
+        got.append((out.cpu(), st.cpu()))
+    assert _rel(got[1][0], got[0][0]) < 1e-6        # four products in fp32 and an exponential
+    assert torch.equal(got[1][1], got[0][1])
