@@ -27,7 +27,7 @@
 // barriers, cost 5 to 15 % instead of gaining; without the rescaling of the sums 8 % less, without the
 // exponentials 5 %.  8 x 2048 tokens, 16 / 4 heads of 128, causal: 187 us (0.73 PFLOP/s; fragments
 // straight from the caches took 331), 5 prompts of up to 3001 tokens through a window of 1024 and pooled
-// blocks of 64: 165 us (553).  Tried for the pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
+// blocks of 64: 161 us (553).  Tried for the pooled form's small weights: the minimum of a step's scores and a branch to a full exponential 16 us
 // more, the step's body twice 170 us more (spills); roots and squares cost 4.
 #include <type_traits>
 
@@ -182,13 +182,13 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
 
-  // one step of 64 keys: scores against the staged keys, weights of those that `seen` admits.  Keys
-  // before klo or past khi are seen by no query of the wave (later tokens, and what a page's last owner
-  // left behind the sequence's end); a weight of 0 would not hide values that are not finite, so their
-  // groups are read as the nearest that the wave sees, and pooled entries, which every wave's queries
-  // see to another end, are cleared one by one.
+  // one step of 64 keys: scores against the staged keys, weights of those from lo to hi, a lane's own
+  // (masked: not all of them; low: some are before lo).  Keys before klo or past khi are seen by no query of
+  // the wave (later tokens, and what a page's last owner left behind the sequence's end); a weight of 0
+  // would not hide values that are not finite, so their groups are read as the nearest that the wave sees,
+  // and pooled entries, which every wave's queries see to another end, are cleared one by one.
   auto compute = [&](const bf16* kl, const bf16* vl, bool masked, int klo, int khi, auto pooled,
-                     auto seen) {
+                     bool low, int lo, int hi) {
     f32x16 s[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -220,17 +220,21 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     // maximum, weights and products of 32 keys at a time
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      float mx = -INFINITY;
       if (masked) {
+        if (32 * k > khi || 32 * k + 31 < klo) continue;   // (no lane sees any of them)
+        const int last = hi - 8 * hf, first = lo - 8 * hf;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          if (!seen(32 * k + 16 * (i >> 3) + 8 * hf + (i & 7))) s[k][i] = -INFINITY;
-          mx = fmaxf(mx, s[k][i]);
+        for (int i = 0; i < 16; ++i)
+          if (32 * k + 16 * (i >> 3) + (i & 7) > last) s[k][i] = -INFINITY;
+        if (low) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (32 * k + 16 * (i >> 3) + (i & 7) < first) s[k][i] = -INFINITY;
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[k][i]);
       }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[k][i]);
       mx = both_max(mx);
       const float m_new = fmaxf(m_run, POOL ? mx : mx * sc2);
       float sum[2] = {0.f, 0.f};
@@ -303,7 +307,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
       }
       __syncthreads();
       if (active && c0 < w_nb)
-        compute(kl, vl, c0 + kKeys > w_all, 0, min(w_nb - 1 - c0, kKeys - 1), std::true_type{}, [&](int key) { return c0 + key < mine; });
+        compute(kl, vl, c0 + kKeys > w_all, 0, min(w_nb - 1 - c0, kKeys - 1), std::true_type{},
+                false, 0, mine - 1 - c0);
     }
   }
 
@@ -320,8 +325,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     if (active && key0 <= w_last && key0 + kKeys > w_lo0) {
       const bf16* kl = lds + (t & 1) * kBuf;
       compute(kl, kl + kKeys * D, key0 + kKeys - 1 > w_first || key0 < w_lo1, max(w_lo0 - key0, 0),
-              min(w_last - key0, kKeys - 1), std::false_type{},
-              [&](int key) { return key0 + key <= limit && key0 + key >= lo_l; });
+              min(w_last - key0, kKeys - 1), std::false_type{}, key0 < w_lo1, lo_l - key0, limit - key0);
     }
   }
 
