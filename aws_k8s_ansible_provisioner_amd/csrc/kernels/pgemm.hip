@@ -47,8 +47,10 @@
 // and grouped rasterisation (8 M-tiles x N-tiles per block, M fastest), so the WGs of one XCD
 // stream the same K slices of 8 X panels and 4 W panels together (pg_tile).
 // Grouped (MoE): group g owns rows [offs[g-1], offs[g]) of X and weight W + g*N*K; the same
-// raster runs over the concatenated list of every group's M tiles; the grid is an upper bound
-// (sum of ceil(rows_g / 256) <= ceil(M / 256) + G) and surplus WGs exit.
+// raster runs over the concatenated list of every group's M tiles, the last round in quarters where it
+// has few tiles (pg_tile_cut); the grid is an upper bound
+// (sum of ceil(rows_g / 256) <= ceil(M / 256) + G) and surplus WGs exit.  A last round with few
+// tiles goes in quarters (pg_tile_cut).
 // With PGemmArgs.rows a tile's X rows are gathered by the DMA's per-lane offsets (a row's 128 bytes of
 // a K tile are one line wherever it lies): 16384 tokens of 2048, 2 of 8 experts of 1408 383 us up and
 // 238 us down; the 64 x 128 tiles of moe_dgemm.hip 626 and 290.
@@ -66,6 +68,8 @@ namespace akap {
 constexpr int PG_T = 256;        // tile rows / cols
 constexpr int PG_BK = 64;        // K tile
 constexpr int PG_THREADS = 512;  // 8 waves
+constexpr int kPgCus = 256;      // workgroups that run at a time, one per CU
+constexpr int kPgCut = 128;      // a last round of up to so many tiles goes in quarters (pg_tile_cut)
 constexpr int PG_BUF = 2 * PG_T * 8;  // 16-B units per LDS buffer (A 256 rows + W 256 rows)
 
 __device__ __forceinline__ int pg_unit(int row, int chunk) {
@@ -165,6 +169,51 @@ __device__ __forceinline__ bool pg_tile(const PGemmArgs& p, int& tm, int& tn, in
     }
     return false;
   }
+}
+
+// Grouped, with the last round of tiles cut: the tiles that go beyond a multiple of the CUs, where they are
+// few, run as four quarters each (pg_quarter), which spreads them over the CUs that would be idle.  The
+// tiles' number is known on the device alone, so every workgroup counts them; whole tiles go first.
+// quarter: -1, or 0 .. 3; the four of a tile are workgroups of one XCD.  A round of quarters takes less than
+// half a round of tiles, so up to 128 tiles are cut, two rounds of quarters: 8 experts of 1408 x 2048, 2 of
+// 8, both products of 1165 / 2679 / 5365 / 8657 tokens 118 / 176 / 229 / 382 us uncut, 112 / 148 / 219 / 341;
+// up to 64 119 / 149 / 225 / 340, up to 160 112 / 150 / 221 / 342.
+__device__ __forceinline__ bool pg_tile_cut(const PGemmArgs& p, int& tm, int& tn, int& group, int& row_lo,
+                                            int& row_hi, int& quarter) {
+  const int GM = p.gm > 0 ? p.gm : 8, tiles_n = p.N / PG_T;
+  int tiles_m = 0;
+  for (int g = 0, lo = 0; g < p.groups; ++g) {
+    const int hi = min(p.offs[g], p.M);
+    tiles_m += max((hi - lo + PG_T - 1) / PG_T, 0);
+    lo = hi;
+  }
+  const int all = tiles_m * tiles_n, rest = all % kPgCus;
+  const int whole = rest <= kPgCut ? all - rest : all;
+  const int b = blockIdx.x;
+  int id;
+  quarter = -1;
+  if (b < whole) {
+    id = xcd_remap(b, whole);
+  } else {
+    const int q = b - whole;
+    id = whole + (q >> 5) * 8 + (q & 7);
+    quarter = (q >> 3) & 3;
+    if (id >= all) return false;
+  }
+  const int per_block = GM * tiles_n, first_m = (id / per_block) * GM;
+  const int gm = min(tiles_m - first_m, GM), in = id % per_block;
+  int mt = first_m + in % gm;
+  tn = in / gm;
+  row_lo = 0;
+  for (group = 0;; ++group) {
+    row_hi = min(p.offs[group], p.M);
+    const int nt = max((row_hi - row_lo + PG_T - 1) / PG_T, 0);
+    if (mt < nt) break;
+    mt -= nt;
+    row_lo = row_hi;
+  }
+  tm = mt;
+  return true;
 }
 
 // The 256 x 256 main loop over K tiles [kt0, kt0 + nk): X rows from m0 (rows past the X
@@ -442,6 +491,80 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
   }
 }
 
+// A quarter of the tile: of every wave's 128 x 64 outputs the 64 rows hm and the 32 columns hn, so one
+// A and one W half-tile per K tile (32 KB), which the four half buffers hold three K tiles ahead.
+// Leaves its outputs in acc[0 .. 3][0 .. 1], summed as in the whole tile.
+template <bool SILU_ROWS, typename ACC>
+__device__ __forceinline__ void pg_quarter(bf16x8* lds, const __amdgpu_buffer_rsrc_t rx,
+                                           const __amdgpu_buffer_rsrc_t rw, int ldx, int K, int nhalf,
+                                           int m0, int n0, int hm, int hn, ACC& accs, const PgRows rows) {
+  auto& acc = accs.v;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w / 4, wn = w % 4, fr = lane & 15, fg = lane >> 4, nk = K / PG_BK;
+  uint32_t va[2], vw[2];
+  int da[2], dw[2];      // places in the first half of a buffer
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int q = 2 * w + e, ra = (q >> 3) * 128 + (q & 7) * 8, rw0 = (q >> 2) * 64 + (q & 3) * 8;
+    const int row = ra + hm * 64 + (lane >> 3), v = n0 + rw0 + hn * 32 + (lane >> 3);
+    int wr = v;
+    if constexpr (SILU_ROWS) wr = ((v >> 4) & 1) * nhalf + (v >> 5) * 16 + (v & 15);
+    va[e] = (uint32_t)((rows(m0 + row) * ldx + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2);
+    vw[e] = (uint32_t)((wr * K + ((lane & 7) ^ ((v >> 1) & 7)) * 8) * 2);
+    da[e] = ra * 8;
+    dw[e] = PG_T * 8 + rw0 * 8;
+  }
+  auto issue = [&](int j) {
+    if (j >= nk) return;
+    bf16x8* buf = lds + (j & 1) * PG_BUF;
+    const int half = (j >> 1) & 1;
+    const uint32_t kb = (uint32_t)(j * PG_BK * 2);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rx, (__attribute__((address_space(3))) void*)(buf + da[e] + half * 64 * 8), 16, va[e], kb, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rw, (__attribute__((address_space(3))) void*)(buf + dw[e] + half * 32 * 8), 16, vw[e], kb, 0, 0);
+#endif
+  };
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  issue(0);
+  issue(1);
+  issue(2);
+  for (int t = 0; t < nk; ++t) {
+    if (t + 2 < nk) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (t + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    pg_sync();  // every wave's pieces of t landed; every read of tile t - 1 (slot of t + 3) retired
+    issue(t + 3);
+    const bf16x8* buf = lds + (t & 1) * PG_BUF;
+    const int half = (t >> 1) & 1;
+    bf16x8 a[4][2], b[2][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i][s] = buf[pg_unit(wm * 128 + half * 64 + i * 16 + fr, fg + 4 * s)];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        b[j][s] = buf[PG_T * 8 + pg_unit(wn * 64 + half * 32 + j * 16 + fr, fg + 4 * s)];
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j][s], a[i][s], acc[i][j], 0, 0, 0);
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // SCHED 3: the unit-pipelined 4-wave body (4 waves of 128 x 128, one wave per SIMD, 256
 // accumulators, every LDS fragment read and every LDS-DMA piece issued BETWEEN MFMAs, 3 vmcnt
@@ -585,6 +708,23 @@ __device__ __forceinline__ void pg_mainloop_u(bf16x8* lds, const __amdgpu_buffer
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-DMA outlives the main loop
 }
 
+__device__ __forceinline__ void pg_store(bf16* to, f32x4 y) {
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = f2bf(y[r]);
+  *reinterpret_cast<bf16x4*>(to) = o;
+}
+__device__ __forceinline__ void pg_store_silu(bf16* to, f32x4 gate, f32x4 up) {
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float g = bf2f(f2bf(gate[r]));
+    const float u = bf2f(f2bf(up[r]));
+    o[r] = f2bf(bf2f(f2bf(g / (1.f + __expf(-g)))) * u);
+  }
+  *reinterpret_cast<bf16x4*>(to) = o;
+}
+
 template <int EPI, bool GROUPED, int NB, int WAVES, int SCHED = 1>
 __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   using G = PgGeo<WAVES>;
@@ -596,8 +736,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   const int fr = lane & 15, fg = lane >> 4;
 
   // ---- tile of this workgroup --------------------------------------------------------------
-  int tm, tn, group, row_lo, row_hi;
-  if (!pg_tile<GROUPED>(p, tm, tn, group, row_lo, row_hi)) return;  // surplus WG (uniform)
+  constexpr bool CUT = GROUPED && WAVES == 8 && SCHED == 4;
+  int tm, tn, group, row_lo, row_hi, quarter = -1;
+  if constexpr (CUT) {
+    if (!pg_tile_cut(p, tm, tn, group, row_lo, row_hi, quarter)) return;   // surplus WG (uniform)
+  } else {
+    if (!pg_tile<GROUPED>(p, tm, tn, group, row_lo, row_hi)) return;
+  }
   const int m0 = row_lo + tm * PG_T, n0 = tn * PG_T;
   const bf16* X = static_cast<const bf16*>(p.X);
   const bf16* W = static_cast<const bf16*>(p.W) + (GROUPED ? (size_t)group * p.N * p.K : 0);
@@ -609,6 +754,25 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   if (GROUPED) rows = {p.rows, p.top, row_hi};
   PgAcc<2 * PgGeo<WAVES>::NJ> accs;
   auto& acc = accs.v;
+  bf16* Y = static_cast<bf16*>(p.Y);
+  if constexpr (CUT) {
+    if (quarter >= 0) {
+      const int hm = quarter & 1, hn = quarter >> 1;
+      pg_quarter<EPI == EPI_SILU>(lds, rx, rw, p.ldx, p.K, p.N >> 1, m0, n0, hm, hn, accs, rows);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = m0 + wm * 128 + hm * 64 + i * 16 + fr;
+        if (row >= row_hi) continue;
+        if constexpr (EPI == EPI_SILU)
+          pg_store_silu(Y + (size_t)row * p.ldy + (n0 >> 1) + wn * 32 + hn * 16 + fg * 4, acc[i][0], acc[i][1]);
+        else
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            pg_store(Y + (size_t)row * p.ldy + n0 + wn * 64 + hn * 32 + j * 16 + fg * 4, acc[i][j]);
+      }
+      return;
+    }
+  }
   if constexpr (SCHED == 3) {
     static_assert(WAVES == 4, "the unit-pipelined body is the 4-wave 128 x 128 form");
     const int nu = p.K / 32;
@@ -624,7 +788,6 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   }
 
   // ---- epilogue: lane holds rows wm*128 + i*16 + fr, 4 consecutive cols per fragment ---------
-  bf16* Y = static_cast<bf16*>(p.Y);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int row = m0 + wm * 128 + i * 16 + fr;
@@ -632,26 +795,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
     if constexpr (EPI == EPI_SILU) {
       // fragments j (gate) and j+1 (up) of one 32-column group -> 16 output columns
 #pragma unroll
-      for (int jj = 0; jj < NJ; ++jj) {
-        const int col = (n0 >> 1) + wn * (G::WCOLS / 2) + jj * 16 + fg * 4;
-        bf16x4 o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float g = bf2f(f2bf(acc[i][2 * jj][r]));
-          const float u = bf2f(f2bf(acc[i][2 * jj + 1][r]));
-          o[r] = f2bf(bf2f(f2bf(g / (1.f + __expf(-g)))) * u);
-        }
-        *reinterpret_cast<bf16x4*>(Y + (size_t)row * p.ldy + col) = o;
-      }
+      for (int jj = 0; jj < NJ; ++jj)
+        pg_store_silu(Y + (size_t)row * p.ldy + (n0 >> 1) + wn * (G::WCOLS / 2) + jj * 16 + fg * 4,
+                      acc[i][2 * jj], acc[i][2 * jj + 1]);
     } else {
 #pragma unroll
-      for (int j = 0; j < 2 * NJ; ++j) {
-        const int col = n0 + wn * G::WCOLS + j * 16 + fg * 4;
-        bf16x4 o;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = f2bf(acc[i][j][r]);
-        *reinterpret_cast<bf16x4*>(Y + (size_t)row * p.ldy + col) = o;
-      }
+      for (int j = 0; j < 2 * NJ; ++j)
+        pg_store(Y + (size_t)row * p.ldy + n0 + wn * G::WCOLS + j * 16 + fg * 4, acc[i][j]);
     }
   }
 }
@@ -963,8 +1113,12 @@ void launch_pgemm(const PGemmArgs& a, int epi, hipStream_t st) {
     return;
   }
   if (pgemm_sched() == 4) {  // stream-first body (AKAP_PGEMM_WAVES 8 | 4)
-    if (pgemm_waves() == 4) launch_pgemm_w<4, 4>(p, epi, grid, st);
-    else launch_pgemm_w<8, 4>(p, epi, grid, st);
+    if (pgemm_waves() == 4) {
+      launch_pgemm_w<4, 4>(p, epi, grid, st);
+    } else {
+      // (three workgroups more per tile that may be cut, and whole rows of eight tiles)
+      launch_pgemm_w<8, 4>(p, epi, p.groups > 0 ? grid + 3 * min(grid, kPgCut) + 28 : grid, st);
+    }
     return;
   }
   // two barriers per K tile (measured 1-4 % faster than four, profiles/r4_pgemm_nb_ab.log); the
