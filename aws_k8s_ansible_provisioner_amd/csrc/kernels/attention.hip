@@ -452,6 +452,9 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
     __builtin_amdgcn_sched_barrier(0);
   }
   const int pend = min(kv_len, pstart + p.part_size);
+  // A partition without keys: the reduction reads those with keys alone.  A step is cut for the longest
+  // sequence the model allows, so most partitions of short ones are empty.
+  if (p.num_parts > 1 && pstart >= kv_len) return;
   ChunkT<F8> cur;
   {
     // issued unconditionally (a wave with no chunk reads block 0, never used): a branch here
@@ -1126,8 +1129,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
     }
 }
 
-// Combine split-KV partitions: grid (num_seqs, Hkv), 256 threads = (16 rows x 16 lanes x 8 dims).
+// Combine split-KV partitions: grid (num_seqs, Hkv), 256 threads = (16 rows x 16 lanes x 8 dims).  Bound by
+// the latency of its reads: eight partitions' maxima, sums and rows are requested together.
 __global__ __launch_bounds__(256) void paged_attn_reduce_kernel(AttnParams p) {
+  constexpr int U = 8;
   const int seq = blockIdx.x;
   const int kvh = blockIdx.y;
   const int G = p.G;
@@ -1135,26 +1140,52 @@ __global__ __launch_bounds__(256) void paged_attn_reduce_kernel(AttnParams p) {
   const int d0 = (threadIdx.x & 15) * 8;
   if (row >= G) return;
   const int kv_len = p.seq_lens[seq];
+  const int q_tok = p.q_start ? p.q_start[seq] : seq;
   const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
   const size_t base = ((size_t)(seq * p.Hkv + kvh) * p.num_parts) * G + row;
   float M = -1e30f;
-  for (int q = 0; q < nparts; ++q) M = fmaxf(M, p.part_m[base + (size_t)q * G]);
   float L = 0.f;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int q = 0; q < nparts; ++q) {
-    const size_t idx = base + (size_t)q * G;
-    const float f = exp2f(p.part_m[idx] - M) * p.part_l[idx];
-    L += f;
-    const f32x4* po = reinterpret_cast<const f32x4*>(p.part_o + idx * kD + d0);
-    f32x4 a = po[0], b = po[1];
+  if (nparts > 0) {
+    float m[U], l[U];
+    f32x4 o[U][2];
+    auto load = [&](int q0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[j] += f * a[j];
-      acc[4 + j] += f * b[j];
+      for (int u = 0; u < U; ++u) {
+        const size_t idx = base + (size_t)min(q0 + u, nparts - 1) * G;
+        m[u] = p.part_m[idx];
+        l[u] = p.part_l[idx];
+        const f32x4* po = reinterpret_cast<const f32x4*>(p.part_o + idx * kD + d0);
+        o[u][0] = po[0];
+        o[u][1] = po[1];
+      }
+    };
+    load(0);
+    for (int q0 = U; q0 < nparts; q0 += U) {
+      float x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = p.part_m[base + (size_t)min(q0 + u, nparts - 1) * G];
+#pragma unroll
+      for (int u = 0; u < U; ++u) M = fmaxf(M, x[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) M = fmaxf(M, m[u]);
+    for (int q0 = 0; q0 < nparts; q0 += U) {
+      if (q0 > 0) load(q0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (q0 + u >= nparts) break;
+        const float f = exp2f(m[u] - M) * l[u];
+        L += f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc[j] += f * o[u][0][j];
+          acc[4 + j] += f * o[u][1][j];
+        }
+      }
     }
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  const int q_tok = p.q_start ? p.q_start[seq] : seq;
   bf16* op = p.out + ((size_t)q_tok * p.Hq + kvh * G + row) * kD + d0;
   bf16x8 o8;
 #pragma unroll

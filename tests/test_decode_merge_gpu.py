@@ -100,3 +100,32 @@ def test_talking_attention(dtype, parts, H, G, D, Dv):
         sops.talking_attention_decode(got, *dev, mix.cuda() if mix is not None else None, gate.cuda(),
                                       D ** -0.5, ws, parts)
         _close(got, want, dtype)
+
+
+@pytest.mark.parametrize("part_size,parts", [(768, 3), (256, 9), (128, 18), (128, 33), (512, 64)])
+@pytest.mark.parametrize("G", [1, 2, 4])
+def test_paged_attention(part_size, parts, G):
+    """Against the same kernel unsplit.  A weight is rounded to bf16 against its partition's maximum, so to
+    other bits than unsplit: at most 2^-9 of it on either side, 2^-8 of the weighted mean of |v| in all;
+    the outputs are rounded once on either side."""
+    from aws_k8s_ansible_provisioner_amd import ops
+
+    g = torch.Generator().manual_seed(parts)
+    bt, sl, NB = _table(g)
+    H, D, T, bf = 3, 128, len(LENS), torch.bfloat16
+    k = torch.randn(NB, H, BS, D, generator=g).to(bf).cuda()
+    v = torch.randn(NB, H, BS // 8, D, 8, generator=g).to(bf).cuda()
+    q = torch.randn(T, H * G, D, generator=g).to(bf).cuda()
+    bt, sl = bt.cuda(), sl.cuda()
+    got, want = (torch.full((T, H * G, D), 7.0, dtype=bf, device="cuda") for _ in range(2))
+    ops.paged_attention_decode(want, q, k, v, bt, sl, G, D ** -0.5, part_size=2304)
+    ws = ops.decode_workspace(T, H, G, parts, "cuda")
+    for t in ws:
+        t.fill_(float("nan"))
+    ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, ws, parts, part_size)
+    got, want = got.float(), want.float()
+    assert bool((got[2] == 0).all()) and bool((want[2] == 0).all())       # a row without keys
+    mag = torch.empty_like(q)
+    ops.paged_attention_decode(mag, q, k, v.abs(), bt, sl, G, D ** -0.5, part_size=2304)
+    assert bool(((got - want).abs() <= 2.0 ** -8 * (1.02 * mag.float() + want.abs())).all())
+    assert (got - want).norm() <= 6e-3 * want.norm()      # independent roundings, as above
