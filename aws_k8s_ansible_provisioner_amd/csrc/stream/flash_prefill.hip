@@ -3,8 +3,9 @@
 // pieces): causal, with a lower bound of visible keys from chunks counted from position 0 and / or a
 // window, pooled entries before the window, a sink in the softmax's denominator, a gate per head.
 //
-// A workgroup takes 4 units of (32 tokens, query head) of one key/value head: with 4 heads to a group
-// the heads of 32 tokens.  64 keys and values at a time arrive by LDS-DMA while the 64 before are
+// Four waves, a team, take 4 units of (32 tokens, query head) of one key/value head: with 4 heads to a
+// group the heads of 32 tokens; a workgroup is one team, or in small grids two that take the steps in turn
+// and add up their sums at the end.  64 keys and values at a time arrive by LDS-DMA while the 64 before are
 // computed (two buffers, one barrier per step); each staged byte feeds 4 waves, where fragments taken
 // straight from the caches cost every wave its own loads.  Two workgroups of 4 waves on a CU instead of
 // one of 8 stage twice the bytes, but one starts or ends under the other's steps and a tile's masked
@@ -45,7 +46,8 @@ using akap::u32x4;
 namespace {
 
 constexpr int kKeys = 64;              // keys per step
-constexpr int NW = 4;                  // waves of a workgroup
+constexpr int NW = 4;                  // waves of a team
+constexpr int kTeamSteps = 4;          // steps up to which one team takes them all
 constexpr float kLog2e = 1.44269504088896f;
 constexpr float kLowest = -3.402823466e38f;   // a running maximum over no keys
 
@@ -75,14 +77,15 @@ __device__ __forceinline__ int swz(int key, int c) {
 }
 
 // POOL: the pooled form (positions given, pooled entries before the window if there are any)
-template <int D, bool POOL>
-__global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashParams p) {
+// TEAMS: of four waves, which take the steps in turn
+template <int D, bool POOL, int TEAMS>
+__global__ __launch_bounds__(64 * NW * TEAMS, 2) void flash_prefill_kernel(const FlashParams p) {
   constexpr int KS = D / 16, DT = D / 32;       // contraction steps of a score, tiles of an output
   constexpr int PIECES = kKeys * D * 2 / 1024;  // 1-KB pieces of the keys (and of the values)
   constexpr int PW = PIECES / NW;               // of a wave
   static_assert(PIECES % NW == 0 && PW >= 1, "pieces");
   constexpr int kBuf = 2 * kKeys * D;           // elements of a buffer: keys, values
-  __shared__ __align__(16) bf16 lds[2 * kBuf];
+  __shared__ __align__(16) bf16 lds_all[TEAMS * 2 * kBuf];
   const int rep = p.H / p.G;
   const int subs = p.tile_rows / 32;            // 32-token pieces of a tile
   const int parts = subs * rep / NW;
@@ -91,8 +94,10 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int flat = (int)gridDim.x - 1 - (int)blockIdx.x;
   const int tile = flat / (p.G * parts), rest = flat - tile * (p.G * parts);
   const int part = rest / p.G, g = rest - part * p.G;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & (64 * NW - 1), lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);      // in its team
+  const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / (64 * NW)) : 0;
+  bf16* const lds = lds_all + team * 2 * kBuf;
   const int r = lane & 31, hf = lane >> 5;
   const int b = __builtin_amdgcn_readfirstlane(p.tile_seq[tile]);
   if (b < 0 || b >= p.B) return;                        // (every exit here is the workgroup's)
@@ -101,7 +106,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int ctx = p.positions ? (int)p.positions[q0] : p.seq_lens[b] - q_len;
   if (ctx < 0 && !p.positions) return;                  // fewer keys than rows
   const int kv_len = ctx + q_len;
-  const int unit = part * NW + w, sub = unit / rep, h = g * rep + unit - sub * rep;
+  const int item = part * NW + w, sub = item / rep, h = g * rep + item - sub * rep;
   const int tok0 = p.tile_row[tile] + 32 * sub;        // the wave's first token of the chunk
   const int tok = tok0 + r;
   const bool valid = tok < q_len, active = tok0 < q_len;
@@ -121,6 +126,9 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
   const int key_first = lower(ctx + g_tok0) & ~31;      // staging starts at a 32-key piece
   const int w_lo0 = lower(w_first), w_lo1 = lower(w_last);
   const int steps = max((g_last - key_first) / kKeys + 1, 1);
+  // teams at work: few steps are not worth the second's sums
+  const int teams = TEAMS > 1 && steps > kTeamSteps ? 2 : 1;
+  if (team >= teams) return;
   const int32_t* bt = p.block_tables + (size_t)b * p.max_blocks;
   const int BS = p.BS, G = p.G;
   const int last_piece = max(kv_len - 1, 0) >> 5;
@@ -153,8 +161,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
 #pragma unroll
     for (int i = 0; i < PW; ++i) dma16(vb + voff[i], vl + (w * PW + i) * 512);
   };
-  stage(0, 0, page_of(0));
-  int page_next = page_of(1);
+  stage(team, 0, page_of(team));
+  int page_next = page_of(team + teams);
 
   bf16x8 qf[KS];
   {
@@ -174,8 +182,9 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     const float root = __builtin_amdgcn_exp2f(below * (0.5f * sc2));
     return root * root;
   };
-  float m_run = p.unit_sink ? 0.f : kLowest;
-  float l_run = p.unit_sink && hf == 0 ? 1.f : 0.f;   // (a lane's own keys; the halves meet at the end)
+  const bool unit = p.unit_sink && team == 0;
+  float m_run = unit ? 0.f : kLowest;
+  float l_run = unit && hf == 0 ? 1.f : 0.f;   // (a lane's own keys; the halves meet at the end)
   f32x16 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d)
@@ -283,7 +292,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     const int mine = valid ? before(pos) : 0;          // (the wave's last and first token above)
     bf16* kl = lds + kBuf;
     bf16* vl = kl + kKeys * D;
-    for (int c0 = 0; c0 < nb; c0 += kKeys) {
+    for (int ca = 0; ca < nb; ca += teams * kKeys) {
+      const int c0 = ca + team * kKeys;
       constexpr int F4 = D / 4, NE = kKeys * F4 / (64 * NW);   // float4 pieces of a row, per thread
       float4 kk[NE], vv[NE];
 #pragma unroll
@@ -295,7 +305,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
         vv[u] = *(const float4*)(p.v_pool + at);
         if (c0 + key >= nb) vv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
       }
-      if (c0 > 0) __syncthreads();            // every wave has read the 64 before
+      if (ca > 0) __syncthreads();            // every wave has read the 64 before
 #pragma unroll
       for (int u = 0; u < NE; ++u) {
         const int e = u * 64 * NW + tid, key = e / F4, d = (e % F4) * 4;
@@ -312,25 +322,50 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_prefill_kernel(const FlashPa
     }
   }
 
-  for (int t = 0; t < steps; ++t) {
+  for (int u = 0; u * teams < steps; ++u) {
+    const int t = u * teams + team;
     // step t has landed for this wave; every wave has read the buffer that step t + 1 goes to
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    if (t + 1 < steps) {
-      stage(t + 1, (t + 1) & 1, page_next);
-      page_next = page_of(t + 2);
+    if (t + teams < steps) {
+      stage(t + teams, (u + 1) & 1, page_next);
+      page_next = page_of(t + 2 * teams);
     }
     const int key0 = key_first + t * kKeys;
-    if (active && key0 <= w_last && key0 + kKeys > w_lo0) {
-      const bf16* kl = lds + (t & 1) * kBuf;
+    if (t < steps && active && key0 <= w_last && key0 + kKeys > w_lo0) {
+      const bf16* kl = lds + (u & 1) * kBuf;
       compute(kl, kl + kKeys * D, key0 + kKeys - 1 > w_first || key0 < w_lo1, max(w_lo0 - key0, 0),
               min(w_last - key0, kKeys - 1), std::false_type{}, key0 < w_lo1, lo_l - key0, limit - key0);
     }
   }
 
-  if (!active) return;
   l_run = both_sum(l_run);
+  if (TEAMS > 1 && teams > 1) {
+    // the second team's maxima and sums into the first's, through the buffers
+    float* to = (float*)lds_all + w * (16 * DT + 2) * 64 + lane;
+    __syncthreads();
+    if (team == 1) {
+      to[0] = m_run;
+      to[64] = l_run;
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) to[(2 + 16 * d + i) * 64] = o[d][i];
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float m1 = to[0], m = fmaxf(m_run, m1);
+    const float fa = POOL ? weight(m_run - m) : __builtin_amdgcn_exp2f(m_run - m);
+    const float fb = POOL ? weight(m1 - m) : __builtin_amdgcn_exp2f(m1 - m);
+    l_run = l_run * fa + to[64] * fb;
+    m_run = m;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] = o[d][i] * fa + to[(2 + 16 * d + i) * 64] * fb;
+  }
+  if (!active) return;
   float corr = 1.f;
   if (p.sink) {
     const float sk = p.sink[h], mk = m_run * 0.693147180559945f;   // back from log2 units
@@ -385,7 +420,16 @@ bool flash_prefill_sizes(int H, int G, int D, int Dv, int BS, int tile_rows, flo
 void launch_flash_prefill(const FlashParams& p, hipStream_t s) {
   if (p.num_tiles <= 0) return;
   const dim3 grid((unsigned)p.num_tiles * p.G * (p.tile_rows / 32 * (p.H / p.G) / NW));
-#define AKAP_FP(DD, PL) flash_prefill_kernel<DD, PL><<<grid, 64 * NW, 0, s>>>(p)
+  // Two teams of four waves, which take the steps in turn, where the grid leaves CUs to one team each: a
+  // prompt of 700 tokens behind 300, 16 / 4 heads of 128, the layer 39.5 -> 35.2 us, one of 2000 67.5 ->
+  // 59.2, the pooled form's 45.1 -> 41.3 and 57.1 -> 54.6.  At up to 512 workgroups 32 / 8 heads lost (8
+  // prompts of 150 30.8 -> 36.6, 4 of 500 behind 600 66.4 -> 72.0).
+  const bool two = grid.x <= 256;
+#define AKAP_FP(DD, PL)                                                             \
+  do {                                                                              \
+    if (two) flash_prefill_kernel<DD, PL, 2><<<grid, 128 * NW, 0, s>>>(p);          \
+    else flash_prefill_kernel<DD, PL, 1><<<grid, 64 * NW, 0, s>>>(p);               \
+  } while (0)
   if (p.positions) {
     if (p.D == 64) AKAP_FP(64, true); else AKAP_FP(128, true);
   } else {

@@ -310,3 +310,34 @@ def test_values_that_are_not_finite_stay_where_they_are_seen(pooled, D, window, 
             unseen = c * pool + pool - 1 > last - window
             assert torch.equal(got[unseen], clean[150:].view(171, H, D)[unseen])
             assert not got[c * pool + pool - 1 <= i - window][:, H // 2:, 5].isfinite().any()
+
+
+@pytest.mark.parametrize("shape,H,G", [([(0, 256)], 8, 2), ([(0, 257)], 4, 4), ([(200, 121)], 8, 2),
+                                       ([(0, 700), (333, 90), (0, 40)], 4, 1), ([(0, 130)] * 20, 8, 4)])
+@pytest.mark.parametrize("D,window,pool", [(128, 0, 0), (64, 290, 0), (128, 300, 8), (64, 330, 16)])
+def test_two_teams(shape, H, G, D, window, pool):
+    """Steps around the number from which two teams share them, odd and even, a pooled part of more than 64
+    entries, and a grid that one team takes whatever its steps; values that no query sees are not finite."""
+    s = _step(shape, G, D, 32, 128, seed=H * D + window)
+    T = int(s["q_start"][-1])
+    q = torch.randn(T, H, D, generator=s["gen"]).bfloat16()
+    for b, (p, n) in enumerate(shape):
+        if (p + n) % 32:
+            s["v"][int(s["bt"][b, (p + n) // 32]), :, ((p + n) % 32 + 7) // 8:] = float("nan")
+    outs = []
+    for dev in ("cpu", DEV):
+        m = {k: v.to(dev) for k, v in s.items() if torch.is_tensor(v)}
+        out = torch.zeros(T, H * D, dtype=torch.bfloat16, device=dev)
+        if pool:
+            g = torch.Generator().manual_seed(T)
+            kp, vp = (torch.randn(s["k"].shape[0], G, sops.pool_slots(32, pool), D, generator=g).to(dev)
+                      for _ in range(2))
+            sops.pooled_window_attention_prefill(out, q.to(dev), m["k"], m["v"], kp, vp, m["bt"],
+                                                 m["q_start"], m["pos"], m["slots"], m["ts"], m["tr"],
+                                                 128, D ** -0.5, window, pool, True)
+        else:
+            sops.sink_attention_prefill(out, q.to(dev), m["k"], m["v"], m["bt"], m["lens"],
+                                        m["q_start"], m["ts"], m["tr"], 128, None,
+                                        torch.linspace(-2, 3, H).to(dev), D ** -0.5, 0, window)
+        outs.append(out)
+    _close(outs[1], outs[0])
