@@ -49,8 +49,7 @@
 // Grouped (MoE): group g owns rows [offs[g-1], offs[g]) of X and weight W + g*N*K; the same
 // raster runs over the concatenated list of every group's M tiles, the last round in quarters where it
 // has few tiles (pg_tile_cut); the grid is an upper bound
-// (sum of ceil(rows_g / 256) <= ceil(M / 256) + G) and surplus WGs exit.  A last round with few
-// tiles goes in quarters (pg_tile_cut).
+// (sum of ceil(rows_g / 256) <= ceil(M / 256) + G) and surplus WGs exit.
 // With PGemmArgs.rows a tile's X rows are gathered by the DMA's per-lane offsets (a row's 128 bytes of
 // a K tile are one line wherever it lies): 16384 tokens of 2048, 2 of 8 experts of 1408 383 us up and
 // 238 us down; the 64 x 128 tiles of moe_dgemm.hip 626 and 290.
