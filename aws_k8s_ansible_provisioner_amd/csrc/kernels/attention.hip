@@ -668,6 +668,7 @@ __device__ __forceinline__ int fa_row_key(int r) {
 }
 
 constexpr int kFaRows = 128;
+constexpr int kFaTeamTiles = 8;   // key tiles up to which one team takes them all
 constexpr int kFaKeys = 64;
 constexpr int kFaBtCache = 1024;  // chunk -> block id cache in LDS (32768 keys)
 
@@ -693,18 +694,23 @@ __device__ __forceinline__ void fa_glds16(const void* g, void* lds_wave_base) {
 // work (MI355X_MICROARCH.md "Two waves per SIMD" item 9).  The deferred P V re-reads V(t) from
 // LDS, so the ring has THREE buffers (tile t's survives until the barrier of t + 2); only the
 // bf16 P fragments and the rescale factor stay in registers (+17 VGPRs).
-template <bool F8, bool GL, int NW = 4, bool STAG = false>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(AttnParams p) {
+// TEAMS = 2 (small grids of bf16 caches): two teams of NW waves take the key tiles of the same rows in
+// turn, each with its own buffers, maximum and sums, which are added up at the end; subs workgroups
+// share a tile of the map.
+template <bool F8, bool GL, int NW = 4, bool STAG = false, int TEAMS = 1>
+__global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged_attn_prefill_fa_kernel(
+    AttnParams p, int subs) {
   constexpr int ROWS = 32 * NW;
   constexpr int NT = 64 * NW;    // threads
   constexpr int PW = 16 / NW;    // 1-KiB K (and V) DMA pieces per wave per tile
   constexpr int NBUF = STAG ? 3 : 2;
   static_assert(NW == 4 || (NW == 8 && GL), "the register-staged path assumes 256 threads");
   static_assert(!STAG || (NW == 8 && GL), "the ping-pong pairs waves w and w + 4");
+  static_assert(TEAMS == 1 || (GL && !STAG && NW == 4), "teams");
   // [buf][K | V][64 keys * 128 dims] bf16 = 64 KiB (96 KiB with STAG) + the block ids of the
   // first kFaBtCache 32-key chunks; ONE __shared__ object (a second one makes hipcc drain vmcnt)
-  __shared__ __attribute__((aligned(16))) bf16 lds[NBUF * 2 * kFaKeys * kD + 2 * kFaBtCache];
-  int* bt_s = reinterpret_cast<int*>(lds + NBUF * 2 * kFaKeys * kD);
+  __shared__ __attribute__((aligned(16))) bf16 lds_all[TEAMS * NBUF * 2 * kFaKeys * kD + 2 * kFaBtCache];
+  int* bt_s = reinterpret_cast<int*>(lds_all + TEAMS * NBUF * 2 * kFaKeys * kD);
   // One flat grid of (tile, kv head) items, kv head innermost, dispatched back to front: the
   // host map is sorted by ascending causal work (scheduler.cpp), so every head of the longest
   // tiles starts first and the grid's tail is made of the shortest ones (longest-first over
@@ -712,9 +718,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
   // With Hkv = 8 the dispatcher's round-robin over the 8 XCDs keeps one head's tiles -- which
   // read the same K/V -- on one XCD's L2.
   const int flat = gridDim.x - 1 - blockIdx.x;
-  const int tile = flat / p.Hkv;
-  const int kvh = flat - tile * p.Hkv;
-  const int tid = threadIdx.x;
+  const int item = flat / p.Hkv;
+  const int kvh = flat - item * p.Hkv;
+  const int tile = TEAMS > 1 ? item / subs : item;
+  const int tid = TEAMS > 1 ? (int)threadIdx.x & (NT - 1) : (int)threadIdx.x;   // in the team
+  const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT) : 0;
+  bf16* const lds = lds_all + team * NBUF * 2 * kFaKeys * kD;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
   const int r = lane & 31;
@@ -724,7 +733,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
   const int q_len = p.q_start[seq + 1] - q0;
   const int kv_len = p.seq_lens[seq];
   const int G = p.G;
-  const int row0 = p.tile_row[tile];
+  const int row0 = p.tile_row[tile] + (TEAMS > 1 ? (item - tile * subs) * ROWS : 0);
+  if (TEAMS > 1 && row0 >= q_len * G) return;   // (the workgroup's)
   const int R = row0 + 32 * w + r;
   const int pos = R / G;
   const int hig = R % G;
@@ -809,6 +819,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
   const int wg_last_pos = min(q_len - 1, (row0 + ROWS - 1) / G);
   const int wg_limit = ctx0 + wg_last_pos;
   const int ntiles = wg_limit / kFaKeys + 1;
+  // teams at work: few key tiles are not worth the second's sums
+  const int teams = TEAMS > 1 && ntiles > kFaTeamTiles ? 2 : 1;
+  if (team >= teams) return;
   const int w_first_pos = (row0 + 32 * w) / G;
   const int w_last_pos = min(q_len - 1, (row0 + 32 * w + 31) / G);
   const bool wave_active = w_first_pos < q_len;
@@ -903,8 +916,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
 
   int blk_next = 0;
   if constexpr (GL) {
-    stage_glds(0, 0, blk_of(0));
-    blk_next = blk_of(1);
+    stage_glds(team, 0, blk_of(team));
+    blk_next = blk_of(team + teams);
     load_q();
   } else {
     load_q();
@@ -954,9 +967,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
   // hold both sets (it spilled); two loops let each keep only its own
   auto kv_loop = [&](auto late_c) {
   constexpr bool late = decltype(late_c)::value;
-  for (int t = 0; t < ntiles; ++t) {
-    const int buf = STAG ? t % NBUF : (t & 1);
-    const bool more = t + 1 < ntiles;
+  for (int u = 0; u * teams < ntiles; ++u) {
+    const int t = u * teams + team;
+    const int buf = STAG ? t % NBUF : (u & 1);
+    const bool more = t + teams < ntiles;
     if constexpr (GL) {
       // tile t (issued one iteration ago) landed for this wave; every wave's LDS reads of
       // the buffer tile t+1 goes into (tile t-1, or t-2 with STAG) are done -> after the
@@ -965,15 +979,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       if (more) {
-        stage_glds(t + 1, STAG ? (t + 1) % NBUF : (buf ^ 1), blk_next);
-        blk_next = blk_of(t + 2);
+        stage_glds(t + teams, STAG ? (t + 1) % NBUF : (buf ^ 1), blk_next);
+        blk_next = blk_of(t + 2 * teams);
       }
     } else {
       if (more) stage_load(t + 1);
     }
     if (late && pend) deferred_pv(t - 1);
     const int key0 = t * kFaKeys;
-    if (wave_active && key0 <= w_limit) {
+    if (wave_active && key0 <= w_limit && (TEAMS == 1 || t < ntiles)) {
       const bf16* kl = lds + (size_t)buf * 2 * kFaKeys * kD;
       const bf16* vl = kl + kFaKeys * kD;
       // S^T = K . Q^T for the two 32-key sub-tiles (interleaved: independent chains)
@@ -1103,6 +1117,28 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_attn_prefill_fa_kernel(
   } else {
     kv_loop(std::false_type{});
   }
+  if (TEAMS > 1 && teams > 1) {
+    // the second team's maxima and sums into the first's, through the buffers
+    float* to = reinterpret_cast<float*>(lds_all) + w * 66 * 64 + lane;
+    __syncthreads();
+    if (team == 1) {
+      to[0] = m_run;
+      to[64] = l_run;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) to[(2 + 16 * i + j) * 64] = oacc[i][j];
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float m = fmaxf(m_run, to[0]);
+    const float fa = __builtin_amdgcn_exp2f(m_run - m), fb = __builtin_amdgcn_exp2f(to[0] - m);
+    l_run = l_run * fa + to[64] * fb;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) oacc[i][j] = oacc[i][j] * fa + to[(2 + 16 * i + j) * 64] * fb;
+  }
   // O^T accumulator of lane (r, h): row r's dims 32 dt + 8 j4 + 4 h + (0..3).  Each pair of
   // 8-dim groups (j4 = 2 kp, 2 kp + 1) is exchanged between the lane halves with two
   // v_permlane32_swap, after which lane r holds dims 16 kp + 0..7 and lane r + 32 dims
@@ -1208,14 +1244,21 @@ void launch_paged_attn_prefill(const AttnParams& p, int num_tiles, int tile_rows
     const char* e = std::getenv("AKAP_PREFILL_STAGGER");
     return e != nullptr && std::atoi(e) == 1;
   }();
-  if (tile_rows == 2 * kFaRows && !p.kv_fp8) {  // 256 rows, 8 waves (bf16 caches)
-    if (stag) paged_attn_prefill_fa_kernel<false, true, 8, true><<<grid, 512, 0, s>>>(q);
-    else paged_attn_prefill_fa_kernel<false, true, 8><<<grid, 512, 0, s>>>(q);
+  // A map of 256-row tiles (long prompts) whose halves fit one to a CU: a workgroup per half, two teams of
+  // four waves on its keys.  16 / 8 heads of 128, the layer: a prompt of 700 tokens behind 300 39.7 -> 32.2
+  // us (35.1 with one team), of 1500 56 -> 42 (47), of 2000 69.5 -> 51.5 (60); 32 / 8 heads, 700 behind 300
+  // 41.3 -> 32.1.  At up to two workgroups to a CU 4 prompts of 500 behind 600 lost (50 -> 56), and at maps of
+  // 128-row tiles 10 prompts of 200 behind 300 (28.1 -> 28.8).
+  if (tile_rows == 2 * kFaRows && !p.kv_fp8 && !stag && 2 * grid.x <= 256)
+    paged_attn_prefill_fa_kernel<false, true, 4, false, 2><<<2 * grid.x, 512, 0, s>>>(q, 2);
+  else if (tile_rows == 2 * kFaRows && !p.kv_fp8) {  // 256 rows, 8 waves (bf16 caches)
+    if (stag) paged_attn_prefill_fa_kernel<false, true, 8, true><<<grid, 512, 0, s>>>(q, 1);
+    else paged_attn_prefill_fa_kernel<false, true, 8><<<grid, 512, 0, s>>>(q, 1);
   }
   else if (p.kv_fp8)  // fp8 caches: register-staged (widened to bf16 on the way into LDS)
-    paged_attn_prefill_fa_kernel<true, false><<<grid, 256, 0, s>>>(q);
+    paged_attn_prefill_fa_kernel<true, false><<<grid, 256, 0, s>>>(q, 1);
   else  // bf16 caches: LDS-DMA staging
-    paged_attn_prefill_fa_kernel<false, true><<<grid, 256, 0, s>>>(q);
+    paged_attn_prefill_fa_kernel<false, true><<<grid, 256, 0, s>>>(q, 1);
 }
 
 void launch_paged_attn_decode(const AttnParams& p, int num_seqs, hipStream_t s) {

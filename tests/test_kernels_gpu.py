@@ -141,6 +141,22 @@ def test_paged_attention_prefill(bs, hq, hkv, tile_rows):
     _close(out, exp, atol=2e-2, rtol=2e-2)
 
 
+# two teams of waves at the number of key tiles from which they share them (8 and 9, odd and even), and a
+# grid too large for them
+@pytest.mark.parametrize("hq,hkv,seqs", [(16, 8, [(512, 512), (513, 130), (576, 64), (1100, 900)]),
+                                         (32, 8, [(513, 1), (640, 640)]), (8, 2, [(1030, 1030)]),
+                                         (32, 8, [(600, 300)] * 4)])
+def test_paged_attention_prefill_teams(hq, hkv, seqs):
+    q, kc, vc, bt, sl, qs = _setup_attn(seqs, hq, hkv, 32, seed=len(seqs) + hq)
+    scale = 1 / math.sqrt(128)
+    exp = ref.paged_attention(q, kc, vc, bt, sl, qs, scale)
+    ts, tr = _tiles(seqs, hq // hkv, 256)
+    out = torch.empty_like(q).to(DEV)
+    ops.paged_attention_prefill(out, q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), sl.to(DEV),
+                                qs.to(DEV), ts.to(DEV), tr.to(DEV), hq // hkv, scale, tile_rows=256)
+    _close(out, exp, atol=2e-2, rtol=2e-2)
+
+
 # odd GQA groups (8/8, 24/8) take the full rotary-row loads, even ones the lane-pair share
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (32, 8), (8, 8), (24, 8)])
 @pytest.mark.parametrize("qk_norm", [True, False])
