@@ -519,28 +519,44 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const ConvArgs a, co
 
 // eight channels per thread (16-byte accesses of bf16), TAPS at compile time: a tile of rb rows
 // inside one sequence is fetched four rows at a time ahead of its products; tiles with a
-// sequence's start or end go row by row with the history from the tile or the slot
+// sequence's start or end go row by row with the history from the tile or the slot.  Memory bounds it.
+// With fp32 results a thread's channels are two groups of four, half of the workgroup's columns
+// apart: eight in a row would leave as two stores that each fill every other 16 bytes (16384 rows of 4352
+// channels 114 us, 102 this way, 4.2 TB/s; the next four rows fetched before the products as well: no less)
 constexpr int kConvRows8 = 32;
 
 template <typename TO, int TAPS>
 __global__ __launch_bounds__(128) void conv_silu_vec8_kernel(const ConvArgs a, int rb) {
-  const int c = (blockIdx.y * 128 + threadIdx.x) * 8;
-  if (c >= a.C) return;
+  const int first = blockIdx.y * 1024, half = min(1024, a.C - first) / 2;
+  constexpr bool SPLIT = sizeof(TO) == 4;
+  if (threadIdx.x * 8 >= half * 2) return;
+  const int c = first + threadIdx.x * (SPLIT ? 4 : 8), hop = SPLIT ? half : 4;
+  auto chan = [&](int k) { return k < 4 ? c + k : c + hop + k - 4; };
   const int tb = blockIdx.x * rb, te = min(a.T, tb + rb);
   const bf16* in = (const bf16*)a.proj + a.off + c;
   TO* out = (TO*)a.out + c;
   float w[TAPS][8], hist[TAPS][8], bias[8];          // hist[j]: the input TAPS - 1 - j rows back
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    bias[k] = a.b ? a.b[c + k] : 0.f;
+    bias[k] = a.b ? a.b[chan(k)] : 0.f;
 #pragma unroll
-    for (int j = 0; j < TAPS; ++j) w[j][k] = a.w[(size_t)(c + k) * TAPS + j];
+    for (int j = 0; j < TAPS; ++j) w[j][k] = a.w[(size_t)chan(k) * TAPS + j];
   }
-  auto load = [&](int t, float (&v)[8]) {
-    const akap::bf16x8 x = *(const akap::bf16x8*)(in + (size_t)t * a.proj_stride);
+  auto fetch = [&](const bf16* p, float (&v)[8]) {
+    if constexpr (SPLIT) {
+      const akap::bf16x4 lo = *(const akap::bf16x4*)p, hi = *(const akap::bf16x4*)(p + hop);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = (float)x[k];
+      for (int k = 0; k < 4; ++k) {
+        v[k] = (float)lo[k];
+        v[k + 4] = (float)hi[k];
+      }
+    } else {
+      const akap::bf16x8 x = *(const akap::bf16x8*)p;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = (float)x[k];
+    }
   };
+  auto load = [&](int t, float (&v)[8]) { fetch(in + (size_t)t * a.proj_stride, v); };
   auto emit = [&](int t, const float (&cur)[8]) {
     float o[8];
 #pragma unroll
@@ -549,10 +565,16 @@ __global__ __launch_bounds__(128) void conv_silu_vec8_kernel(const ConvArgs a, i
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) z += w[j][k] * hist[j][k];
       z += w[TAPS - 1][k] * cur[k];
-      o[k] = c + k >= a.silu_from ? siluf(z) : z;
+      o[k] = chan(k) >= a.silu_from ? siluf(z) : z;
     }
     TO* op = out + (size_t)t * a.C;
-    st8(op, o);
+    if constexpr (SPLIT) {
+      const float lo[4] = {o[0], o[1], o[2], o[3]}, hi[4] = {o[4], o[5], o[6], o[7]};
+      st4(op, lo);
+      st4(op + hop, hi);
+    } else {
+      st8(op, o);
+    }
 #pragma unroll
     for (int j = 0; j < TAPS - 1; ++j)
 #pragma unroll
@@ -578,9 +600,7 @@ __global__ __launch_bounds__(128) void conv_silu_vec8_kernel(const ConvArgs a, i
       if (kk >= 0) {
         load(src, hist[j]);
       } else if (pos0 + kk >= 0) {                   // -1: the input just before the step
-        const akap::bf16x8 x = *(const akap::bf16x8*)(st + (size_t)(TAPS - 1 + kk) * a.C);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) hist[j][k] = (float)x[k];
+        fetch(st + (size_t)(TAPS - 1 + kk) * a.C, hist[j]);
       }
     }
     for (; t + 4 <= r1; t += 4) {
@@ -1088,9 +1108,9 @@ void launch_conv_silu(void* out, bool out_f32, const void* proj, int proj_stride
                     (uintptr_t)proj % 16 == 0 && (uintptr_t)state % 16 == 0 && taps >= 2 &&
                     taps <= 4;
   if (vec8) {
-    // rows of a workgroup, a serial chain: as many as leave 700 workgroups (4352 channels: 400 rows 21 us
-    // with 32, 14 with 16, 10.5 with 8, 10 with 4; 1850 rows 31, 22, 21, 23; 3700 33, 30, 30, 36; 16384
-    // 108, 110, 117, 139)
+    // rows of a workgroup, a serial chain: as many as leave 700 workgroups (4352 channels, fp32 results: 400
+    // rows 19 us with 32, 12 with 16, 8.5 with 8, 7.7 with 4; 1850 rows 28, 17, 16, 16; 3700 28, 24, 24, 26;
+    // 16384 102, 101, 114, 132)
     const unsigned cols = (C / 8 + 127) / 128;
     int rb = kConvRows8;
     while (rb > 8 && (unsigned)(T / rb) * cols < 700) rb /= 2;

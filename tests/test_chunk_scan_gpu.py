@@ -378,3 +378,26 @@ def test_convolution_rows(T, C, taps):
         got.append((out.cpu(), st.cpu()))
     assert _rel(got[1][0], got[0][0]) < 1e-6        # four products in fp32 and an exponential
     assert torch.equal(got[1][1], got[0][1])
+
+
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,first", [(8, 5), (1016, 509), (1024, 600), (1032, 1027), (3080, 0)])
+def test_convolution_columns(C, first, out):
+    """Columns of a workgroup that is not full, and the first one with an activation in either half."""
+    T, taps = 45, 4
+    q_start, pos, slot = _step([40, 5], [0, 7])
+    g = torch.Generator().manual_seed(C)
+    proj = torch.randn(T, C + 16, generator=g).to(torch.bfloat16)
+    w, b = torch.randn(C, taps, generator=g), torch.randn(C, generator=g)
+    state = torch.randn(2, taps - 1, C, generator=g).to(torch.bfloat16)
+    got = []
+    for dev in ("cpu", DEV):
+        st, o = state.clone().to(dev), torch.zeros(T, C, dtype=out, device=dev)
+        sops.conv_silu(o, proj.to(dev), 8, w.to(dev), b.to(dev), st, slot.to(dev), pos.to(dev),
+                       q_start.to(dev), first)
+        got.append((o.cpu(), st.cpu()))
+    # four products in fp32 and an exponential; bf16 neighbours differ by up to 2^-7
+    d = (got[1][0].double() - got[0][0].double()).abs()
+    ulp = 2e-6 if out == torch.float32 else 2.0 ** -7
+    assert (d <= ulp * (got[0][0].double().abs() + 1)).all()
+    assert torch.equal(got[1][1], got[0][1])
