@@ -522,7 +522,8 @@ __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const ConvArgs a, co
 // sequence's start or end go row by row with the history from the tile or the slot.  Memory bounds it.
 // With fp32 results a thread's channels are two groups of four, half of the workgroup's columns
 // apart: eight in a row would leave as two stores that each fill every other 16 bytes (16384 rows of 4352
-// channels 114 us, 102 this way, 4.2 TB/s; the next four rows fetched before the products as well: no less)
+// channels, on its own, 114 us, 102 this way; between the mixer's other kernels 109 and 88,
+// 4.8 TB/s; the next four rows fetched before the products as well: no less)
 constexpr int kConvRows8 = 32;
 
 template <typename TO, int TAPS>
