@@ -79,6 +79,7 @@ class OTLPTracer:
         self.resource = dict(resource or {})
         self._buf: list = []
         self._lock = threading.Lock()
+        self._export = threading.Lock()
         self._wake = threading.Event()
         self._stop = False
         self.exported = 0
@@ -118,6 +119,11 @@ class OTLPTracer:
                             "spans": spans}]}]}
 
     def flush(self) -> int:
+        """Export what is buffered; returns after an export that the thread has under way as well."""
+        with self._export:
+            return self._flush()
+
+    def _flush(self) -> int:
         with self._lock:
             spans, self._buf = self._buf, []
         if not spans:

@@ -185,3 +185,19 @@ def test_gateway_propagates_trace_to_engine(collector):
     req = [s for s in spans if s["name"] == "llm_request"]
     assert len(req) == 1
     assert req[0]["traceId"] == tid and req[0]["parentSpanId"] == gw[0]["spanId"]
+
+
+def test_flush_waits_for_export_under_way(collector):
+    """flush() returns after the thread's export too, also when it finds the buffer empty."""
+    c, tr = collector
+    entered, post = threading.Event(), tr.payload
+
+    def slow(spans):
+        entered.set()
+        time.sleep(0.5)
+        return post(spans)
+    tr.payload = slow
+    tr.record("one", 1.0, 2.0)
+    assert entered.wait(5)
+    assert tr.flush() == 0
+    assert [s["name"] for s in c.spans()] == ["one"]
