@@ -12,8 +12,8 @@
 // others' sums apart where there are registers for it): 2^-26 of a product is left out, and a sum of 16
 // products is rounded once per instruction, where v_mfma_f32_32x32x2_f32 rounds every two.  Against 64 bits,
 // 8 x 2048 rows: scan outputs 1.03e-7 and states 1.12e-7 (in fp32 products 1.04e-7 and 1.14e-7), retention
-// states 1.7e-7 (2.7e-7).  Operands that do not split (not finite, past bf16's range, or so small that
-// parts would be denormal, which the matrix units take as zero) go through the fp32 products.
+// states 1.7e-7 (2.7e-7).  Operands that do not split (not finite, past bf16's range, or one so small that
+// a part would be denormal, which the matrix units take as zero) go through the fp32 products.
 //
 // chunk_frag_kernel prepares every (chunk, key head) side by side: the parts of q and k (rotated and
 // scaled for the retention) as operand fragments and the 32 x 32 products q_i . k_j in fp32; the scan's
@@ -121,10 +121,27 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& h, bf16x8& m
     l[i] = (bf16)(r[i] - (float)m[i]);
   }
 }
-// Magnitudes below this split.  The matrix units take a denormal part as zero, so the largest of the
-// values that meet in a lane has to be above the second limit: then what is lost is 2^-48 of it.
-constexpr float kSplits = 3.38e38f, kWhole = 0x1p-78f;
-__device__ __forceinline__ bool splits(float top) { return top < kSplits && !(top < kWhole && top > 0.f); }
+// Zeros and magnitudes in [kSmall, kSplits) split into three parts that the matrix units take as they are:
+// they take a denormal part as zero, and the last bit of 2^-101 is 2^-124.  One value outside, whatever
+// lies beside it, and the product is formed in fp32: against a large partner it may be what counts.
+constexpr float kSplits = 3.38e38f, kSmall = 0x1p-101f;
+
+// The scan's weights of a chunk's rows in the state after it come this much larger and the keys' parts this
+// much smaller: the largest power that takes every weighted value, however far it decayed, to kSmall.
+constexpr float kUp = 0x1p48f, kDown = 0x1p-48f;
+
+// extremes of magnitudes; a NaN among them makes both NaN
+struct Range {
+  float lo = INFINITY, hi = 0.f;
+  __device__ __forceinline__ void add(float v) {
+    lo = __builtin_elementwise_minimum(lo, fabsf(v));
+    hi = __builtin_elementwise_maximum(hi, fabsf(v));
+  }
+};
+// below `limit` without being zero (zeros are ordinary, so this is asked where the range says so)
+__device__ __forceinline__ bool below(float v, float limit) {
+  return (__float_as_uint(v) << 1) - 1u < (__float_as_uint(limit) << 1) - 1u;
+}
 
 // Products of split operands: the largest go to `big`, the five next to `small`; what is left out is
 // 2^-26 of the product.
@@ -220,9 +237,9 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 
 // ------------------------------------------------------------------ fragments of q and k
 // One workgroup per (chunk, key head).  Buffer of an entry, in pieces of 64 lanes x 16 bytes: [q: 3 parts
-// of N / 16 pieces][k transposed: the same, the retention's already times their weights in the new
-// state][q . k in fp32: 4][1 if a value does not split:
-// then the parts are the fp32 values' upper and lower halves]; rows past the chunk's end are zero.
+// of N / 16 pieces][k transposed: the same, the scan's times kDown, the retention's times their weights
+// in the new state][q . k in fp32: 4][1 if a value does not split: then the parts are the fp32 values'
+// upper and lower halves, without kDown]; rows past the chunk's end are zero.
 template <int MODE, int NT, typename TY>
 __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
@@ -300,7 +317,7 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
   // piece f: contraction step f of q (entries 16 f + 4 hh + 0..3 and 8 on), rows 32 (f / 2) of the state
   // and tokens 16 (f % 2) + 4 hh + 0..3 and 8 on of k
   float v[2][NQ / 4][8];
-  bool bad = false;
+  Range range[2];
 #pragma unroll
   for (int u = 0; u < NQ / 4; ++u) {
     const int f = wave + 4 * u, j0 = 16 * (f & 1) + 4 * hh;
@@ -312,15 +329,19 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
       v[1][u][i] = ks[j * LS + 32 * (f >> 1) + li] * (MODE == 1 ? wt[j] : 1.f);
     }
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
-      float top = 0.f, zero = 0.f;
+    for (int w = 0; w < 2; ++w)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        top = fmaxf(top, fabsf(v[w][u][i]));
-        zero = fmaf(v[w][u][i], 0.f, zero);
-      }
-      bad |= zero != 0.f || !splits(top);
-    }
+      for (int i = 0; i < 8; ++i) range[w].add(v[w][u][i]);
+  }
+  constexpr float scale[2] = {1.f, MODE == 0 ? kDown : 1.f};
+  bool bad = !(range[0].hi < kSplits) || !(range[1].hi < kSplits);
+  if (range[0].lo < kSmall || range[1].lo < kSmall / scale[1]) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int u = 0; u < NQ / 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bad |= below(v[w][u][i], kSmall / scale[w]);
   }
   bad = __syncthreads_or(bad);
 #pragma unroll
@@ -328,7 +349,10 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 #pragma unroll
     for (int u = 0; u < NQ / 4; ++u) {
       bf16x8 part[3];
-      split8(v[w][u], part[0], part[1], part[2]);
+      float e[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = v[w][u][i] * scale[w];
+      split8(e, part[0], part[1], part[2]);
       if (__builtin_expect(bad, 0)) {      // as they are, in two halves
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -381,7 +405,7 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 
 // ------------------------------------------------------------------ step sizes and decays
 // Half a wave per (chunk, head) of the selective scan, a lane per row.  With c the sums of the log2
-// decays (formed in fp64): [32] dt, [32] 2^c, [32] dt 2^(c_end - c), [32] c, [32] what c lost when
+// decays (formed in fp64): [32] dt, [32] 2^c, [32] kUp dt 2^(c_end - c), [32] c, [32] what c lost when
 // it was rounded.  Rows past the end: dt 0, decay 1.
 template <typename TY>
 __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams p) {
@@ -409,7 +433,7 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
     const float hi = (float)l;
     sc[i] = dt;
     sc[kL + i] = exp2f(hi);
-    sc[2 * kL + i] = i < n ? dt * exp2f((float)(end - l)) : 0.f;
+    sc[2 * kL + i] = i < n ? kUp * (dt * exp2f((float)(end - l))) : 0.f;
     sc[3 * kL + i] = hi;
     sc[4 * kL + i] = (float)(l - (double)hi);
   }
@@ -598,10 +622,11 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     const float e[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
     split8(e, to[0], to[1], to[2]);
   };
-  // the values times their weights in the state after the chunk (the retention's are in k), and their
-  // parts
+  // the values times their weights in the state after the chunk (the scan's times kUp, the retention's are
+  // in k), and their parts
   float xw[16];
   bf16x8 w[2][3];
+  Range wr;
   float4 w4[MODE == 0 ? 4 : 1];
   auto fetch_weights = [&](const float* sc) {
     if (MODE == 0) {
@@ -610,7 +635,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     }
   };
   auto weigh = [&] {
-    float zero = 0.f, top = 0.f;
+    wr = Range{};
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float f[4] = {w4[MODE == 0 ? g : 0].x, w4[MODE == 0 ? g : 0].y, w4[MODE == 0 ? g : 0].z,
@@ -619,16 +644,10 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       for (int r = 0; r < 4; ++r) {
         const float v = MODE == 0 ? x[4 * g + r] * f[r] : x[4 * g + r];
         xw[4 * g + r] = v;
-        zero = fmaf(v, 0.f, zero);
-        if (XP == 3) top = fmaxf(top, fabsf(v));
+        if (MODE == 0) wr.hi = __builtin_elementwise_maximum(wr.hi, fabsf(v));
+        else wr.add(v);
       }
     }
-    if (XP == 3) {      // (both halves' tokens: the last of a chunk have weights of their step sizes)
-      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false,
-                                                         false);
-      top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
-    }
-    apart = __any(zero != 0.f || !splits(top));
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       // (parts of the unrounded product)
@@ -651,10 +670,33 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
     }
   };
+  // do the weighted values split (a value of one part: is it one that the matrix units take)?
+  auto judge = [&] {
+    // Of one part they also meet pair weights that may be too small to split, see outputs(): what these
+    // lose, 2^-125, stays far below the normed rows' roundings while the values are no larger.
+    constexpr float least = XP == 3 ? kSmall : __FLT_MIN__, most = XP == 3 ? kSplits : 0x1p20f;
+    apart = __any(!(wr.hi < most));
+    if (MODE == 0) {                  // (kUp: none too small)
+      if (__builtin_expect(apart, 0)) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) xw[s] = x[s] * ((&w4[MODE == 0 ? s >> 2 : 0].x)[s & 3] * kDown);
+      }
+    } else if (__builtin_expect(__any(wr.lo < least), 0)) {
+      bool few = false;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) few |= below(xw[s], least);
+      apart |= __any(few);
+    }
+  };
   // the state after the chunk: dend S + k^T xw
   auto advance = [&](const float4* kb, float dend) {
     const bf16x8* kp = (const bf16x8*)kb + fresh(lane);
     if (__builtin_expect(odd || apart, 0)) {
+      if (MODE == 0 && !apart) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) xw[s] *= kDown;
+      }
+      const float up = MODE == 0 && !odd ? kUp : 1.f;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -664,10 +706,10 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const float4 a = joined(kp, 4 * t + g);
-          S[t] = mfma(a.x, xw[4 * g], S[t]);
-          S[t] = mfma(a.y, xw[4 * g + 1], S[t]);
-          S[t] = mfma(a.z, xw[4 * g + 2], S[t]);
-          S[t] = mfma(a.w, xw[4 * g + 3], S[t]);
+          S[t] = mfma(a.x * up, xw[4 * g], S[t]);
+          S[t] = mfma(a.y * up, xw[4 * g + 1], S[t]);
+          S[t] = mfma(a.z * up, xw[4 * g + 2], S[t]);
+          S[t] = mfma(a.w * up, xw[4 * g + 3], S[t]);
           __builtin_amdgcn_sched_barrier(0);
         }
       return;
@@ -757,13 +799,13 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[i] = O2[i] = 0.f;
     bf16x8 a[2][3];
-    uint32_t seen = 0;                // bits of the lane's part of the state
+    float least = INFINITY;           // of the lane's part of the state
     auto state_parts = [&](int j) {
       float v[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         v[i] = S[j >> 1][8 * (j & 1) + i];
-        seen |= __float_as_uint(v[i]);
+        least = __builtin_elementwise_minimum(least, fabsf(v[i]));
       }
       split8(v, a[j & 1][0], a[j & 1][1], a[j & 1][2]);
     };
@@ -796,6 +838,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       weigh();
       interleave<16, 9>();
       __builtin_amdgcn_sched_barrier(0);
+      judge();
     } else {
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
@@ -807,12 +850,19 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         for (int u = 2; u >= 0; --u) O = mfma16(v, b[u], O);
       }
       weigh();
+      judge();
     }
     float fin = 0.f;
 #pragma unroll
     for (int s = 0; s < 16; ++s) fin = fmaf(O[s], 0.f, fin);
-    seen &= 0x7fffffffu;
-    if (__builtin_expect(odd || __any(fin != 0.f || (seen != 0 && seen < __float_as_uint(kWhole))), 0)) {
+    bool few = false;
+    if (__builtin_expect(__any(!(least >= kSmall)), 0)) {     // (zeros, as before a sequence's first chunk)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) few |= below(S[t][i], kSmall);
+    }
+    if (__builtin_expect(odd || (XP == 1 && apart) || __any(fin != 0.f || few), 0)) {
       // an operand that does not split, or is not finite: the fp32 products
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[i] = 0.f;
@@ -913,6 +963,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       if (MODE == 0) total += sc[4 * kL - 1];
       fetch_weights(sc);
       weigh();
+      judge();
       advance(now, dend);
     };
     stage(0, qbuf);

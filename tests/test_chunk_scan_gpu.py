@@ -401,3 +401,83 @@ def test_convolution_columns(C, first, out):
     ulp = 2e-6 if out == torch.float32 else 2.0 ** -7
     assert (d <= ulp * (got[0][0].double().abs() + 1)).all()
     assert torch.equal(got[1][1], got[0][1])
+
+
+def _beside(rows, what):
+    """Scan inputs of ordinary sizes where one operand has entries of 1e-36 between larger ones, whose last
+    bits are denormal, and the other has ones large enough to make them count, in one row of the state."""
+    H, V, N = 2, 64, 128
+    inp = list(_scan_inputs(rows, 1, H, V, N, 1, torch.float32, 0, seed=12))
+    xbc, state, t = inp[0].clone(), inp[5].clone(), rows - 5
+    inp[2] = inp[2] - 3.0
+    x, k, q = xbc.split([H * V, N, N], 1)
+    if what == "state":
+        state[:, :, 3] *= 1e-36
+        k[:, 3] = 0.0
+        q[:, 3] *= 3e37
+    elif what == "queries":
+        state[:, :, 3] *= 3e37
+        k[:, 3] = 0.0
+        q[:, 3] = 0.0
+        q[1, 3] = 1.2345e-36
+    elif what == "keys":
+        k[t] = 0.0
+        k[t, 3], x[t] = 1.2345e-36, x[t] * 1e37
+    else:                                              # the values of a token
+        k[t] = 0.0
+        k[t, 3], x[t] = 1e37, x[t] * 1e-36
+    inp[0], inp[5] = xbc, state
+    return tuple(inp), H, V, N
+
+
+@pytest.mark.parametrize("rows", [49, 300, 1100])
+@pytest.mark.parametrize("what", ["state", "queries", "keys", "values"])
+def test_small_operands_beside_larger_ones(what, rows):
+    """A part that is denormal is not lost where the other operand is large: every operand as exact as in
+    fp32, row by row of the state and of the outputs (sums of 160 fp32 terms in another order)."""
+    inp, H, V, N = _beside(rows, what)
+    step = _step([rows], [6])
+    want = _run_scan(inp, step, H, V, N, 1, "cpu")
+    got = _run_scan(inp, step, H, V, N, 1, DEV)
+    err = (got[0].cpu() - want[0]).norm(dim=1) / want[0].norm(dim=1)
+    assert float(err.max()) < 1e-5
+    assert _rel(got[1][:, :, 3], want[1][:, :, 3]) < 4e-6
+    assert _rel(got[1], want[1]) < 4e-6
+
+
+@pytest.mark.parametrize("what", ["keys", "values", "denormal values"])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_retention_small_operands_beside_larger_ones(what, dt):
+    """The same of the retention, whose values may be of one part alone, by the state's row of the key."""
+    H, V, T = 2, 128, 96
+    proj = torch.randn(T, 4 * H * V, generator=torch.Generator().manual_seed(6)).to(dt)
+    k, v = proj[:, H * V:2 * H * V], proj[:, 2 * H * V:3 * H * V]
+    k[80].zero_()
+    if what == "keys":
+        k[80, 11], v[80] = 1.2345e-36, v[80] * 1e37
+    else:
+        k[80, 11], v[80] = 1e37, v[80] * (1e-36 if what == "values" else 3e-39)
+    args = (_step([T], [3]), H, V, V, (0, H * V, 2 * H * V, 3 * H * V), None,
+            torch.log2(torch.tensor([0.97, 0.9])))
+    st = torch.randn(1, H, V, V, generator=torch.Generator().manual_seed(7))
+    want = _run_retention((proj, st), *args, "cpu")[1]
+    got = _run_retention((proj, st), *args, DEV)[1].cpu()
+    assert _rel(got, want) < 4e-6
+    assert _rel(got[0, 0, :, 11], want[0, 0, :, 11]) < 4e-6
+
+
+@pytest.mark.parametrize("a_log", [1.5, 2.5, 3.5])
+def test_scan_weights_that_decay_far(a_log):
+    """Decays that take the first rows of a chunk down to denormal weights in the state after it, with a
+    value large enough to count among them."""
+    H, V, N, rows = 2, 64, 128, 64
+    inp = list(_scan_inputs(rows, 1, H, V, N, 1, torch.float32, 0, seed=13))
+    inp[1], inp[2] = torch.zeros_like(inp[1]), torch.zeros(H)      # steps of log 2
+    inp[3] = torch.full((H,), a_log)
+    inp[0] = inp[0].clone()
+    inp[0][rows - 9, :H * V] *= 1e15
+    step = _step([rows], [6])
+    want = _run_scan(tuple(inp), step, H, V, N, 1, "cpu")
+    got = _run_scan(tuple(inp), step, H, V, N, 1, DEV)
+    err = (got[0].cpu() - want[0]).norm(dim=1) / want[0].norm(dim=1)
+    assert float(err.max()) < 1e-5 and _rel(got[1], want[1]) < 4e-6
