@@ -166,6 +166,12 @@ __device__ __forceinline__ void interleave() {
   }
 }
 
+// A retention's decay below 0.41 per token takes the weight of a chunk's first key below 2^-40, and keys times
+// weights to where they do not split.  They then come kLift larger and the values kSink smaller (8 x 2048
+// rows, 8 heads x 128 x 128, decays of 0.003 to 0.07: 215 us as at other decays, 700 with the fp32 products).
+constexpr float kLift = 0x1p80f, kSink = 0x1p-80f;
+__device__ __forceinline__ bool lifted(float l2) { return l2 * (kL - 1) < -40.f; }
+
 // decay^k for a decay given by its log2 (-inf: a decay of zero)
 __device__ __forceinline__ float decay_pow(float l2, int k) {
   return k == 0 ? 1.0f : exp2f(l2 * (float)k);
@@ -238,8 +244,9 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 // ------------------------------------------------------------------ fragments of q and k
 // One workgroup per (chunk, key head).  Buffer of an entry, in pieces of 64 lanes x 16 bytes: [q: 3 parts
 // of N / 16 pieces][k transposed: the same, the scan's times kDown, the retention's times their weights
-// in the new state][q . k in fp32: 4][1 if a value does not split: then the parts are the fp32 values'
-// upper and lower halves, without kDown]; rows past the chunk's end are zero.
+// in the new state (see lifted())][q . k in fp32: 4][1 if a value does not split: then the parts are the
+// fp32 values' upper and lower halves, without kDown, and those of a lifted() head without weights]; rows
+// past the chunk's end are zero.
 template <int MODE, int NT, typename TY>
 __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
@@ -309,7 +316,9 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
     *(float4*)(qs + i * LS + d) = a;
     *(float4*)(ks + i * LS + d) = b4;
   }
-  if (MODE == 1 && tid < kL) wt[tid] = tid < n ? decay_pow(p.log2_decay[kh], n - 1 - tid) : 0.f;
+  const bool lift = MODE == 1 && lifted(p.log2_decay[kh]);
+  if (MODE == 1 && tid < kL)
+    wt[tid] = tid < n ? decay_pow(p.log2_decay[kh], n - 1 - tid) * (lift ? kLift : 1.f) : 0.f;
   __syncthreads();
   const int li = lane & 31, hh = lane >> 5;
   constexpr int NQ = N / 16;
@@ -356,7 +365,11 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
       if (__builtin_expect(bad, 0)) {      // as they are, in two halves
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const uint32_t bits = __float_as_uint(v[w][u][i]);
+          uint32_t bits = __float_as_uint(v[w][u][i]);
+          if (w == 1 && lift) {
+            const int f = wave + 4 * u, j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
+            bits = __float_as_uint(ks[j * LS + 32 * (f >> 1) + li]);
+          }
           part[0][i] = __builtin_bit_cast(bf16, (uint16_t)(bits >> 16));
           part[1][i] = __builtin_bit_cast(bf16, (uint16_t)bits);
         }
@@ -486,6 +499,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
   const int col = (wave % VW) * 32 + li;
   const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
+  const bool lift = MODE == 1 && uniform(lifted(l2));
   // retention: decay^k and decay^(k + 1)
   float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
   if (MODE == 1) {
@@ -622,7 +636,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     const float e[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
     split8(e, to[0], to[1], to[2]);
   };
-  // the values times their weights in the state after the chunk (the scan's times kUp, the retention's are
+  // the values times their weights in the state after the chunk (the scan's times kUp; the retention's are
   // in k), and their parts
   float xw[16];
   bf16x8 w[2][3];
@@ -674,45 +688,66 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   auto judge = [&] {
     // Of one part they also meet pair weights that may be too small to split, see outputs(): what these
     // lose, 2^-125, stays far below the normed rows' roundings while the values are no larger.
-    constexpr float least = XP == 3 ? kSmall : __FLT_MIN__, most = XP == 3 ? kSplits : 0x1p20f;
-    apart = __any(!(wr.hi < most));
-    if (MODE == 0) {                  // (kUp: none too small)
-      if (__builtin_expect(apart, 0)) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) xw[s] = x[s] * ((&w4[MODE == 0 ? s >> 2 : 0].x)[s & 3] * kDown);
-      }
-    } else if (__builtin_expect(__any(wr.lo < least), 0)) {
+    apart = __any(!(wr.hi < (XP == 3 ? kSplits : 0x1p20f)));
+    const float least = (XP == 3 ? kSmall : __FLT_MIN__) * (lift ? kLift : 1.f);
+    if (MODE == 1 && __builtin_expect(__any(wr.lo < least), 0)) {     // (kUp: none of the scan's)
       bool few = false;
 #pragma unroll
-      for (int s = 0; s < 16; ++s) few |= below(xw[s], least);
+      for (int s = 0; s < 16; ++s) few |= below(x[s], least);
       apart |= __any(few);
     }
+    if (MODE == 0 && __builtin_expect(apart, 0)) {
+#pragma unroll
+      for (int s = 0; s < 16; ++s) xw[s] = x[s] * ((&w4[MODE == 0 ? s >> 2 : 0].x)[s & 3] * kDown);
+    }
   };
-  // the state after the chunk: dend S + k^T xw
-  auto advance = [&](const float4* kb, float dend) {
+  // the state after the chunk of n rows: dend S + k^T xw
+  auto advance = [&](const float4* kb, float dend, int n) {
     const bf16x8* kp = (const bf16x8*)kb + fresh(lane);
     if (__builtin_expect(odd || apart, 0)) {
-      if (MODE == 0 && !apart) {
+      if (MODE == 0 && !apart) {       // (judge() did it for others)
 #pragma unroll
         for (int s = 0; s < 16; ++s) xw[s] *= kDown;
       }
-      const float up = MODE == 0 && !odd ? kUp : 1.f;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[t][i] *= dend;
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
+      for (int g = 0; g < 4; ++g) {
+        float up[4];       // undoes the scaling of a key; a lifted() head's values take its weight's exponent
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          up[r] = MODE == 0 && !odd ? kUp : 1.f;
+          if (lift) {
+            const float f = tb[max(n - 1 - (8 * g + 4 * hh + r), 0)];
+            const int e = __builtin_amdgcn_frexp_expf(f);
+            xw[4 * g + r] = odd ? xw[4 * g + r] * f : __builtin_ldexpf(xw[4 * g + r], e);
+            if (!odd) up[r] = __builtin_ldexpf(kSink, -e);
+          }
+        }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const float4 a = joined(kp, 4 * t + g);
-          S[t] = mfma(a.x * up, xw[4 * g], S[t]);
-          S[t] = mfma(a.y * up, xw[4 * g + 1], S[t]);
-          S[t] = mfma(a.z * up, xw[4 * g + 2], S[t]);
-          S[t] = mfma(a.w * up, xw[4 * g + 3], S[t]);
+          S[t] = mfma(a.x * up[0], xw[4 * g], S[t]);
+          S[t] = mfma(a.y * up[1], xw[4 * g + 1], S[t]);
+          S[t] = mfma(a.z * up[2], xw[4 * g + 2], S[t]);
+          S[t] = mfma(a.w * up[3], xw[4 * g + 3], S[t]);
           __builtin_amdgcn_sched_barrier(0);
         }
+      }
       return;
+    }
+    if (lift) {          // (parts anew: scaled where they are formed they would be for every head)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = xw[8 * m + i] * kSink;
+        split8(v, w[m][0], w[m][1], w[m][2]);
+#pragma unroll
+        for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));
+      }
     }
     // piece u: rows 32 (u / 2) of the state, tokens 16 (u % 2) on; the next one's fragments are on
     // their way while a piece's products run, the smallest first
@@ -878,15 +913,23 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         }
 #pragma unroll
       for (int s = 0; s < 16; ++s) O[s] *= e;
-      // a value that is not finite must not reach the rows before its own (0 x inf)
+      float inf = 0.f;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) inf = fmaf(x[s], 0.f, inf);
+      if (__any(inf != 0.f)) {
+        // a value that is not finite must not reach the rows before its own (0 x inf)
 #pragma unroll 1
-      for (int i = 0; i < kL; ++i) {
-        f32x16 one = O;
+        for (int i = 0; i < kL; ++i) {
+          f32x16 one = O;
 #pragma unroll
-        for (int s = 0; s < 16; ++s)
-          one = mfma(8 * (s >> 2) + 4 * hh + (s & 3) <= i ? x[s] : 0.f, P[s], one);
+          for (int s = 0; s < 16; ++s)
+            one = mfma(8 * (s >> 2) + 4 * hh + (s & 3) <= i ? x[s] : 0.f, P[s], one);
 #pragma unroll
-        for (int s = 0; s < 16; ++s) O[s] = li == i ? one[s] : O[s];
+          for (int s = 0; s < 16; ++s) O[s] = li == i ? one[s] : O[s];
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) O = mfma(x[s], P[s], O);
       }
     }
   };
@@ -925,7 +968,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       }
       arrive();                       // the keys are there, the queries were used
       if (c + 1 < chunks) stage_q(c + 1);
-      advance(kbuf, dend);
+      advance(kbuf, dend, n);
       if (kNorm) {
         float ss = 0.f;
 #pragma unroll
@@ -964,7 +1007,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       fetch_weights(sc);
       weigh();
       judge();
-      advance(now, dend);
+      advance(now, dend, n);
     };
     stage(0, qbuf);
 #pragma unroll 1

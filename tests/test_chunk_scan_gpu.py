@@ -481,3 +481,53 @@ def test_scan_weights_that_decay_far(a_log):
     got = _run_scan(tuple(inp), step, H, V, N, 1, DEV)
     err = (got[0].cpu() - want[0]).norm(dim=1) / want[0].norm(dim=1)
     assert float(err.max()) < 1e-5 and _rel(got[1], want[1]) < 4e-6
+
+
+# decays on both sides of the one from which keys times weights are scaled, ones whose weights run out, zero
+@pytest.mark.parametrize("dt,V", [(torch.float32, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("lens,starts", [([64, 33], [0, 5]), ([1100], [3])])
+def test_retention_strong_decays(lens, starts, dt, V):
+    """Tokens whose weight in the state is far below the last ones'.  Then a value among them so large that
+    it counts all the same, for the states alone: rows that it rules and rows where it fades are normed, so
+    their outputs say nothing about a single product."""
+    H, D, T, B = 5, 128, sum(lens), len(lens)
+    g = torch.Generator().manual_seed(T + V)
+    proj = torch.randn(T, 2 * H * D + 2 * H * V, generator=g)
+    state = torch.randn(B, H, V, D, generator=g)
+    l2 = torch.log2(torch.tensor([0.42, 0.4, 0.05, 0.01, 0.0]))
+    args = (_step(lens, starts), H, D, V, (0, H * D, 2 * H * D, 2 * H * D + H * V), None, l2)
+    for large in (False, True):
+        if large:
+            proj[torch.tensor(lens).cumsum(0) - 17, 2 * H * D:2 * H * D + H * V] *= 3e30
+        want = _run_retention((proj.to(dt), state), *args, "cpu")
+        got = _run_retention((proj.to(dt), state), *args, DEV)
+        for h in range(H):
+            a, b = (y[0][:, h * V:(h + 1) * V].float() for y in (got, want))
+            assert large or _rel(a, b) < (6e-3 if dt == torch.bfloat16 else 4e-6)
+            assert _rel(got[1][:, h], want[1][:, h]) < 2e-6
+
+
+def test_retention_strong_decays_take_no_longer():
+    """Keys times weights split however small the weights are."""
+    H, D, T = 8, 128, 4096
+    g = torch.Generator(device=DEV).manual_seed(1)
+    proj = torch.randn(T, 4 * H * D, device=DEV, generator=g).bfloat16()
+    state, out = torch.randn(4, H, D, D, device=DEV, generator=g), proj.new_empty(T, H * D)
+    q_start, pos, slot = (t.to(DEV) for t in _step([T // 4] * 4, [0] * 4))
+
+    def time(decay):
+        l2 = torch.full((H,), math.log2(decay), device=DEV)
+        spent = []
+        for _ in range(9):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                sops.retention(out, proj, 0, H * D, 2 * H * D, 3 * H * D, state, slot, pos, q_start, None,
+                               l2, H, D, D, 1e-5)
+            b.record()
+            b.synchronize()
+            spent.append(a.elapsed_time(b))
+        return min(spent)
+    usual = time(0.97)
+    for decay in (0.2, 0.05, 0.01, 0.003):
+        assert time(decay) < 1.3 * usual       # (3.6 times as long with its products in fp32)
