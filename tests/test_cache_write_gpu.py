@@ -174,3 +174,31 @@ def test_pooled_blocks(D, Dv, pool, BS):
 
     for a, b in zip(run(DEV), run("cpu")):
         assert float((a.cpu() - b).abs().max()) <= pool * 2.0 ** -24 * 5
+
+
+def test_fp32_rows_take_no_longer_than_head_by_head():
+    """The norm over whole rows moves a sixth less than the norm per head with values of their own."""
+    T, H, G, D, BS = 13000, 16, 4, 128, 32
+    slots, pos = torch.arange(T, device=DEV), torch.arange(T, device=DEV) % 2000
+    cs = sops.rotary_table(2048, D, 1e4, None, "cpu").to(DEV)
+    proj = torch.randn(T, (H + 2 * G) * D, device=DEV)
+    q, kc = torch.empty(T, H, D, device=DEV), torch.zeros(T // BS + 1, G, BS, D, device=DEV)
+    vc = torch.zeros(T // BS + 1, G, BS // 8, D, 8, device=DEV)
+    qw, kw = torch.ones(H * D, device=DEV), torch.ones(G * D, device=DEV)
+
+    def time(step):
+        spent = []
+        for _ in range(9):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                step()
+            b.record()
+            b.synchronize()
+            spent.append(a.elapsed_time(b))
+        return min(spent)
+    whole = time(lambda: sops.proj_norm_rope_cache(proj, q, kc, vc, pos, slots, cs, qw, kw, H, G, D, 0,
+                                                   H * D, 1e-5))
+    heads = time(lambda: sops.head_norm_cache(proj, q, kc, vc, slots, H, G, D, D, 0, H * D, (H + G) * D,
+                                              1e-5, cos_sin=cs, positions=pos))
+    assert whole < 1.12 * heads
