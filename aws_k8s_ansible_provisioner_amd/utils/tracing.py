@@ -119,11 +119,19 @@ class OTLPTracer:
                             "spans": spans}]}]}
 
     def flush(self) -> int:
-        """Export what is buffered; returns after an export that the thread has under way as well."""
-        with self._export:
-            return self._flush()
+        """Export what is buffered; returns after an export that another thread has under way as well,
+        unless that one takes longer than an export's own timeout."""
+        return self._flush(self.timeout + 1)
 
-    def _flush(self) -> int:
+    def _flush(self, wait: float) -> int:
+        mine = self._export.acquire(timeout=max(wait, 0.0))
+        try:
+            return self._send()
+        finally:
+            if mine:
+                self._export.release()
+
+    def _send(self) -> int:
         with self._lock:
             spans, self._buf = self._buf, []
         if not spans:
@@ -148,8 +156,9 @@ class OTLPTracer:
     def shutdown(self) -> None:
         self._stop = True
         self._wake.set()
+        until = time.monotonic() + self.timeout + 1
         self._thread.join(timeout=self.timeout + 1)
-        self.flush()
+        self._flush(until - time.monotonic())
 
 
 _TRACER: Optional[OTLPTracer] = None

@@ -201,3 +201,30 @@ def test_flush_waits_for_export_under_way(collector):
     assert entered.wait(5)
     assert tr.flush() == 0
     assert [s["name"] for s in c.spans()] == ["one"]
+
+
+def test_shutdown_does_not_wait_for_a_stuck_export(collector):
+    """An export that never ends (a name that does not resolve, a reply that trickles) holds neither flush()
+    nor shutdown() for longer than the timeout and a second; what is buffered meanwhile still leaves."""
+    c, tr = collector
+    tr.timeout = 0.2
+    entered, go, post = threading.Event(), threading.Event(), tr.payload
+
+    def stuck(spans):
+        if threading.current_thread() is tr._thread:
+            entered.set()
+            go.wait(30)
+        return post(spans)
+    tr.payload = stuck
+    try:
+        tr.record("first", 1.0, 2.0)
+        assert entered.wait(5)
+        tr.record("second", 2.0, 3.0)
+        for call in (tr.flush, tr.shutdown):
+            t = threading.Thread(target=call, daemon=True)
+            t.start()
+            t.join(5)
+            assert not t.is_alive()
+        assert "second" in [s["name"] for s in c.spans()]
+    finally:
+        go.set()
