@@ -230,23 +230,21 @@ __global__ __launch_bounds__(64) void latent_decode_mfma_kernel(LatentAttnParams
   bf16* qs = reinterpret_cast<bf16*>(smem);
   LatentState<NV> st;
   init(st);
-  if (jb <= je) {
-    // column col is head c0 + col of token b: per-column head, one token
-    {
-      constexpr int DK = R + 16 * NKR, CH = DK / 8, P = q_pitch(DK);
-      for (int idx = lane; idx < 32 * CH; idx += 64) {
-        const int cc = idx / CH, ch = idx - cc * CH;
-        const int hh = c0 + cc < p.H ? c0 + cc : c0;
-        const bf16* src = ch * 8 < R
-            ? (const bf16*)p.q_lat + ((size_t)hh * p.T + b) * R + ch * 8
-            : (const bf16*)p.q + (size_t)b * p.q_stride + (size_t)hh * p.q_head + p.rot_off +
-                  ch * 8 - R;
-        *reinterpret_cast<bf16x8*>(qs + cc * P + ch * 8) = *reinterpret_cast<const bf16x8*>(src);
-      }
-      __builtin_amdgcn_wave_barrier();
+  // column col is head c0 + col of token b: per-column head, one token
+  {
+    constexpr int DK = R + 16 * NKR, CH = DK / 8, P = q_pitch(DK);
+    for (int idx = lane; idx < 32 * CH; idx += 64) {
+      const int cc = idx / CH, ch = idx - cc * CH;
+      const int hh = c0 + cc < p.H ? c0 + cc : c0;
+      const bf16* src = ch * 8 < R
+          ? (const bf16*)p.q_lat + ((size_t)hh * p.T + b) * R + ch * 8
+          : (const bf16*)p.q + (size_t)b * p.q_stride + (size_t)hh * p.q_head + p.rot_off +
+                ch * 8 - R;
+      *reinterpret_cast<bf16x8*>(qs + cc * P + ch * 8) = *reinterpret_cast<const bf16x8*>(src);
     }
-    attend<NV, NKR>(st, p, p.block_tables + (size_t)b * p.max_blocks, qs, pos1, pos1, jb, je);
+    __builtin_amdgcn_wave_barrier();
   }
+  attend<NV, NKR>(st, p, p.block_tables + (size_t)b * p.max_blocks, qs, pos1, pos1, jb, je);
   if (!valid) return;
   if (p.num_parts == 1) {
     store<NV>(st, (bf16*)p.out + ((size_t)h * p.T + b) * R);
@@ -266,9 +264,9 @@ __global__ __launch_bounds__(64) void latent_decode_mfma_kernel(LatentAttnParams
 
 
 // ---- wide latents (R >= 256): four waves share one tile of 32 query columns
-// (R = 512, r = 64: latent_prefill.hip, latent_decode.hip.)
-// At R = 512 a single wave's output accumulators alone are 256 registers.  Four waves split the
-// work of a 128-key step instead: wave w scores keys [32 w, 32 w + 32) of the step against the
+// (R = 256 alone: R = 512, r = 64 is latent_prefill.hip and latent_decode.hip.)
+// A single wave's output accumulators alone would be 128 registers.  Four waves split the work of a
+// 128-key step instead: wave w scores keys [32 w, 32 w + 32) of the step against the
 // whole query tile (S^T = K Q^T over all R + r dimensions), the waves agree on the running
 // maximum through LDS, publish their bf16 P fragments there, and each wave then accumulates
 // O^T for ITS quarter of the latent dimensions over all 128 keys.  No matrix product is computed
@@ -554,15 +552,12 @@ __global__ __launch_bounds__(256) void latent_decode_coop_kernel(LatentAttnParam
   if (jb > je && p.num_parts > 1) return;            // (the merge reads partitions with keys alone)
   CoopState<NVW> st;
   coop_init(st);
-  if (jb <= je) {                                    // (workgroup-uniform)
-    coop_load_rows<NV, NKR>(smem, p, p.block_tables + (size_t)b * p.max_blocks, jb, je);
-    coop_load_queries<NV, NKR>(smem, p, [&](int c, int& t, int& hh) {
-      t = b;
-      hh = c0 + c < p.H ? c0 + c : c0;
-    });
-    coop_attend<NV, NKR, 12>(st, p, p.block_tables + (size_t)b * p.max_blocks, smem, pos1, pos1, jb,
-                            je);
-  }
+  coop_load_rows<NV, NKR>(smem, p, p.block_tables + (size_t)b * p.max_blocks, jb, je);
+  coop_load_queries<NV, NKR>(smem, p, [&](int c, int& t, int& hh) {
+    t = b;
+    hh = c0 + c < p.H ? c0 + c : c0;
+  });
+  coop_attend<NV, NKR, 12>(st, p, p.block_tables + (size_t)b * p.max_blocks, smem, pos1, pos1, jb, je);
   if (!valid) return;
   if (p.num_parts == 1) {
     const float f = st.l > 0.f ? 1.0f / st.l : 0.f;
