@@ -668,7 +668,10 @@ __device__ __forceinline__ int fa_row_key(int r) {
 }
 
 constexpr int kFaRows = 128;
-constexpr int kFaTeamTiles = 8;   // key tiles up to which one team takes them all
+// Key tiles up to which one team takes them all: a prompt of 640 tokens of 16 / 8 heads, the layer, 26.5 us
+// with 0, 4 and 8, 27.3 with 16; of 800 28.7 and 30.6, 700 behind 300 32.0 and 35.3 (shorter ones have no
+// tiles of 256 rows)
+constexpr int kFaTeamTiles = 8;
 constexpr int kFaKeys = 64;
 constexpr int kFaBtCache = 1024;  // chunk -> block id cache in LDS (32768 keys)
 
@@ -819,7 +822,8 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   const int wg_last_pos = min(q_len - 1, (row0 + ROWS - 1) / G);
   const int wg_limit = ctx0 + wg_last_pos;
   const int ntiles = wg_limit / kFaKeys + 1;
-  // teams at work: few key tiles are not worth the second's sums
+  // teams at work: few key tiles are not worth the second's sums.  (Where one works the other's waves end
+  // here, and the barriers count the waves that have not ended.)
   const int teams = TEAMS > 1 && ntiles > kFaTeamTiles ? 2 : 1;
   if (team >= teams) return;
   const int w_first_pos = (row0 + 32 * w) / G;

@@ -38,9 +38,11 @@ class LatentPaths:
 
     def _latent_parts(self, rows: int, heads: int) -> int:
         """Key partitions of a decode row: static in the batch size and the model length
-        (hipGraph-capturable).  One workgroup per (row, 32 heads, partition); about one
-        workgroup per CU measured best (64 rows x 2112 keys, 16 heads, latent 512 + 64: 138 us
-        unsplit, 64 us at 4 partitions, 80 at 8, 87 at 16), a partition never under 128 keys."""
+        (hipGraph-capturable).  One workgroup per (row, 32 heads, partition), about one workgroup
+        per CU, a partition never under 128 keys.  16 heads, latent 512 + 64, ~2010 keys, the
+        rows' norms and the merge with it: 64 rows 87 us unsplit, 61 at 2 partitions, 48 at 4, 46
+        at 8, 56 at 16; 16 rows 85 unsplit, 31 at 8, 29 at 16, 37 at 33; one row 73 and 22 at 32.
+        ~285 keys: 64 rows 23 us unsplit and 24 at 4, 200 rows 30 unsplit and 37 at 2."""
         max_parts = max(1, math.ceil(self.max_model_len / 128))
         groups = max(1, rows * math.ceil(heads / 32))
         return min(max_parts, 64, max(1, math.ceil(256 / groups)))

@@ -516,8 +516,9 @@ def latent_attention_decode(out: torch.Tensor, q_lat: torch.Tensor, q: torch.Ten
                             num_parts: int = 1) -> None:
     """latent_attention with one query per sequence, at position seq_lens[b] - 1 (0: a padding
     row, left unwritten).  On the matrix cores (latent_mfma_ok) the heads of a token are the
-    columns of one tile and the keys are cut into num_parts partitions of whole 32-key blocks,
-    one wave each, merged by a second launch (workspace from latent_decode_workspace)."""
+    columns of one tile and the keys are cut into num_parts partitions of whole 32-key blocks (128
+    at a latent of 256), a workgroup each (of one wave up to a latent of 128, four at 256, four or
+    eight at 512), merged by a second launch (workspace from latent_decode_workspace)."""
     if latent_mfma_ok(cache, vgroups, q_lat.shape[2], q, rot_off, scale, block_tables.shape[1]):
         ws_ml, ws_o = workspace if (workspace is not None and num_parts > 1) else (None, None)
         torch.ops.akap_stream.latent_attention_decode_mfma(
