@@ -519,6 +519,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
                   : p.state + ((size_t)slot * p.H + h) * N * V;
   f32x16 S[NT];
   const bool load = FULL && (cut || goes_on(p, first));
+  const bool anew = FULL && (cut ? r0 == first && !goes_on(p, first) : !load);   // a state of zeros
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -891,7 +892,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
     for (int s = 0; s < 16; ++s) fin = fmaf(O[s], 0.f, fin);
     bool few = false;
-    if (__builtin_expect(__any(!(least >= kSmall)), 0)) {     // (zeros, as before a sequence's first chunk)
+    if (__builtin_expect((c > 0 || !anew) && __any(!(least >= kSmall)), 0)) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
