@@ -689,7 +689,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   auto judge = [&] {
     // Of one part they also meet pair weights that may be too small to split, see outputs(): what these
     // lose, 2^-125, stays far below the normed rows' roundings while the values are no larger.
-    apart = __any(!(wr.hi < (XP == 3 ? kSplits : 0x1p20f)));
+    apart = __any(!(wr.hi < (XP == 3 ? kSplits : 0x1p40f)));
     const float least = (XP == 3 ? kSmall : __FLT_MIN__) * (lift ? kLift : 1.f);
     if (MODE == 1 && __builtin_expect(__any(wr.lo < least), 0)) {     // (kUp: none of the scan's)
       bool few = false;

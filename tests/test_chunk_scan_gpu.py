@@ -531,3 +531,26 @@ def test_retention_strong_decays_take_no_longer():
     usual = time(0.97)
     for decay in (0.2, 0.05, 0.01, 0.003):
         assert time(decay) < 1.3 * usual       # (3.6 times as long with its products in fp32)
+
+
+@pytest.mark.parametrize("what", ["large values", "small pairs", "both"])
+def test_retention_pair_weights_of_any_size(what):
+    """bf16 values meet the products of queries and keys in three parts, which lose 2^-125 of a small one:
+    outputs against 64 bits, with values of 1e12, products of 1e-30 and both, no further off than a rounding
+    to bf16 on either side of the norm."""
+    H, V, T = 2, 128, 70
+    proj = torch.randn(T, 4 * H * V, generator=torch.Generator().manual_seed(8))
+    if what != "large values":
+        proj[:, :2 * H * V] *= 1e-15
+    if what != "small pairs":
+        proj[:, 2 * H * V:3 * H * V] *= 3e11
+    proj = proj.bfloat16()
+    l2 = torch.log2(torch.tensor([0.97, 0.3]))
+    args = (_step([T], [0]), H, V, V, (0, H * V, 2 * H * V, 3 * H * V), None, l2)
+    got = _run_retention((proj, torch.zeros(1, H, V, V)), *args, DEV)[0].cpu().double().view(T, H, V)
+    q, k, v, gate = (t.view(T, H, V).transpose(0, 1) for t in proj.double().split(H * V, 1))
+    i = torch.arange(T)
+    w = torch.exp2((i[:, None] - i).clamp_min(0) * l2.double()[:, None, None]).tril()
+    o = ((q @ k.transpose(1, 2)) * V ** -0.5 * w) @ v
+    o = o / torch.sqrt((o * o).mean(2, keepdim=True) + 1e-5) * torch.nn.functional.silu(gate)
+    assert _rel(got.transpose(0, 1), o) < 3e-3
