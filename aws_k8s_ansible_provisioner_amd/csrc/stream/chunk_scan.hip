@@ -107,19 +107,29 @@ __device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// Two values rounded to bf16, as a word: where entries of a vector are used again the compiler converts them one
+// by one and packs them afterwards (a third of all vector work here).
+__device__ __forceinline__ uint32_t pair(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, akap::bf16x2));
+}
+__device__ __forceinline__ float lower(uint32_t two) { return __uint_as_float(two << 16); }
+__device__ __forceinline__ float upper(uint32_t two) { return __uint_as_float(two & 0xffff0000u); }
+
 // v = h + m + l exactly (8 bits each, rounded to nearest) unless v is too large for bf16 or not finite
 __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& h, bf16x8& m, bf16x8& l) {
-  float r[8];
+  u32x4 a, b, c;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    h[i] = (bf16)v[i];
-    r[i] = v[i] - (float)h[i];
+  for (int i = 0; i < 4; ++i) {
+    a[i] = pair(v[2 * i], v[2 * i + 1]);
+    const float r = v[2 * i] - lower(a[i]), s = v[2 * i + 1] - upper(a[i]);
+    b[i] = pair(r, s);
+    c[i] = pair(r - lower(b[i]), s - upper(b[i]));
   }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    m[i] = (bf16)r[i];
-    l[i] = (bf16)(r[i] - (float)m[i]);
-  }
+  h = __builtin_bit_cast(bf16x8, a);
+  m = __builtin_bit_cast(bf16x8, b);
+  l = __builtin_bit_cast(bf16x8, c);
 }
 // Zeros and magnitudes in [kSmall, kSplits) split into three parts that the matrix units take as they are:
 // they take a denormal part as zero, and the last bit of 2^-101 is 2^-124.  One value outside, whatever
@@ -666,21 +676,21 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       // (parts of the unrounded product)
-      float rest[8];
+      u32x4 part[3];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int g = 2 * m + (i >> 2);
-        const float f = MODE == 0 ? (&w4[MODE == 0 ? g : 0].x)[i & 3] : 1.f;
-        w[m][0][i] = (bf16)xw[8 * m + i];
-        rest[i] = fmaf(x[8 * m + i], f, -(float)w[m][0][i]);
-      }
-      if (XP == 3) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          w[m][1][i] = (bf16)rest[i];
-          w[m][2][i] = (bf16)(rest[i] - (float)w[m][1][i]);
+      for (int i = 0; i < 4; ++i) {
+        const int at = 8 * m + 2 * i;
+        const float* f = MODE == 0 ? &w4[MODE == 0 ? at >> 2 : 0].x + (at & 3) : nullptr;
+        part[0][i] = pair(xw[at], xw[at + 1]);
+        if (XP == 3) {
+          const float r = fmaf(x[at], MODE == 0 ? f[0] : 1.f, -lower(part[0][i]));
+          const float s = fmaf(x[at + 1], MODE == 0 ? f[1] : 1.f, -upper(part[0][i]));
+          part[1][i] = pair(r, s);
+          part[2][i] = pair(r - lower(part[1][i]), s - upper(part[1][i]));
         }
       }
+#pragma unroll
+      for (int u = 0; u < XP; ++u) w[m][u] = __builtin_bit_cast(bf16x8, part[u]);
 #pragma unroll
       for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
     }
