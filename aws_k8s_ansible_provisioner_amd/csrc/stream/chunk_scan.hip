@@ -26,10 +26,10 @@
 //
 // Bound by vector work (1000 instructions per chunk, half of them the state's parts) and products (4100
 // cycles per chunk) of a wave that has its SIMD alone or shares it with one other; the next step's
-// parts are formed between a step's products.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 347 us
+// parts are formed between a step's products.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
 // where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
-// 128 x 128 (segments) 110 + 48 for the pass before it, of 136 + 66, while the fragments, half as large
-// again, take 66 of 52.
+// 128 x 128 (segments) 87 + 36 for the pass before it, while the fragments, half as large as fp32 ones again,
+// take 66.
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
 // where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
@@ -218,16 +218,64 @@ __device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int r
 constexpr int kFill = 768;
 constexpr int kScanWaves = 2048, kRetentionWaves = 1024;   // see chunk_scan_piece()
 
-__device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
-  if (n <= p.SEG) return true;
+// are the long sequences of the step cut?
+__device__ __forceinline__ bool long_ones_cut(const ChunkScanParams& p) {
   const int per = p.H * (p.V / 32);
-  if (p.B * per < kFill) return false;
+  if (p.B * per < kFill) return true;
   int count = 0;
   for (int b0 = 0; b0 < p.B; b0 += 64) {
     const int b = b0 + (int)(threadIdx.x & 63);
     count += __popcll(__ballot(b < p.B && p.q_start[b + 1] - p.q_start[b] > p.SEG));
   }
-  return count * per >= kFill;
+  return count * per < kFill;
+}
+__device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
+  return n <= p.SEG || !long_ones_cut(p);
+}
+
+// The step's item-th walk: of the sequences that are not cut (WHOLE: else none of these) first, then of the cut
+// ones' segments, without gaps.  True: there is one, of rows [r0, r1) of sequence b.  A lane looks at a
+// sequence.
+template <bool WHOLE>
+__device__ __forceinline__ bool walk_of(const ChunkScanParams& p, int item, int& b, int& r0, int& r1, bool& cut) {
+  const int lane = threadIdx.x & 63;
+  const bool cuts = long_ones_cut(p);
+  if (p.B == 1) {
+    const ScalarInts q_start = (ScalarInts)p.q_start;
+    const int first = q_start[0], end = q_start[1];
+    cut = cuts && end - first > p.SEG;
+    b = 0;
+    r0 = first + (cut ? item * p.PIECE : 0);
+    r1 = cut ? min(r0 + p.PIECE, end) : end;
+    return r1 > r0 && (cut || (WHOLE && item == 0));
+  }
+  for (int turn = WHOLE ? 0 : 1; turn < 2; ++turn)
+    for (int b0 = 0; b0 < p.B; b0 += 64) {
+      const int from = p.q_start[min(b0 + lane, p.B)], n = p.q_start[min(b0 + lane + 1, p.B)] - from;
+      const bool long_one = cuts && n > p.SEG;
+      const int walks = n <= 0 ? 0 : turn == 0 ? !long_one : long_one ? (n + p.PIECE - 1) / p.PIECE : 0;
+      // sums up to a lane: within rows of 16, then the last lane of one row or two to the next
+      int upto = walks;
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xc, 0xf, false);
+      const int total = __builtin_amdgcn_readlane(upto, 63);
+      if (item < total) {
+        const int at = __ffsll((unsigned long long)__ballot(upto > item)) - 1;
+        const int first = __builtin_amdgcn_readlane(from, at), end = first + __builtin_amdgcn_readlane(n, at);
+        const int k = item - __builtin_amdgcn_readlane(upto - walks, at);
+        cut = turn == 1;
+        b = b0 + at;
+        r0 = first + (cut ? k * p.PIECE : 0);
+        r1 = cut ? min(r0 + p.PIECE, end) : end;
+        return true;
+      }
+      item -= total;
+    }
+  return false;
 }
 
 // first segment of sequence b in the buffers (long sequences alone have any): counted like the
@@ -485,24 +533,29 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, hh = lane >> 5;
-  // SEGM: a workgroup per segment of a cut sequence and head, FULL ahead of all of them one per sequence
-  // and head for those that are not cut (side by side, so that they spread over the CUs as without
-  // SEGM: between workgroups that only leave, 24 sequences of 600 rows took 275 us and not 187)
-  const int whole = SEGM && !FULL ? 0 : p.B * (p.H / HW);
-  const bool cut = SEGM && (int)blockIdx.x >= whole;
-  const int entry = blockIdx.x - (cut ? whole : 0), entries = cut ? p.T / p.PIECE + p.B : p.B;
-  const int h0 = entry / entries * HW, hw = wave / VW, h = h0 + hw;
-  int b = entry % entries, r0, r1;
-  if (cut) {
-    b = locate(p, b, p.PIECE, r0, r1);
+  // SEGM: a workgroup per head and segment of a cut sequence (FULL: or sequence that is not cut), those that
+  // find none last.  One that leaves at once shifts the turns in which the next ones are dealt out to the
+  // CUs, and some then wait behind a full one: with such between them a tenth of the waves of 8 x 2048 rows,
+  // 8 heads x 128 x 128 began when others had ended (passes of 48 and 111 us, now 36 and 87).  Heads of eight
+  // walks side by side: a walk keeps to one XCD, whose cache then holds what the scan's heads share
+  // (24 sequences of 100 rows, 8 heads: 45.6 us, heads side by side 49.3).
+  const int heads = p.H / HW;
+  int b, r0, r1, h0;
+  bool cut = false;
+  if (SEGM) {
+    constexpr int kSide = 8;
+    const int at = blockIdx.x % (kSide * heads);
+    h0 = at / kSide * HW;
+    if (!walk_of<FULL>(p, (int)blockIdx.x / (kSide * heads) * kSide + at % kSide, b, r0, r1, cut)) return;
   } else {
-    b = uniform(b);
+    h0 = (int)blockIdx.x / p.B * HW;
+    b = blockIdx.x % p.B;
     r0 = ((ScalarInts)p.q_start)[b];
     r1 = ((ScalarInts)p.q_start)[b + 1];
+    if (r1 <= r0) return;
   }
-  if (r1 <= r0) return;
+  const int hw = wave / VW, h = h0 + hw;
   const int first = ((ScalarInts)p.q_start)[b];
-  if (SEGM && walked_whole(p, ((ScalarInts)p.q_start)[b + 1] - first) == cut) return;
   const size_t seg = cut ? (size_t)uniform((int)seg_base(p, b) + (r0 - first) / p.PIECE) : 0;
   const int slot = uniform(p.seq_slot[first]);
   if (!live_slot(p, slot)) return;
@@ -1095,10 +1148,11 @@ void run(const ChunkScanParams& p, hipStream_t s) {
     chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
     return;
   }
-  const int segs = p.T / p.PIECE + p.B;
-  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<segs * (p.H / HW), nt, 0, s>>>(p);
+  // (whole multiples of eight walks)
+  const int walks = (p.T / p.PIECE + p.B + 7) / 8 * 8 * (p.H / HW);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<walks, nt, 0, s>>>(p);
   chunk_join_kernel<<<dim3(p.B, p.H, (p.V * p.N + 1023) / 1024), 256, 0, s>>>(p);
-  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<(p.B + segs) * (p.H / HW), nt, 0, s>>>(p);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true><<<walks, nt, 0, s>>>(p);
 }
 
 // two heads of 64 columns that share their keys go through one workgroup: the keys' fragments

@@ -75,10 +75,13 @@ def test_selective_scan_chunks(lens, starts, H, V, N, G, dt):
 
 # lens, starts, heads of the scan and of the retention (V 64): two cut sequences of five, one continued, a
 # padding sequence; one long continued one; a prompt among rows of one token (whose number alone would
-# fill the chip); as many long sequences as fill it, so that none is cut
+# fill the chip); as many long sequences as fill it, so that none is cut; more sequences than a wave has lanes
 CUT = [([700, 600, 1, 3, 257], [0, 10, 0, -1, 4], 4, 4), ([1100], [9], 4, 4),
        ([1] * 50 + [1100] + [1] * 10 + [300], [7] * 50 + [0] + [5] * 10 + [40], 8, 8),
-       ([300] * 24 + [1] * 10, [0, 3] * 12 + [9] * 10, 16, 16)]
+       ([300] * 24 + [1] * 10, [0, 3] * 12 + [9] * 10, 16, 16),
+       # cut sequences on both sides of the 64th, sequences without rows among them and at the ends
+       ([0, 1100, 0, 2] + [1] * 58 + [0, 520, 700] + [3] * 5 + [300, 0], [0, 4, 0, 9] + [6] * 58 + [0, 0, 8]
+        + [2] * 5 + [0, 0], 2, 2)]
 
 
 @pytest.mark.parametrize("lens,starts,H,_", CUT)
