@@ -10,12 +10,14 @@
 // "half-tile" is 128 rows x 64 k (16 KB: two 1-KiB DMA instructions per wave), issued in the
 // order the phases consume them, so every wait is a counted `s_waitcnt vmcnt` (never 0 in
 // steady state: cdna_hip_programming.md "Pipelining across barriers", T3+T4).
-// DEFAULT K loop (SCHED 4, "stream-first"): one counted wait + one barrier per K tile,
-// then the whole next K tile (four half-tiles, 64 KiB) is requested at once and streams into the
-// other buffer under this tile's 64 MFMAs per wave.  A no-math probe of exactly this operand
-// stream runs as fast as hipBLASLt's whole GEMM, and the phase pipeline below measured ~stream +
-// math; the stream-first loop is 5-14 % faster than it (0.70-0.88x hipBLASLt dense, 0.97-1.11x
-// with the SwiGLU epilogue).  The phase pipeline (SCHED 1):
+// DEFAULT K loop (SCHED 4): the two waves of a SIMD alternate, one reads fragments and requests data while the
+// other multiplies (pg_mainloop has the order).  Bound by what passes through LDS, 192 KB of fragments and
+// 64 KB of data a K tile, beside 2048 cycles of products: 3200 cycles a K tile.  One counted wait and one
+// barrier per K tile, with the whole next tile requested behind it (what 4 waves still run), had every wave
+// read at the same time and multiply at the same time: 8 experts of 2816 x 2048 and 2048 x 1408, 31 thousand rows,
+// 356 + 194 us, now 348 + 191; dense 31232 x 7168 x 4096 1483 -> 1430, 8192 cubed 799 -> 792 (hipBLASLt
+// 1218 and 674).  Workgroups that stay and request their next tile's data before they store gained nothing.
+// The phase pipeline (SCHED 1):
 // NB = 2 (plain store; two raw s_barriers per K tile):
 //   phase | counted wait + barrier           | ds_reads issued            | DMA issued
 //   1     | W right + A bottom of tile t     | B right + A bottom (t)     | W right, A bottom (t+1)
@@ -334,6 +336,84 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     __builtin_amdgcn_s_setprio(0);
   };
 
+  if constexpr (SCHED == 4 && WAVES == 8) {
+    // ---- alternating schedule: the two waves of a SIMD (rows 0 .. 127 and 128 .. 255 of the tile) take turns,
+    // one reads the next quadrant's fragments and requests a half-tile while the other multiplies a
+    // quadrant.  A turn ends with a barrier; the second four waves are one turn behind.
+    //   turn pair | read                 | requested      | product
+    //   1         | W right (t)          | A top (t+2)    | A top x W left
+    //   2         | A bottom (t)         | W left (t+2)   | A top x W right
+    //   3         | A top (t+1)          | W right (t+2)  | A bottom x W left
+    //   4         | W left (t+1)         | A bottom (t+2) | A bottom x W right
+    // A half-tile's place is requested again two turns after the later group's reads of it have
+    // completed (they are waited for where a product's turn begins), and it has landed for every wave a
+    // turn before the earlier group reads it: five half-tiles are younger then.
+    auto turn = [&] {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto read = [&] {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(H0{}, 0);
+    issue(H1{}, 0);
+    issue(H2{}, 0);
+    issue(H3{}, 0);
+    issue(H0{}, 1);
+    issue(H1{}, 1);
+    issue(H2{}, 1);
+    issue(H3{}, 1);
+    if (nk > 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    turn();
+    rd_a(at, lds, 0);
+    rd_b(bl, lds, 0);
+    if (wm) turn();
+    for (int t = 0; t < nk; ++t) {
+      const bf16x8* cur = lds + (t & 1) * PG_BUF;
+      const bf16x8* nxt = lds + ((t + 1) & 1) * PG_BUF;
+      // the half-tile of the next turn but one has landed (2 instructions per half-tile)
+      auto landed = [&](auto last) {
+        if (t + 2 < nk) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+        else if (t + 2 == nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(last)::value) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      };
+      issue(H0{}, t + 2);
+      rd_b(br, cur, 1);
+      landed(HalfTile<8>{});
+      turn();
+      read();
+      mma(at, bl, 0, 0);
+      turn();
+      issue(H1{}, t + 2);
+      rd_a(ab, cur, 1);
+      landed(HalfTile<6>{});
+      turn();
+      read();
+      mma(at, br, 0, NJ);
+      turn();
+      issue(H2{}, t + 2);
+      if (t + 1 < nk) rd_a(at, nxt, 0);
+      landed(HalfTile<4>{});
+      turn();
+      read();
+      mma(ab, bl, 4, 0);
+      turn();
+      issue(H3{}, t + 2);
+      if (t + 1 < nk) rd_b(bl, nxt, 0);
+      landed(HalfTile<2>{});
+      turn();
+      read();
+      mma(ab, br, 4, NJ);
+      turn();
+    }
+    if (!wm) turn();
+    return;
+  }
   if constexpr (SCHED == 4) {
     // ---- stream-first schedule: the whole next K tile (all four half-tiles, 64 KiB) is
     // requested right after this tile's barrier and streams under this tile's MFMAs.  The
@@ -713,15 +793,24 @@ __device__ __forceinline__ void pg_store(bf16* to, f32x4 y) {
   for (int r = 0; r < 4; ++r) o[r] = f2bf(y[r]);
   *reinterpret_cast<bf16x4*>(to) = o;
 }
+// (Conversions in pairs, as words whose halves are taken out by shift and mask; the reciprocal as it comes, one
+// unit in the last place of fp32: half the vector work of an output; 31 thousand rows of 2816 x 2048 348 -> 337 us.)
 __device__ __forceinline__ void pg_store_silu(bf16* to, f32x4 gate, f32x4 up) {
-  bf16x4 o;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  auto two = [](float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+  };
+  auto lower = [](uint32_t v) { return __uint_as_float(v << 16); };
+  auto upper = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+  uint32_t o[2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float g = bf2f(f2bf(gate[r]));
-    const float u = bf2f(f2bf(up[r]));
-    o[r] = f2bf(bf2f(f2bf(g / (1.f + __expf(-g)))) * u);
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t g = two(gate[2 * r], gate[2 * r + 1]), u = two(up[2 * r], up[2 * r + 1]);
+    auto silu = [](float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); };
+    const uint32_t sg = two(silu(lower(g)), silu(upper(g)));
+    o[r] = two(lower(sg) * lower(u), upper(sg) * upper(u));
   }
-  *reinterpret_cast<bf16x4*>(to) = o;
+  *reinterpret_cast<uint2*>(to) = make_uint2(o[0], o[1]);
 }
 
 template <int EPI, bool GROUPED, int NB, int WAVES, int SCHED = 1>
@@ -1031,10 +1120,9 @@ long pgemm_sk_ws_floats(int M, int N, int splits) {
 // Wave form of the 256 x 256 body: AKAP_PGEMM_WAVES = 8 (2 x 4 waves of 128 x 64) or 4 (2 x 2
 // waves of 128 x 128), read once per process.
 // K-loop issue schedule: AKAP_PGEMM_SCHED = 1 (phase pipeline, half-tiles requested 1.0-1.25
-// tiles ahead), 2 (early issue, 1.25-1.75 tiles ahead), 3 (4-wave unit body), 4 (default,
-// stream-first: the whole next tile under this tile's math, 5-14 % faster than 1 on the dense
-// verdict shapes; pg_mainloop), read once per process.  The
-// decode split-K form (launch_pgemm_sk) keeps 1 / 2.
+// tiles ahead), 2 (early issue, 1.25-1.75 tiles ahead), 3 (4-wave unit body), 4 (default:
+// with 8 waves the alternating body, with 4 the whole next tile under this tile's math; pg_mainloop), read
+// once per process.  The decode split-K form (launch_pgemm_sk) keeps 1 / 2.
 int pgemm_sched() {
   static int v = [] {
     const char* e = getenv("AKAP_PGEMM_SCHED");
