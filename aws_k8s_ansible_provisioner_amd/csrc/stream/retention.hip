@@ -1013,73 +1013,89 @@ __global__ __launch_bounds__(1024) void route_topk_kernel(int32_t* __restrict__ 
   if (threadIdx.x == 0) route_pick(lds, n, top, ids + (size_t)t * top, wout + (size_t)t * top);
 }
 
-// The same sums in the same order with the router's pieces used for kRouteRows rows at a time (large
-// steps; d a multiple of 4, rows of whole 4-element pieces).  A wave takes two logits per turn.  Bound
-// by its vector instructions (about 20 of 37 us at 16384 rows of 2048, 8 experts); with a row per
-// workgroup the fp32 router is read from L2 once per row, 86 us; 8 rows at a time 40.
-constexpr int kRouteRows = 4;
-
-template <typename T>
+// The same sums in the same order for large steps (d a multiple of 4, rows of whole 4-element pieces): a wave
+// takes R rows and eight logits per turn, so that a row's entries are widened once for eight sums and the
+// router's pieces serve R rows.  The sums' lanes meet as in wave_sum, but of 8 R values at once: at each
+// distance a lane hands on the half of its values that its partner goes on with, 32 exchanges for 192.
+// Bound by vector work and the latency of a wave's own loads, which are one piece ahead: 15600 rows of 2048, 8
+// logits 21.4 us (64: 121), 6000 of 4096 17.4; four waves that shared their rows' logits, each widening the
+// entries for two, took 27.5 (146) and 27.7.
+template <typename T, int R>
 __global__ __launch_bounds__(256) void route_topk_rows_kernel(int32_t* __restrict__ ids,
                                                               float* __restrict__ wout,
                                                               const T* __restrict__ h, int h_stride,
                                                               const float* __restrict__ router,
                                                               const float* __restrict__ bias,
                                                               int rows, int d, int n, int top) {
-  extern __shared__ __align__(16) unsigned char route_smem[];   // [R][n] logits, [R][d] rows
+  extern __shared__ float route_z[];   // [4 waves][R][n] logits
   typedef T Piece __attribute__((ext_vector_type(4)));
-  float* z = (float*)route_smem;
-  Piece* hs = (Piece*)(route_smem + ((kRouteRows * n * 4 + 15) & ~15));
-  const int t0 = blockIdx.x * kRouteRows, nr = min(kRouteRows, rows - t0), dp = d >> 2;
+  constexpr int E = 8;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int c = threadIdx.x; c < dp; c += 256) {
-    Piece x[kRouteRows];
+  const int t0 = (blockIdx.x * 4 + wave) * R;
+  float* z = route_z + wave * R * n;
+  const T* hr[R];
 #pragma unroll
-    for (int r = 0; r < kRouteRows; ++r)
-      x[r] = *(const Piece*)(h + (size_t)(t0 + min(r, nr - 1)) * h_stride + c * 4);
+  for (int r = 0; r < R; ++r) hr[r] = h + (size_t)min(t0 + r, rows - 1) * h_stride;
+  for (int e0 = 0; e0 < n; e0 += E) {
+    float a0[R * E], a1[R * E];
 #pragma unroll
-    for (int r = 0; r < kRouteRows; ++r) hs[r * dp + c] = x[r];
-  }
-  __syncthreads();
-  for (int e0 = wave; e0 < n; e0 += 8) {
-    const float* wr[2] = {router + (size_t)e0 * d, router + (size_t)min(e0 + 4, n - 1) * d};
-    float a0[2][kRouteRows], a1[2][kRouteRows];
+    for (int v = 0; v < R * E; ++v) a0[v] = a1[v] = 0.f;
+    struct Pieces {
+      Piece x[R];
+      float4 w[E];
+    };
+    auto load = [&](int c, Pieces& in) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int r = 0; r < R; ++r) in.x[r] = *(const Piece*)(hr[r] + c);
 #pragma unroll
-      for (int r = 0; r < kRouteRows; ++r) a0[u][r] = a1[u][r] = 0.f;
-    auto add = [&](int c, float (&a)[2][kRouteRows]) {
-      float4 w4[2];
+      for (int e = 0; e < E; ++e) in.w[e] = *(const float4*)(router + (size_t)min(e0 + e, n - 1) * d + c);
+    };
+    auto add = [&](const Pieces& in, float (&a)[R * E]) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) w4[u] = *(const float4*)(wr[u] + c);
+      for (int r = 0; r < R; ++r) {
+        const float x[4] = {(float)in.x[r][0], (float)in.x[r][1], (float)in.x[r][2], (float)in.x[r][3]};
 #pragma unroll
-      for (int r = 0; r < kRouteRows; ++r) {
-        const Piece x = hs[r * dp + (c >> 2)];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          a[u][r] = fmaf((float)x[0], w4[u].x,
-                         fmaf((float)x[1], w4[u].y,
-                              fmaf((float)x[2], w4[u].z, fmaf((float)x[3], w4[u].w, a[u][r]))));
+        for (int e = 0; e < E; ++e)
+          a[r * E + e] = fmaf(x[0], in.w[e].x, fmaf(x[1], in.w[e].y,
+                         fmaf(x[2], in.w[e].z, fmaf(x[3], in.w[e].w, a[r * E + e]))));
       }
     };
+    // (a piece is on its way while the one before is used; past the end the first again)
     int c = lane * 4;
+    Pieces in0, in1;
+    load(c < d ? c : 0, in0);
     for (; c + 256 < d; c += 512) {
-      add(c, a0);
-      add(c + 256, a1);
+      load(c + 256, in1);
+      __builtin_amdgcn_sched_barrier(0);
+      add(in0, a0);
+      load(c + 512 < d ? c + 512 : 0, in0);
+      __builtin_amdgcn_sched_barrier(0);
+      add(in1, a1);
     }
-    if (c < d) add(c, a0);
+    if (c < d) add(in0, a0);
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int v = 0; v < R * E; ++v) a0[v] += a1[v];
+    // value v ends in the lanes whose upper bits, from 32 down, are v's lower ones
+    constexpr int kHalvings = R == 4 ? 5 : 4;
 #pragma unroll
-      for (int r = 0; r < kRouteRows; ++r) {
-        const float a = wave_sum(a0[u][r] + a1[u][r]);
-        const int e = e0 + 4 * u;
-        if (lane == 0 && e < n) z[r * n + e] = a + (bias ? bias[e] : 0.f);
+    for (int k = 0; k < kHalvings; ++k) {
+      const int o = 32 >> k;
+      const bool up = lane & o;
+#pragma unroll
+      for (int v = 0; v < (R * E) >> (k + 1); ++v) {
+        const float mine = up ? a0[2 * v + 1] : a0[2 * v], other = up ? a0[2 * v] : a0[2 * v + 1];
+        a0[v] = mine + __shfl_xor(other, o, 64);
       }
+    }
+#pragma unroll
+    for (int o = 32 >> kHalvings; o > 0; o >>= 1) a0[0] += __shfl_xor(a0[0], o, 64);
+    const int v = __brev((unsigned)lane) >> 26 & (R * E - 1);
+    const int e = e0 + v % E;
+    if ((lane & ((64 >> kHalvings) - 1)) == 0 && e < n) z[v / E * n + e] = a0[0] + (bias ? bias[e] : 0.f);
   }
   __syncthreads();
-  const int r = threadIdx.x;
-  if (r < nr) route_pick(z + r * n, n, top, ids + (size_t)(t0 + r) * top, wout + (size_t)(t0 + r) * top);
+  if (lane < R && t0 + lane < rows)
+    route_pick(z + lane * n, n, top, ids + (size_t)(t0 + lane) * top, wout + (size_t)(t0 + lane) * top);
 }
 
 // out[t, e F + f] = w_e(t) act(gu[t, e 2F + f]) gu[t, e 2F + F + f]; ids null: weight 1;
@@ -1288,17 +1304,21 @@ void launch_route_topk(int32_t* ids, float* w, const void* h, int h_stride, cons
                        hipStream_t s) {
   if (rows <= 0) return;
   const size_t es = f32 ? 4 : 2;
-  const size_t rlds = (((size_t)kRouteRows * n * 4 + 15) & ~(size_t)15) + (size_t)kRouteRows * d * es;
-  // (from 1024 rows on the chip is full with 4 rows to a workgroup)
-  if (rows >= 256 * kRouteRows && d % 4 == 0 && h_stride % 4 == 0 && rlds <= 65536 &&
+  if (rows >= 1024 && d % 4 == 0 && h_stride % 4 == 0 && n <= 1024 &&
       ((uintptr_t)h & (4 * es - 1)) == 0 && ((uintptr_t)router & 15) == 0) {
-    const int grid = (rows + kRouteRows - 1) / kRouteRows;
-    if (f32)
-      route_topk_rows_kernel<float><<<grid, 256, rlds, s>>>(ids, w, (const float*)h, h_stride, router,
-                                                            bias, rows, d, n, top);
-    else
-      route_topk_rows_kernel<bf16><<<grid, 256, rlds, s>>>(ids, w, (const bf16*)h, h_stride, router,
-                                                           bias, rows, d, n, top);
+    // (8 logits, a wave of two rows / four: 2000 rows of 4096 10.0 / 11.6 us, 3000 of 2048 9.8 / 9.1)
+    const int R = rows >= 2560 ? 4 : 2;
+    const int grid = (rows + 4 * R - 1) / (4 * R);
+    const size_t zlds = (size_t)4 * R * n * sizeof(float);
+#define AKAP_RR(TY, N)                                                                              \
+  route_topk_rows_kernel<TY, N><<<grid, 256, zlds, s>>>(ids, w, (const TY*)h, h_stride, router, bias, rows, \
+                                                        d, n, top)
+    if (f32) {
+      if (R == 4) AKAP_RR(float, 4); else AKAP_RR(float, 2);
+    } else {
+      if (R == 4) AKAP_RR(bf16, 4); else AKAP_RR(bf16, 2);
+    }
+#undef AKAP_RR
     return;
   }
   const size_t lds = (size_t)(((n + 3) & ~3) + d) * sizeof(float);

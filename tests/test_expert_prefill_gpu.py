@@ -59,7 +59,9 @@ def test_large_steps(T, d, F, pad):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,d,n,top", [(1023, 256, 8, 2), (1024, 260, 9, 3), (1025, 1000, 3, 1)])
+@pytest.mark.parametrize("T,d,n,top", [(1023, 256, 8, 2), (1024, 260, 9, 3), (1025, 1000, 3, 1),
+                                       (2559, 512, 8, 2), (2561, 516, 17, 4), (2563, 4, 2, 1),
+                                       (2560, 768, 40, 8)])
 def test_routing(T, d, n, top, dt):
     """Sums of d products in fp32 on both sides: logits within d 2^-24 of the products' sum of
     magnitudes; the winners agree where the logits differ by more."""
