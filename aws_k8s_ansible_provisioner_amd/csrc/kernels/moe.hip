@@ -263,12 +263,13 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
   }
 }
 
-// The same for up to 32 experts without atomics, over 16 workgroups that need no word from each
-// other: every one counts all ids by segments, each wave one segment, and places its own.  A wave counts
-// by ballots into its own row of counters; a second walk puts every id at its cursor plus its rank among
-// the lanes with the same id -- a stable sort.  Bound by latencies: 32768 ids of 8 experts 19 us; in one
-// workgroup 26 us with an LDS atomic per id, 29 us with ballots.
-constexpr int kAlignE = 32;
+// The same for up to 32 experts without a word between its 64 workgroups: every one counts all ids by segments,
+// each wave four, with LDS adds to several counters of an id so that few lanes meet at one, and places its
+// own segment's.  There a wave counts its run of ids by ballots, a lane an id, and a second walk puts every id at
+// its cursor plus its rank among the lanes with the same id -- a stable sort.  Bound by latencies: 31200 ids of
+// 8 experts 12.4 us, 60000 of 16 19.7; 16 workgroups that counted by ballots, a read and a write after each other
+// per 64 ids, 17 and 32; one workgroup 26 us at 32768 ids with an LDS atomic per id.
+constexpr int kAlignE = 32, kAlignSegs = 64;
 
 __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __restrict__ ids, int n,
                                                              int E, int block,
@@ -278,7 +279,8 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
                                                              int32_t* __restrict__ inv,
                                                              int32_t* __restrict__ tile_expert,
                                                              int max_tiles) {
-  __shared__ int seg[16][kAlignE], run[16][kAlignE];   // ids per segment, per wave of my segment
+  __shared__ int hist[kAlignSegs][64];                          // ids per segment, 2^(6 - bits) counters each
+  __shared__ int seg[kAlignSegs][kAlignE], run[16][kAlignE];   // their sums; ids per wave of my segment
   __shared__ int total[kAlignE], mine[kAlignE], offs[kAlignE + 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x;
@@ -314,21 +316,37 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
     __builtin_amdgcn_wave_barrier();
   };
   auto count = [&](int* row, int lo, int hi) {
-    if (lane < E) row[lane] = 0;
-    wave_sync();
+    int sum = 0;
     walk(lo, hi, [&](int id, int) {
-      const uint64_t same = peers(id);
-      if (same && !(same & below)) row[id] += __popcll(same);   // the first of them
-      wave_sync();
+      uint64_t mine = __ballot((unsigned)id < (unsigned)E);
+      for (int k = 0; k < bits; ++k) {
+        const uint64_t m = __ballot((id >> k) & 1);
+        mine &= (lane >> k) & 1 ? m : ~m;
+      }
+      sum += __popcll(mine);
     });
+    if (lane < E) row[lane] = sum;
   };
   // segments and, in mine, runs of whole 64s
-  const int sper = (((n + 15) >> 4) + 63) & ~63;
+  const int sper = ((n + kAlignSegs - 1) / kAlignSegs + 63) & ~63;
   const int s0 = min(b * sper, n), s1 = min(s0 + sper, n);
   const int rper = (((s1 - s0 + 15) >> 4) + 63) & ~63;
   const int r0 = min(s0 + wave * rper, s1), r1 = min(r0 + rper, s1);
-  count(seg[wave], min(wave * sper, n), min(wave * sper + sper, n));
+  for (int i = tid; i < kAlignSegs * 64; i += 1024) (&hist[0][0])[i] = 0;
+  __syncthreads();
+  const int copy = (lane << bits) & 63;
+  walk(min(4 * wave * sper, n), min((4 * wave + 4) * sper, n), [&](int id, int i) {
+    const int s = __builtin_amdgcn_readfirstlane((i - lane) / sper);
+    if ((unsigned)id < (unsigned)E) atomicAdd(&hist[s][copy | id], 1);
+  });
   count(run[wave], r0, r1);
+  __syncthreads();
+  for (int i = tid; i < kAlignSegs * E; i += 1024) {
+    const int s = i / E, e = i % E;
+    int sum = 0;
+    for (int c = 0; c < 64; c += 1 << bits) sum += hist[s][c | e];
+    seg[s][e] = sum;
+  }
   __syncthreads();
   if (tid < E) {
     int sum = 0;
@@ -339,7 +357,7 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
     }
     int before = 0;
     sum = 0;
-    for (int s = 0; s < 16; ++s) {
+    for (int s = 0; s < kAlignSegs; ++s) {
       if (s == b) before = sum;
       sum += seg[s][tid];
     }
@@ -541,9 +559,9 @@ void launch_moe_combine(const void* Y, const float* wts, const int32_t* inv, voi
 void launch_moe_align(const int32_t* topk_ids, int n, int E, int block, int32_t* sorted_ids,
                       int32_t* expert_offsets, int32_t* num_padded, int32_t* inv,
                       int32_t* tile_expert, int max_tiles, hipStream_t s) {
-  // (4096 ids 5.7 -> 6.9 us, 32768 ids 26 -> 19: below 8192 one workgroup is done sooner)
+  // (below 8192 ids one workgroup is done as soon)
   if (E <= kAlignE && n >= 8192) {
-    moe_align_few_kernel<<<16, 1024, 0, s>>>(topk_ids, n, E, block, sorted_ids, expert_offsets,
+    moe_align_few_kernel<<<kAlignSegs, 1024, 0, s>>>(topk_ids, n, E, block, sorted_ids, expert_offsets,
                                             num_padded, inv, tile_expert, max_tiles);
     return;
   }

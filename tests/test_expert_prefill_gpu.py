@@ -79,7 +79,8 @@ def test_routing(T, d, n, top, dt):
     assert torch.equal(few[0].cpu().long(), ids[:100]) and torch.equal(few[1].cpu(), w[:100])
 
 
-@pytest.mark.parametrize("n,E,run", [(8192, 32, 1), (9000, 8, 64), (16500, 3, 4000)])
+@pytest.mark.parametrize("n,E,run", [(8192, 32, 1), (9000, 8, 64), (16500, 3, 4000), (8193, 1, 7),
+                                     (70001, 17, 3)])
 def test_align_runs(n, E, run):
     """Ids by turns in runs: a counter goes from lane to lane of a wave, or stays with one for long."""
     ids = (torch.arange(n) // run % E).to(torch.int32)
