@@ -10,6 +10,7 @@ using akap::bf16;
 using akap::bf16x4;
 using akap::bf16x8;
 using akap::f32x16;
+using akap::f32x4;
 
 namespace {
 
@@ -313,46 +314,70 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
 }
 
 // out = talk x the heads' normalised sums, times the gate.  A lane takes 4 value entries of a token,
-// all heads' sums of them in flight together.  Bound by reading the sums: 90 us for 8000 rows of
-// 16 x 512 fp32 (262 MB), their gates and outputs; a workgroup per token with 4-byte loads took 174.
+// all heads' sums of them in flight together, past the caches: they are read once, and lines that the
+// attention just wrote need not make room for them.  Bound by reading the sums: 60 us for 7300 rows of
+// 16 x 512 fp32 (240 MB), their gates and outputs, 81 us for 2500 rows of 32 x 1024 (328 MB); through the
+// caches 67 and 109.  No branch, coefficient or gate stands between a head's loads: with one of each per
+// head 91 and 142 us, and 10.1 for 6.6 where the step is 200 rows.
 template <int HM>
 __global__ __launch_bounds__(256) void talk_mix_kernel(TalkParams p) {
   const int t = ((p.row0 >> 5) + blockIdx.x) * 32 + (threadIdx.x & 31);
   const int e4 = blockIdx.y * 8 + (threadIdx.x >> 5), GV = p.G * p.Dv;
   if (e4 * 4 >= GV || t < p.row0 || t >= p.T) return;
-  if (p.seq_lens[sequence_of(p.q_start, p.B, t)] <= 0) return;
   const int c = __builtin_amdgcn_readfirstlane(e4 * 4 / p.Dv);   // (a wave's: Dv is whole 32s)
   const int dv = e4 * 4 - c * p.Dv, rep = p.H / p.G;
-  float4 o[HM];
+  f32x4 o[HM];
 #pragma unroll
   for (int g = 0; g < HM; ++g)
-    if (g < p.H) o[g] = *(const float4*)(p.ws_o + ws_at(p, t, g, e4));
+    o[g] = akap::ld_nt((const f32x4*)(p.ws_o + ws_at(p, t, min(g, p.H - 1), e4)));
   const bool wide = ((p.gate_stride & 3) | ((uintptr_t)p.gate & 7) | (p.out_stride & 3) |
                      ((uintptr_t)p.out & 7)) == 0;
+  const __attribute__((address_space(4))) float* talk =
+      (const __attribute__((address_space(4))) float*)p.talk;
+  bf16x4 next = {};
+  auto gates = [&](int i) __attribute__((always_inline)) {
+    if (!p.gate || i >= rep) return;
+    const bf16* gp = (const bf16*)p.gate + (size_t)t * p.gate_stride + (c * rep + i) * p.Dv + dv;
+    if (wide) {
+      next = *(const bf16x4*)gp;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) next[e] = gp[e];
+    }
+  };
+  gates(0);
+  if (p.seq_lens[sequence_of(p.q_start, p.B, t)] <= 0) return;
+#pragma unroll
+  for (int g = 0; g < HM; ++g)
+    if (g >= p.H) o[g] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int i = 0; i < rep; ++i) {
     const int h = c * rep + i;
+    const bf16x4 z = next;
+    gates(i + 1);                         // (asked for before the stores that it could alias)
     float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.talk) {
+      float f[HM];
 #pragma unroll
-    for (int g = 0; g < HM; ++g)
-      if (g < p.H && (p.talk || g == h)) {
-        const float f = p.talk ? p.talk[(size_t)h * p.H + g] : 1.f;
-        v[0] = fmaf(f, o[g].x, v[0]); v[1] = fmaf(f, o[g].y, v[1]);
-        v[2] = fmaf(f, o[g].z, v[2]); v[3] = fmaf(f, o[g].w, v[3]);
+      for (int g = 0; g < HM; ++g) f[g] = talk[(size_t)h * p.H + min(g, p.H - 1)];
+#pragma unroll
+      for (int g = 0; g < HM; ++g) {
+        const float fg = g < p.H ? f[g] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = fmaf(fg, o[g][e], v[e]);
       }
-    const int col = h * p.Dv + dv;
+    } else {
+#pragma unroll
+      for (int g = 0; g < HM; ++g)
+        if (g == h) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += o[g][e];
+        }
+    }
     if (p.gate) {
-      const bf16* gp = (const bf16*)p.gate + (size_t)t * p.gate_stride + col;
-      bf16x4 z;
-      if (wide) {
-        z = *(const bf16x4*)gp;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) z[e] = gp[e];
-      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] *= 1.0f / (1.0f + __expf(-(float)z[e]));
     }
-    bf16* at = (bf16*)p.out + (size_t)t * p.out_stride + col;
+    bf16* at = (bf16*)p.out + (size_t)t * p.out_stride + h * p.Dv + dv;
     const bf16x4 ob = {(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
     if (wide) {
       *(bf16x4*)at = ob;
