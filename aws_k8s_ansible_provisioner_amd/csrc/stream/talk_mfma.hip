@@ -14,6 +14,8 @@
 // operand).  A workgroup thus forms, for its query head, the unnormalised sums of ALL value
 // heads; they go to a workspace (fp32) with the head's (max, sum), and the merge launch of the
 // split row kernel normalises, mixes the heads and gates.
+#include <type_traits>
+
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -444,12 +446,228 @@ __global__ __launch_bounds__(256) void talk_decode_mfma_kernel(TalkParams p) {
   }
 }
 
+// The same with eight waves, for D = 16 KS entries, at most 16 / KB key heads and pages of a power of two:
+// a step takes 32 KB keys, a wave scores ONE key head's 32 of them, the waves of a key head agree on the
+// maximum through LDS, and a wave accumulates TPW column tiles.
+//
+// Bound by reading keys and values; in steps of few rows by the chain of a step and, as its code runs
+// about once, by fetching instructions: 3 to 6 KB of them run where the kernel above has 29.  The keys and
+// values of the next step are asked for while this one is computed, their pages a step before that.  16 / 4
+// heads of 128: one row at 900 keys 16.6 -> 9.4 us, 64 rows at ~850 36.4 -> 23.2 (4.8 TB/s), 150 at ~2250
+// 214 -> 146 (4.7 TB/s); 32 / 8 heads, 32 rows at ~360 33.7 -> 18.2.  Sixteen waves of half the registers
+// (some spill, and every reload waits for the loads in flight) took 11.6, 28.8, 191 and 26.4 us.
+template <int KB, int TPW, int KS>
+__global__ __launch_bounds__(512, 2) void talk_decode_step_kernel(TalkParams p) {
+  constexpr int NW = 8, D = 16 * KS, NP = 2 * KB;   // waves, 16-key pieces of a step
+  __shared__ __align__(16) bf16x8 qs[KS * 64];       // Q operands (column = head)
+  __shared__ __align__(16) bf16x8 ps[NP * 64];       // weights of a step
+  __shared__ __align__(16) float alpha_s[32], max_s[NW * 32];
+  const int t = blockIdx.x, part = blockIdx.y;
+  int len = p.seq_lens[t], last = (int)p.positions[t];         // the row sees keys 0 .. last
+  asm volatile("" : "+s"(len), "+s"(last));                    // (asked for together)
+  if (len <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hf = lane >> 5;
+  const int steps = (last + 128) >> 7;
+  const int per = (steps + p.num_parts - 1) / p.num_parts;
+  const int lo = part * per * 128;
+  const int hi = min(last + 1, lo + per * 128);    // keys [lo, hi)
+  if (lo >= hi) return;                            // (the merge reads partitions with keys alone)
+  const int BS = p.BS, G = p.G, Dv = p.Dv, DVT = Dv >> 5, NT = G * DVT, rep = p.H / G;
+  const int cc = wave / KB, blk = wave % KB;       // key head and keys that the wave scores
+  const int ck = min(cc, G - 1);                   // (waves past the last key head score it along)
+  const bool act = col < p.H && col / rep == cc;   // its columns
+  const float sc2 = p.scale * 1.44269504088896f;
+  bf16x8 zero;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) zero[i] = (bf16)0.f;
+  bf16x8 q8 = zero;
+  if (wave < KS && col < p.H)
+    q8 = *(const bf16x8*)((const bf16*)p.q + ((size_t)t * p.H + col) * D + 16 * wave + 8 * hf);
+
+  // A step's pieces of 16 keys (pages are whole pieces), a piece per lane, past the range its last one:
+  // scores of rows past it are masked below, value groups past it are read as the last, their weights are
+  // zero.  Pages are asked for two steps ahead, keys and values one.
+  const char* bt = (const char*)(p.block_tables + (size_t)t * p.max_blocks);
+  const int last_piece = (hi - 1) >> 4, shift = __builtin_ctz(BS);   // (BS is a power of two)
+  auto piece_at = [&](int key0) { return min((key0 >> 4) + (lane & (NP - 1)), last_piece) << 4; };
+  auto page_at = [&](int key0) { return *(const uint32_t*)(bt + ((uint32_t)(piece_at(key0) >> shift) << 2)); };
+  uint32_t rows;                                   // first row of the next step's pieces, key head 0
+  auto rows_at = [&](uint32_t page, int key0) {
+    rows = page * (uint32_t)(G * BS) + (uint32_t)(piece_at(key0) & (BS - 1));
+  };
+  bf16x8 kf[KS], vf[TPW][NP];
+  const char* kl = (const char*)p.k_cache + ((ck * BS + swap23(col & 15)) * D + 8 * hf) * 2;
+  auto keys = [&]() __attribute__((always_inline)) {
+    const uint32_t r0 = __builtin_amdgcn_readlane((int)rows, 2 * blk);
+    const uint32_t r1 = __builtin_amdgcn_readlane((int)rows, 2 * blk + 1);
+    const char* at = kl + (uint64_t)(col & 16 ? r1 : r0) * (uint32_t)(D * 2);
+#pragma unroll
+    for (int c = 0; c < KS; ++c) kf[c] = *(const bf16x8*)(at + 32 * c);
+  };
+  auto values = [&](int key0) __attribute__((always_inline)) {
+    // the second group of the range's last piece may lie past it
+    const int whole = ((hi - 1) >> 3) & 1 ? NP : last_piece - (key0 >> 4);
+    const uint32_t l0 = col * 16, l1 = l0 + hf * Dv * 16;    // (in bytes: uniform base, 32-bit offset)
+#pragma unroll
+    for (int k = 0; k < TPW; ++k) {
+      const int ti = min(wave + NW * k, NT - 1), cv = ti / DVT, dv0 = (ti - cv * DVT) << 5;
+      const char* base = (const char*)p.v_cache + ((size_t)cv * BS * Dv + dv0 * 8) * 2;
+#pragma unroll
+      for (int j = 0; j < NP; ++j) {
+        const char* at = base + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)rows, j) * (Dv * 2);
+        vf[k][j] = *(const bf16x8*)(at + (j < whole ? l1 : l0));
+      }
+    }
+  };
+  uint32_t page = page_at(lo), page2 = page_at(lo + 32 * KB);
+  rows_at(page, lo);
+  keys();
+  __builtin_amdgcn_sched_barrier(0);
+  values(lo);
+  if (wave < KS) qs[tid] = q8;
+  if (wave < NP) ps[tid] = zero;                   // columns past H stay zero
+  if (tid < 32) alpha_s[tid] = 1.f;                // rows past H: never rescaled
+  f32x16 acc[TPW];
+#pragma unroll
+  for (int k = 0; k < TPW; ++k)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[k][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // (the last step apart: it alone is masked, and the counts of loads in flight are known in the others)
+  int key0 = lo;
+  auto step = [&](auto more) __attribute__((always_inline)) {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < KS; ++c)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c], qs[c * 64 + lane], s, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more()) {
+      rows_at(page2, key0 + 32 * KB);
+      page2 = page_at(key0 + 64 * KB);
+      keys();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int left = hi - key0 - 32 * blk - 8 * hf;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = more() || 16 * (i >> 3) + (i & 7) < left ? s[i] * sc2 : -INFINITY;
+      mx = fmaxf(mx, s[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (KB > 1 && hf == 0) max_s[wave * 32 + col] = mx;
+    // (with one wave to a key head: the weights of the step before have been read)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // (lanes of other heads' columns compute along; what they get is never stored)
+    float mn = fmaxf(m_run, mx);
+    if (KB > 1) {
+#pragma unroll
+      for (int u = 0; u < KB; ++u) mn = fmaxf(mn, max_s[(cc * KB + u) * 32 + col]);
+    }
+    const float ms = mn == -INFINITY ? 0.f : mn;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - ms);
+    float psum = 0.f;
+    bf16x8 pb[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = __builtin_amdgcn_exp2f(s[i] - ms);
+      psum += e;
+      pb[i >> 3][i & 7] = (bf16)e;
+    }
+    m_run = mn;
+    l_run = l_run * alpha + psum;
+    if (act) {
+      ps[(2 * blk + 0) * 64 + lane] = pb[0];
+      ps[(2 * blk + 1) * 64 + lane] = pb[1];
+      if (blk == 0) alpha_s[col] = alpha;          // (both halves, the same)
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // the accumulators are rescaled only when some head's maximum moved (wave-uniform)
+    if (__any(alpha_s[col] != 1.0f)) {
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const float4 a4 = *(const float4*)(alpha_s + 4 * hf + 8 * (i4 & 1) + 16 * (i4 >> 1));
+#pragma unroll
+        for (int k = 0; k < TPW; ++k) {
+          acc[k][4 * i4] *= a4.x; acc[k][4 * i4 + 1] *= a4.y;
+          acc[k][4 * i4 + 2] *= a4.z; acc[k][4 * i4 + 3] *= a4.w;
+        }
+      }
+    }
+    // (pieces past the range are left out: a weight of 0 would not hide a value that is not finite)
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+      if (more() || key0 + 16 * j < hi) {
+#pragma unroll
+        for (int k = 0; k < TPW; ++k)
+          acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ps[j * 64 + lane], vf[k][j], acc[k], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more()) values(key0 + 32 * KB);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (; key0 + 32 * KB < hi; key0 += 32 * KB) step(std::true_type{});
+  step(std::false_type{});
+  // (max, sum) of the columns, and the sums of the wave's column tiles
+  const size_t cell = (size_t)t * p.num_parts + part;
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (KB > 1) {                                    // (max_s was last read before the barrier before)
+    if (hf == 0) max_s[wave * 32 + col] = l_run;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  if (act && blk == 0 && hf == 0) {
+#pragma unroll
+    for (int u = 1; u < KB; ++u) l_run += max_s[(wave + u) * 32 + col];
+    p.ws_ml[(cell * p.H + col) * 2] = m_run * 0.6931471805599453f;
+    p.ws_ml[(cell * p.H + col) * 2 + 1] = l_run;
+  }
+  const int GV = G * Dv;
+#pragma unroll
+  for (int k = 0; k < TPW; ++k) {
+    const int ti = wave + NW * k;
+    if (ti < NT) {
+      float* o = p.ws_o + cell * p.H * GV + (ti << 5) + col;
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int row = 4 * hf + 8 * i4;
+        if (8 * i4 + 8 <= p.H) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[(size_t)(row + i) * GV] = acc[k][4 * i4 + i];
+        } else if (8 * i4 < p.H) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (row + i < p.H) o[(size_t)(row + i) * GV] = acc[k][4 * i4 + i];
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
 
 void launch_talking_decode_mfma(const TalkParams& p, hipStream_t s) {
   if (p.T <= 0) return;
   const int NT = p.G * (p.Dv / 32);
   const dim3 grid(p.T, p.num_parts);
+  // (sizes whose loads are all known at compile time; the others run the general kernel)
+  if ((p.D == 64 || p.D == 128) && p.G <= 8 && (p.BS & (p.BS - 1)) == 0) {
+#define AKAP_TS(KB, TP)                                                          \
+  do {                                                                           \
+    if (p.D == 128) talk_decode_step_kernel<KB, TP, 8><<<grid, 512, 0, s>>>(p);  \
+    else talk_decode_step_kernel<KB, TP, 4><<<grid, 512, 0, s>>>(p);             \
+  } while (0)
+    if (p.G > 4) AKAP_TS(1, 4);
+    else if (NT <= 16) AKAP_TS(2, 2);
+    else AKAP_TS(2, 4);
+#undef AKAP_TS
+    return;
+  }
   const size_t lds = (size_t)(p.D / 16) * 64 * 16 + 2 * 4 * 2 * 64 * 16 + 2 * 32 * sizeof(float);
   if (NT <= 8) talk_decode_mfma_kernel<2><<<grid, 256, lds, s>>>(p);
   else if (NT <= 16) talk_decode_mfma_kernel<4><<<grid, 256, lds, s>>>(p);

@@ -247,7 +247,10 @@ def test_talking_attention_matrix_core_kernel(H, G, D, Dv, BS):
 
 @pytest.mark.parametrize("H,G,D,Dv,BS", [(6, 2, 80, 96, 32), (4, 1, 16, 32, 16), (8, 8, 32, 64, 32),
                                          (16, 4, 128, 128, 32), (2, 2, 48, 160, 16),
-                                         (32, 8, 64, 128, 32)])
+                                         (32, 8, 64, 128, 32), (32, 8, 128, 128, 16),
+                                         (10, 5, 64, 160, 64), (12, 3, 128, 96, 32),
+                                         (8, 4, 64, 256, 128), (7, 1, 128, 32, 32),
+                                         (16, 4, 128, 128, 48)])
 def test_talking_attention_matrix_core_decode_kernel(H, G, D, Dv, BS):
     """One query per sequence on the matrix cores (heads as columns), several partition counts,
     sequences of 1 key, of a few and of many steps, a padding row."""
