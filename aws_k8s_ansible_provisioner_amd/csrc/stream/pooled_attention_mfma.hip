@@ -11,6 +11,8 @@
 // walked as pooled entries first (fp32 in memory, rounded to bf16 operands, gathered), then
 // window tokens in steps aligned to 32 positions; the sink of score 0 is the starting state of
 // the online softmax.
+#include <type_traits>
+
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -297,6 +299,224 @@ __global__ __launch_bounds__(DEC ? 64 * kDecWaves : 256) void pooled_window_mfma
   }
 }
 
+// Decode rows of D = 16 KS and Dv = 32 DVT entries, at most 8 query heads to a key/value head, pages of whole
+// 32-token steps: the steps of the general kernel's DEC form, of which a wave's next one is on its way while
+// one is computed, and the waves' shares added in order.
+//
+// Bound by the chain of a wave's steps (page, keys, products, weights, values), one after the other 5 us
+// each in the general form, and in large steps by reading.  16 / 4 heads of 128, window 1024, pooled blocks
+// of 64: 10 rows at ~1800 keys 28.2 -> 15.9 us, one at 500 16.7 -> 9.1, 64 at ~2000 34.2 -> 24.4, 150 at ~2200
+// 113 -> 70 (4.4 TB/s); 32 / 8 heads, 32 rows at ~630 24.1 -> 17.2.
+template <int KS, int DVT>
+__global__ __launch_bounds__(64 * kDecWaves, 2) void pooled_decode_kernel(const PoolAttnParams p) {
+  constexpr int NW = kDecWaves, D = 16 * KS, Dv = 32 * DVT, LS = Dv + 4;
+  __shared__ __align__(16) bf16x8 qs[KS * 64];
+  __shared__ __align__(16) float shares[NW * 8 * LS];
+  __shared__ float m_s[NW * 32], l_s[NW * 32];
+  const int t = blockIdx.x, g = blockIdx.y;
+  int slot = (int)(p.slots[t] >> 32), pos = (int)p.positions[t];
+  asm volatile("" : "+s"(slot), "+s"(pos));        // (asked for together)
+  if (slot < 0) return;                            // a padding row (the whole workgroup)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hf = lane >> 5, rep = p.H / p.G;
+  const bool used = col < rep;
+  const int W = p.window, P = p.pool, BS = p.BS, G = p.G;
+  const int32_t* bt = p.block_tables + (size_t)t * p.max_blocks;
+  const float sc2 = p.scale * 1.44269504088896f;   // scores -> log2 units
+  bf16x8 q8 = zero8();
+  if (wave < KS && used)
+    q8 = *(const bf16x8*)((const bf16*)p.q + ((size_t)t * p.H + g * rep + col) * D + 16 * wave + 8 * hf);
+
+  const int nb = (P > 0 && W > 0 && pos - W + 1 > 0) ? (pos - W + 1) / P : 0;    // pooled entries
+  const int pool_steps = (nb + 31) >> 5;
+  const int lo = W > 0 ? max(0, pos - W + 1) : 0, first = lo & ~31, steps = ((pos - first) >> 5) + 1;
+  // the wave's window steps: sw, sw + NW, ...; pages of 64 of them by lanes
+  int sw = (wave - pool_steps) & (NW - 1), base = sw;
+  auto pages_at = [&](int s) { return bt[min(first + 32 * (s + NW * lane), pos) / BS]; };
+  int pages = pages_at(base);
+  bf16x8 kf[KS], vf[2][DVT];
+  const char* kl = (const char*)p.k_cache + (swap23(col) * D + 8 * hf) * 2;
+  auto page_row = [&](int s) __attribute__((always_inline)) {     // first row of the step
+    const int j = (s - base) / NW, key = first + 32 * s;
+    return ((size_t)__builtin_amdgcn_readlane(pages, j) * G + g) * BS + key % BS;
+  };
+  auto keys = [&](int s) __attribute__((always_inline)) {
+    const char* at = kl + page_row(s) * (D * 2);
+#pragma unroll
+    for (int c = 0; c < KS; ++c) kf[c] = *(const bf16x8*)(at + 32 * c);
+  };
+  auto values = [&](int s) __attribute__((always_inline)) {
+    const char* at = (const char*)p.v_cache + page_row(s) * (Dv * 2);
+#pragma unroll
+    for (int c2 = 0; c2 < 2; ++c2) {
+      // groups of 8 keys past the row are read as its last, their weights are zero
+      const int grp = min(2 * c2 + hf, (pos - first - 32 * s) >> 3);
+      const uint32_t off = (uint32_t)(grp * Dv + col) * 16;
+#pragma unroll
+      for (int k = 0; k < DVT; ++k) vf[c2][k] = *(const bf16x8*)(at + (off + 512 * k));
+    }
+  };
+  if (wave < KS) qs[tid] = q8;
+  f32x16 acc[DVT];
+#pragma unroll
+  for (int k = 0; k < DVT; ++k)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[k][i] = 0.f;
+  float m_run = p.unit_sink ? 0.f : -INFINITY;
+  // the two lanes of a column and the waves are added at the end: the sink counts once
+  float l_run = p.unit_sink && hf == 0 && wave == 0 ? 1.f : 0.f;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // scores of the keys from first_key to last_key (of 32) -> weights; false: none of a used column is above 0
+  auto softmax = [&](f32x16& s, int first_key, int last_key, bf16x8 (&pb)[2])
+      __attribute__((always_inline)) {
+    const int from = 8 * hf - first_key;
+    const uint32_t upto = (uint32_t)(last_key - first_key);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = (uint32_t)(16 * (i >> 3) + (i & 7) + from) <= upto ? s[i] * sc2 : -INFINITY;
+      mx = fmaxf(mx, s[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx);
+    const bool any = m_new != -INFINITY;
+    const float alpha = any ? exp2f(m_run - m_new) : 1.f;
+    float sum = 0.f;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float w = any ? exp2f(s[8 * c + e] - m_new) : 0.f;
+        sum += w;
+        pb[c][e] = (bf16)w;
+      }
+    l_run = l_run * alpha + sum;
+    m_run = m_new;
+    if (__any(alpha != 1.f)) {
+#pragma unroll
+      for (int k = 0; k < DVT; ++k)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[k][i] *= alpha;
+    }
+    return __any(used && sum > 0.f);
+  };
+  for (int cb = 32 * wave; cb < nb; cb += 32 * NW) {
+    // an entry per lane, in the order of the score rows; past the last one the last
+    const int key = min(cb + swap23(col), nb - 1) * P;
+    const uint32_t row = (uint32_t)(bt[key / BS] * G + g) * (uint32_t)p.PS + (uint32_t)(key % BS / P);
+    const float* kp = p.k_pool + (size_t)row * D + 8 * hf;
+    float4 k4[KS][2];
+#pragma unroll
+    for (int c = 0; c < KS; ++c) {
+      k4[c][0] = *(const float4*)(kp + 16 * c);
+      k4[c][1] = *(const float4*)(kp + 16 * c + 4);
+    }
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < KS; ++c) {
+      const float4 a = k4[c][0], b = k4[c][1];
+      const bf16x8 k8 = {(bf16)a.x, (bf16)a.y, (bf16)a.z, (bf16)a.w,
+                         (bf16)b.x, (bf16)b.y, (bf16)b.z, (bf16)b.w};
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k8, qs[c * 64 + lane], s, 0, 0, 0);
+    }
+    // values: entry rows gathered one by one, on their way under the softmax
+    float v4[2][8][DVT];
+#pragma unroll
+    for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t r0 = __builtin_amdgcn_readlane((int)row, swap23(16 * c2 + e));
+        const uint32_t r1 = __builtin_amdgcn_readlane((int)row, swap23(16 * c2 + 8 + e));
+        const float* at = p.v_pool + (size_t)(hf ? r1 : r0) * Dv + col;
+#pragma unroll
+        for (int k = 0; k < DVT; ++k) v4[c2][e][k] = at[32 * k];
+      }
+    bf16x8 pb[2];
+    if (!softmax(s, 0, min(nb - 1 - cb, 31), pb)) continue;
+#pragma unroll
+    for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+      for (int k = 0; k < DVT; ++k) {
+        bf16x8 v8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v8[e] = (bf16)v4[c2][e][k];
+        acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v8, pb[c2], acc[k], 0, 0, 0);
+      }
+  }
+  // (the last step apart: the counts of loads in flight are known in the others)
+  auto step = [&](auto more) __attribute__((always_inline)) {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < KS; ++c)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c], qs[c * 64 + lane], s, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more()) {
+      keys(sw + NW);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 pb[2];
+    if (softmax(s, max(lo - first - 32 * sw, 0), min(pos - first - 32 * sw, 31), pb)) {
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+        for (int k = 0; k < DVT; ++k)
+          acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c2][k], pb[c2], acc[k], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more()) values(sw + NW);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  while (sw < steps) {
+    keys(sw);
+    __builtin_amdgcn_sched_barrier(0);
+    values(sw);
+    __builtin_amdgcn_sched_barrier(0);
+    const int end = min(steps, base + 64 * NW);
+    for (; sw + NW < end; sw += NW) step(std::true_type{});
+    step(std::false_type{});
+    sw += NW;
+    base = sw;
+    if (sw < steps) pages = pages_at(base);
+  }
+
+  // the waves' shares: register j of tile k is value entry 32 k + 8 (j / 4) + 4 hf + j % 4 of head col
+  const float l = l_run + __shfl_xor(l_run, 32, 64);
+  if (hf == 0) {
+    m_s[wave * 32 + col] = m_run;
+    l_s[wave * 32 + col] = l;
+  }
+  if (used) {
+    float* at = shares + (wave * 8 + col) * LS + 4 * hf;
+#pragma unroll
+    for (int k = 0; k < DVT; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *(float4*)(at + 32 * k + 8 * j) = make_float4(acc[k][4 * j], acc[k][4 * j + 1],
+                                                      acc[k][4 * j + 2], acc[k][4 * j + 3]);
+  }
+  __syncthreads();
+  bf16* o = (bf16*)p.out + (size_t)t * p.out_stride + (size_t)g * rep * Dv;
+  for (int e = tid; e < rep * Dv; e += 64 * NW) {
+    const int c = e / Dv, d = e % Dv;
+    float mg = -INFINITY, lg = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mg = fmaxf(mg, m_s[w * 32 + c]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float mw = m_s[w * 32 + c], f = mw == -INFINITY ? 0.f : exp2f(mw - mg);
+      lg += l_s[w * 32 + c] * f;
+      sum += f > 0.f ? shares[(w * 8 + c) * LS + d] * f : 0.f;
+    }
+    o[e] = (bf16)(lg > 0.f ? sum / lg : 0.f);
+  }
+}
+
 }  // namespace
 
 bool pooled_mfma_supported(int H, int G, int D, int Dv, int BS) {
@@ -341,6 +561,17 @@ void launch_pooled_window_prefill_mfma(const PoolAttnParams& p, const int32_t* t
 void launch_pooled_window_decode_mfma(const PoolAttnParams& p, int rows, hipStream_t s) {
   if (rows <= 0) return;
   const dim3 grid(rows, p.G);
+  // (sizes whose loads are all known at compile time and whose shares fit LDS; the others run the general form)
+  if ((p.D == 64 || p.D == 128) && (p.Dv == 64 || p.Dv == 128) && p.BS % 32 == 0 && p.H <= 8 * p.G) {
+#define AKAP_PD(KS, N) pooled_decode_kernel<KS, N><<<grid, 64 * kDecWaves, 0, s>>>(p)
+    if (p.D == 64) {
+      if (p.Dv == 64) AKAP_PD(4, 2); else AKAP_PD(4, 4);
+    } else {
+      if (p.Dv == 64) AKAP_PD(8, 2); else AKAP_PD(8, 4);
+    }
+#undef AKAP_PD
+    return;
+  }
   const size_t q_bytes = (size_t)(p.D >> 4) * 64 * sizeof(bf16x8);
   const size_t m_bytes = (size_t)(2 * kDecWaves * 32 + p.Dv * 32) * sizeof(float);
   const size_t lds = q_bytes > m_bytes ? q_bytes : m_bytes;

@@ -386,7 +386,8 @@ def test_large_batches_take_the_grouped_expert_gemms():
 @pytest.mark.parametrize("H,G,D,Dv,rot,window,pool,BS", [
     (6, 3, 64, 64, 32, 44, 12, 32), (4, 2, 32, 32, 16, 24, 8, 32), (8, 2, 128, 128, 64, 100, 48, 32),
     (2, 1, 16, 256, 0, 0, 0, 16), (4, 4, 80, 64, 16, 33, 0, 8), (3, 1, 48, 32, 48, 7, 5, 16),
-    (4, 1, 128, 128, 128, 200, 4, 32)])
+    (4, 1, 128, 128, 128, 200, 4, 32), (8, 1, 64, 128, 0, 32, 3, 96), (5, 1, 128, 64, 64, 0, 0, 64),
+    (9, 1, 64, 64, 32, 1, 64, 32)])
 def test_attention_matrix_core_kernel(H, G, D, Dv, rot, window, pool, BS):
     """Prompt chunks on the matrix cores against the row ops on the CPU: chunks that start in
     the middle of a sequence, tiles cut by a chunk's end, more than one tile per chunk, leading
@@ -453,6 +454,23 @@ def test_attention_matrix_core_kernel(H, G, D, Dv, rot, window, pool, BS):
                                         True)
     close(got[:B], want[last], "bfloat16", scale=2.0)
     assert (got[B] == 3.0).all()                     # the padding row is left unwritten
+
+
+@pytest.mark.parametrize("window", [0, 16500])
+def test_decode_row_of_many_steps(window):
+    """More keys than 64 steps of 32 for each of a workgroup's eight waves."""
+    g, H, G, D, BS, n = gen(11), 2, 1, 64, 64, 64 * 32 * 8 + 700
+    NB = -(-n // BS)
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    a = [rnd(1, H, D), rnd(NB, G, BS, D), rnd(NB, G, BS // 8, D, 8), None, None,
+         torch.randperm(NB, generator=g).int()[None]]
+    at = [torch.tensor([n - 1]), torch.tensor([0])]
+    want = torch.zeros(1, H * D, dtype=torch.bfloat16)
+    got = torch.zeros_like(want, device="cuda")
+    sops.pooled_window_attention(want, *a, None, *at, 0.3, window, 0, True)
+    sops.pooled_window_attention_decode(got, *(None if x is None else x.cuda() for x in a + at), 0.3,
+                                        window, 0, True)
+    close(got, want, "bfloat16", scale=2.0)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
