@@ -12,12 +12,14 @@
 // maximum, weights go to LDS; then every wave sums ITS part of the latent dimensions over all keys of the
 // step (O^T = C^T P^T, v_mfma_f32_32x32x16_bf16).
 //
-// Bound by reading the rows (39 us for 64 sequences of ~2010 keys, 148 MB at 3.8 TB/s: a step's 74 KB
-// take 3.8 us of the 4.3 at the card's copy rate); the kernel that read rows and groups took 51.  With
-// eight waves and steps of 64 keys, as four waves' chain of barriers, fragment reads and exponentials
-// takes 2.8 us per 32 keys (48 us in all, four slots ahead).  Grids that do not fit one workgroup to a CU
-// run two of four waves there: 200 rows of ~2250 keys 219 -> 136 us with the layer's other launches, 100
-// of ~1200 79 -> 54.
+// Bound by reading the rows: 32 us for 64 sequences of ~2010 keys (148 MB at 4.6 TB/s), 93 for 150 of ~2120
+// under 32 heads (3.9), 108 for 200 of ~2250 (4.8); 39, 116 and 121 where a wait for the queries stood in
+// the loop and every step asked whether it is masked; the kernel that read rows and groups took 51 for the
+// first.  With eight waves and steps of 64 keys, as four waves' chain of barriers, fragment reads and
+// exponentials takes longer per 32 keys (48 for 39 us, four slots ahead).  Grids that do not fit one
+// workgroup to a CU run two of four waves there.
+#include <type_traits>
+
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -119,6 +121,10 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_decode_rows_kernel(LatentAt
 #pragma unroll
     for (int c = 0; c < kKs; ++c)
       qf[c] = *(const bf16x8*)(c < kR / 32 ? ql + 32 * c : qr + 32 * (c - kR / 32));
+    // arrived here, once: a wait at the first product would stand in the loop, where it waits for the
+    // rows of the next step as well
+#pragma unroll
+    for (int c = 0; c < kKs; ++c) asm volatile("" : "+v"(qf[c]));
   }
   const float sc2 = p.scale * 1.44269504088896f;
   float m = -INFINITY, l = 0.f;                           // of query 16 qh + n16; l: this lane's keys
@@ -134,7 +140,9 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_decode_rows_kernel(LatentAt
   const unsigned va = (8 * hf + jr) * kRowBytes + w * DT * 64 +
                       ((2 * (g & 1) + ((lane & 3) >> 1)) ^ turn(8 * hf + jr)) * 16 + (lane & 1) * 8;
 
-  for (int t = 0; t < steps; ++t) {
+  // (masked: the last step, whose rows may lie past the partition's end; without the question the
+  // others' reads of value operands run ahead of their products)
+  auto step = [&](int t, auto masked) __attribute__((always_inline)) {
     // the step's rows have landed for this wave; every wave is through with the step before
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
@@ -147,12 +155,11 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_decode_rows_kernel(LatentAt
       const bf16x8 kf = *(const bf16x8*)(slot + (ka ^ (c & 1) * 64) + (c >> 1) * 128);
       s[c & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[c], s[c & 1], 0, 0, 0);
     }
-    const bool masked = j0 + kStep > end;
     float sv[4], mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {                         // key j0 + 16 kq + 4 g + i
       sv[i] = s[0][i] + s[1][i];
-      if (masked && j0 + 16 * kq + 4 * g + i >= end) sv[i] = -INFINITY;
+      if (masked() && j0 + 16 * kq + 4 * g + i >= end) sv[i] = -INFINITY;
       mx = fmaxf(mx, sv[i]);
     }
     mx = rows_max(mx);
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_decode_rows_kernel(LatentAt
 #pragma unroll
           for (int e = 0; e < 4; ++e) vf[4 * i + e] = v[e];
         }
-        if (masked) {      // what lies behind the partition's end may hold values that are not finite
+        if (masked()) {    // what lies behind the partition's end may hold values that are not finite
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (j0 + 16 * sl + 8 * hf + e >= end) vf[e] = (bf16)0.f;
@@ -206,7 +213,9 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_decode_rows_kernel(LatentAt
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[dt], 0, 0, 0);
       }
     }
-  }
+  };
+  for (int t = 0; t + 1 < steps; ++t) step(t, std::false_type{});
+  step(steps - 1, std::true_type{});
   l = rows_sum(l);
   if (g == 0) sum_s[kq * 32 + 16 * qh + n16] = l;
   lds_barrier();
