@@ -1,6 +1,8 @@
 // Head-mixed attention of prompt chunks on the matrix cores, 128 queries of one query head against
 // all value heads at a time (bf16 caches K [NB, G, BS, D], V [NB, G, BS / 8, Dv, 8], D = 64 or 128,
 // pages of whole 32-token pieces), and the launch that mixes the heads and gates.
+#include <type_traits>
+
 #include "../kernels/common.h"
 #include "stream.h"
 
@@ -66,10 +68,10 @@ __device__ __forceinline__ size_t ws_at(const TalkParams& p, int t, int g, int e
 //
 // Bound by the chain of a step (score products, maximum, barrier, exponentials, barrier: half of the time
 // alone) beside the products (116 us of the matrix units' time): 8 chunks of 1000 tokens behind 1000
-// cached, 16 / 4 heads of 128 352 us; 64 queries per workgroup with every fragment from the caches
+// cached, 16 / 4 heads of 128 330 us; 64 queries per workgroup with every fragment from the caches
 // took 919.  Opposite order of matrix and vector work in a SIMD's two waves gained nothing (24 us
-// more).  A query tile's own end costs 8 us of them (a branch per tile; by pairs of tiles or by 16 keys
-// the same; a second body without branches spills).
+// more).  The steps that all four query tiles see whole have a body of their own, without a branch per
+// tile; with one body for all 352 us, and 290 for 4 chunks of 700 behind 300 of 32 / 8 heads, now 273.
 template <int D, int TPW>
 __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const int32_t* tile_seq,
                                                              const int32_t* tile_row, int num_tiles,
@@ -105,12 +107,11 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
       (const __attribute__((address_space(4))) int*)(p.block_tables + (size_t)b * p.max_blocks);
   const int last_piece = last >> 5;
 
-  int koff[PW];
-#pragma unroll
-  for (int i = 0; i < PW; ++i) {
-    const int s = (w * PW + i) * 64 + lane, key = s / (D / 8), c = swz<D>(key, s % (D / 8));
-    koff[i] = (key & 31) * D + c * 8;
-  }
+  // a lane's element of the wave's first piece of a step's keys; the second's, 4 rows on, has another bit of
+  // the turned column as well (formed in the loop: it lacks the register)
+  static_assert(PW == 1 || (PW == 2 && D == 128), "pieces");
+  const int koff = ((w * PW * 64 + lane) / (D / 8) & 31) * D +
+                   swz<D>((w * PW * 64 + lane) / (D / 8), (w * PW * 64 + lane) % (D / 8)) * 8;
   // page and row in it of the 32-key piece a walk stands at; past the last piece it stays there
   struct Walk {
     int piece, idx, row;
@@ -127,8 +128,10 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
     const bf16* kc = (const bf16*)p.k_cache +
                      (((size_t)bt[kw.idx] * G + kvh) * BS + kw.row) * D;
     bf16* kl = kl0 + buf * (kK / 2);
-#pragma unroll
-    for (int i = 0; i < PW; ++i) dma16(kc + koff[i], kl + (w * PW + i) * 512);
+    int off = koff;
+    asm volatile("" : "+v"(off));
+    dma16(kc + off, kl + w * PW * 512);
+    if (PW > 1) dma16(kc + ((off ^ 32) + 4 * D), kl + (w * PW + 1) * 512);
     advance(kw);
     advance(kw);
   };
@@ -231,13 +234,13 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
     }
     alpha_s[32 * qt + r] = alpha;           // (as both key halves' waves do)
   };
-  auto products = [&](int t, int half) {
+  auto products = [&](int t, int half, auto whole) __attribute__((always_inline)) {
     const bf16x8* ps = ps0 + (t & 1) * (kP / 16);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       // keys past a query tile's last take no part: a weight of 0 would not hide a value that is not
       // finite
-      if (t * kKeys + 32 * half > last_of(q)) continue;
+      if (!whole() && t * kKeys + 32 * half > last_of(q)) continue;
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const bf16x8 pf = ps[(4 * q + 2 * half + e) * 64 + lane];
@@ -249,14 +252,14 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
   };
 
   values(0);
-  values(1);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   scores(0);
   maximum(0);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   weights(0);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  for (int t = 0, b1 = 1, b0 = 0; t < steps; ++t) {
+  int t = 0, b1 = 1, b0 = 0;
+  auto step = [&](auto whole) __attribute__((always_inline)) {
     {
       float a[4];
       bool moved = false;
@@ -274,9 +277,15 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
             for (int i = 0; i < 16; ++i) acc[k][q][i] *= a[q];
       }
     }
-    const bool ahead = t + 1 < steps;
+    const bool ahead = whole() || t + 1 < steps;
     if (ahead) scores(b1);
-    products(t, 0);
+    // (beside DMA in flight the compiler waits for every load where it needs one: the first half's values
+    // arrive here, and only then the second half's are asked for, which have the first products' time)
+#pragma unroll
+    for (int k = 0; k < TPW; ++k) asm volatile("" : "+v"(vf[0][k][0]), "+v"(vf[0][k][1]));
+    values(1);
+    __builtin_amdgcn_sched_barrier(0);
+    products(t, 0, whole);
     if (ahead) maximum(t + 1);
     // the keys of step t + 2 have landed, those of step t were last read before the barrier before
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -285,12 +294,14 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
       stage(b0);
       weights(t + 1);
     }
-    products(t, 1);
-    if (ahead) values(1);
+    products(t, 1, whole);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     b0 = b0 == 2 ? 0 : b0 + 1;
     b1 = b1 == 2 ? 0 : b1 + 1;
-  }
+  };
+  const int all = min(steps - 1, (last_of(0) - 32) / kKeys + 1);
+  for (; t < all; ++t) step(std::true_type{});
+  for (; t < steps; ++t) step(std::false_type{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (nothing may land after the end)
   // both key halves' sums; the normalised sums of the wave's value entries
   l_run = both_sum(l_run);
