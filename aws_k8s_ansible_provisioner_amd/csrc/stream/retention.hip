@@ -646,6 +646,106 @@ __global__ __launch_bounds__(DREG == 16 ? 256 : 512) void retention_kernel(Reten
   }
 }
 
+// One row per sequence, heads of D x V entries: the same thread owns the same pieces of the state, but
+// everything a workgroup reads is asked for at once, the row's entries and angles ahead of the state, whose
+// arrival no barrier waits for (slot, position, angles and state in turn, each behind the others' loads, and
+// a branch per piece took 18.2 us for 64 rows of 8 heads of 128 x 128, now 10.0; 8 rows 10.8 -> 5.9, 150
+// rows 38 -> 25.8; 64 rows of 16 heads 34 -> 22).  Bound by reading and writing the states: 6.1 TB/s.
+template <typename T, int D, int V>
+__global__ __launch_bounds__(V / 4 * (D / 16)) void retention_step_kernel(RetentionParams p) {
+  constexpr int DP = D / 16, NT = V / 4 * DP;
+  __shared__ __align__(16) float qs[D], ks[D];
+  __shared__ float part_ss[NT / 64];
+  const int b = blockIdx.x, h = blockIdx.y;
+  int slot = p.seq_slot[b];
+  int64_t pos = p.positions[b];
+  asm volatile("" : "+s"(slot), "+s"(pos));        // (asked for together)
+  if (slot < 0 || slot >= p.num_slots) return;
+  const int tid = threadIdx.x, v0 = tid / DP * 4, part = tid % DP;
+  // four dimensions of q and k (every D / 4 threads the same ones), with their partners in the rotation
+  const int d = tid % (D / 4) * 4, half = p.rot_dims >> 1;
+  const bool rot = d < p.rot_dims, low = d < half;
+  const int d2 = rot ? (low ? d + half : d - half) : d;
+  const T* row = (const T*)p.proj + (size_t)b * p.proj_stride;
+  const T *q = row + p.q_off + h * D, *k = row + p.k_off + h * D;
+  float q4[4], k4[4], q2[4], k2[4], vr[4], z4[4], c4[4] = {1.f, 1.f, 1.f, 1.f}, s4[4] = {};
+  ld4(q + d, q4);
+  ld4(k + d, k4);
+  ld4(q + d2, q2);
+  ld4(k + d2, k2);
+  ld4(row + p.v_off + h * V + v0, vr);
+  ld4(row + p.g_off + h * V + v0, z4);
+  if (half > 0) {
+    const float* cs = p.cos_sin + (size_t)pos * p.rot_dims + (rot ? (low ? d : d - half) : 0);
+    ld4(cs, c4);
+    ld4(cs + half, s4);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float* st = p.state + ((size_t)slot * p.H + h) * V * D + v0 * D + 4 * part;
+  float4 S[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r][j] = *(const float4*)(st + r * D + 4 * j * DP);
+  __builtin_amdgcn_sched_barrier(0);
+  const float decay = exp2f(p.log2_decay[h]), kscale = 1.0f / sqrtf((float)D);
+  if (rot) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float sn = low ? -s4[u] : s4[u];
+      q4[u] = q4[u] * c4[u] + q2[u] * sn;
+      k4[u] = k4[u] * c4[u] + k2[u] * sn;
+    }
+  }
+  if (tid < D / 4) {
+    *(float4*)(qs + d) = make_float4(q4[0], q4[1], q4[2], q4[3]);
+    *(float4*)(ks + d) = make_float4(k4[0] * kscale, k4[1] * kscale, k4[2] * kscale, k4[3] * kscale);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const bool fresh = pos == 0;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float4 kj = *(const float4*)(ks + 4 * (j * DP + part)), qj = *(const float4*)(qs + 4 * (j * DP + part));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float4 x = S[r][j];
+      if (fresh) x = make_float4(0.f, 0.f, 0.f, 0.f);
+      x.x = fmaf(decay, x.x, kj.x * vr[r]);
+      x.y = fmaf(decay, x.y, kj.y * vr[r]);
+      x.z = fmaf(decay, x.z, kj.z * vr[r]);
+      x.w = fmaf(decay, x.w, kj.w * vr[r]);
+      *(float4*)(st + r * D + 4 * j * DP) = x;
+      acc[r] = fmaf(x.x, qj.x, acc[r]);
+      acc[r] = fmaf(x.y, qj.y, acc[r]);
+      acc[r] = fmaf(x.z, qj.z, acc[r]);
+      acc[r] = fmaf(x.w, qj.w, acc[r]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int o = DP >> 1; o > 0; o >>= 1) acc[r] += __shfl_xor(acc[r], o, 64);
+    ss += acc[r] * acc[r];
+  }
+  // the head's norm over its V entries and the silu gate
+#pragma unroll
+  for (int o = DP; o < 64; o <<= 1) ss += __shfl_xor(ss, o, 64);
+  if (NT > 64) {
+    if ((tid & 63) == 0) part_ss[tid >> 6] = ss;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) ss += part_ss[w];
+  }
+  if (part != 0) return;
+  const float inv = 1.0f / sqrtf(ss / (float)V + p.eps);
+  T* o = (T*)p.out + (size_t)b * p.out_stride + h * V + v0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) stf(o + r, acc[r] * inv * z4[r] * sigmoidf(z4[r]));
+}
+
 // state before each segment from the segments' own states, per (sequence, head); the state
 // after the last segment goes to the sequence's slot
 __global__ __launch_bounds__(256) void retention_scan_kernel(RetentionParams p) {
@@ -1243,6 +1343,27 @@ int retention_dreg(int D, int V) {
 
 void launch_retention(RetentionParams p, bool f32, hipStream_t s) {
   if (p.num_seqs <= 0) return;
+  // (heads whose pieces divide among a workgroup's threads at compile time, every read one of 4 elements)
+  const size_t es = f32 ? 4 : 2;
+  if (p.q_start == nullptr && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) &&
+      ((p.proj_stride | p.q_off | p.k_off | p.v_off | p.g_off) & 3) == 0 &&
+      p.rot_dims % 8 == 0 && ((uintptr_t)p.proj & (4 * es - 1)) == 0 &&
+      (((uintptr_t)p.state | (uintptr_t)p.cos_sin) & 15) == 0) {
+    const dim3 grid(p.num_seqs, p.H);
+#define AKAP_RS1(TY, DD, VV) retention_step_kernel<TY, DD, VV><<<grid, VV / 4 * (DD / 16), 0, s>>>(p)
+#define AKAP_RS(DD, VV)                                                    \
+  do {                                                                     \
+    if (f32) AKAP_RS1(float, DD, VV); else AKAP_RS1(bf16, DD, VV);         \
+  } while (0)
+    if (p.D == 64) {
+      if (p.V == 64) AKAP_RS(64, 64); else AKAP_RS(64, 128);
+    } else {
+      if (p.V == 64) AKAP_RS(128, 64); else AKAP_RS(128, 128);
+    }
+#undef AKAP_RS
+#undef AKAP_RS1
+    return;
+  }
   const int dreg = retention_dreg(p.D, p.V);
   int dp = 1;
   while (dp * dreg < p.D) dp <<= 1;

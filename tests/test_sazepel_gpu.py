@@ -116,6 +116,30 @@ def test_retention_kernel(dtype, H, D, V, rot):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,D,V,rot", [(2, 64, 64, 32), (3, 64, 128, 64), (1, 128, 64, 0), (2, 128, 128, 8)])
+def test_retention_single_rows(dtype, H, D, V, rot):
+    """Rows whose pieces are aligned: slots continued, one started at position 0 over what lies in it, two
+    padding rows (a negative slot, one past the last)."""
+    g, dt = gen(H * D + V), DT[dtype]
+    N, slot = H * (2 * D + 2 * V), torch.tensor([2, 0, -1, 4, 1, 5], dtype=torch.int32)
+    T = len(slot)
+    state, proj = torch.randn(5, H, V, D, generator=g), torch.randn(T, N, generator=g).to(dt)
+    pos = torch.tensor([7, 0, 3, 900, 1, 2])
+    cs, decay = sops.rotary_table(1024, rot, 10000.0) if rot else None, torch.linspace(-0.2, -0.01, H)
+    res = []
+    for dev in ("cpu", "cuda"):
+        out, st = torch.zeros(T, H * V + 3, dtype=dt, device=dev), state.to(dev, copy=True)
+        sops.retention(out[:, 1:H * V + 1], proj.to(dev), 0, H * D, 2 * H * D, 2 * H * D + H * V, st,
+                       (slot if dev == "cuda" else slot.where(slot < 5, -1)).to(dev), pos.to(dev), None,
+                       cs.to(dev) if rot else None, decay.to(dev), H, D, V, 1e-6)
+        res.append((out, st))
+    live = torch.tensor([0, 1, 3, 4])
+    close(res[1][0][live.cuda()], res[0][0][live], dtype, scale=3.0)
+    close(res[1][1], res[0][1], "float32")
+    assert (res[1][0][[2, 5]] == 0).all() and torch.equal(res[1][1][3].cpu(), state[3])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,D,V,rot", [(3, 64, 32, 16), (2, 128, 128, 64), (2, 24, 40, 8)])
 def test_retention_kernel_in_segments(dtype, H, D, V, rot):
     """A step long enough for the segmented form: sequences of many segments, one that goes on
