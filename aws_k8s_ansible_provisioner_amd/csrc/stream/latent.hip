@@ -198,6 +198,83 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepParams p) {
   }
 }
 
+// The same for steps of few rows at the sizes below: a wave per row, all of its loads together but the
+// angles, which wait for the position.  Bound by that chain: 64 rows of 768 + 512 + 64 4.0 us (6.2 with a
+// workgroup per row, two sums over it and every entry read twice), 150 of 1536 5.5 (10.4), 600 of 768 6.2
+// (7.2), 1800 10.8 (11.0).
+template <int NQ>
+__global__ __launch_bounds__(64) void latent_prep_wave_kernel(LatentPrepParams p) {
+  const int t = blockIdx.x, lane = threadIdx.x, qc = p.q_rank >> 3, kc = p.kv_rank >> 3;
+  const bf16* row = (const bf16*)p.proj + (size_t)t * p.proj_stride;
+  const bf16* kv = row + p.kv_off;
+  const bool store = p.cache != nullptr;
+  int64_t slot = store ? p.slots[t] : -1, pos = store ? p.positions[t] : 0;
+  asm volatile("" : "+s"(slot), "+s"(pos));          // (asked for together)
+  if (slot >= p.num_slots) slot = -1;
+  // pieces past a rank read its last, rotated pairs past the last the last
+  bf16x8 q[NQ], k8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  float4 qw[NQ][2], kw[2] = {};
+  const int half = p.rot_dim >> 1, i0 = min(lane, max(half - 1, 0));
+  auto first = [&](int i) { return p.half_pairs ? i : 2 * i; };
+  auto second = [&](int i) { return p.half_pairs ? i + half : 2 * i + 1; };
+  float u = 0.f, v = 0.f, cs = 0.f, sn = 0.f;
+#pragma unroll
+  for (int c = 0; c < NQ; ++c) {
+    const int at = min(lane + 64 * c, qc - 1) * 8;
+    q[c] = *(const bf16x8*)(row + p.q_off + at);
+    qw[c][0] = *(const float4*)(p.q_w + at);
+    qw[c][1] = *(const float4*)(p.q_w + at + 4);
+  }
+  if (slot >= 0) {
+    const int at = min(lane, kc - 1) * 8;
+    k8 = *(const bf16x8*)(kv + at);
+    kw[0] = *(const float4*)(p.kv_w + at);
+    kw[1] = *(const float4*)(p.kv_w + at + 4);
+    if (half > 0) {
+      const float* angles = p.cos_sin + (size_t)min(max(pos, (int64_t)0), (int64_t)p.max_pos - 1) * p.rot_dim;
+      u = (float)kv[p.kv_rank + first(i0)];
+      v = (float)kv[p.kv_rank + second(i0)];
+      cs = angles[i0];
+      sn = angles[half + i0];
+    }
+  }
+  float ss = 0.f, sk = 0.f;
+#pragma unroll
+  for (int c = 0; c < NQ; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += lane + 64 * c < qc ? (float)q[c][e] * (float)q[c][e] : 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sk += lane < kc ? (float)k8[e] * (float)k8[e] : 0.f;
+  const float inv = 1.0f / sqrtf(akap::wave_sum_dpp(ss) / (float)p.q_rank + p.eps);
+  const float invk = 1.0f / sqrtf(akap::wave_sum_dpp(sk) / (float)p.kv_rank + p.eps);
+  auto normed = [](const bf16x8& x, const float4 (&w)[2], float f) __attribute__((always_inline)) {
+    const float wv[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (bf16)((float)x[e] * f * wv[e]);
+    return o;
+  };
+#pragma unroll
+  for (int c = 0; c < NQ; ++c)
+    if (lane + 64 * c < qc)
+      *(bf16x8*)((bf16*)p.cq_out + (size_t)t * p.q_rank + (lane + 64 * c) * 8) = normed(q[c], qw[c], inv);
+  if (slot < 0) return;
+  bf16* dst = (bf16*)p.cache + (size_t)slot * (p.kv_rank + p.rot_dim);
+  if (lane < kc) {
+    const bf16x8 o = normed(k8, kw, invk);
+    *(bf16x8*)(dst + lane * 8) = o;
+    if (p.vgroups) {
+      bf16* grp = (bf16*)p.vgroups + (size_t)(slot >> 3) * p.kv_rank * 8 + (slot & 7) + lane * 64;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) grp[e * 8] = o[e];
+    }
+  }
+  if (lane < half) {
+    dst[p.kv_rank + first(lane)] = (bf16)(u * cs - v * sn);
+    dst[p.kv_rank + second(lane)] = (bf16)(v * cs + u * sn);
+  }
+}
+
 // The same for large steps (bf16, ranks and offsets of whole 16-byte pieces, q_rank up to 512 NQ,
 // kv_rank up to 512): 32 rows per workgroup, a wave for 4 of them with all their loads in flight.  The
 // normed latents pass through LDS, where 8 rows that fill one group are transposed and leave as whole
@@ -872,15 +949,23 @@ void launch_token_shift(void* out, const void* h, const float* mu, void* state,
 
 void launch_latent_prep(const LatentPrepParams& p, bool f32, hipStream_t s) {
   if (p.T <= 0) return;
-  // (fewer rows leave most CUs without one of these workgroups)
-  if (!f32 && p.T >= 2048 && ((p.q_rank | p.q_off | p.proj_stride) & 7) == 0 && p.q_rank <= 2048 &&
+  if (!f32 && ((p.q_rank | p.q_off | p.proj_stride) & 7) == 0 && p.q_rank <= 2048 &&
       (((uintptr_t)p.proj | (uintptr_t)p.cq_out) & 15) == 0 &&
       (!p.cache || (((p.kv_rank | p.kv_off | p.rot_dim) & 7) == 0 && p.kv_rank <= 512 &&
                     (((uintptr_t)p.cache | (uintptr_t)p.vgroups) & 15) == 0))) {
-    const int n = (p.T + 31) / 32;
-    if (p.q_rank <= 1024) latent_prep_rows_kernel<2><<<n, 512, 0, s>>>(p);
-    else latent_prep_rows_kernel<4><<<n, 512, 0, s>>>(p);
-    return;
+    // (below 2048 rows most CUs lack one of the workgroups of 32)
+    if (p.T >= 2048) {
+      const int n = (p.T + 31) / 32;
+      if (p.q_rank <= 1024) latent_prep_rows_kernel<2><<<n, 512, 0, s>>>(p);
+      else latent_prep_rows_kernel<4><<<n, 512, 0, s>>>(p);
+      return;
+    }
+    if (p.q_rank > 0 && p.rot_dim <= 128 && (!p.cache || p.kv_rank > 0) &&
+        (((uintptr_t)p.q_w | (uintptr_t)p.kv_w) & 15) == 0) {
+      if (p.q_rank <= 1024) latent_prep_wave_kernel<2><<<p.T, 64, 0, s>>>(p);
+      else latent_prep_wave_kernel<4><<<p.T, 64, 0, s>>>(p);
+      return;
+    }
   }
   if (f32) latent_prep_kernel<float><<<p.T, 256, 0, s>>>(p);
   else latent_prep_kernel<bf16><<<p.T, 256, 0, s>>>(p);
