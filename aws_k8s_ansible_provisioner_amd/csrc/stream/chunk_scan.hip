@@ -1185,8 +1185,19 @@ int chunk_scan_segment(int mode, int T, int B, int H, int V) {
   // scan, whose many heads fill the chip with a few prompts, takes them only where the mean length
   // says that most sequences are short (64 heads x 128 x 64, 64 rows and a prompt of 2048: 263 us, 441
   // whole).
-  const bool full = (int64_t)B * H * (V / 32) >= kFill;
-  if (!full) return T >= 1024 || T >= 384 * (int64_t)B ? 256 : 0;
+  const int64_t waves = (int64_t)B * H * (V / 32);
+  if (waves < kFill) {
+    if (T >= 1024 || T >= 384 * (int64_t)B) return 256;
+    // Few short prompts, whose segments are of 64 rows, are cut from 129 rows on: the retention's from a mean
+    // of 160 (8 heads x 128 x 128: a prompt of 160 rows 33 us either way, of 200 41.6 whole and 33.7 cut, of 350
+    // 59.8 and 34.6; three of 256 50 and 41, four of 250 55 and 42), the scan's, whose two launches more weigh
+    // more, of one or two prompts (64 heads x 128 x 64: one of 200 60.9 and 63, of 240 67.5 and 62.3, of 300 76
+    // and 62.5, two of 256 73.4 and 68.3, three of 256 74.5 and 84; 128 heads: one of 256 71.7 and 79.8, of 350
+    // 85.5 and 82).
+    const bool longer = mode == 1 ? T >= 160 * (int64_t)B
+                                  : waves <= 256 && T >= (waves <= 128 ? 240 : 320) * (int64_t)B;
+    return longer && chunk_scan_piece(mode, T, B, H, V) == 64 ? 128 : 0;
+  }
   return T - B >= 1024 && (mode == 1 || T < 256 * (int64_t)B) ? 256 : 0;
 }
 

@@ -557,3 +557,24 @@ def test_retention_pair_weights_of_any_size(what):
     o = ((q @ k.transpose(1, 2)) * V ** -0.5 * w) @ v
     o = o / torch.sqrt((o * o).mean(2, keepdim=True) + 1e-5) * torch.nn.functional.silu(gate)
     assert _rel(got.transpose(0, 1), o) < 3e-3
+
+
+@pytest.mark.parametrize("mode,lens,starts", [
+    (0, [383, 129], [0, 7]), (0, [253], [3]), (1, [320, 129, 128, 257], [0, 4, 9, 0]), (1, [161], [0])])
+def test_few_short_prompts_in_segments(mode, lens, starts):
+    """Sequences of 129 rows and more in segments of 64 where all are short, beside one of 128, whole."""
+    H, V, N, T, B = 4, 64, 64, sum(lens), len(lens)
+    assert torch.ops.akap_stream.chunk_scan_segment(mode, T, B, H, V) == 128
+    step = _step(lens, starts)
+    if mode == 0:
+        inp = _scan_inputs(T, B, H, V, N, 2, torch.bfloat16, 0, seed=T)
+        want, got = (_run_scan(inp, step, H, V, N, 2, d) for d in ("cpu", DEV))
+    else:
+        g = torch.Generator().manual_seed(T)
+        proj, state = torch.randn(T, 4 * H * V, generator=g), torch.randn(B, H, V, N, generator=g)
+        args = (step, H, N, V, (0, H * V, 2 * H * V, 3 * H * V), None,
+                torch.log2(torch.linspace(0.9, 0.999, H)))
+        want, got = (_run_retention((proj, state), *args, d) for d in ("cpu", DEV))
+    assert _rel(got[0], want[0]) < 4e-6
+    for b in range(B):
+        assert _rel(got[1][b], want[1][b]) < 1e-5
