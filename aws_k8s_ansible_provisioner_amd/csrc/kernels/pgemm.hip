@@ -346,8 +346,9 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     //   3         | A top (t+1)          | W right (t+2)  | A bottom x W left
     //   4         | W left (t+1)         | A bottom (t+2) | A bottom x W right
     // A half-tile's place is requested again two turns after the later group's reads of it have
-    // completed (they are waited for where a product's turn begins), and it has landed for every wave a
-    // turn before the earlier group reads it: five half-tiles are younger then.
+    // completed (they are waited for where a product's turn begins; those of tile 0's A top and W left by
+    // both groups ahead of the first turn, whose request takes the same place), and it has landed for
+    // every wave a turn before the earlier group reads it: five half-tiles are younger then.
     auto turn = [&] {
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("" ::: "memory");
@@ -372,6 +373,8 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     turn();
     rd_a(at, lds, 0);
     rd_b(bl, lds, 0);
+    read();
+    turn();
     if (wm) turn();
     for (int t = 0; t < nk; ++t) {
       const bf16x8* cur = lds + (t & 1) * PG_BUF;

@@ -1388,6 +1388,25 @@ def test_pgemm_grouped(counts):
         assert (y - exp).abs().max().item() <= 3e-2 * exp.abs().max().item() + 1e-2, silu
 
 
+@pytest.mark.parametrize("counts", [None, [1100, 3, 900, 0, 300]])
+@pytest.mark.parametrize("K", [64, 128, 192, 320])
+def test_pgemm_few_k_tiles(K, counts):
+    """One to five K tiles: two that fill both LDS buffers, a third that takes the first one's place,
+    odd counts.  Small integers, whose sums fp32 holds: the products are exact but for their rounding
+    to bf16, and a fragment of another K tile shows.  Grouped with enough tiles that they run whole."""
+    M, N = sum(counts or [300]), 4096 if counts else 512
+    g = torch.Generator().manual_seed(K)
+    x = torch.randint(-1, 2, (M, K), generator=g).bfloat16()
+    w = torch.randint(-1, 2, (*([len(counts)] if counts else []), N, K), generator=g).bfloat16()
+    offs = torch.tensor(counts).cumsum(0).int() if counts else None
+    dev = [t if t is None else t.to(DEV) for t in (x, w, offs)]
+    assert torch.equal(ops.pgemm(*dev[:2], offs=dev[2]).cpu(), ref.pgemm(x, w, False, offs))
+    y = ops.pgemm(*dev[:2], silu=True, offs=dev[2]).float().cpu()
+    exp = ref.pgemm(x, w, True, offs).float()
+    # (silu and its product are rounded to bf16 on both sides, 2^-9 each; exp of gates up to 320)
+    assert bool(((y - exp).abs() <= 2 ** -7 * exp.abs() + 1e-30).all())
+
+
 def test_h2d_stage_kernel_copies_pinned_host_memory():
     """The in-stream staging copy (a kernel reading the pinned buffer's device mapping)."""
     for n in (1, 15, 16, 4099, 65536 + 7):
