@@ -299,7 +299,8 @@ __global__ __launch_bounds__(512, 2) void talk_staged_kernel(TalkParams p, const
     b0 = b0 == 2 ? 0 : b0 + 1;
     b1 = b1 == 2 ? 0 : b1 + 1;
   };
-  const int all = min(steps - 1, (last_of(0) - 32) / kKeys + 1);
+  // (whole: step t's second half starts no later than the first query tile's last key; that may be key 31)
+  const int all = min(steps - 1, (last_of(0) + 32) / kKeys);
   for (; t < all; ++t) step(std::true_type{});
   for (; t < steps; ++t) step(std::false_type{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (nothing may land after the end)

@@ -118,3 +118,20 @@ def test_values_that_are_not_finite_stay_where_they_are_seen(Dv, bad):
         out_of_reach = last < (j & ~31)
         assert torch.equal(got[200:][out_of_reach], clean[200:][out_of_reach])
         assert not got[200:][row + 77 >= j].view(-1, 8, Dv)[:, 2:4, 5].isfinite().any()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("D,Dv", [(128, 64), (128, 128), (64, 64)])
+def test_values_that_are_not_finite_in_a_prompt_from_its_start(D, Dv, bad):
+    """The same for a prompt at position 0: its first 32 rows see half of the first step's 64 keys."""
+    a, run = _two_prompts(torch.Generator().manual_seed(8), D=D, Dv=Dv)
+    clean, v = run(DEV), a["v"].clone()
+    row = torch.arange(200)
+    for j in (3, 31, 32, 40, 63, 64, 100, 131, 199):
+        a["v"] = v.clone()
+        a["v"][a["bt"][0, j // 32], 1, j % 32 // 8, 5, j % 8] = bad
+        got = run(DEV)
+        assert torch.equal(got[200:], clean[200:])
+        out_of_reach = (row | 31) < (j & ~31)
+        assert torch.equal(got[:200][out_of_reach], clean[:200][out_of_reach]), j
+        assert not got[:200][row >= j].view(-1, 8, Dv)[:, 2:4, 5].isfinite().any()
