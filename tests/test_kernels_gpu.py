@@ -1407,6 +1407,26 @@ def test_pgemm_few_k_tiles(K, counts):
     assert bool(((y - exp).abs() <= 2 ** -7 * exp.abs() + 1e-30).all())
 
 
+def test_pgemm_silu_of_every_gate():
+    """Each finite bf16 gate whose exponential fp32 holds, times 1, to the bit what the plain product and
+    the activation give: among them the gates where silu is near the smallest fp32 holds, as is the
+    reciprocal of 1 + exp."""
+    K = 256
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    gates[~(gates.float().abs() <= 3e38) | (gates.float() < -88.5)] = 1.0
+    x = torch.eye(K, dtype=torch.bfloat16)
+    w = torch.cat([gates.view(K, K).t(), torch.ones(K, K, dtype=torch.bfloat16)]).contiguous()
+    plain = ops.pgemm(x.to(DEV), w.to(DEV))
+    assert torch.equal(plain[:, :K].cpu()[gates.view(K, K).float().abs() > 2 ** -126],
+                       gates[gates.float().abs() > 2 ** -126])
+    y = ops.pgemm(x.to(DEV), w.to(DEV), silu=True)
+    assert torch.equal(y, ops.silu_and_mul(plain))
+    low = gates.view(K, K).double()
+    want = low / (1 + torch.exp(-low))
+    normal = want.abs() > 2 ** -125
+    assert bool(((y.cpu().double() - want).abs() <= 2 ** -8 * want.abs())[normal].all())
+
+
 def test_h2d_stage_kernel_copies_pinned_host_memory():
     """The in-stream staging copy (a kernel reading the pinned buffer's device mapping)."""
     for n in (1, 15, 16, 4099, 65536 + 7):
