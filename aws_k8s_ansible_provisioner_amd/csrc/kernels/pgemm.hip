@@ -10,13 +10,16 @@
 // "half-tile" is 128 rows x 64 k (16 KB: two 1-KiB DMA instructions per wave), issued in the
 // order the phases consume them, so every wait is a counted `s_waitcnt vmcnt` (never 0 in
 // steady state: cdna_hip_programming.md "Pipelining across barriers", T3+T4).
-// DEFAULT K loop (SCHED 4): the two waves of a SIMD alternate, one reads fragments and requests data while the
-// other multiplies (pg_mainloop has the order).  Bound by what passes through LDS, 192 KB of fragments and
-// 64 KB of data a K tile, beside 2048 cycles of products: 3200 cycles a K tile.  One counted wait and one
-// barrier per K tile, with the whole next tile requested behind it (what 4 waves still run), had every wave
-// read at the same time and multiply at the same time: 8 experts of 2816 x 2048 and 2048 x 1408, 31 thousand rows,
-// 356 + 194 us, now 348 + 191; dense 31232 x 7168 x 4096 1483 -> 1430, 8192 cubed 799 -> 792 (hipBLASLt
-// 1218 and 674).  Workgroups that stay and request their next tile's data before they store gained nothing.
+// DEFAULT K loops: up to 16 K tiles stream-first (SCHED 4): one counted wait and one barrier per K tile,
+// the whole next tile (four half-tiles, 64 KB) requested behind it; every wave reads at the same time and
+// multiplies at the same time.  Beyond, alternating (SCHED 5): the two waves of a SIMD take turns, one reads
+// fragments and requests data while the other multiplies (pg_mainloop has the order).  A K tile then takes 1.14
+// us where stream-first takes 1.23 (one round of tiles, N = 256 .. 4096), its products alone 0.85 (2048 cycles at
+// 2.4 GHz) and what passes through LDS as much (192 KB of fragments, 64 KB of data, 128 bytes a cycle); what the
+// rest goes into is not known.  But a tile's ten turns beside the loop take 1.4 us more: see launch_pgemm.  Long
+// runs, where the clock falls: 8 experts of 2816 x 2048 and 2048 x 1408, 31 thousand rows, 358 + 179 us
+// stream-first, 351 + 176 alternating; dense 31232 x 4096 x 8192 1701 and 1632.  Workgroups that stay and request
+// their next tile's data before they store gained nothing.
 // The phase pipeline (SCHED 1):
 // NB = 2 (plain store; two raw s_barriers per K tile):
 //   phase | counted wait + barrier           | ds_reads issued            | DMA issued
@@ -336,7 +339,7 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     __builtin_amdgcn_s_setprio(0);
   };
 
-  if constexpr (SCHED == 4 && WAVES == 8) {
+  if constexpr (SCHED == 5) {
     // ---- alternating schedule: the two waves of a SIMD (rows 0 .. 127 and 128 .. 255 of the tile) take turns,
     // one reads the next quadrant's fragments and requests a half-tile while the other multiplies a
     // quadrant.  A turn ends with a barrier; the second four waves are one turn behind.
@@ -368,8 +371,7 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     issue(H1{}, 1);
     issue(H2{}, 1);
     issue(H3{}, 1);
-    if (nk > 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (launch_pgemm: there are more than two K tiles)
     turn();
     rd_a(at, lds, 0);
     rd_b(bl, lds, 0);
@@ -421,8 +423,8 @@ __device__ __forceinline__ void pg_mainloop(bf16x8* lds, const __amdgpu_buffer_r
     // ---- stream-first schedule: the whole next K tile (all four half-tiles, 64 KiB) is
     // requested right after this tile's barrier and streams under this tile's MFMAs.  The
     // no-math stream of these tiles (one tile in flight, the same pattern) runs as fast as
-    // hipBLASLt's whole GEMM, while the phase pipeline above measured stream + math
-    // (the "no-math stream" probe).  One wait, one barrier per K tile.
+    // hipBLASLt's whole GEMM, while the phase pipeline below measured stream + math.
+    // One wait, one barrier per K tile.
     issue(H0{}, 0);
     issue(H1{}, 0);
     issue(H2{}, 0);
@@ -828,7 +830,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void pgemm_kernel(PGemmArgs p) {
   const int fr = lane & 15, fg = lane >> 4;
 
   // ---- tile of this workgroup --------------------------------------------------------------
-  constexpr bool CUT = GROUPED && WAVES == 8 && SCHED == 4;
+  constexpr bool CUT = GROUPED && WAVES == 8 && SCHED >= 4;
   int tm, tn, group, row_lo, row_hi, quarter = -1;
   if constexpr (CUT) {
     if (!pg_tile_cut(p, tm, tn, group, row_lo, row_hi, quarter)) return;   // surplus WG (uniform)
@@ -1125,12 +1127,12 @@ long pgemm_sk_ws_floats(int M, int N, int splits) {
 // waves of 128 x 128), read once per process.
 // K-loop issue schedule: AKAP_PGEMM_SCHED = 1 (phase pipeline, half-tiles requested 1.0-1.25
 // tiles ahead), 2 (early issue, 1.25-1.75 tiles ahead), 3 (4-wave unit body), 4 (default:
-// with 8 waves the alternating body, with 4 the whole next tile under this tile's math; pg_mainloop), read
-// once per process.  The decode split-K form (launch_pgemm_sk) keeps 1 / 2.
+// stream-first, with 8 waves and more than 16 K tiles alternating; launch_pgemm), read once per
+// process.  The decode split-K form (launch_pgemm_sk) keeps 1 / 2.
 int pgemm_sched() {
   static int v = [] {
     const char* e = getenv("AKAP_PGEMM_SCHED");
-    const int x = e ? atoi(e) : 4;  // default: the stream-first body
+    const int x = e ? atoi(e) : 4;
     return (x >= 1 && x <= 4) ? x : 4;
   }();
   return v;
@@ -1203,13 +1205,20 @@ void launch_pgemm(const PGemmArgs& a, int epi, hipStream_t st) {
     launch_pgemm_w<4, 3>(q, epi, grid, st);
     return;
   }
-  if (pgemm_sched() == 4) {  // stream-first body (AKAP_PGEMM_WAVES 8 | 4)
+  if (pgemm_sched() == 4) {
     if (pgemm_waves() == 4) {
       launch_pgemm_w<4, 4>(p, epi, grid, st);
-    } else {
-      // (three workgroups more per tile that may be cut, and whole rows of eight tiles)
-      launch_pgemm_w<8, 4>(p, epi, p.groups > 0 ? grid + 3 * min(grid, kPgCut) + 28 : grid, st);
+      return;
     }
+    // (three workgroups more per tile that may be cut, and whole rows of eight tiles)
+    const int all = p.groups > 0 ? grid + 3 * min(grid, kPgCut) + 28 : grid;
+    // What the alternating loop saves per K tile makes up for its turns beside the loop from about 16 on: 1024 rows x
+    // 4096, K = 64 / 512 / 1024 / 2048 / 4096 stream-first 12.3 / 21.3 / 31.8 / 51.9 / 91.1 us, alternating
+    // 13.6 / 22.1 / 32.1 / 50.7 / 86.9; 16384 rows x 2048, K = 768 / 1408 / 6144 59.6 / 90.2 / 311 and 61.9 / 90.1 /
+    // 308; SwiGLU of 16384 x 4096, K = 1024 / 8192 132 / 836 and 135 / 804; 8 experts, 16 thousand rows x 1024, K = 512
+    // 27.4 and 28.4, x 4096, K = 3584 403 and 391.
+    if (p.K > 16 * PG_BK) launch_pgemm_w<8, 5>(p, epi, all, st);
+    else launch_pgemm_w<8, 4>(p, epi, all, st);
     return;
   }
   // two barriers per K tile (measured 1-4 % faster than four, profiles/r4_pgemm_nb_ab.log); the

@@ -1389,11 +1389,12 @@ def test_pgemm_grouped(counts):
 
 
 @pytest.mark.parametrize("counts", [None, [1100, 3, 900, 0, 300]])
-@pytest.mark.parametrize("K", [64, 128, 192, 320])
-def test_pgemm_few_k_tiles(K, counts):
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 1024, 1088, 1152])
+def test_pgemm_exact_sums(K, counts):
     """One to five K tiles: two that fill both LDS buffers, a third that takes the first one's place,
-    odd counts.  Small integers, whose sums fp32 holds: the products are exact but for their rounding
-    to bf16, and a fragment of another K tile shows.  Grouped with enough tiles that they run whole."""
+    odd counts; 16, 17 and 18, where the K loop becomes the alternating one.  Small integers, whose sums
+    fp32 holds: the products are exact but for their rounding to bf16, and a fragment of another K tile
+    shows.  Grouped with enough tiles that they run whole."""
     M, N = sum(counts or [300]), 4096 if counts else 512
     g = torch.Generator().manual_seed(K)
     x = torch.randint(-1, 2, (M, K), generator=g).bfloat16()
