@@ -315,16 +315,17 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
+  auto lanes = [&](int id) {                             // that hold this lane's number as their id
+    uint64_t mine = __ballot((unsigned)id < (unsigned)E);
+    for (int k = 0; k < bits; ++k) {
+      const uint64_t m = __ballot((id >> k) & 1);
+      mine &= (lane >> k) & 1 ? m : ~m;
+    }
+    return __popcll(mine);
+  };
   auto count = [&](int* row, int lo, int hi) {
     int sum = 0;
-    walk(lo, hi, [&](int id, int) {
-      uint64_t mine = __ballot((unsigned)id < (unsigned)E);
-      for (int k = 0; k < bits; ++k) {
-        const uint64_t m = __ballot((id >> k) & 1);
-        mine &= (lane >> k) & 1 ? m : ~m;
-      }
-      sum += __popcll(mine);
-    });
+    walk(lo, hi, [&](int id, int) { sum += lanes(id); });
     if (lane < E) row[lane] = sum;
   };
   // segments and, in mine, runs of whole 64s
@@ -332,20 +333,37 @@ __global__ __launch_bounds__(1024) void moe_align_few_kernel(const int32_t* __re
   const int s0 = min(b * sper, n), s1 = min(s0 + sper, n);
   const int rper = (((s1 - s0 + 15) >> 4) + 63) & ~63;
   const int r0 = min(s0 + wave * rper, s1), r1 = min(r0 + rper, s1);
-  for (int i = tid; i < kAlignSegs * 64; i += 1024) (&hist[0][0])[i] = 0;
-  __syncthreads();
-  const int copy = (lane << bits) & 63;
-  walk(min(4 * wave * sper, n), min((4 * wave + 4) * sper, n), [&](int id, int i) {
-    const int s = __builtin_amdgcn_readfirstlane((i - lane) / sper);
-    if ((unsigned)id < (unsigned)E) atomicAdd(&hist[s][copy | id], 1);
-  });
-  count(run[wave], r0, r1);
-  __syncthreads();
-  for (int i = tid; i < kAlignSegs * E; i += 1024) {
-    const int s = i / E, e = i % E;
-    int sum = 0;
-    for (int c = 0; c < 64; c += 1 << bits) sum += hist[s][c | e];
-    seg[s][e] = sum;
+  // (a ballot per bit of an id counts few experts sooner than the adds: 8192 ids of 1 / 4 / 8 experts 7.1 / 8.1 /
+  // 8.7 us, with adds 10.1 / 8.6 / 8.4; 32768 ids 10.3 / 14.3 / 16.5 and 15.6 / 13.1 / 12.8)
+  if (E <= (n < 16384 ? 4 : 2)) {
+    int at = 4 * wave, sum = 0;
+    auto put = [&] { if (lane < E) seg[at][lane] = sum; };
+    walk(min(4 * wave * sper, n), min((4 * wave + 4) * sper, n), [&](int id, int i) {
+      if (__builtin_amdgcn_readfirstlane(i - lane) >= (at + 1) * sper) {
+        put();
+        ++at;
+        sum = 0;
+      }
+      sum += lanes(id);
+    });
+    for (; at < 4 * wave + 4; ++at, sum = 0) put();
+    count(run[wave], r0, r1);
+  } else {
+    for (int i = tid; i < kAlignSegs * 64; i += 1024) (&hist[0][0])[i] = 0;
+    __syncthreads();
+    const int copy = (lane << bits) & 63;
+    walk(min(4 * wave * sper, n), min((4 * wave + 4) * sper, n), [&](int id, int i) {
+      const int s = __builtin_amdgcn_readfirstlane((i - lane) / sper);
+      if ((unsigned)id < (unsigned)E) atomicAdd(&hist[s][copy | id], 1);
+    });
+    count(run[wave], r0, r1);
+    __syncthreads();
+    for (int i = tid; i < kAlignSegs * E; i += 1024) {
+      const int s = i / E, e = i % E;
+      int sum = 0;                                       // (from another counter on per segment: other banks)
+      for (int c = 0; c < 64; c += 1 << bits) sum += hist[s][(c + (s << bits)) & 63 | e];
+      seg[s][e] = sum;
+    }
   }
   __syncthreads();
   if (tid < E) {

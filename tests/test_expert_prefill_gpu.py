@@ -1,5 +1,5 @@
 """Routed experts of large steps (GPU): rows sorted without padding and gathered by the 256 x 256 tiles,
-the sort's one and sixteen workgroups, and the logits of four rows at a time, against the same ops on
+the sort's one and 64 workgroups, and the logits of four rows at a time, against the same ops on
 CPU tensors."""
 import pytest
 import torch
@@ -13,7 +13,8 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("n,E,block", [(1, 1, 1), (63, 3, 64), (8191, 8, 1), (8192, 8, 1),
-                                       (8300, 32, 64), (20011, 5, 1), (70001, 17, 32)])
+                                       (8300, 32, 64), (20011, 5, 1), (70001, 17, 32),
+                                       (8192, 1, 1), (12001, 4, 64), (70001, 2, 1)])
 def test_align(n, E, block):
     """Every id in its expert's segment, from 8192 ids on in order; ids that name no expert skipped."""
     g = torch.Generator().manual_seed(n)
