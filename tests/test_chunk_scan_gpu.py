@@ -81,7 +81,10 @@ CUT = [([700, 600, 1, 3, 257], [0, 10, 0, -1, 4], 4, 4), ([1100], [9], 4, 4),
        ([300] * 24 + [1] * 10, [0, 3] * 12 + [9] * 10, 16, 16),
        # cut sequences on both sides of the 64th, sequences without rows among them and at the ends
        ([0, 1100, 0, 2] + [1] * 58 + [0, 520, 700] + [3] * 5 + [300, 0], [0, 4, 0, 9] + [6] * 58 + [0, 0, 8]
-        + [2] * 5 + [0, 0], 2, 2)]
+        + [2] * 5 + [0, 0], 2, 2),
+       # 64 and 65 sequences, which are counted and looked at one by one; 70 that are long, too many to be cut
+       ([900] + [2] * 62 + [400], [0] + [4] * 62 + [7], 2, 2), ([400] + [2] * 63 + [900], [3] + [4] * 63 + [0], 2, 2),
+       ([260] * 70 + [3] * 40, [0, 5] * 35 + [1] * 40, 6, 6)]
 
 
 @pytest.mark.parametrize("lens,starts,H,_", CUT)
