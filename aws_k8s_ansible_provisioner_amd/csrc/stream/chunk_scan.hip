@@ -238,7 +238,7 @@ __device__ __forceinline__ bool walked_whole(const ChunkScanParams& p, int n) {
 // ones' segments, without gaps.  True: there is one, of rows [r0, r1) of sequence b.  A lane looks at a
 // sequence.  Of more sequences than lanes the item-th is looked at itself, and a cut one is a gap: so many are
 // mostly short, and a walk of few rows would take less time than to find it (500 sequences of 30 rows, 16 heads x
-// 128 x 128: 606 us by counting, 561 so; 64 heads x 128 x 64 1014 and 947).
+// 128 x 128: 606 us by counting, 518 so; 64 heads x 128 x 64 with its convolution 1014 and 846).
 constexpr int kCounted = 64;
 template <bool WHOLE>
 __device__ __forceinline__ bool walk_of(const ChunkScanParams& p, int item, int& b, int& r0, int& r1, bool& cut) {

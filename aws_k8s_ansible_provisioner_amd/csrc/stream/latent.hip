@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepParams p) {
 // The same for steps of few rows at the sizes below: a wave per row, all of its loads together but the
 // angles, which wait for the position.  Bound by that chain: 64 rows of 768 + 512 + 64 4.0 us (6.2 with a
 // workgroup per row, two sums over it and every entry read twice), 150 of 1536 5.5 (10.4), 600 of 768 6.2
-// (7.2), 1800 10.8 (11.0).
+// (7.2).
 template <int NQ>
 __global__ __launch_bounds__(64) void latent_prep_wave_kernel(LatentPrepParams p) {
   const int t = blockIdx.x, lane = threadIdx.x, qc = p.q_rank >> 3, kc = p.kv_rank >> 3;
@@ -960,7 +960,11 @@ void launch_latent_prep(const LatentPrepParams& p, bool f32, hipStream_t s) {
       else latent_prep_rows_kernel<4><<<n, 512, 0, s>>>(p);
       return;
     }
-    if (p.q_rank > 0 && p.rot_dim <= 128 && (!p.cache || p.kv_rank > 0) &&
+    // (a wave's 2-byte group entries weigh more than a workgroup's from 512 + q_rank rows on, rows of 512 + 64 behind
+    // q_rank: 64 at 512 / 800 / 2047 rows 5.6 / 6.6 / 11.0 us, a workgroup per row 5.7 / 6.5 / 9.0; 768 at 1024 /
+    // 1500 / 2047 7.7 / 9.6 / 11.5 and 7.8 / 9.1 / 10.7; 1536 at 2047 12.4 and 12.6; rows of 256 + 64 8.1 and 8.8)
+    const bool small = !p.vgroups || p.kv_rank <= 256 || p.T <= 512 + p.q_rank;
+    if (small && p.q_rank > 0 && p.rot_dim <= 128 && (!p.cache || p.kv_rank > 0) &&
         (((uintptr_t)p.q_w | (uintptr_t)p.kv_w) & 15) == 0) {
       if (p.q_rank <= 1024) latent_prep_wave_kernel<2><<<p.T, 64, 0, s>>>(p);
       else latent_prep_wave_kernel<4><<<p.T, 64, 0, s>>>(p);

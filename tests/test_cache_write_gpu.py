@@ -120,9 +120,10 @@ def test_large_steps(form, n, H, G, D, rot, BS):
     (2047, 768, 512, 64, ""), (2048, 768, 512, 64, ""), (2077, 1536, 512, 64, "half"),
     (2050, 1032, 96, 16, ""), (2049, 64, 256, 32, "rows"), (2051, 768, 512, 64, "queries"),
     (70, 768, 512, 64, ""), (300, 8, 8, 8, "half"), (65, 1536, 504, 128, "half"), (71, 520, 64, 32, "rows"),
-    (64, 2048, 512, 64, "queries"), (66, 1032, 512, 136, "")])
+    (64, 2048, 512, 64, "queries"), (66, 1032, 512, 136, ""), (576, 64, 512, 64, ""), (577, 64, 512, 64, ""),
+    (2047, 64, 256, 32, "half"), (2047, 64, 512, 64, "rows")])
 def test_latent_rows(n, q_rank, kv_rank, rot, form):
-    """Both sides of 2048 rows (32 to a workgroup, one to a wave); rows without the grouped copy, and
+    """Both sides of 2048 rows (32 to a workgroup) and of 512 + q_rank (one to a wave); rows without the grouped copy, and
     without any; ranks of one 16-byte piece, of one piece more and less than whole waves."""
     g = torch.Generator().manual_seed(n)
     BS, dt = 64, torch.bfloat16
