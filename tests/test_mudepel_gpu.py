@@ -473,6 +473,44 @@ def test_decode_row_of_many_steps(window):
     close(got, want, "bfloat16", scale=2.0)
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,G,D,window,pool", [(16, 4, 128, 200, 16), (8, 1, 64, 0, 0), (3, 1, 64, 50, 32)])
+def test_decode_rows_beside_values_that_are_not_finite(H, G, D, window, pool, bad):
+    """What lies in a row's pages behind its last key, behind its last group of 8 values, in pooled entries
+    that it does not see and in pages that the window has left reaches nothing."""
+    g, BS, lens = gen(H + D), 32, [1, 700, 129, 128, 333, 64, 41]
+    n = [-(-k // BS) for k in lens]
+    bt, at = torch.zeros(len(lens), max(n), dtype=torch.int32), 0
+    for b, k in enumerate(n):
+        bt[b, :k] = torch.arange(at, at + k)
+        at += k
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    q, k, v = rnd(len(lens), H, D), rnd(at, G, BS, D), rnd(at, G, BS // 8, D, 8)
+    kp, vp = [torch.randn(at, G, BS // pool, D, generator=g) if pool else None for _ in range(2)]
+    pos = torch.tensor(lens) - 1
+    slots = bt[torch.arange(len(lens)), pos // BS].long() * BS + pos % BS
+    out = []
+    for _ in range(2):
+        o = torch.zeros(len(lens), H * D, dtype=torch.bfloat16, device="cuda")
+        sops.pooled_window_attention_decode(o, *(None if x is None else x.cuda() for x in (
+            q, k, v, kp, vp, bt, pos, slots)), 0.1, window, pool, True)
+        out.append(o)
+        for b, end in enumerate(lens):
+            if window:
+                gone = max(0, end - window) // BS
+                k[bt[b, :gone].long()], v[bt[b, :gone].long()] = bad, bad
+            if pool:
+                for c in range(max(0, end - window) // pool, n[b] * BS // pool):
+                    kp[bt[b, c * pool // BS], :, c * pool % BS // pool] = bad
+                    vp[bt[b, c * pool // BS], :, c * pool % BS // pool] = bad
+            if end % BS:
+                k[bt[b, end // BS], :, end % BS:] = bad
+            end = -(-end // 8) * 8
+            if end % BS:
+                v[bt[b, end // BS], :, end % BS // 8:] = bad
+    assert out[0].isfinite().all() and torch.equal(*out)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_mid_size_engine_against_the_cpu_ops(tmp_path, dtype):
     """Sizes between the tiny oracle models and the benchmark's (matrix-core attention, the

@@ -306,6 +306,37 @@ def test_talking_attention_matrix_core_decode_kernel(H, G, D, Dv, BS):
         close(out, want, "bfloat16")
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,G,D,BS", [(16, 4, 128, 32), (8, 8, 64, 64), (6, 2, 80, 32)])
+def test_talking_decode_rows_beside_values_that_are_not_finite(H, G, D, BS, bad):
+    """What lies in a row's pages behind its last key, and behind its last group of 8 values, reaches nothing."""
+    g, lens = gen(H + D), [1, 700, 129, 128, 333, 64, 41]
+    n = [-(-k // BS) for k in lens]
+    bt, at = torch.zeros(len(lens), max(n), dtype=torch.int32), 0
+    for b, k in enumerate(n):
+        bt[b, :k] = torch.arange(at, at + k)
+        at += k
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    q, k, v = rnd(len(lens), H, D), rnd(at, G, BS, D), rnd(at, G, BS // 8, D, 8)
+    pos = torch.tensor(lens) - 1
+    out = []
+    for _ in range(2):
+        for parts in (1, 3):
+            o = torch.zeros(len(lens), H * D, dtype=torch.bfloat16, device="cuda")
+            ws = sops.talking_attention_workspace(len(lens), H, G, D, parts, "cuda")
+            sops.talking_attention_decode(o, q.cuda(), k.cuda(), v.cuda(), bt.cuda(), pos.int().cuda() + 1,
+                                          pos.cuda(), torch.eye(H, device="cuda"), None, 0.1, ws, parts)
+            out.append(o)
+        for b, end in enumerate(lens):
+            if end % BS:
+                k[bt[b, end // BS], :, end % BS:] = bad
+            end = -(-end // 8) * 8
+            if end % BS:
+                v[bt[b, end // BS], :, end % BS // 8:] = bad
+    assert out[0].isfinite().all()
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("E,top,F_,d", [(12, 3, 80, 160), (5, 5, 7, 40), (8, 1, 64, 256), (3, 2, 8, 24)])
 def test_routing_and_gated_activation_kernels(dtype, E, top, F_, d):
