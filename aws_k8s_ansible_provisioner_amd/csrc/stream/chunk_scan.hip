@@ -551,16 +551,20 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   // find none last.  One that leaves at once shifts the turns in which the next ones are dealt out to the
   // CUs, and some then wait behind a full one: with such between them a tenth of the waves of 8 x 2048 rows,
   // 8 heads x 128 x 128 began when others had ended (passes of 48 and 111 us, now 36 and 87).  Heads of eight
-  // walks side by side: a walk keeps to one XCD, whose cache then holds what the scan's heads share
-  // (24 sequences of 100 rows, 8 heads: 45.6 us, heads side by side 49.3).
+  // walks side by side: heads that share their keys walk on one XCD, whose cache then holds these (24
+  // sequences of 100 rows, 8 heads: 45.6 us, heads side by side 49.3).  Other keys' heads, and the next eight walks,
+  // start at another XCD: walks are long and short by turns, or fewer than eight (2 prompts of 500 rows, 128 heads
+  // of 8 keys x 64 x 128: 158 us, all heads of a walk on one XCD 162, turned 130; 8 of 300, 32 heads x 64 x 64 81,
+  // 86, 76).
   const int heads = p.H / HW;
   int b, r0, r1, h0;
   bool cut = false;
   if (SEGM) {
     constexpr int kSide = 8;
-    const int at = blockIdx.x % (kSide * heads);
+    const int round = blockIdx.x / (kSide * heads), at = blockIdx.x % (kSide * heads);
     h0 = at / kSide * HW;
-    if (!walk_of<FULL>(p, (int)blockIdx.x / (kSide * heads) * kSide + at % kSide, b, r0, r1, cut)) return;
+    const int turned = (at + round + (MODE == 0 ? h0 / (p.H / p.KH) : h0)) % kSide;
+    if (!walk_of<FULL>(p, round * kSide + turned, b, r0, r1, cut)) return;
   } else {
     h0 = (int)blockIdx.x / p.B * HW;
     b = blockIdx.x % p.B;
