@@ -24,9 +24,10 @@
 // 16 j + 4 hh + 0..3 and 16 j + 8 + 4 hh + 0..3) eight neighbouring registers are an operand of the next
 // product, so the state, the values and the outputs feed each other without lane traffic.
 //
-// Bound by vector work (1000 instructions per chunk, half of them the state's parts) and products (4100
-// cycles per chunk) of a wave that has its SIMD alone or shares it with one other; the next step's
-// parts are formed between a step's products.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
+// Bound by vector work (1000 instructions per chunk, half of them the state's parts, 5.1 cycles each where a wave
+// has its SIMD alone) and products (4100 cycles per chunk); the next step's parts are formed between a step's
+// products.  That is 9200 of the 11850 cycles a chunk takes (8 sequences of 64 heads, a wave per SIMD); what the
+// rest goes into is not known.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
 // where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
 // 128 x 128 (segments) 87 + 36 for the pass before it, while the fragments, half as large as fp32 ones again,
 // take 66.

@@ -649,8 +649,8 @@ __global__ __launch_bounds__(DREG == 16 ? 256 : 512) void retention_kernel(Reten
 // One row per sequence, heads of D x V entries: the same thread owns the same pieces of the state, but
 // everything a workgroup reads is asked for at once, the row's entries and angles ahead of the state, whose
 // arrival no barrier waits for (slot, position, angles and state in turn, each behind the others' loads, and
-// a branch per piece took 18.2 us for 64 rows of 8 heads of 128 x 128, now 10.0; 8 rows 10.8 -> 5.9, 150
-// rows 38 -> 25.8; 64 rows of 16 heads 34 -> 22).  Bound by reading and writing the states: 6.1 TB/s.
+// a branch per piece took 18.2 us of kernel time for 64 rows of 8 heads of 128 x 128, now 9.1; 8 rows 10.9 -> 5.9,
+// 150 rows 38 -> 26; 64 rows of 16 heads 34 -> 22).  Bound by reading and writing the states: 6.1 TB/s.
 template <typename T, int D, int V>
 __global__ __launch_bounds__(V / 4 * (D / 16)) void retention_step_kernel(RetentionParams p) {
   constexpr int DP = D / 16, NT = V / 4 * DP;
@@ -1141,7 +1141,8 @@ __global__ __launch_bounds__(1024) void route_topk_kernel(int32_t* __restrict__ 
 // distance a lane hands on the half of its values that its partner goes on with, 32 exchanges for 192.
 // Bound by vector work and the latency of a wave's own loads, which are one piece ahead: 15600 rows of 2048, 8
 // logits 21.4 us (64: 121), 6000 of 4096 17.4; four waves that shared their rows' logits, each widening the
-// entries for two, took 27.5 (146) and 27.7.
+// entries for two, took 27.5 (146) and 27.7.  A turn of fewer than eight logits repeats the last one: 16384 rows
+// of 2048, 1 / 2 / 4 / 9 logits 19.3 / 20.1 / 20.7 / 34.5 us, by four waves 22.2 / 24.0 / 27.1 / 37.3.
 template <typename T, int R>
 __global__ __launch_bounds__(256) void route_topk_rows_kernel(int32_t* __restrict__ ids,
                                                               float* __restrict__ wout,

@@ -446,7 +446,7 @@ __global__ __launch_bounds__(256) void talk_decode_mfma_kernel(TalkParams p) {
   }
 }
 
-// The same with eight waves, for D = 16 KS entries, at most 16 / KB key heads and pages of a power of two:
+// The same with eight waves, for D = 16 KS entries, at most 8 / KB key heads and pages of a power of two:
 // a step takes 32 KB keys, a wave scores ONE key head's 32 of them, the waves of a key head agree on the
 // maximum through LDS, and a wave accumulates TPW column tiles.
 //
