@@ -29,8 +29,9 @@
 // products.  That is 9200 of the 11850 cycles a chunk takes (8 sequences of 64 heads, a wave per SIMD); what the
 // rest goes into is not known.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
 // where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
-// 128 x 128 (segments) 87 + 36 for the pass before it, while the fragments, half as large as fp32 ones again,
-// take 66.
+// 128 x 128 (segments) 84 + 33 for the pass before it, and 57 for the fragments: all three wait much for
+// memory, and with entries of one part (HALF) 148 MB of fragments are written and 215 read, of 215 and 316
+// where all have three (87 + 37 and 67 us).
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
 // where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
@@ -188,6 +189,10 @@ __device__ __forceinline__ float decay_pow(float l2, int k) {
   return k == 0 ? 1.0f : exp2f(l2 * (float)k);
 }
 
+// a retention's keys times this
+template <int N>
+constexpr float key_scale() { return N == 64 ? 0.125f : 0.08838834764831845f; }
+
 // entries of the per-chunk buffers: sequence b owns those from base(b) on
 __device__ __forceinline__ int base_of(const int32_t* q_start, int b, int rows) {
   return q_start[b] / rows + b;
@@ -315,12 +320,17 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 }
 
 // ------------------------------------------------------------------ fragments of q and k
+// HALF: bf16 rows of a retention of which at most half the entries turn.  The other half of the queries' and keys'
+// are bf16 numbers, one part instead of three: 36 of a chunk's 52 KB are written here and read by the walk, 16 of
+// 24 by the pass before it.  These keys come as they are (times kDown; if a value of the chunk does not split,
+// without) and the weights go to the values, in three parts.
+//
 // One workgroup per (chunk, key head).  Buffer of an entry, in pieces of 64 lanes x 16 bytes: [q: 3 parts
 // of N / 16 pieces][k transposed: the same, the scan's times kDown, the retention's times their weights
 // in the new state (see lifted())][q . k in fp32: 4][1 if a value does not split: then the parts are the
 // fp32 values' upper and lower halves, without kDown, and those of a lifted() head without weights]; rows
 // past the chunk's end are zero.
-template <int MODE, int NT, typename TY>
+template <int MODE, int NT, typename TY, bool HALF>
 __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
   // q and k, then (once every wave has read them) the waves' shares of the products
@@ -377,14 +387,14 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
       }
     }
   }
-  const float kscale = MODE == 1 ? 1.0f / sqrtf((float)N) : 1.0f;
+  constexpr float kscale = MODE == 1 ? key_scale<N>() : 1.0f;
 #pragma unroll
   for (int u = 0; u < RN; ++u) {
     const int i = i0 + u * RS;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b4 = a;
     if (i < n) {
       a = make_float4(q4[u][0], q4[u][1], q4[u][2], q4[u][3]);
-      b4 = make_float4(k4[u][0] * kscale, k4[u][1] * kscale, k4[u][2] * kscale, k4[u][3] * kscale);
+      b4 = make_float4(k4[u][0], k4[u][1], k4[u][2], k4[u][3]);
     }
     *(float4*)(qs + i * LS + d) = a;
     *(float4*)(ks + i * LS + d) = b4;
@@ -394,7 +404,7 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
     wt[tid] = tid < n ? decay_pow(p.log2_decay[kh], n - 1 - tid) * (lift ? kLift : 1.f) : 0.f;
   __syncthreads();
   const int li = lane & 31, hh = lane >> 5;
-  constexpr int NQ = N / 16;
+  constexpr int NQ = N / 16, XQ = HALF ? NQ / 2 : NQ;
   float* buf = p.frag + ((size_t)entry * p.KH + kh) * p.frag_floats;
   // piece f: contraction step f of q (entries 16 f + 4 hh + 0..3 and 8 on), rows 32 (f / 2) of the state
   // and tokens 16 (f % 2) + 4 hh + 0..3 and 8 on of k
@@ -408,7 +418,8 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int j = j0 + (i & 3) + 8 * (i >> 2);
-      v[1][u][i] = ks[j * LS + 32 * (f >> 1) + li] * (MODE == 1 ? wt[j] : 1.f);
+      const float k = ks[j * LS + 32 * (f >> 1) + li];
+      v[1][u][i] = MODE == 0 ? k : f < XQ ? k * kscale * wt[j] : k * kDown;
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w)
@@ -439,9 +450,10 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           uint32_t bits = __float_as_uint(v[w][u][i]);
-          if (w == 1 && lift) {
-            const int f = wave + 4 * u, j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
-            bits = __float_as_uint(ks[j * LS + 32 * (f >> 1) + li]);
+          const int f = wave + 4 * u;
+          if (w == 1 && (lift || f >= XQ)) {
+            const int j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
+            bits = __float_as_uint(ks[j * LS + 32 * (f >> 1) + li] * (f >= XQ ? 1.f : kscale));
           }
           part[0][i] = __builtin_bit_cast(bf16, (uint16_t)(bits >> 16));
           part[1][i] = __builtin_bit_cast(bf16, (uint16_t)bits);
@@ -449,7 +461,8 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        ((bf16x8*)buf)[(3 * NQ * w + wave + 4 * u + i * NQ) * 64 + lane] = part[i];
+        if (i == 0 || wave + 4 * u < XQ)
+          ((bf16x8*)buf)[(3 * NQ * w + wave + 4 * u + i * NQ) * 64 + lane] = part[i];
     }
   // q . k with the keys as rows: lane (i, hh) register 4 g + r is q_i . k_(8 g + 4 hh + r), the
   // operand the walk needs; the waves contract a part of the entries each.  The scan's in four chains
@@ -464,10 +477,10 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
   for (int f = wave; f < NT * 4; f += 4) {
     const float4 a = *(const float4*)(ks + li * LS + 8 * f + 4 * hh);
     const float4 c = *(const float4*)(qs + li * LS + 8 * f + 4 * hh);
-    acc[0] = mfma(a.x, c.x, acc[0]);
-    acc[1 % NC] = mfma(a.y, c.y, acc[1 % NC]);
-    acc[2 % NC] = mfma(a.z, c.z, acc[2 % NC]);
-    acc[3 % NC] = mfma(a.w, c.w, acc[3 % NC]);
+    acc[0] = mfma(a.x * kscale, c.x, acc[0]);
+    acc[1 % NC] = mfma(a.y * kscale, c.y, acc[1 % NC]);
+    acc[2 % NC] = mfma(a.z * kscale, c.z, acc[2 % NC]);
+    acc[3 % NC] = mfma(a.w * kscale, c.w, acc[3 % NC]);
   }
   __syncthreads();
 #pragma unroll
@@ -531,18 +544,21 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
 // segment's own state from zeros.  Fragments and scalars arrive by LDS-DMA: those of q while the state
 // of the chunk before is formed, those of k (in time for the chunk's state) while its outputs are, so
 // that one buffer of each does and two workgroups share a CU; the values in registers a chunk ahead.
-template <int MODE, int NT, int V, int HW, typename TY, bool FULL, bool SEGM>
+template <int MODE, int NT, int V, int HW, typename TY, bool HALF, bool FULL, bool SEGM>
 __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkScanParams p) {
   constexpr int N = NT * 32, NQ = NT * 2, VW = V / 32, NW = VW * HW;
   constexpr bool kNorm = MODE == 1 && FULL;
   constexpr int XP = MODE == 1 && sizeof(TY) == 2 ? 1 : 3;   // parts of a value (of bf16 rows: itself)
   // pieces of 1 KB: [q parts][q . k][scalars of the heads (scan)] and [k parts]; without outputs
   // twice [k parts][scalars]
+  // (HALF: of the pieces from XQ on the first part alone)
+  constexpr int XQ = HALF ? NQ / 2 : NQ;
   constexpr int KU = 3 * NQ, SU = MODE == 0 ? HW : 0, G0 = 3 * NQ, C0 = FULL ? G0 + 4 : KU;
   constexpr int QB = C0 + SU;
   __shared__ __align__(16) float4 qbuf[QB * 64];
   __shared__ __align__(16) float4 kbuf[(FULL ? KU : QB) * 64];
   __shared__ __align__(16) float tab[MODE == 1 ? NW * 2 * kL : 4];   // per wave, see below
+  __shared__ __align__(16) float wtab[HALF ? NW * 2 * kL : 4];       // per wave, see below
   __shared__ __align__(16) float pd[kNorm ? 1024 : 4];       // retention: 2^(c_i - c_j), by lane
   __shared__ __align__(16) float ssq[kNorm ? 2 * NW * kL : 4];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -584,11 +600,14 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   const bool lift = MODE == 1 && uniform(lifted(l2));
   // retention: decay^k and decay^(k + 1)
   float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
+  // HALF: the weights of a chunk's rows in the state after it, kUp times those of keys as they are, and zeros
+  float* wb = wtab + (HALF ? wave * 2 * kL : 0);
   if (MODE == 1) {
     if (lane < kL) {
       tb[lane] = decay_pow(l2, lane);
       tb[kL + lane] = decay_pow(l2, lane + 1);
     }
+    if (HALF) wb[lane] = lane < kL ? decay_pow(l2, kL - 1 - lane) * (key_scale<N>() * kUp) : 0.f;
     if (kNorm) {
       for (int e = tid; e < 1024; e += 64 * NW) {
         const int ln = (e >> 2) & 63, j = 8 * (e >> 8) + 4 * (ln >> 5) + (e & 3), i = ln & 31;
@@ -633,14 +652,21 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     if (MODE == 0 && wave < HW)
       dma16((const char*)(p.scal + ((cb + c) * p.H + h0 + wave) * kScal) + l16, to + wave * 64);
   };
+  auto parts_of = [&](const char* src, float4* to) {
+    if (!HALF) {
+      pieces(src, to, std::integral_constant<int, 3 * NQ>{});
+      return;
+    }
+    pieces(src, to, std::integral_constant<int, NQ>{});
+    pieces(src + NQ * 1024, to + NQ * 64, std::integral_constant<int, XQ>{});
+    pieces(src + 2 * NQ * 1024, to + 2 * NQ * 64, std::integral_constant<int, XQ>{});
+  };
   auto stage_q = [&](int c) {
-    pieces(frag_of(c), qbuf, std::integral_constant<int, 3 * NQ>{});
+    parts_of(frag_of(c), qbuf);
     pieces(frag_of(c) + 6 * NQ * 1024, qbuf + G0 * 64, std::integral_constant<int, 4>{});
     stage_scalars(c, qbuf + C0 * 64);
   };
-  auto stage_k = [&](int c, float4* to) {
-    pieces(frag_of(c) + 3 * NQ * 1024, to, std::integral_constant<int, KU>{});
-  };
+  auto stage_k = [&](int c, float4* to) { parts_of(frag_of(c) + 3 * NQ * 1024, to); };
   // values of a chunk's rows 8 g + 4 hh + r at a lane's column
   const int ld = MODE == 0 ? p.x_stride : p.proj_stride;
   constexpr int es = MODE == 0 ? 4 : sizeof(TY);
@@ -701,7 +727,10 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   auto joined = [&](const bf16x8* parts, int f) {
     typedef uint32_t Words __attribute__((ext_vector_type(2)));   // two entries each
     const Words* at = (const Words*)(parts + (f >> 1) * 64) + (f & 1);
-    const Words a = at[0], b = at[NQ * 128], d = at[NQ * 256];
+    const Words a = at[0];
+    if (f >> 1 >= XQ)
+      return make_float4(lower(a[0]), upper(a[0]), lower(a[1]), upper(a[1]));
+    const Words b = at[NQ * 128], d = at[NQ * 256];
     float v[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -722,14 +751,26 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   // the values times their weights in the state after the chunk (the scan's times kUp; the retention's are
   // in k), and their parts
   float xw[16];
-  bf16x8 w[2][3];
+  bf16x8 w[2][3], wh[HALF ? 2 : 1][3];       // (wh: of values times wb, for keys as they are)
   Range wr;
-  float4 w4[MODE == 0 ? 4 : 1];
-  auto fetch_weights = [&](const float* sc) {
+  float4 w4[MODE == 0 || HALF ? 4 : 1];
+  auto fetch_weights = [&](const float* sc, int n) {
     if (MODE == 0) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) w4[g] = *(const float4*)(sc + 2 * kL + 8 * g + 4 * hh);
+    } else if (HALF) {
+      const float* at = wb + (kL - n) + 4 * hh;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) w4[g] = make_float4(at[8 * g], at[8 * g + 1], at[8 * g + 2], at[8 * g + 3]);
     }
+  };
+  // values s and s + 1 times their weights, in parts (of the unrounded products)
+  auto weigh_two = [&](int s, uint32_t (&part)[3]) {
+    const float f0 = (&w4[s >> 2].x)[s & 3], f1 = (&w4[s >> 2].x)[(s & 3) + 1];
+    part[0] = pair(x[s] * f0, x[s + 1] * f1);
+    const float r0 = fmaf(x[s], f0, -lower(part[0])), r1 = fmaf(x[s + 1], f1, -upper(part[0]));
+    part[1] = pair(r0, r1);
+    part[2] = pair(r0 - lower(part[1]), r1 - upper(part[1]));
   };
   auto weigh = [&] {
     wr = Range{};
@@ -766,6 +807,24 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
       for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
     }
+    if constexpr (HALF) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        u32x4 part[3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t two[3];
+          weigh_two(8 * m + 2 * i, two);
+#pragma unroll
+          for (int u = 0; u < 3; ++u) part[u][i] = two[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+          wh[m][u] = __builtin_bit_cast(bf16x8, part[u]);
+          asm volatile("" : "+v"(wh[m][u]));
+        }
+      }
+    }
   };
   // do the weighted values split (a value of one part: is it one that the matrix units take)?
   auto judge = [&] {
@@ -798,6 +857,12 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         for (int i = 0; i < 16; ++i) S[t][i] *= dend;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
+        float xe[4];       // values of keys as they are
+        if (HALF) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            xe[r] = x[4 * g + r] * (wb[kL - n + 8 * g + 4 * hh + r] * kDown);
+        }
         float up[4];       // undoes the scaling of a key; a lifted() head's values take its weight's exponent
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -812,6 +877,15 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const float4 a = joined(kp, 4 * t + g);
+          if (HALF && t >= NT / 2) {
+            const float whole = odd ? 1.f : kUp;
+            S[t] = mfma(a.x * whole, xe[0], S[t]);
+            S[t] = mfma(a.y * whole, xe[1], S[t]);
+            S[t] = mfma(a.z * whole, xe[2], S[t]);
+            S[t] = mfma(a.w * whole, xe[3], S[t]);
+            __builtin_amdgcn_sched_barrier(0);
+            continue;
+          }
           S[t] = mfma(a.x * up[0], xw[4 * g], S[t]);
           S[t] = mfma(a.y * up[1], xw[4 * g + 1], S[t]);
           S[t] = mfma(a.z * up[2], xw[4 * g + 2], S[t]);
@@ -837,7 +911,8 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     bf16x8 k[2][3];
     auto fetch = [&](int u) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i) k[u & 1][i] = kp[(u + i * NQ) * 64];
+      for (int i = 0; i < 3; ++i)
+        if (i == 0 || u < XQ) k[u & 1][i] = kp[(u + i * NQ) * 64];
     };
     auto decay = [&](int t) {
 #pragma unroll
@@ -853,7 +928,11 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       constexpr int ka[6] = {2, 0, 1, 1, 0, 0}, wa[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
       for (int i = 0; i < 6; ++i)
-        if (wa[i] < XP) S[t] = mfma16(k[m][ka[i]], w[m][wa[i]], S[t]);
+        if (HALF && t >= NT / 2) {
+          if (ka[i] == 0) S[t] = mfma16(k[m][0], wh[m][wa[i]], S[t]);
+        } else if (wa[i] < XP) {
+          S[t] = mfma16(k[m][ka[i]], w[m][wa[i]], S[t]);
+        }
       if (m == 0 && t + 1 < NT) {
         decay(t + 1);
         interleave<XP == 3 ? 6 : 3, XP == 3 ? 3 : 6>();
@@ -869,7 +948,8 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     bf16x8 q[2][3];                   // (the next fragments are on their way while a step's products run)
     auto fetch = [&](int j) {
 #pragma unroll
-      for (int u = 0; u < 3; ++u) q[j & 1][u] = qp[(j + u * NQ) * 64];
+      for (int u = 0; u < 3; ++u)
+        if (u == 0 || j < XQ) q[j & 1][u] = qp[(j + u * NQ) * 64];
     };
     fetch(0);
     float P[16];
@@ -935,17 +1015,23 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       if (j + 1 < NQ) fetch(j + 1);
       if (PG == 1 ? j > 0 : j % PG == 1 && j + 1 < NQ) fetch_pairs(PG == 1 ? j : j / PG + 1);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_split(a[j & 1], q[j & 1], O, O2);
+      if (j < XQ) {
+        mfma_split(a[j & 1], q[j & 1], O, O2);
+      } else {
+        O2 = mfma16(a[j & 1][2], q[j & 1][0], O2);
+        O = mfma16(a[j & 1][0], q[j & 1][0], O);
+        O2 = mfma16(a[j & 1][1], q[j & 1][0], O2);
+      }
       if (j + 1 < NQ) state_parts(j + 1);
       if (j % PG == 0) {
         pair_weights(j / PG);
-        interleave<6, MODE == 0 ? 18 : 12>();
+        if (j < XQ) interleave<6, MODE == 0 ? 18 : 12>(); else interleave<3, 24>();
       } else {
-        interleave<6, 9>();
+        if (j < XQ) interleave<6, 9>(); else interleave<3, 18>();
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    fetch_weights(sc);
+    fetch_weights(sc, n);
 #pragma unroll
     for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
     __builtin_amdgcn_sched_barrier(0);
@@ -1087,7 +1173,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       const float* sc = MODE == 0 ? (const float*)(now + (C0 + hw) * 64) : nullptr;
       const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
       if (MODE == 0) total += sc[4 * kL - 1];
-      fetch_weights(sc);
+      fetch_weights(sc, n);
       weigh();
       judge();
       advance(now, dend, n);
@@ -1156,23 +1242,23 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
   *st = prev;
 }
 
-template <int MODE, int NT, int V, int HW, typename TY>
+template <int MODE, int NT, int V, int HW, typename TY, bool HALF = false>
 void run(const ChunkScanParams& p, hipStream_t s) {
   const int chunks = p.T / kL + p.B;
-  chunk_frag_kernel<MODE, NT, TY><<<dim3(chunks, p.KH), 256, 0, s>>>(p);
+  chunk_frag_kernel<MODE, NT, TY, HALF><<<dim3(chunks, p.KH), 256, 0, s>>>(p);
   if (MODE == 0)
     chunk_scalar_kernel<TY><<<dim3(chunks, (p.H + 31) / 32), 256, 0, s>>>(p);
   constexpr int nt = 2 * V * HW;
   if (p.SEG == 0) {
-    chunk_walk_kernel<MODE, NT, V, HW, TY, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
+    chunk_walk_kernel<MODE, NT, V, HW, TY, HALF, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
     return;
   }
   // at most so many sequences are cut, and so many segments theirs; whole multiples of eight walks
   const int cut = min(p.B, p.T / p.SEG), segs = p.T / p.PIECE + cut;
   auto grid = [&](int walks) { return (walks + 7) / 8 * 8 * (p.H / HW); };
-  chunk_walk_kernel<MODE, NT, V, HW, TY, false, true><<<grid(segs), nt, 0, s>>>(p);
+  chunk_walk_kernel<MODE, NT, V, HW, TY, HALF, false, true><<<grid(segs), nt, 0, s>>>(p);
   chunk_join_kernel<<<dim3(p.B, p.H, (p.V * p.N + 1023) / 1024), 256, 0, s>>>(p);
-  chunk_walk_kernel<MODE, NT, V, HW, TY, true, true>
+  chunk_walk_kernel<MODE, NT, V, HW, TY, HALF, true, true>
       <<<grid(p.B > kCounted ? p.B + segs : p.T / p.PIECE + p.B), nt, 0, s>>>(p);
 }
 
@@ -1180,6 +1266,15 @@ void run(const ChunkScanParams& p, hipStream_t s) {
 // are staged once for both
 template <int MODE, int NT, typename TY>
 void pick_v(const ChunkScanParams& p, hipStream_t s) {
+  if constexpr (MODE == 1 && sizeof(TY) == 2) {
+    // (which pieces have one part is fixed when the kernels are built: half of them, as the models turn half
+    // of the entries or fewer; 8 x 2048 rows, 8 heads x 128 x 128: 176 us, 197 where all have three)
+    if (p.rot_dims * 2 <= p.N) {
+      if (p.V == 128) run<MODE, NT, 128, 1, TY, true>(p, s);
+      else run<MODE, NT, 64, 1, TY, true>(p, s);
+      return;
+    }
+  }
   if (p.V == 128) run<MODE, NT, 128, 1, TY>(p, s);
   else if (MODE == 0 && (p.H / p.KH) % 2 == 0) run<MODE, NT, 64, MODE == 0 ? 2 : 1, TY>(p, s);
   else run<MODE, NT, 64, 1, TY>(p, s);

@@ -581,3 +581,37 @@ def test_few_short_prompts_in_segments(mode, lens, starts):
     assert _rel(got[0], want[0]) < 4e-6
     for b in range(B):
         assert _rel(got[1][b], want[1][b]) < 1e-5
+
+
+@pytest.mark.parametrize("D,V,rot", [(128, 128, 64), (128, 64, 40), (64, 128, 32), (64, 64, 8)])
+@pytest.mark.parametrize("what", ["usual", "small keys", "odd key", "odd query"])
+def test_retention_entries_that_do_not_turn(D, V, rot, what):
+    """bf16 rows of which at most half the entries turn keep the others as they are, with the weights on the
+    values; the same rows in fp32 go the general way.  Keys of 2^-60 and 2^-100 are below what is scaled
+    down exactly, those of 3e38 and the infinite do not split.  Outputs: a rounding to bf16; states: both sides
+    sum in fp32 (module comment)."""
+    H, lens, starts = 4, [1, 33, 300, 64], [9, 0, 5, 0]
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(D + V + rot)
+    proj = torch.randn(T, 2 * H * D + 2 * H * V, generator=g)
+    q, k = (proj[:, i * H * D:(i + 1) * H * D].view(T, H, D) for i in range(2))
+    if what == "small keys":
+        k[:, 0, rot:] *= 2.0 ** -60
+        k[::3, 1, D - 1] *= 2.0 ** -100
+    elif what == "odd key":
+        k[-3, 0, D - 1], k[40, 1, rot] = float("inf"), 3e38
+    elif what == "odd query":
+        q[-3, 0, D - 1], q[40, 1, rot] = float("nan"), 2.0 ** -110
+    proj = proj.bfloat16()
+    state = torch.randn(B, H, V, D, generator=g)
+    ang = torch.arange(2048)[:, None] * (0.5 ** torch.arange(rot // 2))[None, :]
+    args = (_step(lens, starts), H, D, V, (0, H * D, 2 * H * D, 2 * H * D + H * V),
+            torch.cat([torch.cos(ang), torch.sin(ang)], 1), torch.log2(torch.tensor([0.97, 0.42, 0.2, 0.999])), DEV)
+    got, want = _run_retention((proj, state), *args), _run_retention((proj.float(), state), *args)
+    for a, b, limit in zip((got[0].float(), got[1]), want, (3e-3, 2e-6)):
+        ok = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), ok)
+        # (a product of 3e38 rules its head's sums: heads apart)
+        for h in range(H):
+            part = (slice(None), slice(h * V, (h + 1) * V)) if a.dim() == 2 else (slice(None), h)
+            assert _rel(torch.where(ok, a, 0.)[part], torch.where(ok, b, 0.)[part].cpu()) < limit
