@@ -15,9 +15,9 @@
 // states 1.7e-7 (2.7e-7).  Operands that do not split (not finite, past bf16's range, or one so small that
 // a part would be denormal, which the matrix units take as zero) go through the fp32 products.
 //
-// chunk_frag_kernel prepares every (chunk, key head) side by side: the parts of q and k (rotated and
+// chunk_prep_kernel prepares every (chunk, key head) side by side: the parts of q and k (rotated and
 // scaled for the retention) as operand fragments and the 32 x 32 products q_i . k_j in fp32; the scan's
-// keys belong to a group, so its heads share them.  chunk_scalar_kernel sums the scan's decays.
+// keys belong to a group, so its heads share them.  It also sums the scan's decays.
 // chunk_walk_kernel then walks the chunks of a (sequence, head): a wave owns 32 state columns in
 // accumulators.  An accumulator lane holds column l & 31 and rows 8 g + 4 (l >> 5) + r in
 // register 4 g + r: with the fragments' entries in that order (lane (i, hh) of step j: entries
@@ -331,7 +331,7 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 // fp32 values' upper and lower halves, without kDown, and those of a lifted() head without weights]; rows
 // past the chunk's end are zero.
 template <int MODE, int NT, typename TY, bool HALF>
-__global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p) {
+__device__ __forceinline__ void fragments(const ChunkScanParams& p, const int entry, const int kh) {
   constexpr int N = NT * 32, LS = N + 4;   // rows 4 banks apart: 16-byte reads of 32 rows are free
   // q and k, then (once every wave has read them) the waves' shares of the products
   using TR = typename std::conditional<MODE == 0, double, float>::type;
@@ -340,7 +340,6 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
   __shared__ float wt[kL];     // retention: the rows' weights in the state after the chunk
   float *qs = rows, *ks = rows + kL * LS;
   TR* red = (TR*)rows;
-  const int entry = blockIdx.x, kh = blockIdx.y;
   int r0, r1;
   const int b = locate(p, entry, kL, r0, r1);
   if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
@@ -507,8 +506,8 @@ __global__ __launch_bounds__(256) void chunk_frag_kernel(const ChunkScanParams p
 // decays (formed in fp64): [32] dt, [32] 2^c, [32] kUp dt 2^(c_end - c), [32] c, [32] what c lost when
 // it was rounded.  Rows past the end: dt 0, decay 1.
 template <typename TY>
-__global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams p) {
-  const int entry = blockIdx.x, i = threadIdx.x & 31;
+__device__ __forceinline__ void scalars(const ChunkScanParams& p, const int entry, const int heads) {
+  const int i = threadIdx.x & 31;
   int r0, r1;
   const int b = locate(p, entry, kL, r0, r1);
   if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
@@ -516,7 +515,7 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
   const TY* src = (const TY*)p.proj + (size_t)(r0 + min(i, n - 1)) * p.proj_stride + p.dt_off;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const int h = blockIdx.y * 32 + u * 8 + (threadIdx.x >> 5);
+    const int h = heads * 32 + u * 8 + (threadIdx.x >> 5);
     if (h >= p.H) return;   // (all lanes of a half wave share h)
     const float v = ldv(src + h) + p.dt_bias[h];
     const float dt = i < n ? (v > 20.f ? v : log1pf(expf(v))) : 0.f;
@@ -536,6 +535,15 @@ __global__ __launch_bounds__(256) void chunk_scalar_kernel(const ChunkScanParams
     sc[3 * kL + i] = hi;
     sc[4 * kL + i] = (float)(l - (double)hi);
   }
+}
+
+// Both wait for chains of loads (8 x 2048 rows, 64 heads x 128 x 64: 13 us each, one launch after the other), so
+// they run side by side in one, 21 us: the key heads' workgroups first, then those of 32 heads (in turns 23).
+// Short steps gain the launch: a prompt of 200 rows 61 -> 55 us with its convolution, 64 of 26 106 -> 100.
+template <int MODE, int NT, typename TY, bool HALF>
+__global__ __launch_bounds__(256) void chunk_prep_kernel(const ChunkScanParams p) {
+  if (MODE == 1 || (int)blockIdx.y < p.KH) fragments<MODE, NT, TY, HALF>(p, blockIdx.x, blockIdx.y);
+  else scalars<TY>(p, blockIdx.x, blockIdx.y - p.KH);
 }
 
 // ------------------------------------------------------------------ the walk
@@ -1245,9 +1253,8 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
 template <int MODE, int NT, int V, int HW, typename TY, bool HALF = false>
 void run(const ChunkScanParams& p, hipStream_t s) {
   const int chunks = p.T / kL + p.B;
-  chunk_frag_kernel<MODE, NT, TY, HALF><<<dim3(chunks, p.KH), 256, 0, s>>>(p);
-  if (MODE == 0)
-    chunk_scalar_kernel<TY><<<dim3(chunks, (p.H + 31) / 32), 256, 0, s>>>(p);
+  chunk_prep_kernel<MODE, NT, TY, HALF>
+      <<<dim3(chunks, p.KH + (MODE == 0 ? (p.H + 31) / 32 : 0)), 256, 0, s>>>(p);
   constexpr int nt = 2 * V * HW;
   if (p.SEG == 0) {
     chunk_walk_kernel<MODE, NT, V, HW, TY, HALF, true, false><<<p.B * (p.H / HW), nt, 0, s>>>(p);
