@@ -29,9 +29,9 @@
 // products.  That is 9200 of the 11850 cycles a chunk takes (8 sequences of 64 heads, a wave per SIMD); what the
 // rest goes into is not known.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
 // where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
-// 128 x 128 (segments) 84 + 33 for the pass before it, and 57 for the fragments: all three wait much for
+// 128 x 128 (segments) 76 + 33 for the pass before it, and 57 for the fragments: all three wait much for
 // memory, and with entries of one part (HALF) 148 MB of fragments are written and 215 read, of 215 and 316
-// where all have three (87 + 37 and 67 us).
+// where all have three (walks 3 + 4 us more, fragments 67).
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
 // where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
@@ -193,14 +193,14 @@ __device__ __forceinline__ float decay_pow(float l2, int k) {
 template <int N>
 constexpr float key_scale() { return N == 64 ? 0.125f : 0.08838834764831845f; }
 
-// entries of the per-chunk buffers: sequence b owns those from base(b) on
-__device__ __forceinline__ int base_of(const int32_t* q_start, int b, int rows) {
-  return q_start[b] / rows + b;
-}
-
 // the sequence that owns an entry (the same in all lanes), and the rows [r0, r1) of the entry (r1 <= r0:
 // none): a chain of scalar loads
 typedef const __attribute__((address_space(4))) int32_t* ScalarInts;
+
+// entries of the per-chunk buffers: sequence b (the same in all lanes) owns those from base(b) on
+__device__ __forceinline__ int base_of(const int32_t* q_start, int b, int rows) {
+  return ((ScalarInts)q_start)[b] / rows + b;
+}
 
 __device__ __forceinline__ int locate(const ChunkScanParams& p, int entry, int rows, int& r0, int& r1) {
   const ScalarInts q_start = (ScalarInts)p.q_start;
@@ -304,16 +304,20 @@ __device__ __forceinline__ bool walk_of(const ChunkScanParams& p, int item, int&
 __host__ __device__ __forceinline__ bool few_long(int T, int B, int PIECE) { return B > T / PIECE + 2; }
 
 __device__ __forceinline__ size_t seg_base(const ChunkScanParams& p, int b) {
-  return few_long(p.T, p.B, p.PIECE) ? (size_t)(2 * (int64_t)p.q_start[b] / p.PIECE)
+  return few_long(p.T, p.B, p.PIECE) ? (size_t)(2 * (int64_t)((ScalarInts)p.q_start)[b] / p.PIECE)
                                      : (size_t)base_of(p.q_start, b, p.PIECE);
 }
 
-// does a sequence whose first row is t go on from its slot's state?  (The scan's row form starts anew
-// at positions below 0 too.)
+// does a sequence whose first row is t (the same in all lanes) go on from its slot's state?  (The scan's row
+// form starts anew at positions below 0 too.)
 __device__ __forceinline__ bool goes_on(const ChunkScanParams& p, int t) {
-  const int64_t pos = p.positions[t];
+  typedef const __attribute__((address_space(4))) int64_t* ScalarLongs;
+  const int64_t pos = ((ScalarLongs)p.positions)[t];
   return p.mode == 0 ? pos > 0 : pos != 0;
 }
+
+// the slot of the sequence with first row t
+__device__ __forceinline__ int slot_of(const ChunkScanParams& p, int t) { return ((ScalarInts)p.seq_slot)[t]; }
 
 __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
   return slot >= 0 && slot < p.num_slots;
@@ -342,7 +346,9 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
   TR* red = (TR*)rows;
   int r0, r1;
   const int b = locate(p, entry, kL, r0, r1);
-  if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
+  if (r1 <= r0) return;
+  // (looked at once the rows are on their way; the positions of a sequence without a slot are not used)
+  const bool live = live_slot(p, slot_of(p, ((ScalarInts)p.q_start)[b]));
   const int n = r1 - r0, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int half = p.rot_dims / 2;
   // a thread keeps to four columns; its rows' loads are in flight together
@@ -374,7 +380,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
     const int a = low ? d : d - half;
 #pragma unroll
     for (int u = 0; u < RN; ++u) {
-      const float* cs = p.cos_sin + (size_t)pos[u] * p.rot_dims + a;
+      const float* cs = p.cos_sin + (size_t)(live ? pos[u] : 0) * p.rot_dims + a;
       float c4[4], s4[4];
       ld4(cs, c4);
       ld4(cs + half, s4);
@@ -436,6 +442,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
         for (int i = 0; i < 8; ++i) bad |= below(v[w][u][i], kSmall / scale[w]);
   }
   bad = __syncthreads_or(bad);
+  if (!live) return;
 #pragma unroll
   for (int w = 0; w < 2; ++w)
 #pragma unroll
@@ -510,7 +517,7 @@ __device__ __forceinline__ void scalars(const ChunkScanParams& p, const int entr
   const int i = threadIdx.x & 31;
   int r0, r1;
   const int b = locate(p, entry, kL, r0, r1);
-  if (r1 <= r0 || !live_slot(p, p.seq_slot[p.q_start[b]])) return;
+  if (r1 <= r0 || !live_slot(p, slot_of(p, ((ScalarInts)p.q_start)[b]))) return;
   const int n = r1 - r0;
   const TY* src = (const TY*)p.proj + (size_t)(r0 + min(i, n - 1)) * p.proj_stride + p.dt_off;
 #pragma unroll
@@ -599,54 +606,13 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   }
   const int hw = wave / VW, h = h0 + hw;
   const int first = ((ScalarInts)p.q_start)[b];
-  const size_t seg = cut ? (size_t)uniform((int)seg_base(p, b) + (r0 - first) / p.PIECE) : 0;
-  const int slot = uniform(p.seq_slot[first]);
+  const size_t seg = cut ? (size_t)((int)seg_base(p, b) + (r0 - first) / p.PIECE) : 0;
+  const int slot = slot_of(p, first);
   if (!live_slot(p, slot)) return;
   const int kh = MODE == 0 ? h0 / (p.H / p.KH) : h;
   const int col = (wave % VW) * 32 + li;
-  const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
-  const bool lift = MODE == 1 && uniform(lifted(l2));
-  // retention: decay^k and decay^(k + 1)
-  float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
-  // HALF: the weights of a chunk's rows in the state after it, kUp times those of keys as they are, and zeros
-  float* wb = wtab + (HALF ? wave * 2 * kL : 0);
-  if (MODE == 1) {
-    if (lane < kL) {
-      tb[lane] = decay_pow(l2, lane);
-      tb[kL + lane] = decay_pow(l2, lane + 1);
-    }
-    if (HALF) wb[lane] = lane < kL ? decay_pow(l2, kL - 1 - lane) * (key_scale<N>() * kUp) : 0.f;
-    if (kNorm) {
-      for (int e = tid; e < 1024; e += 64 * NW) {
-        const int ln = (e >> 2) & 63, j = 8 * (e >> 8) + 4 * (ln >> 5) + (e & 3), i = ln & 31;
-        pd[e] = j <= i ? decay_pow(l2, i - j) : 0.f;
-      }
-    }
-  }
-  // entry (row, column) of the state: the scan keeps [N, V], the retention [V, N]
-  float* sp = cut ? p.seg + (seg * p.H + h) * N * V
-                  : p.state + ((size_t)slot * p.H + h) * N * V;
-  f32x16 S[NT];
-  const bool load = FULL && (cut || goes_on(p, first));
-  const bool anew = FULL && (cut ? r0 == first && !goes_on(p, first) : !load);   // a state of zeros
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int row = 32 * t + 8 * g + 4 * hh;
-      if (!load) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = 0.f;
-      } else if (MODE == 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = sp[(size_t)(row + r) * V + col];
-      } else {
-        const float4 v = *(const float4*)(sp + (size_t)col * N + row);
-        S[t][4 * g] = v.x; S[t][4 * g + 1] = v.y; S[t][4 * g + 2] = v.z; S[t][4 * g + 3] = v.w;
-      }
-    }
   const int c0 = (r0 - first) / kL, chunks = (r1 - r0 + kL - 1) / kL;
-  const size_t cb = (size_t)uniform(base_of(p.q_start, b, kL) + c0);
+  const size_t cb = (size_t)(base_of(p.q_start, b, kL) + c0);
   const uint32_t l16 = lane * 16;
   auto frag_of = [&](int c) { return (const char*)(p.frag + ((cb + c) * p.KH + kh) * p.frag_floats); };
   auto pieces = [&](const char* src, float4* to, auto count) {
@@ -695,6 +661,54 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       o += (s & 3) == 3 ? 5 * step : step;
     }
   };
+  // (the first chunk's are on their way while the state is asked for)
+  values(0);
+  auto stage = [&](int c, float4* to) {
+    stage_k(c, to);
+    stage_scalars(c, to + C0 * 64);
+  };
+  if (FULL) stage_q(0); else stage(0, qbuf);
+  const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
+  const bool lift = MODE == 1 && uniform(lifted(l2));
+  // retention: decay^k and decay^(k + 1)
+  float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
+  // HALF: the weights of a chunk's rows in the state after it, kUp times those of keys as they are, and zeros
+  float* wb = wtab + (HALF ? wave * 2 * kL : 0);
+  if (MODE == 1) {
+    if (lane < kL) {
+      tb[lane] = decay_pow(l2, lane);
+      tb[kL + lane] = decay_pow(l2, lane + 1);
+    }
+    if (HALF) wb[lane] = lane < kL ? decay_pow(l2, kL - 1 - lane) * (key_scale<N>() * kUp) : 0.f;
+    if (kNorm) {
+      for (int e = tid; e < 1024; e += 64 * NW) {
+        const int ln = (e >> 2) & 63, j = 8 * (e >> 8) + 4 * (ln >> 5) + (e & 3), i = ln & 31;
+        pd[e] = j <= i ? decay_pow(l2, i - j) : 0.f;
+      }
+    }
+  }
+  // entry (row, column) of the state: the scan keeps [N, V], the retention [V, N]
+  float* sp = cut ? p.seg + (seg * p.H + h) * N * V
+                  : p.state + ((size_t)slot * p.H + h) * N * V;
+  f32x16 S[NT];
+  const bool load = FULL && (cut || goes_on(p, first));
+  const bool anew = FULL && (cut ? r0 == first && !goes_on(p, first) : !load);   // a state of zeros
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 32 * t + 8 * g + 4 * hh;
+      if (!load) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = 0.f;
+      } else if (MODE == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][4 * g + r] = sp[(size_t)(row + r) * V + col];
+      } else {
+        const float4 v = *(const float4*)(sp + (size_t)col * N + row);
+        S[t][4 * g] = v.x; S[t][4 * g + 1] = v.y; S[t][4 * g + 2] = v.z; S[t][4 * g + 3] = v.w;
+      }
+    }
   const float dsk = MODE == 0 ? p.d_skip[h] : 0.f;
   float total = 0.f;   // log2 decay of the segment
   // outputs transposed: row 8 g + 4 hh + r of the accumulator is a column of the state, lane li the
@@ -948,7 +962,14 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto outputs = [&](int c) {
+  // hand_on() lets the next chunk's queries into the buffer.  A retention's segments do so as soon as the queries
+  // were used and norm a chunk's outputs when the next one's keys were asked for: what follows the queries'
+  // products is short (walk of 8 x 2048 rows, 8 heads x 128 x 128 84 -> 76 us, 40 prompts of 300 rows 139 -> 129).
+  // The scan has more to do there (half a per cent slower so), and a few heads alone wait for each step and not
+  // for memory (a retention's prompt of 100 rows 28.9 us, so 29.9).
+  constexpr bool kEarly = MODE == 1 && SEGM;
+  float dend;
+  auto outputs = [&](int c, auto hand_on) {
     const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
     const int lane_ = (int)fresh(lane), li = lane_ & 31, hh = lane_ >> 5;
     const bf16x8* qp = (const bf16x8*)qbuf + lane_;
@@ -1040,9 +1061,14 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       __builtin_amdgcn_sched_barrier(0);
     }
     fetch_weights(sc, n);
+    dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
 #pragma unroll
     for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
     __builtin_amdgcn_sched_barrier(0);
+    if (kEarly) {
+      hand_on();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if constexpr (XP == 3) {
       // (values and weights would take as long to split)
 #pragma unroll
@@ -1075,14 +1101,15 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         for (int i = 0; i < 16; ++i) few |= below(S[t][i], kSmall);
     }
     if (__builtin_expect(odd || (XP == 1 && apart) || __any(fin != 0.f || few), 0)) {
-      // an operand that does not split, or is not finite: the fp32 products
+      // an operand that does not split, or is not finite: the fp32 products (queries from memory)
+      const bf16x8* qg = (const bf16x8*)frag_of(c) + fresh(lane);
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[i] = 0.f;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const float4 a = joined(qp, 4 * t + g);
+          const float4 a = joined(qg, 4 * t + g);
           O = mfma(S[t][4 * g], a.x, O);
           O = mfma(S[t][4 * g + 1], a.y, O);
           O = mfma(S[t][4 * g + 2], a.z, O);
@@ -1110,43 +1137,13 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       }
     }
   };
-  values(0);
   if constexpr (FULL) {
-    stage_q(0);
-#pragma unroll 1
-    for (int c = 0; c < chunks; ++c) {
-      const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
-      arrive();                       // the queries are there, the keys before were used
-      take(c);
-      stage_k(c, kbuf);
-      if (c > 0) write(c - 1);
-      akap::bf16x4 zb[kNorm ? 4 : 1];
-      float4 zf[kNorm ? 4 : 1];
+    akap::bf16x4 zb[kNorm ? 4 : 1];
+    float4 zf[kNorm ? 4 : 1];
+    // the head's root mean square: a lane's columns, the other half's, the other waves'
+    auto finish = [&](int c) {
       if (kNorm) {
-        const TY* zr = (const TY*)p.proj + (size_t)(t0 + min(li, n - 1)) * p.proj_stride + p.g_off +
-                       h * V + (wave % VW) * 32 + 4 * hh;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if (sizeof(TY) == 2) zb[g] = *(const akap::bf16x4*)(zr + 8 * g);
-          else zf[g] = *(const float4*)(zr + 8 * g);
-        }
-      }
-      outputs(c);
-      const float* sc = MODE == 0 ? (const float*)(qbuf + (C0 + hw) * 64) : nullptr;
-      const float dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
-      // the head's root mean square: a lane's columns, the other half's, the other waves'
-      float* sq = ssq + (c & 1) * NW * kL;
-      if (kNorm) {
-        float ss = 0.f;
-#pragma unroll
-        for (int s = 0; s < 16; ++s) ss = fmaf(O[s], O[s], ss);
-        ss += __shfl_xor(ss, 32, 64);
-        if (hh == 0) sq[wave * kL + li] = ss;
-      }
-      arrive();                       // the keys are there, the queries were used
-      if (c + 1 < chunks) stage_q(c + 1);
-      advance(kbuf, dend, n);
-      if (kNorm) {
+        const float* sq = ssq + (c & 1) * NW * kL;
         float ss = 0.f;
 #pragma unroll
         for (int w = 0; w < VW; ++w) ss += sq[(hw * VW + w) * kL + li];
@@ -1165,12 +1162,48 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
             O[4 * g + r] = O[4 * g + r] * inv * zv[r] * (1.0f / (1.0f + __expf(-zv[r])));
         }
       }
-    }
-  } else {
-    auto stage = [&](int c, float4* to) {
-      stage_k(c, to);
-      stage_scalars(c, to + C0 * 64);
     };
+#pragma unroll 1
+    for (int c = 0; c < chunks; ++c) {
+      const int t0 = r0 + c * kL, n = min(kL, r1 - t0);
+      arrive();                       // the queries are there, the keys before were used
+      take(c);
+      stage_k(c, kbuf);
+      if (c > 0) {
+        if (kEarly) finish(c - 1);
+        write(c - 1);
+      }
+      if (kNorm) {
+        const TY* zr = (const TY*)p.proj + (size_t)(t0 + min(li, n - 1)) * p.proj_stride + p.g_off +
+                       h * V + (wave % VW) * 32 + 4 * hh;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if (sizeof(TY) == 2) zb[g] = *(const akap::bf16x4*)(zr + 8 * g);
+          else zf[g] = *(const float4*)(zr + 8 * g);
+        }
+      }
+      auto hand_on = [&] {
+        arrive();                     // the keys are there, the queries were used
+        if (c + 1 < chunks) stage_q(c + 1);
+      };
+      outputs(c, hand_on);
+      if (kNorm) {
+        float ss = 0.f;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) ss = fmaf(O[s], O[s], ss);
+        ss += __shfl_xor(ss, 32, 64);
+        if (hh == 0) ssq[(c & 1) * NW * kL + wave * kL + li] = ss;
+      }
+      if (!kEarly) hand_on();
+      advance(kbuf, dend, n);
+      if (!kEarly) finish(c);
+    }
+    if (kEarly) {
+      arrive();
+      finish(chunks - 1);
+    }
+    write(chunks - 1);
+  } else {
     // (now and next are restrict so that the reads of one buffer are known not to touch the other:
     // else every read would wait for the DMA under way)
     auto step = [&](int c, const float4* __restrict__ now, float4* __restrict__ next) {
@@ -1186,14 +1219,12 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       judge();
       advance(now, dend, n);
     };
-    stage(0, qbuf);
 #pragma unroll 1
     for (int c = 0; c < chunks; c += 2) {
       step(c, qbuf, kbuf);
       if (c + 1 < chunks) step(c + 1, kbuf, qbuf);
     }
   }
-  if (FULL) write(chunks - 1);
   if (FULL && cut) return;   // the slots were written when the segments were joined
   // (addresses formed anew: kept since the state was read they would take the loop's registers)
   const uint32_t first_at = fresh(MODE == 0 ? 4 * hh * V + col : col * N + 4 * hh);
@@ -1220,9 +1251,9 @@ __global__ __launch_bounds__(256) void chunk_join_kernel(const ChunkScanParams p
   const int b = blockIdx.x, h = blockIdx.y;
   const size_t hs = (size_t)p.V * p.N;
   const size_t e = ((size_t)blockIdx.z * 256 + threadIdx.x) * 4;
-  const int r0 = p.q_start[b], r1 = p.q_start[b + 1];
+  const int r0 = ((ScalarInts)p.q_start)[b], r1 = ((ScalarInts)p.q_start)[b + 1];
   if (r1 <= r0 || walked_whole(p, r1 - r0) || e >= hs) return;
-  const int slot = p.seq_slot[r0];
+  const int slot = slot_of(p, r0);
   if (!live_slot(p, slot)) return;
   const int nseg = (r1 - r0 + p.PIECE - 1) / p.PIECE;
   const size_t sb = seg_base(p, b);
