@@ -710,10 +710,13 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   static_assert(NW == 4 || (NW == 8 && GL), "the register-staged path assumes 256 threads");
   static_assert(!STAG || (NW == 8 && GL), "the ping-pong pairs waves w and w + 4");
   static_assert(TEAMS == 1 || (GL && !STAG && NW == 4), "teams");
-  // [buf][K | V][64 keys * 128 dims] bf16 = 64 KiB (96 KiB with STAG) + the block ids of the
+  // [buf][K | V][64 keys * 128 dims] bf16 = 64 KiB (96 KiB with STAG), room for those of 256 q rows that
+  // the buffers behind the first do not take, + the block ids of the
   // first kFaBtCache 32-key chunks; ONE __shared__ object (a second one makes hipcc drain vmcnt)
-  __shared__ __attribute__((aligned(16))) bf16 lds_all[TEAMS * NBUF * 2 * kFaKeys * kD + 2 * kFaBtCache];
-  int* bt_s = reinterpret_cast<int*>(lds_all + TEAMS * NBUF * 2 * kFaKeys * kD);
+  constexpr int kBuf = 2 * kFaKeys * kD;
+  constexpr int kMore = ROWS * kD > (NBUF - 1) * kBuf ? ROWS * kD - (NBUF - 1) * kBuf : 0;
+  __shared__ __attribute__((aligned(16))) bf16 lds_all[TEAMS * NBUF * kBuf + kMore + 2 * kFaBtCache];
+  int* bt_s = reinterpret_cast<int*>(lds_all + TEAMS * NBUF * kBuf + kMore);
   // One flat grid of (tile, kv head) items, kv head innermost, dispatched back to front: the
   // host map is sorted by ascending causal work (scheduler.cpp), so every head of the longest
   // tiles starts first and the grid's tail is made of the shortest ones (longest-first over
@@ -726,11 +729,20 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   const int tile = TEAMS > 1 ? item / subs : item;
   const int tid = TEAMS > 1 ? (int)threadIdx.x & (NT - 1) : (int)threadIdx.x;   // in the team
   const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT) : 0;
-  bf16* const lds = lds_all + team * NBUF * 2 * kFaKeys * kD;
+  bf16* const lds = lds_all + team * NBUF * kBuf;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
   const int r = lane & 31;
   const int h = lane >> 5;
+  // the q norm's weights, for the wave in fp32 in LDS: asked for first, while the item is looked up
+  const bool prep = p.qkv != nullptr, qn = prep && p.q_w != nullptr;
+  float* const w_s = GL ? reinterpret_cast<float*>(bt_s) + (team * NW + w) * kD
+                        : reinterpret_cast<float*>(lds) + w * kD;
+  bf16 wq[2] = {};
+  if (qn) {
+    wq[0] = p.q_w[2 * lane];
+    wq[1] = p.q_w[2 * lane + 1];
+  }
   const int seq = __builtin_amdgcn_readfirstlane(p.tile_seq[tile]);  // scalar: bt is uniform
   const int q0 = p.q_start[seq];
   const int q_len = p.q_start[seq + 1] - q0;
@@ -745,78 +757,94 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   const int ctx0 = kv_len - q_len;  // keys before this chunk's first query token
   const int limit = valid ? ctx0 + pos : -1;
 
-  // Q^T fragments (B operand): lane (r, h) holds Q[row][16 s + 8 h + j].  Loaded after the
-  // first K/V tile's DMA is issued, so the q round trips (and the fused q prep) overlap it.
+  // Q^T fragments (B operand): lane (r, h) holds Q[row][16 s + 8 h + j].  Requested after the
+  // first K/V tile's DMA is issued, so the q round trips overlap it: the wave's rows whole, four to an
+  // instruction, into the buffers behind the first (16-B column c of a row at c ^ (row & 15)), and read
+  // from there.  (A lane that loads its own columns takes 32 bytes of 32 lines in each of eight
+  // instructions.)  Short prompts see few key tiles, and what stands before and behind these is much of the
+  // time: of 12.6 thousand rows, 37 prompts, 16 / 8 heads, 40 of 58 us where every workgroup took one tile.
+  // With rows in and out as whole lines and an instruction in three less in the preparation (weights in fp32
+  // from LDS, its norm a branch) 56.4 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
+  // prompts of ~115 61.8 -> 55.8, one of 48 12.4 -> 12.0.
   bf16x8 qf[8];
+  bf16* const q_s = lds + kBuf + w * 32 * kD;
   auto load_q = [&]() {
-  if (p.qkv != nullptr) {
-    // fused q prep (the standalone qk_norm_rope_cache pass then skips these tokens' q heads):
-    // the raw q row straight from the QKV projection, per-head RMSNorm over the lane pair
-    // (r, r + 32) that holds its 128 dims (one v_permlane32_swap), bf16-rounded like the
-    // standalone kernel, then NeoX rotary -- dims d < 64 (s8 < 4) pair with d + 64 (s8 + 4)
-    // in the same lane, so the rotation is lane-local.  Same arithmetic as rope_cache.hip
-    // qk_tok.
-    const int tok = q0 + (valid ? pos : 0);
-    const bf16* src = p.qkv + (size_t)tok * p.qkv_stride + (size_t)(kvh * G + hig) * kD + 8 * h;
-    // rotary position = the token's key index ctx0 + pos -- the invariant the causal limit
-    // above already relies on (positions[tok] holds the same value): no dependent load
-    const float* cs = p.cos_sin + (size_t)(valid ? ctx0 + pos : 0) * kD + 8 * h;
-    // every operand load issued up front, unconditionally (one round trip; without a q norm
-    // the weight loads read valid rotary-table bytes and are ignored)
-    const bool qn = p.q_w != nullptr;
-    const bf16* wsrc = qn ? p.q_w : reinterpret_cast<const bf16*>(p.cos_sin);
-    bf16x8 raw[8], w8[8];
-    f32x4 cv[4][2], sv[4][2];
+  const bf16* rows = prep ? p.qkv : p.q;
+  const uint32_t stride = prep ? p.qkv_stride : p.Hq * kD;
+  // (aligned the projection's rows are always; a prompt has at most 32768 tokens)
+  const bool whole = ((uintptr_t)rows & 15) == 0 && stride < (1u << 16);
+  const bf16* first = rows + (size_t)q0 * stride + (size_t)kvh * G * kD;   // of the sequence and kv head
+  bf16x8 raw[8];
+  if (whole) {
+    const int mine = (valid ? pos : 0) << 16 | hig;
 #pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) raw[s8] = *reinterpret_cast<const bf16x8*>(src + 16 * s8);
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) {
-      // both 8-dim halves at wave-uniform addresses (scalar loads: 512 B per wave instead of
-      // 8 KB of vector loads of the same 256-B weight row), then the lane's half selected
-      typedef const __attribute__((address_space(4))) bf16x8 cbf16x8;  // constant: s_load
-      const bf16x8 wl = *(cbf16x8*)(size_t)(wsrc + 16 * s8);
-      const bf16x8 wh = *(cbf16x8*)(size_t)(wsrc + 16 * s8 + 8);
-      w8[s8] = h ? wh : wl;
+    for (int i = 0; i < 8; ++i) {
+      const int row = 4 * i + (lane >> 4), at = __shfl(mine, row);
+      const uint32_t off = (((uint32_t)at >> 16) * stride + (at & 0xffff) * kD + ((lane & 15) ^ (row & 15)) * 8) * 2u;
+      fa_glds16(reinterpret_cast<const char*>(first) + off, q_s + i * 4 * kD);
     }
+  }
+  // rotary position = the token's key index ctx0 + pos -- the invariant the causal limit above already
+  // relies on (positions[tok] holds the same value): no dependent load
+  f32x4 cv[4][2], sv[4][2];
+  if (prep) {
+    const uint32_t cs = ((valid ? ctx0 + pos : 0) * kD + 8 * h) * 4u;
 #pragma unroll
     for (int s8 = 0; s8 < 4; ++s8)
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        cv[s8][k] = *reinterpret_cast<const f32x4*>(cs + 16 * s8 + 4 * k);
-        sv[s8][k] = *reinterpret_cast<const f32x4*>(cs + 64 + 16 * s8 + 4 * k);
+        const char* at = reinterpret_cast<const char*>(p.cos_sin);
+        cv[s8][k] = *reinterpret_cast<const f32x4*>(at + cs + (16 * s8 + 4 * k) * 4);
+        sv[s8][k] = *reinterpret_cast<const f32x4*>(at + cs + (64 + 16 * s8 + 4 * k) * 4);
       }
+  }
+  if (whole) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8)
+      raw[s8] = *reinterpret_cast<const bf16x8*>(q_s + r * kD + ((2 * s8 + h) ^ (r & 15)) * 8);
+  } else {
+    const bf16* mine = first + (size_t)(valid ? pos : 0) * stride + hig * kD + 8 * h;
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) raw[s8] = *reinterpret_cast<const bf16x8*>(mine + 16 * s8);
+  }
+  // (rows that are not valid hold those of the sequence's first token; they are not stored)
+  if (!prep) {
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) qf[s8] = raw[s8];
+    return;
+  }
+  // fused q prep (the standalone qk_norm_rope_cache pass then skips these tokens' q heads): per-head RMSNorm
+  // over the lane pair (r, r + 32) that holds the row's 128 dims (one v_permlane32_swap), bf16-rounded like
+  // the standalone kernel, then NeoX rotary -- dims d < 64 (s8 < 4) pair with d + 64 (s8 + 4) in the same
+  // lane, so the rotation is lane-local.  Same arithmetic as rope_cache.hip qk_tok.
+  if (qn) {
     float ss = 0.f;
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8)
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss += bf2f(raw[s8][j]) * bf2f(raw[s8][j]);
     const float inv = rsqrtf(xor32_sum(ss) / (float)kD + p.eps);
-    // normed value of dim (s8, j), bf16-rounded like the standalone kernel (raw without a norm)
-    auto xn = [&](int s8, int j) {
-      const float v = bf2f(raw[s8][j]);
-      return qn ? bf2f(f2bf(v * inv * bf2f(w8[s8][j]))) : v;
-    };
 #pragma unroll
-    for (int s8 = 0; s8 < 4; ++s8) {
-      bf16x8 lo, hi;
+    for (int s8 = 0; s8 < 8; ++s8) {
+      const f32x4 wa = *reinterpret_cast<const f32x4*>(w_s + 16 * s8 + 8 * h);
+      const f32x4 wb = *reinterpret_cast<const f32x4*>(w_s + 16 * s8 + 8 * h + 4);
+      float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float c = cv[s8][j >> 2][j & 3], sn = sv[s8][j >> 2][j & 3];
-        const float x1 = xn(s8, j), x2 = xn(s8 + 4, j);
-        lo[j] = f2bf(x1 * c + -1.f * x2 * sn);
-        hi[j] = f2bf(x2 * c + 1.f * x1 * sn);
-      }
-      const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-      qf[s8] = valid ? lo : z;
-      qf[s8 + 4] = valid ? hi : z;
+      for (int j = 0; j < 8; ++j) v[j] = bf2f(raw[s8][j]) * inv * (j < 4 ? wa[j & 3] : wb[j & 3]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) raw[s8][j] = f2bf(v[j]);
     }
-  } else {
-    const bf16* qrow = p.q + ((size_t)(q0 + (valid ? pos : 0)) * p.Hq + kvh * G + hig) * kD;
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8)
-      qf[s8] = valid ? *reinterpret_cast<const bf16x8*>(qrow + 16 * s8 + 8 * h)
-                     : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
+#pragma unroll
+  for (int s8 = 0; s8 < 4; ++s8)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float c = cv[s8][j >> 2][j & 3], sn = sv[s8][j >> 2][j & 3];
+      const float x1 = bf2f(raw[s8][j]), x2 = bf2f(raw[s8 + 4][j]);
+      qf[s8][j] = f2bf(x1 * c + -1.f * x2 * sn);
+      qf[s8 + 4][j] = f2bf(x2 * c + 1.f * x1 * sn);
+    }
   };
 
   const int wg_last_pos = min(q_len - 1, (row0 + ROWS - 1) / G);
@@ -919,8 +947,13 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   };
 
   int blk_next = 0;
+  const int blk_first = GL ? blk_of(team) : 0;
+  if (qn) {
+    w_s[2 * lane] = bf2f(wq[0]);
+    w_s[2 * lane + 1] = bf2f(wq[1]);
+  }
   if constexpr (GL) {
-    stage_glds(team, 0, blk_of(team));
+    stage_glds(team, 0, blk_first);
     blk_next = blk_of(team + teams);
     load_q();
   } else {
@@ -1146,14 +1179,19 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // O^T accumulator of lane (r, h): row r's dims 32 dt + 8 j4 + 4 h + (0..3).  Each pair of
   // 8-dim groups (j4 = 2 kp, 2 kp + 1) is exchanged between the lane halves with two
   // v_permlane32_swap, after which lane r holds dims 16 kp + 0..7 and lane r + 32 dims
-  // 16 kp + 8..15 of the same row: one 16-B store per pair instead of two 8-B stores (the
-  // epilogue is store-issue bound: 18 us of 117 at 32 x 512, profiles/r2_pmc_prefill_v2.md)
+  // 16 kp + 8..15 of the same row.  The wave's rows then go through LDS, 64 dims at a time (16-B column c of
+  // row r at c ^ (r & 7)), and are stored as whole 128-byte lines, eight to an instruction.
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  bf16* orow = p.out + ((size_t)(q0 + (valid ? pos : 0)) * p.Hq + kvh * G + hig) * kD;
+  // (a place that no other wave reads: the buffer of the tile before the last, or the wave's own sums)
+  bf16* o_s = lds_all + w * 66 * 64 * 2;
+  if (TEAMS == 1 || teams == 1) o_s = lds + (STAG ? ntiles % NBUF : ntiles & 1) * kBuf + w * 32 * 64;
+  const int mine = valid ? (q0 + pos) * p.Hq + kvh * G + hig : -1;
+  asm volatile("" ::: "memory");   // (sums of the second team are read from the same place, as another type)
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+  for (int half = 0; half < 2; ++half) {
 #pragma unroll
-    for (int kp = 0; kp < 2; ++kp) {
+    for (int c2 = 0; c2 < 4; ++c2) {
+      const int dt = 2 * half + (c2 >> 1), kp = c2 & 1;
       bf16x4 oa, ob;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1164,9 +1202,16 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
       const auto r0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
       const auto r1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
       const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
-      // every lane takes part in the swaps; only rows of this chunk store
-      if (valid) *reinterpret_cast<u32x4*>(orow + 32 * dt + 16 * kp + 8 * h) = o;
+      *reinterpret_cast<u32x4*>(o_s + r * 64 + ((2 * c2 + h) ^ (r & 7)) * 8) = o;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 8 * i + (lane >> 3), at = __shfl(mine, row);
+      const u32x4 o = *reinterpret_cast<const u32x4*>(o_s + row * 64 + ((lane & 7) ^ (row & 7)) * 8);
+      // every lane takes part in the exchange; only rows of this chunk store
+      if (at >= 0) *reinterpret_cast<u32x4*>(p.out + (size_t)at * kD + 64 * half + (lane & 7) * 8) = o;
+    }
+  }
 }
 
 // Combine split-KV partitions: grid (num_seqs, Hkv), 256 threads = (16 rows x 16 lanes x 8 dims).  Bound by

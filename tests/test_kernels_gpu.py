@@ -141,6 +141,24 @@ def test_paged_attention_prefill(bs, hq, hkv, tile_rows):
     _close(out, exp, atol=2e-2, rtol=2e-2)
 
 
+# query rows that the kernel cannot take whole (not on 16 bytes) are read column by column: the same bits;
+# groups of more heads than a tile has rows between two of its waves
+@pytest.mark.parametrize("hq,hkv,tile_rows", [(16, 8, 128), (64, 1, 128), (24, 8, 256), (64, 2, 256)])
+def test_paged_attention_prefill_unaligned_rows(hq, hkv, tile_rows):
+    seqs = [(1, 1), (37, 37), (129, 64), (600, 590)]
+    q, kc, vc, bt, sl, qs = _setup_attn(seqs, hq, hkv, 32, seed=hq)
+    scale = 1 / math.sqrt(128)
+    ts, tr = _tiles(seqs, hq // hkv, tile_rows)
+    args = [t.to(DEV) for t in (kc, vc, bt, sl, qs, ts, tr)]
+    exp, out = (torch.empty(q.shape, dtype=q.dtype, device=DEV) for _ in range(2))
+    ops.paged_attention_prefill(exp, q.to(DEV), *args, hq // hkv, scale, tile_rows=tile_rows)
+    _close(exp, ref.paged_attention(q, kc, vc, bt, sl, qs, scale), atol=2e-2, rtol=2e-2)
+    odd = torch.empty(q.numel() + 1, dtype=q.dtype, device=DEV)[1:].view(q.shape).copy_(q)
+    assert odd.data_ptr() % 16 == 2
+    ops.paged_attention_prefill(out, odd, *args, hq // hkv, scale, tile_rows=tile_rows)
+    assert torch.equal(out, exp)
+
+
 # two teams of waves at the number of key tiles from which they share them (8 and 9, odd and even), and a
 # grid too large for them
 @pytest.mark.parametrize("hq,hkv,seqs", [(16, 8, [(512, 512), (513, 130), (576, 64), (1100, 900)]),
