@@ -794,41 +794,42 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
     part[1] = pair(r0, r1);
     part[2] = pair(r0 - lower(part[1]), r1 - upper(part[1]));
   };
+  // (in twelve pieces, which stand between products)
+  auto weigh_four = [&](int g) __attribute__((always_inline)) {
+    if (g == 0) wr = Range{};
+    const float f[4] = {w4[MODE == 0 ? g : 0].x, w4[MODE == 0 ? g : 0].y, w4[MODE == 0 ? g : 0].z,
+                        w4[MODE == 0 ? g : 0].w};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float v = MODE == 0 ? x[4 * g + r] * f[r] : x[4 * g + r];
+      xw[4 * g + r] = v;
+      if (MODE == 0) wr.hi = __builtin_elementwise_maximum(wr.hi, fabsf(v));
+      else wr.add(v);
+    }
+  };
+  u32x4 wp[3];
+  auto weigh_pair = [&](int m, int i) __attribute__((always_inline)) {
+    // (parts of the unrounded product)
+    const int at = 8 * m + 2 * i;
+    const float* f = MODE == 0 ? &w4[MODE == 0 ? at >> 2 : 0].x + (at & 3) : nullptr;
+    wp[0][i] = pair(xw[at], xw[at + 1]);
+    if (XP == 3) {
+      const float r = fmaf(x[at], MODE == 0 ? f[0] : 1.f, -lower(wp[0][i]));
+      const float s = fmaf(x[at + 1], MODE == 0 ? f[1] : 1.f, -upper(wp[0][i]));
+      wp[1][i] = pair(r, s);
+      wp[2][i] = pair(r - lower(wp[1][i]), s - upper(wp[1][i]));
+    }
+    if (i < 3) return;
+#pragma unroll
+    for (int u = 0; u < XP; ++u) w[m][u] = __builtin_bit_cast(bf16x8, wp[u]);
+#pragma unroll
+    for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
+  };
   auto weigh = [&] {
-    wr = Range{};
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float f[4] = {w4[MODE == 0 ? g : 0].x, w4[MODE == 0 ? g : 0].y, w4[MODE == 0 ? g : 0].z,
-                          w4[MODE == 0 ? g : 0].w};
+    for (int g = 0; g < 4; ++g) weigh_four(g);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = MODE == 0 ? x[4 * g + r] * f[r] : x[4 * g + r];
-        xw[4 * g + r] = v;
-        if (MODE == 0) wr.hi = __builtin_elementwise_maximum(wr.hi, fabsf(v));
-        else wr.add(v);
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      // (parts of the unrounded product)
-      u32x4 part[3];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int at = 8 * m + 2 * i;
-        const float* f = MODE == 0 ? &w4[MODE == 0 ? at >> 2 : 0].x + (at & 3) : nullptr;
-        part[0][i] = pair(xw[at], xw[at + 1]);
-        if (XP == 3) {
-          const float r = fmaf(x[at], MODE == 0 ? f[0] : 1.f, -lower(part[0][i]));
-          const float s = fmaf(x[at + 1], MODE == 0 ? f[1] : 1.f, -upper(part[0][i]));
-          part[1][i] = pair(r, s);
-          part[2][i] = pair(r - lower(part[1][i]), s - upper(part[1][i]));
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < XP; ++u) w[m][u] = __builtin_bit_cast(bf16x8, part[u]);
-#pragma unroll
-      for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w[m][u]));   // (formed here, beside products)
-    }
+    for (int i = 0; i < 8; ++i) weigh_pair(i >> 2, i & 3);
     if constexpr (HALF) {
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
@@ -936,9 +937,13 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       for (int i = 0; i < 3; ++i)
         if (i == 0 || u < XQ) k[u & 1][i] = kp[(u + i * NQ) * 64];
     };
+    // (of a factor that the compiler knows nothing about: else all of them, common to both ways through here,
+    // stand ahead of the branch and not between the products)
+    float by = dend;
+    asm volatile("" : "+v"(by));
     auto decay = [&](int t) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) S[t][i] *= dend;
+      for (int i = 0; i < 16; ++i) S[t][i] *= by;
     };
     fetch(0);
     decay(0);
@@ -1037,12 +1042,14 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       split8(v, a[j & 1][0], a[j & 1][1], a[j & 1][2]);
     };
     constexpr int PG = NQ / 4;        // steps per group of pairs
+    constexpr bool kEarlyWeights = XP == 3 && PG > 1;
     fetch_pairs(0);
     state_parts(0);
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
       if (j + 1 < NQ) fetch(j + 1);
       if (PG == 1 ? j > 0 : j % PG == 1 && j + 1 < NQ) fetch_pairs(PG == 1 ? j : j / PG + 1);
+      if (kEarlyWeights && j + 2 == NQ) fetch_weights(sc, n);
       __builtin_amdgcn_sched_barrier(0);
       if (j < XQ) {
         mfma_split(a[j & 1], q[j & 1], O, O2);
@@ -1052,7 +1059,11 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         O2 = mfma16(a[j & 1][1], q[j & 1][0], O2);
       }
       if (j + 1 < NQ) state_parts(j + 1);
-      if (j % PG == 0) {
+      if (kEarlyWeights && j + 1 == NQ) {   // (their factors were asked for a step before)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) weigh_four(g);
+        interleave<6, 6>();
+      } else if (j % PG == 0) {
         pair_weights(j / PG);
         if (j < XQ) interleave<6, MODE == 0 ? 18 : 12>(); else interleave<3, 24>();
       } else {
@@ -1060,7 +1071,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    fetch_weights(sc, n);
+    if (!kEarlyWeights) fetch_weights(sc, n);
     dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
 #pragma unroll
     for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
@@ -1070,12 +1081,15 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (XP == 3) {
-      // (values and weights would take as long to split)
+      // (Values and weights would take as long to split.  The pieces are set between the products by hand: asked
+      // to, the compiler left all of them behind the last, 8 x 2048 rows, 64 heads 525 -> 520 us with the decays.)
 #pragma unroll
-      for (int s = 0; s < 16; ++s) O = mfma(x[s], P[s], O);
-      weigh();
-      interleave<16, 9>();
-      __builtin_amdgcn_sched_barrier(0);
+      for (int s = 0; s < 16; ++s) {
+        O = mfma(x[s], P[s], O);
+        if (s < 4 && !kEarlyWeights) weigh_four(s);
+        if (s >= 4 && s < 12) weigh_pair((s - 4) >> 2, s & 3);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       judge();
     } else {
 #pragma unroll
