@@ -419,6 +419,82 @@ __device__ __forceinline__ void deferred_kv_stores(const AttnParams& p, int kvh,
 // the caches leaves the L2 / MALL to the block tables, q rows and weights)
 constexpr bool kDecodeNT = true;
 
+// Merge the partitions of a (sequence, kv head): 256 threads = (16 rows x 16 lanes x 8 dims).  Bound by the
+// latency of its reads: eight partitions' maxima, sums and rows are requested together.  SHARED: partitions
+// that other workgroups of the launch wrote past their caches, read past this one's.
+constexpr int kPartSc1 = 16;   // buffer instructions past this XCD's caches
+template <bool SHARED>
+__device__ __forceinline__ float part_load(const float* at) {
+  return SHARED ? __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *at;
+}
+template <bool SHARED>
+__device__ __forceinline__ void merge_parts(const AttnParams& p, int seq, int kvh, int kv_len, int q_tok) {
+  constexpr int U = 8;
+  const int G = p.G;
+  const int row = threadIdx.x >> 4;
+  const int d0 = (threadIdx.x & 15) * 8;
+  if (row >= G) return;
+  const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
+  const size_t base = ((size_t)(seq * p.Hkv + kvh) * p.num_parts) * G + row;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.part_o + ((size_t)(seq * p.Hkv + kvh) * p.num_parts) * G * kD), (short)0,
+      SHARED ? p.num_parts * G * kD * 4 : 0, 0x00020000);
+  float M = -1e30f;
+  float L = 0.f;
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (nparts > 0) {
+    float m[U], l[U];
+    f32x4 o[U][2];
+    auto load = [&](int q0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const size_t idx = base + (size_t)min(q0 + u, nparts - 1) * G;
+        m[u] = part_load<SHARED>(p.part_m + idx);
+        l[u] = part_load<SHARED>(p.part_l + idx);
+        const float* po = p.part_o + idx * kD + d0;
+        if constexpr (SHARED) {
+          const int at = (int)((idx - (base - row)) * kD + d0) * 4;
+          o[u][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, kPartSc1));
+          o[u][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, at + 16, 0, kPartSc1));
+        } else {
+          o[u][0] = reinterpret_cast<const f32x4*>(po)[0];
+          o[u][1] = reinterpret_cast<const f32x4*>(po)[1];
+        }
+      }
+    };
+    load(0);
+    for (int q0 = U; q0 < nparts; q0 += U) {
+      float x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = part_load<SHARED>(p.part_m + base + (size_t)min(q0 + u, nparts - 1) * G);
+#pragma unroll
+      for (int u = 0; u < U; ++u) M = fmaxf(M, x[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) M = fmaxf(M, m[u]);
+    for (int q0 = 0; q0 < nparts; q0 += U) {
+      if (q0 > 0) load(q0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (q0 + u >= nparts) break;
+        const float f = exp2f(m[u] - M) * l[u];
+        L += f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc[j] += f * o[u][0][j];
+          acc[4 + j] += f * o[u][1][j];
+        }
+      }
+    }
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  bf16* op = p.out + ((size_t)q_tok * p.Hq + kvh * G + row) * kD + d0;
+  bf16x8 o8;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o8[j] = f2bf(acc[j] * inv);
+  *reinterpret_cast<bf16x8*>(op) = o8;
+}
+
 // One (seq, kv head, partition) work item of the decode grid.
 //  head: what the item needs before its first K/V byte can be requested -- the sequence's
 //    length, the cache block ids of the wave's chunks (lane j: chunk pstart + 32 w + 128 j,
@@ -454,7 +530,10 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
   const int pend = min(kv_len, pstart + p.part_size);
   // A partition without keys: the reduction reads those with keys alone.  A step is cut for the longest
   // sequence the model allows, so most partitions of short ones are empty.
-  if (p.num_parts > 1 && pstart >= kv_len) return;
+  if (p.num_parts > 1 && pstart >= kv_len) {
+    if (p.tickets != nullptr && part == 0) merge_parts<true>(p, seq, kvh, 0, p.q_start ? p.q_start[seq] : seq);
+    return;
+  }
   ChunkT<F8> cur;
   {
     // issued unconditionally (a wave with no chunk reads block 0, never used): a branch here
@@ -579,7 +658,11 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
   __syncthreads();
   // combine: thread -> (row, 8 dims)
   const int row = threadIdx.x >> 4;
-  const int d0 = (threadIdx.x & 15) * 8;
+  // (with tickets a row whose keys are all in the first partition needs no merge)
+  const bool alone = p.num_parts == 1 || (p.tickets != nullptr && kv_len <= p.part_size);
+  // dims d0 .. + 3 and d0 + d4 .. + 3; partial rows go past the caches in whole lines
+  const bool lines = p.tickets != nullptr && !alone;
+  const int d0 = (threadIdx.x & 15) * (lines ? 4 : 8), d4 = lines ? 64 : 4;
   if (row < G) {
     float M = -1e30f;
 #pragma unroll
@@ -591,10 +674,10 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
       const float f = exp2f(m_s[ww * G + row] - M);
       L += f * l_s[ww * G + row];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] += f * OS(ww, row, d0 + j);
+      for (int j = 0; j < 8; ++j) acc[j] += f * OS(ww, row, d0 + (j >> 2) * d4 + (j & 3));
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    if (p.num_parts == 1) {
+    if (alone) {
       bf16* op = p.out + ((size_t)q_tok * p.Hq + kvh * G + row) * kD + d0;
       bf16x8 o8;
 #pragma unroll
@@ -603,13 +686,49 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
     } else {
       const size_t pidx = ((size_t)(seq * p.Hkv + kvh) * p.num_parts + part) * G + row;
       float* po = p.part_o + pidx * kD + d0;
+      const float mp = L > 0.f ? M : -1e30f;
+      if (p.tickets != nullptr) {       // past this XCD's cache: another's workgroup may read them
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(p.part_o + (((size_t)(seq * p.Hkv + kvh) * p.num_parts + part) * G) * kD), (short)0,
+            G * kD * 4, 0x00020000);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) po[j] = acc[j] * inv;
-      if ((threadIdx.x & 15) == 0) {
-        p.part_m[pidx] = L > 0.f ? M : -1e30f;
-        p.part_l[pidx] = L;
+        for (int u = 0; u < 2; ++u)
+          __builtin_amdgcn_raw_buffer_store_b128(
+              u32x4{__float_as_uint(acc[4 * u] * inv), __float_as_uint(acc[4 * u + 1] * inv),
+                    __float_as_uint(acc[4 * u + 2] * inv), __float_as_uint(acc[4 * u + 3] * inv)},
+              rs, (row * kD + d0 + 64 * u) * 4, 0, kPartSc1);
+        if ((threadIdx.x & 15) == 0) {
+          __hip_atomic_store(p.part_m + pidx, mp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(p.part_l + pidx, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) po[j] = acc[j] * inv;
+        if ((threadIdx.x & 15) == 0) {
+          p.part_m[pidx] = mp;
+          p.part_l[pidx] = L;
+        }
       }
     }
+  }
+  if (p.tickets != nullptr && !alone) {
+    // The last of the row's partitions to get here merges them (a launch and its gap less: one row of 16 / 8 heads
+    // at 900 keys 10.3 -> 8.8 us, at 240, which one partition holds, 10.4 -> 7.7; 60 at ~450 21.2 -> 18.5, 200 at
+    // ~560 83 -> 77, 64 at ~2000 87 either way; with the partial rows stored in pieces of 8 bytes that last one took
+    // 2 us more).  Every wave's stores have been acknowledged
+    // where all XCDs see them before the workgroup takes its ticket, and the last one puts it back
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* flag = reinterpret_cast<int*>(m_s);
+    if (threadIdx.x == 0) {
+      int* ticket = p.tickets + (size_t)(seq * p.Hkv + kvh) * kCtrStride;
+      const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
+      const int last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
+      if (last) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = last;
+    }
+    __syncthreads();
+    if (*flag != 0) merge_parts<true>(p, seq, kvh, kv_len, q_tok);
   }
   if constexpr (FUSED && !F8) {
     if (use_img && p.defer_kv) deferred_kv_stores<F8>(p, kvh, pp, k_img, v_img);
@@ -1214,68 +1333,10 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   }
 }
 
-// Combine split-KV partitions: grid (num_seqs, Hkv), 256 threads = (16 rows x 16 lanes x 8 dims).  Bound by
-// the latency of its reads: eight partitions' maxima, sums and rows are requested together.
+// Combine split-KV partitions: grid (num_seqs, Hkv).
 __global__ __launch_bounds__(256) void paged_attn_reduce_kernel(AttnParams p) {
-  constexpr int U = 8;
   const int seq = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int G = p.G;
-  const int row = threadIdx.x >> 4;
-  const int d0 = (threadIdx.x & 15) * 8;
-  if (row >= G) return;
-  const int kv_len = p.seq_lens[seq];
-  const int q_tok = p.q_start ? p.q_start[seq] : seq;
-  const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
-  const size_t base = ((size_t)(seq * p.Hkv + kvh) * p.num_parts) * G + row;
-  float M = -1e30f;
-  float L = 0.f;
-  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (nparts > 0) {
-    float m[U], l[U];
-    f32x4 o[U][2];
-    auto load = [&](int q0) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const size_t idx = base + (size_t)min(q0 + u, nparts - 1) * G;
-        m[u] = p.part_m[idx];
-        l[u] = p.part_l[idx];
-        const f32x4* po = reinterpret_cast<const f32x4*>(p.part_o + idx * kD + d0);
-        o[u][0] = po[0];
-        o[u][1] = po[1];
-      }
-    };
-    load(0);
-    for (int q0 = U; q0 < nparts; q0 += U) {
-      float x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = p.part_m[base + (size_t)min(q0 + u, nparts - 1) * G];
-#pragma unroll
-      for (int u = 0; u < U; ++u) M = fmaxf(M, x[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) M = fmaxf(M, m[u]);
-    for (int q0 = 0; q0 < nparts; q0 += U) {
-      if (q0 > 0) load(q0);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (q0 + u >= nparts) break;
-        const float f = exp2f(m[u] - M) * l[u];
-        L += f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[j] += f * o[u][0][j];
-          acc[4 + j] += f * o[u][1][j];
-        }
-      }
-    }
-  }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
-  bf16* op = p.out + ((size_t)q_tok * p.Hq + kvh * G + row) * kD + d0;
-  bf16x8 o8;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) o8[j] = f2bf(acc[j] * inv);
-  *reinterpret_cast<bf16x8*>(op) = o8;
+  merge_parts<false>(p, seq, blockIdx.y, p.seq_lens[seq], p.q_start ? p.q_start[seq] : seq);
 }
 
 void launch_paged_attn_prefill(const AttnParams& p, int num_tiles, int tile_rows,
@@ -1330,7 +1391,7 @@ void launch_paged_attn_decode(const AttnParams& p, int num_seqs, hipStream_t s) 
     if (p.qkv != nullptr) paged_attn_decode_kernel<true, false><<<grid, 256, smem, s>>>(q);
     else paged_attn_decode_kernel<false, false><<<grid, 256, smem, s>>>(q);
   }
-  if (p.num_parts > 1) paged_attn_reduce_kernel<<<dim3(num_seqs, p.Hkv), 256, 0, s>>>(q);
+  if (p.num_parts > 1 && p.tickets == nullptr) paged_attn_reduce_kernel<<<dim3(num_seqs, p.Hkv), 256, 0, s>>>(q);
 }
 
 }  // namespace akap

@@ -60,6 +60,7 @@ struct AttnParams {
   float* part_m;  // [B, Hkv, parts, G]
   float* part_l;
   float* part_o;  // [B, Hkv, parts, G, D]
+  int* tickets;   // [B, Hkv] of kCtrStride, zeros between launches (nullptr: merged by a second launch)
   int flags;      // reserved (0)
   int kv_fp8;     // caches hold OCP e4m3fn bytes (scale 1) instead of bf16
   // fused decode (qkv != nullptr): the kernel itself applies per-head q/k RMSNorm + RoPE to

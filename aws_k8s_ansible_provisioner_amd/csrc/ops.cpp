@@ -139,6 +139,19 @@ static void set_v_tail(akap::AttnParams& p, const std::optional<Tensor>& v_tail,
   p.tail_slot = tail_slot->data_ptr<int>();
 }
 
+// Tickets of the in-launch merge of split decode rows: a workspace's own, kCtrStride int32 per (row, kv head),
+// zeros between launches.  Without enough of them, or with partial rows that do not lie on 16 bytes, the
+// partitions are merged by a second launch.
+static void set_tickets(akap::AttnParams& p, const std::optional<Tensor>& tickets, int rows) {
+  p.tickets = nullptr;
+  if (!tickets) return;
+  TORCH_CHECK(tickets->is_cuda() && tickets->scalar_type() == at::kInt && tickets->is_contiguous(),
+              "tickets: contiguous int32 on the GPU");
+  if (tickets->numel() >= (int64_t)rows * p.Hkv * akap::kCtrStride && (uintptr_t)p.part_o % 16 == 0 &&
+      (int64_t)p.num_parts * p.G * 128 * 4 < (1LL << 31))
+    p.tickets = tickets->data_ptr<int>();
+}
+
 akap::AttnParams attn_params(Tensor& out, Tensor& q, Tensor& k_cache, Tensor& v_cache,
                              Tensor& block_tables, Tensor& seq_lens, int64_t G, double scale) {
   CHECK_GPU(q); CHECK_BF16(q); CHECK_CONTIG(q); CHECK_CONTIG(out); CHECK_CONTIG(k_cache);
@@ -242,7 +255,8 @@ void paged_attention_decode(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache
                             Tensor block_tables, Tensor seq_lens, std::optional<Tensor> q_start,
                             Tensor part_m, Tensor part_l, Tensor part_o, int64_t num_parts,
                             int64_t part_size, int64_t G, double scale,
-                            std::optional<Tensor> v_tail, std::optional<Tensor> tail_slot) {
+                            std::optional<Tensor> v_tail, std::optional<Tensor> tail_slot,
+                            std::optional<Tensor> tickets) {
   auto p = attn_params(out, q, k_cache, v_cache, block_tables, seq_lens, G, scale);
   TORCH_CHECK(G <= 16, "decode kernel supports up to 16 q heads per kv head");
   set_v_tail(p, v_tail, tail_slot, seq_lens.numel());
@@ -259,6 +273,7 @@ void paged_attention_decode(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache
     p.part_m = part_m.data_ptr<float>();
     p.part_l = part_l.data_ptr<float>();
     p.part_o = part_o.data_ptr<float>();
+    set_tickets(p, tickets, B);
   }
   const c10::DeviceGuard g(q.device());
   akap::launch_paged_attn_decode(p, B, cur_stream());
@@ -273,7 +288,7 @@ void paged_attention_decode_fused(Tensor out, Tensor qkv, Tensor k_cache, Tensor
                                   std::optional<Tensor> k_w, Tensor part_m, Tensor part_l,
                                   Tensor part_o, int64_t num_parts, int64_t part_size, int64_t G,
                                   double scale, double eps, std::optional<Tensor> v_tail,
-                                  std::optional<Tensor> tail_slot) {
+                                  std::optional<Tensor> tail_slot, std::optional<Tensor> tickets) {
   auto p = attn_params(out, out, k_cache, v_cache, block_tables, seq_lens, G, scale);
   set_v_tail(p, v_tail, tail_slot, seq_lens.numel());
   CHECK_GPU(qkv); CHECK_BF16(qkv); CHECK_LAST_CONTIG(qkv);
@@ -305,6 +320,7 @@ void paged_attention_decode_fused(Tensor out, Tensor qkv, Tensor k_cache, Tensor
     p.part_m = part_m.data_ptr<float>();
     p.part_l = part_l.data_ptr<float>();
     p.part_o = part_o.data_ptr<float>();
+    set_tickets(p, tickets, B);
   }
   const c10::DeviceGuard g(qkv.device());
   akap::launch_paged_attn_decode(p, B, cur_stream());
@@ -1316,13 +1332,13 @@ TORCH_LIBRARY(akap, m) {
       "paged_attention_decode(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, "
       "Tensor block_tables, Tensor seq_lens, Tensor? q_start, Tensor(b!) part_m, Tensor(c!) part_l, "
       "Tensor(d!) part_o, int num_parts, int part_size, int G, float scale, "
-      "Tensor? v_tail=None, Tensor? tail_slot=None) -> ()");
+      "Tensor? v_tail=None, Tensor? tail_slot=None, Tensor(e!)? tickets=None) -> ()");
   m.def(
       "paged_attention_decode_fused(Tensor(a!) out, Tensor qkv, Tensor(b!) k_cache, "
       "Tensor(c!) v_cache, Tensor block_tables, Tensor seq_lens, Tensor positions, Tensor slots, "
       "Tensor cos_sin, Tensor? q_w, Tensor? k_w, Tensor(d!) part_m, Tensor(e!) part_l, "
       "Tensor(f!) part_o, int num_parts, int part_size, int G, float scale, float eps, "
-      "Tensor(g!)? v_tail=None, Tensor? tail_slot=None) -> ()");
+      "Tensor(g!)? v_tail=None, Tensor? tail_slot=None, Tensor(h!)? tickets=None) -> ()");
   m.def(
       "sample(Tensor logits, Tensor temperature, Tensor top_k, Tensor top_p, Tensor seeds, "
       "Tensor steps, Tensor(a!) out_tokens, Tensor(b!) out_logprobs, "

@@ -218,12 +218,13 @@ def paged_attention_decode(out, q, k_cache, v_cache, block_tables, seq_lens, gqa
         if workspace is None:
             B = seq_lens.numel()
             Hkv = k_cache.shape[1]
-            workspace = decode_workspace(B, Hkv, gqa_group, num_parts, q.device)
+            workspace = _decode_workspace(B, Hkv, gqa_group, num_parts, q.device)
         pm, pl, po = workspace
         torch.ops.akap.paged_attention_decode(out, q, k_cache, v_cache, block_tables, seq_lens,
                                               q_start, pm, pl, po, num_parts, part_size,
                                               gqa_group, scale, v_tail,
-                                              tail_slot if v_tail is not None else None)
+                                              tail_slot if v_tail is not None else None,
+                                              getattr(workspace, "tickets", None))
         return out
     if q_start is None:
         q_start = torch.arange(seq_lens.numel() + 1, dtype=torch.int32)
@@ -241,14 +242,15 @@ def paged_attention_decode_fused(out, qkv, k_cache, v_cache, block_tables, seq_l
     goes to its sequence's tail row and the cache gets whole 8-token groups only."""
     if _native(qkv):
         if workspace is None:
-            workspace = decode_workspace(seq_lens.numel(), k_cache.shape[1], gqa_group,
-                                         num_parts, qkv.device)
+            workspace = _decode_workspace(seq_lens.numel(), k_cache.shape[1], gqa_group,
+                                          num_parts, qkv.device)
         pm, pl, po = workspace
         torch.ops.akap.paged_attention_decode_fused(out, qkv, k_cache, v_cache, block_tables,
                                                     seq_lens, positions, slots, cos_sin, q_w, k_w,
                                                     pm, pl, po, num_parts, part_size, gqa_group,
                                                     scale, eps, v_tail,
-                                                    tail_slot if v_tail is not None else None)
+                                                    tail_slot if v_tail is not None else None,
+                                                    getattr(workspace, "tickets", None))
         return out
     B, Hq = out.shape[0], out.shape[1]
     q = torch.empty_like(out)
@@ -259,8 +261,29 @@ def paged_attention_decode_fused(out, qkv, k_cache, v_cache, block_tables, seq_l
     return out
 
 
+class DecodeWorkspace(tuple):
+    """(part_m, part_l, part_o) of a split decode step, and the tickets that merge its partitions
+    within the launch (zeros between launches; None: merged by a second one).  One step at a time
+    may use it, as ever."""
+
+    tickets = None
+
+
 def decode_workspace(max_seqs: int, num_kv_heads: int, gqa_group: int, num_parts: int,
                      device) -> tuple:
+    ws = DecodeWorkspace(_decode_workspace(max_seqs, num_kv_heads, gqa_group, num_parts, device))
+    if num_parts > 1 and torch.device(device).type == "cuda":
+        ws.tickets = torch.zeros(max(1, max_seqs * num_kv_heads) * DECODE_TICKET_INTS,
+                                 dtype=torch.int32, device=device)
+    return ws
+
+
+# int32 of a (row, kv head)'s ticket, a cache line of its own (csrc/kernels/kernels.h kCtrStride)
+DECODE_TICKET_INTS = 32
+
+
+def _decode_workspace(max_seqs: int, num_kv_heads: int, gqa_group: int, num_parts: int,
+                      device) -> tuple:
     n = max(1, max_seqs * num_kv_heads * max(num_parts, 1) * gqa_group)
     pm = torch.empty(n, dtype=torch.float32, device=device)
     pl = torch.empty(n, dtype=torch.float32, device=device)

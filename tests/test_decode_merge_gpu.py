@@ -129,3 +129,39 @@ def test_paged_attention(part_size, parts, G):
     ops.paged_attention_decode(mag, q, k, v.abs(), bt, sl, G, D ** -0.5, part_size=2304)
     assert bool(((got - want).abs() <= 2.0 ** -8 * (1.02 * mag.float() + want.abs())).all())
     assert (got - want).norm() <= 6e-3 * want.norm()      # independent roundings, as above
+
+
+@pytest.mark.parametrize("part_size,parts,G", [(128, 18, 2), (256, 9, 4), (1024, 3, 1), (768, 2, 16)])
+def test_paged_attention_tickets(part_size, parts, G):
+    """The merge within the launch: the values of the second launch (a workspace without tickets) but for
+    the order of one fp32 product, so at most one bf16 step apart; tickets that are zeros again after every
+    launch; and the same bits from every replay of a captured step, whoever comes last."""
+    from aws_k8s_ansible_provisioner_amd import ops
+
+    g = torch.Generator().manual_seed(parts)
+    bt, sl, NB = _table(g)
+    H, D, T, bf = 3, 128, len(LENS), torch.bfloat16
+    k = torch.randn(NB, H, BS, D, generator=g).to(bf).cuda()
+    v = torch.randn(NB, H, BS // 8, D, 8, generator=g).to(bf).cuda()
+    q = torch.randn(T, H * G, D, generator=g).to(bf).cuda()
+    bt, sl = bt.cuda(), sl.cuda()
+    want, got = (torch.full((T, H * G, D), 7.0, dtype=bf, device="cuda") for _ in range(2))
+    ws = ops.decode_workspace(T, H, G, parts, "cuda")
+    ops.paged_attention_decode(want, q, k, v, bt, sl, G, D ** -0.5, tuple(ws), parts, part_size)
+
+    def step():
+        ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, ws, parts, part_size)
+
+    step()
+    assert not bool(ws.tickets.any())
+    d = (got.float() - want.float()).abs()
+    assert bool((d <= 2.0 ** -7 * want.float().abs()).all())
+    first = got.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for _ in range(4):
+        got.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, first) and not bool(ws.tickets.any())
