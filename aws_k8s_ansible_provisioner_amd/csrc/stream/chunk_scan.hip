@@ -24,10 +24,11 @@
 // 16 j + 4 hh + 0..3 and 16 j + 8 + 4 hh + 0..3) eight neighbouring registers are an operand of the next
 // product, so the state, the values and the outputs feed each other without lane traffic.
 //
-// Bound by vector work (1000 instructions per chunk, half of them the state's parts, 5.1 cycles each where a wave
-// has its SIMD alone) and products (4100 cycles per chunk); the next step's parts are formed between a step's
-// products.  That is 9200 of the 11850 cycles a chunk takes (8 sequences of 64 heads, a wave per SIMD); what the
-// rest goes into is not known.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 335 us
+// Bound by vector work (900 instructions per chunk, half of them the state's parts) and products (4100 cycles per
+// chunk); the next step's parts are formed between a step's products.  Of the 11200 cycles a chunk takes (8
+// sequences of 64 heads, a wave per SIMD) 5100 issue, 4000 wait to issue, most of them behind products with nothing
+// beside them (the state's own), 2000 wait for LDS, memory and barriers, of which fragments asked for a chunk
+// earlier took none away.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 330 us
 // where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
 // 128 x 128 (segments) 76 + 33 for the pass before it, and 57 for the fragments: all three wait much for
 // memory, and with entries of one part (HALF) 148 MB of fragments are written and 215 read, of 215 and 316
