@@ -853,15 +853,13 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
   const int r = lane & 31;
   const int h = lane >> 5;
-  // the q norm's weights, for the wave in fp32 in LDS: asked for first, while the item is looked up
+  // the q norm's weights (dims 16 s + 8 h + 0..7): asked for first, while the item is looked up
   const bool prep = p.qkv != nullptr, qn = prep && p.q_w != nullptr;
-  float* const w_s = GL ? reinterpret_cast<float*>(bt_s) + (team * NW + w) * kD
-                        : reinterpret_cast<float*>(lds) + w * kD;
-  bf16 wq[2] = {};
-  if (qn) {
-    wq[0] = p.q_w[2 * lane];
-    wq[1] = p.q_w[2 * lane + 1];
-  }
+  // (without a branch, behind which they would be waited for: where there are none, some bytes of the cache)
+  const bf16* wsrc = qn ? p.q_w : static_cast<const bf16*>(p.k_cache);
+  bf16x8 wq[8];
+#pragma unroll
+  for (int s8 = 0; s8 < 8; ++s8) wq[s8] = *reinterpret_cast<const bf16x8*>(wsrc + 16 * s8 + 8 * (lane >> 5));
   const int seq = __builtin_amdgcn_readfirstlane(p.tile_seq[tile]);  // scalar: bt is uniform
   const int q0 = p.q_start[seq];
   const int q_len = p.q_start[seq + 1] - q0;
@@ -882,8 +880,8 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // from there.  (A lane that loads its own columns takes 32 bytes of 32 lines in each of eight
   // instructions.)  Short prompts see few key tiles, and what stands before and behind these is much of the
   // time: of 12.6 thousand rows, 37 prompts, 16 / 8 heads, 40 of 58 us where every workgroup took one tile.
-  // With rows in and out as whole lines and an instruction in three less in the preparation (weights in fp32
-  // from LDS, its norm a branch) 56.4 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
+  // With rows in and out as whole lines and an instruction in four less in the preparation (its norm a branch,
+  // its weights a lane's own loads) 56 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
   // prompts of ~115 61.8 -> 55.8, one of 48 12.4 -> 12.0.
   bf16x8 qf[8];
   bf16* const q_s = lds + kBuf + w * 32 * kD;
@@ -946,11 +944,9 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
     const float inv = rsqrtf(xor32_sum(ss) / (float)kD + p.eps);
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8) {
-      const f32x4 wa = *reinterpret_cast<const f32x4*>(w_s + 16 * s8 + 8 * h);
-      const f32x4 wb = *reinterpret_cast<const f32x4*>(w_s + 16 * s8 + 8 * h + 4);
       float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = bf2f(raw[s8][j]) * inv * (j < 4 ? wa[j & 3] : wb[j & 3]);
+      for (int j = 0; j < 8; ++j) v[j] = bf2f(raw[s8][j]) * inv * bf2f(wq[s8][j]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) raw[s8][j] = f2bf(v[j]);
     }
@@ -1067,10 +1063,6 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
 
   int blk_next = 0;
   const int blk_first = GL ? blk_of(team) : 0;
-  if (qn) {
-    w_s[2 * lane] = bf2f(wq[0]);
-    w_s[2 * lane + 1] = bf2f(wq[1]);
-  }
   if constexpr (GL) {
     stage_glds(team, 0, blk_first);
     blk_next = blk_of(team + teams);
