@@ -190,6 +190,14 @@ __device__ __forceinline__ float decay_pow(float l2, int k) {
   return k == 0 ? 1.0f : exp2f(l2 * (float)k);
 }
 
+// Keys in one bf16 part take the power of two in their weight, exactly, and values the rest of it, 1 to 2 times
+// key_scale(), so that both split however small the weight is.  Keys come kEven smaller and values kEven larger:
+// the power that takes every value of FLT_MIN and more to kSmall.
+constexpr float kEven = 0x1p29f;
+__device__ __forceinline__ int decay_exponent(float l2, int k) {
+  return k == 0 ? 0 : (int)fmaxf(floorf(l2 * (float)k), -512.f);
+}
+
 // a retention's keys times this
 template <int N>
 constexpr float key_scale() { return N == 64 ? 0.125f : 0.08838834764831845f; }
@@ -327,8 +335,8 @@ __device__ __forceinline__ bool live_slot(const ChunkScanParams& p, int slot) {
 // ------------------------------------------------------------------ fragments of q and k
 // HALF: bf16 rows of a retention of which at most half the entries turn.  The other half of the queries' and keys'
 // are bf16 numbers, one part instead of three: 36 of a chunk's 52 KB are written here and read by the walk, 16 of
-// 24 by the pass before it.  These keys come as they are (times kDown; if a value of the chunk does not split,
-// without) and the weights go to the values, in three parts.
+// 24 by the pass before it.  These keys come times the powers of two in their weights (see kEven; if a value of the
+// chunk does not split, as they are) and what is left of the weights goes to the values, in three parts.
 //
 // One workgroup per (chunk, key head).  Buffer of an entry, in pieces of 64 lanes x 16 bytes: [q: 3 parts
 // of N / 16 pieces][k transposed: the same, the scan's times kDown, the retention's times their weights
@@ -343,6 +351,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
   constexpr int kRed = 4096 * sizeof(TR) / 4;
   __shared__ __align__(16) float rows[2 * kL * LS > kRed ? 2 * kL * LS : kRed];
   __shared__ float wt[kL];     // retention: the rows' weights in the state after the chunk
+  __shared__ float wp[HALF ? kL : 1];   // of keys in one part
   float *qs = rows, *ks = rows + kL * LS;
   TR* red = (TR*)rows;
   int r0, r1;
@@ -406,8 +415,12 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
     *(float4*)(ks + i * LS + d) = b4;
   }
   const bool lift = MODE == 1 && lifted(p.log2_decay[kh]);
-  if (MODE == 1 && tid < kL)
-    wt[tid] = tid < n ? decay_pow(p.log2_decay[kh], n - 1 - tid) * (lift ? kLift : 1.f) : 0.f;
+  if (MODE == 1 && tid < kL) {
+    const float l2 = p.log2_decay[kh], by = lift ? kLift : 1.f;
+    const float w = tid < n ? decay_pow(l2, n - 1 - tid) * by : 0.f;
+    wt[tid] = w;
+    if (HALF) wp[tid] = w != 0.f ? __builtin_ldexpf(by / kEven, decay_exponent(l2, n - 1 - tid)) : 0.f;
+  }
   __syncthreads();
   const int li = lane & 31, hh = lane >> 5;
   constexpr int NQ = N / 16, XQ = HALF ? NQ / 2 : NQ;
@@ -425,7 +438,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
     for (int i = 0; i < 8; ++i) {
       const int j = j0 + (i & 3) + 8 * (i >> 2);
       const float k = ks[j * LS + 32 * (f >> 1) + li];
-      v[1][u][i] = MODE == 0 ? k : f < XQ ? k * kscale * wt[j] : k * kDown;
+      v[1][u][i] = MODE == 0 ? k : f < XQ ? k * kscale * wt[j] : k * wp[HALF ? j : 0];
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w)
@@ -440,7 +453,13 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
 #pragma unroll
       for (int u = 0; u < NQ / 4; ++u)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) bad |= below(v[w][u][i], kSmall / scale[w]);
+        for (int i = 0; i < 8; ++i) {
+          const int f = wave + 4 * u, j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
+          bad |= below(v[w][u][i], f < XQ ? kSmall / scale[w] : __FLT_MIN__);
+          // (a key of which nothing is left beside its weight)
+          if (MODE == 1 && w == 1)
+            bad |= v[1][u][i] == 0.f && wt[j] != 0.f && ks[j * LS + 32 * (f >> 1) + li] != 0.f;
+        }
   }
   bad = __syncthreads_or(bad);
   if (!live) return;
@@ -673,14 +692,17 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   const bool lift = MODE == 1 && uniform(lifted(l2));
   // retention: decay^k and decay^(k + 1)
   float* tb = tab + (MODE == 1 ? wave * 2 * kL : 0);
-  // HALF: the weights of a chunk's rows in the state after it, kUp times those of keys as they are, and zeros
+  // HALF: what the values of a chunk's rows take of their weights in the state after it, and zeros
   float* wb = wtab + (HALF ? wave * 2 * kL : 0);
   if (MODE == 1) {
     if (lane < kL) {
       tb[lane] = decay_pow(l2, lane);
       tb[kL + lane] = decay_pow(l2, lane + 1);
     }
-    if (HALF) wb[lane] = lane < kL ? decay_pow(l2, kL - 1 - lane) * (key_scale<N>() * kUp) : 0.f;
+    if (HALF) {
+      const float rest = __builtin_ldexpf(decay_pow(l2, kL - 1 - lane), -decay_exponent(l2, kL - 1 - lane));
+      wb[lane] = lane < kL ? rest * (key_scale<N>() * kEven * (lift ? kSink : 1.f)) : 0.f;
+    }
     if (kNorm) {
       for (int e = tid; e < 1024; e += 64 * NW) {
         const int ln = (e >> 2) & 63, j = 8 * (e >> 8) + 4 * (ln >> 5) + (e & 3), i = ln & 31;
@@ -774,7 +796,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
   // the values times their weights in the state after the chunk (the scan's times kUp; the retention's are
   // in k), and their parts
   float xw[16];
-  bf16x8 w[2][3], wh[HALF ? 2 : 1][3];       // (wh: of values times wb, for keys as they are)
+  bf16x8 w[2][3], wh[HALF ? 2 : 1][3];       // (wh: of values times wb, for keys in one part)
   Range wr;
   float4 w4[MODE == 0 || HALF ? 4 : 1];
   auto fetch_weights = [&](const float* sc, int n) {
@@ -881,39 +903,30 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         for (int i = 0; i < 16; ++i) S[t][i] *= dend;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        float xe[4];       // values of keys as they are
-        if (HALF) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            xe[r] = x[4 * g + r] * (wb[kL - n + 8 * g + 4 * hh + r] * kDown);
-        }
         float up[4];       // undoes the scaling of a key; a lifted() head's values take its weight's exponent
+        float upe[4];      // the same of a key in one part, which takes its own weight's rest besides
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          const float f = HALF || lift ? tb[max(n - 1 - (8 * g + 4 * hh + r), 0)] : 1.f;
           up[r] = MODE == 0 && !odd ? kUp : 1.f;
+          if (HALF) upe[r] = odd ? key_scale<N>() * (lift ? 1.f : f) : wb[kL - n + 8 * g + 4 * hh + r];
           if (lift) {
-            const float f = tb[max(n - 1 - (8 * g + 4 * hh + r), 0)];
             const int e = __builtin_amdgcn_frexp_expf(f);
             xw[4 * g + r] = odd ? xw[4 * g + r] * f : __builtin_ldexpf(xw[4 * g + r], e);
-            if (!odd) up[r] = __builtin_ldexpf(kSink, -e);
+            if (!odd) {
+              up[r] = __builtin_ldexpf(kSink, -e);
+              if (HALF) upe[r] = __builtin_ldexpf(upe[r], -e);
+            }
           }
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const float4 a = joined(kp, 4 * t + g);
-          if (HALF && t >= NT / 2) {
-            const float whole = odd ? 1.f : kUp;
-            S[t] = mfma(a.x * whole, xe[0], S[t]);
-            S[t] = mfma(a.y * whole, xe[1], S[t]);
-            S[t] = mfma(a.z * whole, xe[2], S[t]);
-            S[t] = mfma(a.w * whole, xe[3], S[t]);
-            __builtin_amdgcn_sched_barrier(0);
-            continue;
-          }
-          S[t] = mfma(a.x * up[0], xw[4 * g], S[t]);
-          S[t] = mfma(a.y * up[1], xw[4 * g + 1], S[t]);
-          S[t] = mfma(a.z * up[2], xw[4 * g + 2], S[t]);
-          S[t] = mfma(a.w * up[3], xw[4 * g + 3], S[t]);
+          const float* by = HALF && t >= NT / 2 ? upe : up;
+          S[t] = mfma(a.x * by[0], xw[4 * g], S[t]);
+          S[t] = mfma(a.y * by[1], xw[4 * g + 1], S[t]);
+          S[t] = mfma(a.z * by[2], xw[4 * g + 2], S[t]);
+          S[t] = mfma(a.w * by[3], xw[4 * g + 3], S[t]);
           __builtin_amdgcn_sched_barrier(0);
         }
       }

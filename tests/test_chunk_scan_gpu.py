@@ -586,10 +586,10 @@ def test_few_short_prompts_in_segments(mode, lens, starts):
 @pytest.mark.parametrize("D,V,rot", [(128, 128, 64), (128, 64, 40), (64, 128, 32), (64, 64, 8)])
 @pytest.mark.parametrize("what", ["usual", "small keys", "odd key", "odd query"])
 def test_retention_entries_that_do_not_turn(D, V, rot, what):
-    """bf16 rows of which at most half the entries turn keep the others as they are, with the weights on the
-    values; the same rows in fp32 go the general way.  Keys of 2^-60 and 2^-100 are below what is scaled
-    down exactly, those of 3e38 and the infinite do not split.  Outputs: a rounding to bf16; states: both sides
-    sum in fp32 (module comment)."""
+    """bf16 rows of which at most half the entries turn keep the others in one part, with a power of two of their
+    weights; the same rows in fp32 go the general way.  Keys of 2^-100 are too small for that and infinite ones do
+    not split; those of 2^-60 and of 3e38 do.  Outputs: a rounding to bf16; states: both sides sum in fp32 (module
+    comment)."""
     H, lens, starts = 4, [1, 33, 300, 64], [9, 0, 5, 0]
     T, B = sum(lens), len(lens)
     g = torch.Generator().manual_seed(D + V + rot)
@@ -615,3 +615,60 @@ def test_retention_entries_that_do_not_turn(D, V, rot, what):
         for h in range(H):
             part = (slice(None), slice(h * V, (h + 1) * V)) if a.dim() == 2 else (slice(None), h)
             assert _rel(torch.where(ok, a, 0.)[part], torch.where(ok, b, 0.)[part].cpu()) < limit
+
+
+@pytest.mark.parametrize("what,decay,size", [
+    ("values", 0.42, 1.2e-36), ("values", 0.06, 1.3e-9),
+    ("denormal values", 0.97, 3e-39), ("large values", 0.42, 1e13), ("large values", 0.06, 1e13),
+    ("small keys", 0.42, 1e-25), ("small keys", 0.06, 1e-17), ("odd", 0.42, 1.2e-36)])
+@pytest.mark.parametrize("V", [64, 128])
+@pytest.mark.parametrize("T", [96, 1120])
+def test_retention_small_operands_that_do_not_turn(T, V, what, decay, size):
+    """The oldest row of a chunk of bf16, whose weight in the state is the smallest, with a value or a key of
+    any size, alone in one row of the state of an entry that does not turn, beside a key or a value that makes
+    it count: as exact as the operands in fp32.  (The row form rounds the entry 31 times and has the decay's own
+    rounding 31 times, 3.7e-6 in all; a weight's exponent of up to 126 is rounded to 2^-18, 2.6e-6 of the weight;
+    some roundings of the products besides.)"""
+    H, row, at = 2, T - 32, 3 * V // 4 + 4
+    proj = torch.randn(T, 4 * H * V, generator=torch.Generator().manual_seed(16)).bfloat16()
+    k, v = proj[:, H * V:2 * H * V], proj[:, 2 * H * V:3 * H * V]
+    k[:, at] = 0.0
+    k[row, at], v[row] = (size, v[row] * 1e30) if what == "small keys" else (1e37, v[row] * size)
+    if what == "large values":
+        k[row, at] = 1.0
+    elif what == "odd":
+        k[row + 1, at - 1] = float("inf")
+    args = (_step([T], [0]), H, V, V, (0, H * V, 2 * H * V, 3 * H * V), None,
+            torch.log2(torch.tensor([decay, 0.9])))
+    st = torch.zeros(1, H, V, V)
+    want = _run_retention((proj, st), *args, "cpu")[1][0, 0, :, at]
+    got = _run_retention((proj, st), *args, DEV)[1].cpu()[0, 0, :, at]
+    assert float(want.abs().max()) > 0
+    assert float(((got - want).abs() - 8e-6 * want.abs()).max()) <= 0
+
+
+def test_retention_small_keys_take_no_longer():
+    """Keys that one bf16 part holds do not send a chunk through the fp32 products, however small they are."""
+    H, D, T = 8, 128, 4096
+    g = torch.Generator(device=DEV).manual_seed(1)
+    proj = torch.randn(T, 4 * H * D, device=DEV, generator=g)
+    state, out = torch.randn(4, H, D, D, device=DEV, generator=g), proj.new_empty(T, H * D).bfloat16()
+    q_start, pos, slot = (t.to(DEV) for t in _step([T // 4] * 4, [0] * 4))
+    l2 = torch.full((H,), math.log2(0.97), device=DEV)
+
+    def time(rows):
+        spent = []
+        for _ in range(9):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                sops.retention(out, rows, 0, H * D, 2 * H * D, 3 * H * D, state, slot, pos, q_start, None,
+                               l2, H, D, D, 1e-5)
+            b.record()
+            b.synchronize()
+            spent.append(a.elapsed_time(b))
+        return min(spent)
+    usual = time(proj.bfloat16())
+    for size in (2.0 ** -60, 2.0 ** -90):
+        proj[:, H * D:2 * H * D].view(T, H, D)[::7, :, D - 3] = size
+        assert time(proj.bfloat16()) < 1.3 * usual      # (3.6 times as long with its products in fp32)
