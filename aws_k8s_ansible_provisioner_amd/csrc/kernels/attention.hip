@@ -715,17 +715,17 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
     // The last of the row's partitions to get here merges them (a launch and its gap less: one row of 16 / 8 heads
     // at 900 keys 10.3 -> 8.8 us, at 240, which one partition holds, 10.4 -> 7.7; 60 at ~450 21.2 -> 18.5, 200 at
     // ~560 83 -> 77, 64 at ~2000 87 either way; with the partial rows stored in pieces of 8 bytes that last one took
-    // 2 us more).  Every wave's stores have been acknowledged
-    // where all XCDs see them before the workgroup takes its ticket, and the last one puts it back
+    // 2 us more).  Every wave's stores have been acknowledged where all XCDs see them before the workgroup adds its
+    // share to the row's ticket: 1, the first partition 1 - nparts, so that nothing but all of them leave what was
+    // there, a zero, and whatever steps ran at once on one workspace, spoiling each other, the next one finds it.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     int* flag = reinterpret_cast<int*>(m_s);
     if (threadIdx.x == 0) {
       int* ticket = p.tickets + (size_t)(seq * p.Hkv + kvh) * kCtrStride;
       const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
-      const int last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
-      if (last) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *flag = last;
+      const int share = part == 0 ? 1 - nparts : 1;
+      *flag = __hip_atomic_fetch_add(ticket, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + share == 0;
     }
     __syncthreads();
     if (*flag != 0) merge_parts<true>(p, seq, kvh, kv_len, q_tok);

@@ -165,3 +165,28 @@ def test_paged_attention_tickets(part_size, parts, G):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, first) and not bool(ws.tickets.any())
+
+
+def test_paged_attention_tickets_are_left_as_found():
+    """A whole step adds nothing to its tickets, whatever stands in them when it starts and however many
+    partitions its rows have: one whose tickets another step was using (with outputs that mean nothing) leaves
+    them to that one, and the step after both finds zeros."""
+    from aws_k8s_ansible_provisioner_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    bt, sl, NB = _table(g)
+    H, G, D, T, bf = 3, 2, 128, len(LENS), torch.bfloat16
+    k = torch.randn(NB, H, BS, D, generator=g).to(bf).cuda()
+    v = torch.randn(NB, H, BS // 8, D, 8, generator=g).to(bf).cuda()
+    q = torch.randn(T, H * G, D, generator=g).to(bf).cuda()
+    bt, sl = bt.cuda(), sl.cuda()
+    ws = ops.decode_workspace(T, H, G, 18, "cuda")
+    first, out = (torch.empty(T, H * G, D, dtype=bf, device="cuda") for _ in range(2))
+    ops.paged_attention_decode(first, q, k, v, bt, sl, G, D ** -0.5, ws, 18, 128)
+    for parts, size in ((18, 128), (9, 256), (2, 1152)):
+        ws.tickets.fill_(3)
+        ops.paged_attention_decode(out, q, k, v, bt, sl, G, D ** -0.5, ws, parts, size)
+        assert bool((ws.tickets == 3).all())
+    ws.tickets.fill_(0)
+    ops.paged_attention_decode(out, q, k, v, bt, sl, G, D ** -0.5, ws, 18, 128)
+    assert torch.equal(out, first)
