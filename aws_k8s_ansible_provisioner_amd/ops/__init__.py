@@ -263,8 +263,8 @@ def paged_attention_decode_fused(out, qkv, k_cache, v_cache, block_tables, seq_l
 
 class DecodeWorkspace(tuple):
     """(part_m, part_l, part_o) of a split decode step, and the tickets that merge its partitions
-    within the launch (zeros between launches; None: merged by a second one).  One step at a time
-    may use it, as ever."""
+    within the launch (zeros between steps; None: merged by a second launch).  One step at a time
+    may use it, as ever; on which stream, and which stream made it, does not matter."""
 
     tickets = None
 
@@ -272,9 +272,13 @@ class DecodeWorkspace(tuple):
 def decode_workspace(max_seqs: int, num_kv_heads: int, gqa_group: int, num_parts: int,
                      device) -> tuple:
     ws = DecodeWorkspace(_decode_workspace(max_seqs, num_kv_heads, gqa_group, num_parts, device))
-    if num_parts > 1 and torch.device(device).type == "cuda":
+    # (made while a graph is captured its zeros would be a node of the graph: no tickets)
+    if num_parts > 1 and torch.device(device).type == "cuda" \
+            and not torch.cuda.is_current_stream_capturing():
         ws.tickets = torch.zeros(max(1, max_seqs * num_kv_heads) * DECODE_TICKET_INTS,
                                  dtype=torch.int32, device=device)
+        # a step on another stream must not run ahead of the zeros
+        torch.cuda.current_stream(ws.tickets.device).synchronize()
     return ws
 
 

@@ -190,3 +190,45 @@ def test_paged_attention_tickets_are_left_as_found():
     ws.tickets.fill_(0)
     ops.paged_attention_decode(out, q, k, v, bt, sl, G, D ** -0.5, ws, 18, 128)
     assert torch.equal(out, first)
+
+
+def test_paged_attention_workspace_of_another_stream():
+    """A workspace made on a stream with much to do, used on another one at once: its tickets are there.  One
+    made while a graph is captured has none, and merges by the second launch."""
+    from aws_k8s_ansible_provisioner_amd import ops
+
+    g = torch.Generator().manual_seed(4)
+    bt, sl, NB = _table(g)
+    H, G, D, T, bf = 3, 2, 128, len(LENS), torch.bfloat16
+    k = torch.randn(NB, H, BS, D, generator=g).to(bf).cuda()
+    v = torch.randn(NB, H, BS // 8, D, 8, generator=g).to(bf).cuda()
+    q = torch.randn(T, H * G, D, generator=g).to(bf).cuda()
+    bt, sl = bt.cuda(), sl.cuda()
+    want, got = (torch.full((T, H * G, D), 7.0, dtype=bf, device="cuda") for _ in range(2))
+    ops.paged_attention_decode(want, q, k, v, bt, sl, G, D ** -0.5,
+                               ops.decode_workspace(T, H, G, 9, "cuda"), 9, 256)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        a = torch.randn(4096, 4096, device="cuda")
+        left = torch.full((T * H * ops.DECODE_TICKET_INTS,), 5, dtype=torch.int32, device="cuda")
+        del left                                   # (the tickets may be given this memory)
+        for _ in range(20):
+            a = (a @ a).clamp_(-1, 1)
+        ws = ops.decode_workspace(T, H, G, 9, "cuda")
+    ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, ws, 9, 256)
+    assert ws.tickets is not None and torch.equal(got, want)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ws = ops.decode_workspace(T, H, G, 9, "cuda")
+        ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, ws, 9, 256)
+    assert ws.tickets is None
+    plain = torch.empty_like(want)
+    ops.paged_attention_decode(plain, q, k, v, bt, sl, G, D ** -0.5,
+                               tuple(ops.decode_workspace(T, H, G, 9, "cuda")), 9, 256)
+    for _ in range(3):
+        got.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, plain)
