@@ -672,3 +672,22 @@ def test_retention_small_keys_take_no_longer():
     for size in (2.0 ** -60, 2.0 ** -90):
         proj[:, H * D:2 * H * D].view(T, H, D)[::7, :, D - 3] = size
         assert time(proj.bfloat16()) < 1.3 * usual      # (3.6 times as long with its products in fp32)
+
+
+@pytest.mark.parametrize("D,V,rot", [(128, 128, 64), (64, 64, 32), (128, 64, 128), (64, 128, 64), (128, 128, 96)])
+@pytest.mark.parametrize("lens,starts", [([700, 420], [5, 0]), ([300, 161, 33], [0, 4, 2])])
+def test_retention_segments_of_turned_rows(D, V, rot, lens, starts):
+    """bf16 rows in segments, half of the entries turned and more, against the same rows in fp32."""
+    H, T, B = 4, sum(lens), len(lens)
+    assert torch.ops.akap_stream.chunk_scan_segment(1, T, B, H, V) > 0
+    g = torch.Generator().manual_seed(D + V + rot)
+    proj = torch.randn(T, 2 * H * D + 2 * H * V, generator=g).bfloat16()
+    state = torch.randn(B, H, V, D, generator=g)
+    ang = torch.arange(2048)[:, None] * (0.5 ** torch.arange(rot // 2))[None, :]
+    args = (_step(lens, starts), H, D, V, (0, H * D, 2 * H * D, 2 * H * D + H * V),
+            torch.cat([torch.cos(ang), torch.sin(ang)], 1), torch.log2(torch.tensor([0.97, 0.42, 0.2, 0.999])), DEV)
+    got, want = _run_retention((proj, state), *args), _run_retention((proj.float(), state), *args)
+    for h in range(H):
+        part = slice(h * V, (h + 1) * V)
+        assert _rel(got[0].float()[:, part], want[0][:, part].cpu()) < 3e-3
+        assert _rel(got[1][:, h], want[1][:, h].cpu()) < 2e-6

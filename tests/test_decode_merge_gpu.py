@@ -232,3 +232,39 @@ def test_paged_attention_workspace_of_another_stream():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("T,H,G,parts,size,fp8", [
+    (4, 8, 2, 16, 128, False), (3, 1, 8, 70, 128, False), (1, 2, 16, 140, 128, False), (2, 1, 4, 513, 128, True),
+    (9, 4, 5, 3, 1024, True)])
+def test_paged_attention_merge_of_many_partitions(T, H, G, parts, size, fp8):
+    """Rows of all partitions, all but a key, one key, one whole partition, one key more and none: the values of the
+    second launch but for the order of one fp32 product; its own where there are tickets for fewer rows or the
+    partial rows lie off 16 bytes, whatever the tickets hold."""
+    from aws_k8s_ansible_provisioner_amd import ops
+
+    g = torch.Generator().manual_seed(T + parts)
+    D, bf, most = 128, torch.bfloat16, parts * size
+    lens = [most, size + 1, most - 1, 1, 0, size, most // 2, 3, most][:T]
+    NB = most // BS
+    bt = torch.stack([torch.randperm(NB, generator=g) for _ in range(T)]).int().cuda()
+    k = torch.randn(NB, H, BS, D, generator=g).to(bf).cuda()
+    v = torch.randn(NB, H, BS // 8, D, 8, generator=g).to(bf).cuda()
+    if fp8:
+        k, v = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (k, v))
+    q = torch.randn(T, H * G, D, generator=g).to(bf).cuda()
+    sl = torch.tensor(lens, dtype=torch.int32).cuda()
+    want, got = (torch.full((T, H * G, D), 7.0, dtype=bf, device="cuda") for _ in range(2))
+    ws = ops.decode_workspace(T, H, G, parts, "cuda")
+    ops.paged_attention_decode(want, q, k, v, bt, sl, G, D ** -0.5, tuple(ws), parts, size)
+    ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, ws, parts, size)
+    assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs()).all())
+    assert not bool(ws.tickets.any())
+    short = ops.DecodeWorkspace(tuple(ws))
+    short.tickets = torch.full((T * H * ops.DECODE_TICKET_INTS - 1,), 5, dtype=torch.int32, device="cuda")
+    odd = ops.DecodeWorkspace((ws[0], ws[1], torch.empty(ws[2].numel() + 1, device="cuda")[1:]))
+    odd.tickets = torch.full_like(ws.tickets, 5)
+    for w in (short, odd):
+        got.fill_(7.0)
+        ops.paged_attention_decode(got, q, k, v, bt, sl, G, D ** -0.5, w, parts, size)
+        assert torch.equal(got, want) and bool((w.tickets == 5).all())

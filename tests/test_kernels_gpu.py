@@ -4,6 +4,9 @@ Every test here runs the HIP kernel (torch.ops.akap.*) on the GPU and compares i
 with ops.reference on the same inputs.  Requires an MI355X.
 """
 import math
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -173,6 +176,36 @@ def test_paged_attention_prefill_teams(hq, hkv, seqs):
     ops.paged_attention_prefill(out, q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), sl.to(DEV),
                                 qs.to(DEV), ts.to(DEV), tr.to(DEV), hq // hkv, scale, tile_rows=256)
     _close(out, exp, atol=2e-2, rtol=2e-2)
+
+
+def _prefill_in_turns():
+    """256-row tiles of 1 to 6 key tiles, whole and cut, against the reference and against rows that are read
+    column by column."""
+    ops.load_native(required=True)
+    for hq, hkv, seqs in [(16, 8, [(n, n) for n in (1, 64, 65, 128, 129, 192, 193, 256, 257)]),
+                          (32, 8, [(64, 64), (320, 200), (384, 3)]), (64, 2, [(65, 40), (200, 129)])]:
+        q, kc, vc, bt, sl, qs = _setup_attn(seqs, hq, hkv, 32, seed=hq)
+        scale = 1 / math.sqrt(128)
+        ts, tr = _tiles(seqs, hq // hkv, 256)
+        args = [t.to(DEV) for t in (kc, vc, bt, sl, qs, ts, tr)]
+        odd = torch.empty(q.numel() + 1, dtype=q.dtype, device=DEV)[1:].view(q.shape).copy_(q)
+        out = [torch.empty(q.shape, dtype=q.dtype, device=DEV) for _ in range(2)]
+        for rows, o in zip((q.to(DEV), odd), out):
+            ops.paged_attention_prefill(o, rows, *args, hq // hkv, scale, tile_rows=256)
+        _close(out[0], ref.paged_attention(q, kc, vc, bt, sl, qs, scale), atol=2e-2, rtol=2e-2)
+        assert torch.equal(*out)
+    print("in turns: same")
+
+
+def test_paged_attention_prefill_waves_in_turns():
+    """The form whose later waves hold back their products by a key tile: asked for by a variable that is read
+    once, so in a process of its own."""
+    env = dict(os.environ, AKAP_PREFILL_STAGGER="1")
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = f"import sys; sys.path[:0] = [{here!r}, {os.path.dirname(here)!r}]; " \
+           "import test_kernels_gpu as t; t._prefill_in_turns()"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, env=env)
+    assert r.returncode == 0 and "in turns: same" in r.stdout, r.stdout + r.stderr
 
 
 # odd GQA groups (8/8, 24/8) take the full rotary-row loads, even ones the lane-pair share
