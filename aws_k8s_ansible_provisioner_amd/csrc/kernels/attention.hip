@@ -16,7 +16,9 @@
 //    softmax rescale is lane-local.
 //  * K operand: K cache [blk, Hkv, BS, D]; each lane loads 16 B per MFMA k-chunk.
 //  * Decode: grid (seq, kv_head, partition); 4 waves split a partition's 32-token
-//    chunks and combine through LDS; partitions are combined by a reduce kernel.  A wave's
+//    chunks and combine through LDS; the last of a row's partitions to finish merges them, or, of
+//    a workspace without tickets (or with too few, or with partial rows off 16 bytes), a second
+//    launch does.  A wave's
 //    cache block ids sit in one VGPR (read by readlane), its K/V chunks alternate between
 //    two named register sets with every load unconditional (exact vmcnt counts), and in the
 //    serving form the new token's K/V reach the chunk registers from LDS images, so no wave
@@ -504,7 +506,8 @@ __device__ __forceinline__ void merge_parts(const AttnParams& p, int seq, int kv
 //    clamped into the block-table row instead of guarded by it), so the chain before the
 //    first K/V load is two round trips.
 //  body: fused q/k-norm + RoPE + new-token K/V write (FUSED), the chunk loop over two named
-//    register sets, the 4-wave LDS combine, the output (or split-KV partial) store.
+//    register sets, the 4-wave LDS combine, then the output of a row that one partition holds,
+//    or the partial row, a ticket, and in the last of the row's workgroups the merge.
 template <bool FUSED, bool F8>
 __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kvh, int part,
                                             float* dyn_lds) {
@@ -712,12 +715,23 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
     }
   }
   if (p.tickets != nullptr && !alone) {
-    // The last of the row's partitions to get here merges them (a launch and its gap less: one row of 16 / 8 heads
-    // at 900 keys 10.3 -> 8.8 us, at 240, which one partition holds, 10.4 -> 7.7; 60 at ~450 21.2 -> 18.5, 200 at
-    // ~560 83 -> 77, 64 at ~2000 87 either way; with the partial rows stored in pieces of 8 bytes that last one took
-    // 2 us more).  Every wave's stores have been acknowledged where all XCDs see them before the workgroup adds its
-    // share to the row's ticket: 1, the first partition 1 - nparts, so that nothing but all of them leave what was
-    // there, a zero, and whatever steps ran at once on one workspace, spoiling each other, the next one finds it.
+    // The last of the row's partitions to get here merges them: a launch and its gap less, 2 to 3 us whatever the
+    // rows hold, and none of what follows for a row of one partition.  Layers of 16 / 8 heads and a maximum of 4096
+    // keys, by a second launch and so: one row at 120 / 900 / 4000 keys 8.7 / 9.5 / 11.3 us and 6.8 / 9.1 / 10.5, 16
+    // rows at 120 / 900 / 4000 9.6 / 16.1 / 49.3 and 7.5 / 15.1 / 50.3, 64 at 450 / 2000 / 4000 24.2 / 82.3 / 161 and
+    // 22 / 82.5 / 160, 200 at 450 / 2000 66.3 / 262 and 63.9 / 257.  What it costs: every workgroup of a row of
+    // several waits for its stores and its ticket, 0.7 us for each round of workgroups on a full chip, and the last
+    // one reads the others' rows, a trip of 0.8 us for eight partitions; in steps of 6 to 60 long rows that is more
+    // than the launch (worst 24 at 3000 keys 49.9 and 51.7; 40 of 32 / 8 heads at 1500 42.8 and 45; e4m3 caches, 32 of
+    // 32 / 8 at 4000 50.2 and 53.9; 16 heads per kv head, 16 rows of 2 kv heads at 8192 in 512s 26.2 and 28.7), and
+    // which rows are long only the device knows.  Many partitions of few rows are no worse for it, as a second launch
+    // then has as few workgroups and colder caches: one row at 8192 / 16384 / 32768 keys in partitions of 256, 16 / 8
+    // heads 13.3 / 25.5 / 47.9 and 11.9 / 23 / 44.4, 8 / 1 heads 16.2 / 27.2 / 47.4 and 12 / 17.5 / 29.1, at 131072
+    // 187 and 99; four rows of 32 / 8 at 16384 54.4 and 55.7.  (Partial rows stored in pieces of 8 bytes took 2 us
+    // more; the merge by all threads of a workgroup, or its maxima and rows in one pass, nothing less.)
+    // Every wave's stores have been acknowledged where all XCDs see them before the workgroup adds its share to the
+    // row's ticket: 1, the first partition 1 - nparts, so that nothing but all of them leave what was there, a zero,
+    // and whatever steps ran at once on one workspace, spoiling each other, the next one finds it.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     int* flag = reinterpret_cast<int*>(m_s);
@@ -880,8 +894,8 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // from there.  (A lane that loads its own columns takes 32 bytes of 32 lines in each of eight
   // instructions.)  Short prompts see few key tiles, and what stands before and behind these is much of the
   // time: of 12.6 thousand rows, 37 prompts, 16 / 8 heads, 40 of 58 us where every workgroup took one tile.
-  // With rows in and out as whole lines and an instruction in four less in the preparation (its norm a branch,
-  // its weights a lane's own loads) 56 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
+  // With rows in and out as whole lines and an instruction in six less in the preparation (929 for 1126: its norm a
+  // branch, its weights a lane's own loads) 56 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
   // prompts of ~115 61.8 -> 55.8, one of 48 12.4 -> 12.0.
   bf16x8 qf[8];
   bf16* const q_s = lds + kBuf + w * 32 * kD;

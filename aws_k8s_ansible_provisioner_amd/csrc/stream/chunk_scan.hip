@@ -28,11 +28,11 @@
 // chunk); the next step's parts are formed between a step's products.  Of the 11200 cycles a chunk takes (8
 // sequences of 64 heads, a wave per SIMD) 5100 issue, 4000 wait to issue, most of them behind products with nothing
 // beside them (the state's own), 2000 wait for LDS, memory and barriers, of which fragments asked for a chunk
-// earlier took none away.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 330 us
-// where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows 86 -> 65; 8 heads x
-// 128 x 128 (segments) 76 + 33 for the pass before it, and 57 for the fragments: all three wait much for
-// memory, and with entries of one part (HALF) 148 MB of fragments are written and 215 read, of 215 and 316
-// where all have three (walks 3 + 4 us more, fragments 67).
+// earlier took none away.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 349 us, 372 on average
+// under a profiler, where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows
+// 86 -> 65; 8 heads x 128 x 128 (segments) 78 + 34 for the pass before it, and 57 for the fragments: all
+// three wait much for memory, and with entries of one part (HALF) 148 MB of fragments are written and 215
+// read, of 215 and 316 where all have three (walks 3 + 4 us more, fragments 67).
 //
 // A walk alone is a serial chain of about 4 us per chunk (128 x 32 state entries per wave), so
 // where the (sequence, head, 32 columns) triples of the long sequences leave SIMDs idle, these run in
@@ -577,7 +577,8 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(const ChunkScanParams p
 // HW heads (of one key head) of V / 32 waves each, a wave per 32 state columns; FULL: outputs,
 // from the state in the slot (or, SEGM and the sequence is cut, from the segment buffer); else the
 // segment's own state from zeros.  Fragments and scalars arrive by LDS-DMA: those of q while the state
-// of the chunk before is formed, those of k (in time for the chunk's state) while its outputs are, so
+// of the chunk before is formed (a retention's segments ask for them once the outputs of the chunk before
+// have used its own, see hand_on()), those of k (in time for the chunk's state) while its outputs are, so
 // that one buffer of each does and two workgroups share a CU; the values in registers a chunk ahead.
 template <int MODE, int NT, int V, int HW, typename TY, bool HALF, bool FULL, bool SEGM>
 __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkScanParams p) {
