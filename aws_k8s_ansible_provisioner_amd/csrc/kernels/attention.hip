@@ -663,6 +663,10 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
   const int row = threadIdx.x >> 4;
   // (with tickets a row whose keys are all in the first partition needs no merge)
   const bool alone = p.num_parts == 1 || (p.tickets != nullptr && kv_len <= p.part_size);
+  // what the workgroup adds to the row's ticket, below (formed here, not between the stores and the ticket)
+  int share = 1;
+  if (part == 0 && !alone) share -= min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
+  asm volatile("" : "+s"(share));
   // dims d0 .. + 3 and d0 + d4 .. + 3; partial rows go past the caches in whole lines
   const bool lines = p.tickets != nullptr && !alone;
   const int d0 = (threadIdx.x & 15) * (lines ? 4 : 8), d4 = lines ? 64 : 4;
@@ -737,8 +741,6 @@ __device__ __forceinline__ void decode_item(const AttnParams& p, int seq, int kv
     int* flag = reinterpret_cast<int*>(m_s);
     if (threadIdx.x == 0) {
       int* ticket = p.tickets + (size_t)(seq * p.Hkv + kvh) * kCtrStride;
-      const int nparts = min(p.num_parts, (kv_len + p.part_size - 1) / p.part_size);
-      const int share = part == 0 ? 1 - nparts : 1;
       *flag = __hip_atomic_fetch_add(ticket, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + share == 0;
     }
     __syncthreads();
