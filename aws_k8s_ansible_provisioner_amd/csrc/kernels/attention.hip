@@ -835,7 +835,8 @@ __device__ __forceinline__ void fa_glds16(const void* g, void* lds_wave_base) {
 // TEAMS = 2 (small grids of bf16 caches): two teams of NW waves take the key tiles of the same rows in
 // turn, each with its own buffers, maximum and sums, which are added up at the end; subs workgroups
 // share a tile of the map.
-template <bool F8, bool GL, int NW = 4, bool STAG = false, int TEAMS = 1>
+// LINES (large grids): outputs go through LDS and are stored as whole lines.
+template <bool F8, bool GL, int NW = 4, bool STAG = false, int TEAMS = 1, bool LINES = false>
 __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged_attn_prefill_fa_kernel(
     AttnParams p, int subs) {
   constexpr int ROWS = 32 * NW;
@@ -845,6 +846,7 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   static_assert(NW == 4 || (NW == 8 && GL), "the register-staged path assumes 256 threads");
   static_assert(!STAG || (NW == 8 && GL), "the ping-pong pairs waves w and w + 4");
   static_assert(TEAMS == 1 || (GL && !STAG && NW == 4), "teams");
+  static_assert(!LINES || (!STAG && TEAMS == 1), "the buffer that no wave reads any more");
   // [buf][K | V][64 keys * 128 dims] bf16 = 64 KiB (96 KiB with STAG), room for those of 256 q rows that
   // the buffers behind the first do not take, + the block ids of the
   // first kFaBtCache 32-key chunks; ONE __shared__ object (a second one makes hipcc drain vmcnt)
@@ -901,6 +903,15 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // prompts of ~115 61.8 -> 55.8, one of 48 12.4 -> 12.0.
   bf16x8 qf[8];
   bf16* const q_s = lds + kBuf + w * 32 * kD;
+  // The tokens and heads of a lane's part of the wave's rows, every 4th (of the outputs every 8th): the first from
+  // the lane that owns it, the next ones by steps.  (Each from its owner was a trip through LDS between the loads:
+  // one prompt of 20 tokens, 16 / 8 heads, the layer 14.1 us, so 14.0.)
+  auto next_row = [&](int& t, int& g, int by, int rest) {
+    g += rest;
+    const bool over = g >= G;
+    t += by + over;
+    g -= over ? G : 0;
+  };
   auto load_q = [&]() {
   const bf16* rows = prep ? p.qkv : p.q;
   const uint32_t stride = prep ? p.qkv_stride : p.Hq * kD;
@@ -909,12 +920,14 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   const bf16* first = rows + (size_t)q0 * stride + (size_t)kvh * G * kD;   // of the sequence and kv head
   bf16x8 raw[8];
   if (whole) {
-    const int mine = (valid ? pos : 0) << 16 | hig;
+    const int at = __shfl(pos << 16 | hig, lane >> 4), by = G > 4 ? 0 : G > 2 ? 1 : 4 / G;
+    int t = (uint32_t)at >> 16, g = at & 0xffff;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int row = 4 * i + (lane >> 4), at = __shfl(mine, row);
-      const uint32_t off = (((uint32_t)at >> 16) * stride + (at & 0xffff) * kD + ((lane & 15) ^ (row & 15)) * 8) * 2u;
+      const int row = 4 * i + (lane >> 4);
+      const uint32_t off = ((t < q_len ? t : 0) * stride + g * kD + ((lane & 15) ^ (row & 15)) * 8) * 2u;
       fa_glds16(reinterpret_cast<const char*>(first) + off, q_s + i * 4 * kD);
+      next_row(t, g, by, 4 - by * G);
     }
   }
   // rotary position = the token's key index ctx0 + pos -- the invariant the causal limit above already
@@ -1306,37 +1319,55 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // O^T accumulator of lane (r, h): row r's dims 32 dt + 8 j4 + 4 h + (0..3).  Each pair of
   // 8-dim groups (j4 = 2 kp, 2 kp + 1) is exchanged between the lane halves with two
   // v_permlane32_swap, after which lane r holds dims 16 kp + 0..7 and lane r + 32 dims
-  // 16 kp + 8..15 of the same row.  The wave's rows then go through LDS, 64 dims at a time (16-B column c of
-  // row r at c ^ (r & 7)), and are stored as whole 128-byte lines, eight to an instruction.
+  // 16 kp + 8..15 of the same row: one 16-B store per pair instead of two 8-B stores (the
+  // epilogue is store-issue bound: 18 us of 117 at 32 x 512, profiles/r2_pmc_prefill_v2.md).
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  // (a place that no other wave reads: the buffer of the tile before the last, or the wave's own sums)
-  bf16* o_s = lds_all + w * 66 * 64 * 2;
-  if (TEAMS == 1 || teams == 1) o_s = lds + (STAG ? ntiles % NBUF : ntiles & 1) * kBuf + w * 32 * 64;
-  const int mine = valid ? (q0 + pos) * p.Hq + kvh * G + hig : -1;
-  asm volatile("" ::: "memory");   // (sums of the second team are read from the same place, as another type)
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-#pragma unroll
-    for (int c2 = 0; c2 < 4; ++c2) {
-      const int dt = 2 * half + (c2 >> 1), kp = c2 & 1;
-      bf16x4 oa, ob;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        oa[i] = f2bf(oacc[dt][8 * kp + i] * inv);
-        ob[i] = f2bf(oacc[dt][8 * kp + 4 + i] * inv);
-      }
-      const u32x2 a = __builtin_bit_cast(u32x2, oa), b = __builtin_bit_cast(u32x2, ob);
-      const auto r0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
-      const auto r1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
-      const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
-      *reinterpret_cast<u32x4*>(o_s + r * 64 + ((2 * c2 + h) ^ (r & 7)) * 8) = o;
-    }
+  auto dims = [&](int dt, int kp) {
+    bf16x4 oa, ob;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = 8 * i + (lane >> 3), at = __shfl(mine, row);
-      const u32x4 o = *reinterpret_cast<const u32x4*>(o_s + row * 64 + ((lane & 7) ^ (row & 7)) * 8);
-      // every lane takes part in the exchange; only rows of this chunk store
-      if (at >= 0) *reinterpret_cast<u32x4*>(p.out + (size_t)at * kD + 64 * half + (lane & 7) * 8) = o;
+      oa[i] = f2bf(oacc[dt][8 * kp + i] * inv);
+      ob[i] = f2bf(oacc[dt][8 * kp + 4 + i] * inv);
+    }
+    const u32x2 a = __builtin_bit_cast(u32x2, oa), b = __builtin_bit_cast(u32x2, ob);
+    const auto r0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const auto r1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    return u32x4{r0[0], r1[0], r0[1], r1[1]};
+  };
+  if constexpr (!LINES) {
+    bf16* orow = p.out + ((size_t)(q0 + (valid ? pos : 0)) * p.Hq + kvh * G + hig) * kD;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int kp = 0; kp < 2; ++kp) {
+        const u32x4 o = dims(dt, kp);
+        // every lane takes part in the swaps; only rows of this chunk store
+        if (valid) *reinterpret_cast<u32x4*>(orow + 32 * dt + 16 * kp + 8 * h) = o;
+      }
+  } else {
+    // The wave's rows through LDS, 64 dims at a time (16-B column c of row r at c ^ (r & 7)), in the buffer of the
+    // tile before the last, which no other wave reads: whole 128-byte lines, eight to an instruction.
+    bf16* o_s = lds + (ntiles & 1) * kBuf + w * 32 * 64;
+    int own = pos;                   // (formed anew: kept since the queries it would be a register of the loop's)
+    asm volatile("" : "+v"(own));
+    const int at = __shfl(own << 16 | hig, lane >> 3), by = G > 8 ? 0 : G > 4 ? 1 : G > 2 ? 2 : 8 / G;
+    int t = (uint32_t)at >> 16, g = at & 0xffff, to[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      to[i] = t < q_len ? (q0 + t) * p.Hq + kvh * G + g : -1;
+      next_row(t, g, by, 8 - by * G);
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int c2 = 0; c2 < 4; ++c2)
+        *reinterpret_cast<u32x4*>(o_s + r * 64 + ((2 * c2 + h) ^ (r & 7)) * 8) = dims(2 * half + (c2 >> 1), c2 & 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        const u32x4 o = *reinterpret_cast<const u32x4*>(o_s + row * 64 + ((lane & 7) ^ (row & 7)) * 8);
+        if (to[i] >= 0) *reinterpret_cast<u32x4*>(p.out + (size_t)to[i] * kD + 64 * half + (lane & 7) * 8) = o;
+      }
     }
   }
 }
@@ -1367,16 +1398,27 @@ void launch_paged_attn_prefill(const AttnParams& p, int num_tiles, int tile_rows
   // us (35.1 with one team), of 1500 56 -> 42 (47), of 2000 69.5 -> 51.5 (60); 32 / 8 heads, 700 behind 300
   // 41.3 -> 32.1.  At up to two workgroups to a CU 4 prompts of 500 behind 600 lost (50 -> 56), and at maps of
   // 128-row tiles 10 prompts of 200 behind 300 (28.1 -> 28.8).
+  // Outputs as whole lines (LINES) in large grids; in small ones each workgroup's own chain counts, which the trip
+  // through LDS makes longer.  The layer, lanes' own pieces and lines: 16 / 8 heads, one prompt of 20
+  // tokens 13.5 and 14.1 us, 10 of ~130 (200 workgroups) 18.0 and 18.5, 64 of 26 (512) 21.3 and 21.9, 64 of ~115
+  // (1200) 44.6 and 43.9, 37 of ~340 (1650) 82.4 and 80.6; 32 / 8, 12 of ~200 (800) 31.3 and 32, 64 of ~115 (2400)
+  // 59.7 and 58.5; in tiles of 256 rows 24 of 512 (1536) 135 and 131.2, 3 of ~1200 (600) 74.6 and 75.7; e4m3 caches,
+  // 10 of ~130 (200) 22 and 22.4, 12 of ~200 (450) 33.5 and 33, 37 of ~340 112.8 and 111.1.
+  const bool lines = grid.x > (p.kv_fp8 ? 256 : 1024);
   if (tile_rows == 2 * kFaRows && !p.kv_fp8 && !stag && 2 * grid.x <= 256)
     paged_attn_prefill_fa_kernel<false, true, 4, false, 2><<<2 * grid.x, 512, 0, s>>>(q, 2);
   else if (tile_rows == 2 * kFaRows && !p.kv_fp8) {  // 256 rows, 8 waves (bf16 caches)
     if (stag) paged_attn_prefill_fa_kernel<false, true, 8, true><<<grid, 512, 0, s>>>(q, 1);
+    else if (lines) paged_attn_prefill_fa_kernel<false, true, 8, false, 1, true><<<grid, 512, 0, s>>>(q, 1);
     else paged_attn_prefill_fa_kernel<false, true, 8><<<grid, 512, 0, s>>>(q, 1);
   }
-  else if (p.kv_fp8)  // fp8 caches: register-staged (widened to bf16 on the way into LDS)
-    paged_attn_prefill_fa_kernel<true, false><<<grid, 256, 0, s>>>(q, 1);
-  else  // bf16 caches: LDS-DMA staging
-    paged_attn_prefill_fa_kernel<false, true><<<grid, 256, 0, s>>>(q, 1);
+  else if (p.kv_fp8) {  // fp8 caches: register-staged (widened to bf16 on the way into LDS)
+    if (lines) paged_attn_prefill_fa_kernel<true, false, 4, false, 1, true><<<grid, 256, 0, s>>>(q, 1);
+    else paged_attn_prefill_fa_kernel<true, false><<<grid, 256, 0, s>>>(q, 1);
+  } else {  // bf16 caches: LDS-DMA staging
+    if (lines) paged_attn_prefill_fa_kernel<false, true, 4, false, 1, true><<<grid, 256, 0, s>>>(q, 1);
+    else paged_attn_prefill_fa_kernel<false, true><<<grid, 256, 0, s>>>(q, 1);
+  }
 }
 
 void launch_paged_attn_decode(const AttnParams& p, int num_seqs, hipStream_t s) {

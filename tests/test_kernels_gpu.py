@@ -178,6 +178,43 @@ def test_paged_attention_prefill_teams(hq, hkv, seqs):
     _close(out, exp, atol=2e-2, rtol=2e-2)
 
 
+# outputs stored as whole lines, from more than 1024 workgroups (of e4m3 caches 256) on, and by each lane below
+@pytest.mark.parametrize("hq,hkv,tile_rows,fp8,n", [
+    (16, 8, 128, False, 130), (32, 8, 128, False, 129), (24, 8, 128, False, 128), (5, 1, 128, False, 1030),
+    (16, 8, 256, False, 130), (64, 2, 256, False, 520), (16, 8, 128, True, 33), (28, 4, 128, True, 66)])
+def test_paged_attention_prefill_many_workgroups(hq, hkv, tile_rows, fp8, n):
+    """The same bits from one call as from calls of a few prompts each, and the reference's values."""
+    G = hq // hkv
+    lens = [1 + 7 * i % max(2, tile_rows // G) for i in range(n - 1)] + [200]
+    seqs = [(m + (i % 3) * 40, m) for i, m in enumerate(lens)]
+    q, kc, vc, bt, sl, qs = _setup_attn(seqs, hq, hkv, 32, seed=n)
+    scale = 1 / math.sqrt(128)
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (kc, vc))
+    cache = [t.to(DEV) for t in (kc, vc)]
+
+    def run(part, first):
+        ts, tr = _tiles(part, G, tile_rows)
+        out = torch.full((sum(m for _, m in part), hq, 128), 7.0, dtype=torch.bfloat16, device=DEV)
+        at = int(qs[first])
+        start = (qs[first:first + len(part) + 1] - at).to(DEV)
+        ops.paged_attention_prefill(out, q[at:at + out.shape[0]].to(DEV), *cache, bt[first:first + len(part)].to(DEV),
+                                    sl[first:first + len(part)].to(DEV), start, ts.to(DEV), tr.to(DEV), G, scale,
+                                    tile_rows=tile_rows)
+        return out, len(ts) * hkv
+
+    limit = 256 if fp8 else 1024
+    out, wgs = run(seqs, 0)
+    assert wgs > limit
+    step = max(1, n // 4)
+    parts = [run(seqs[i:i + step], i) for i in range(0, n, step)]
+    assert max(w for _, w in parts) <= limit
+    assert torch.equal(out, torch.cat([o for o, _ in parts]))
+    last = slice(int(qs[n - 3]), None)
+    exp = ref.paged_attention(q[last], kc, vc, bt[n - 3:], sl[n - 3:], qs[n - 3:] - qs[n - 3], scale)
+    _close(out[last], exp, atol=2e-2, rtol=2e-2)
+
+
 def _prefill_in_turns():
     """256-row tiles of 1 to 6 key tiles, whole and cut, against the reference and against rows that are read
     column by column."""
