@@ -193,7 +193,8 @@ __device__ __forceinline__ float decay_pow(float l2, int k) {
 // Keys in one bf16 part take the power of two in their weight, exactly, and values the rest of it, 1 to 2 times
 // key_scale(), so that both split however small the weight is.  Keys come kEven smaller and values kEven larger:
 // the power that takes every value of FLT_MIN and more to kSmall.
-constexpr float kEven = 0x1p29f;
+// (They are looked over times kFirst, as far from infinity and from zero as keys times whole weights.)
+constexpr float kEven = 0x1p29f, kFirst = 0x1p-4f;
 __device__ __forceinline__ int decay_exponent(float l2, int k) {
   return k == 0 ? 0 : (int)fmaxf(floorf(l2 * (float)k), -512.f);
 }
@@ -419,7 +420,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
     const float l2 = p.log2_decay[kh], by = lift ? kLift : 1.f;
     const float w = tid < n ? decay_pow(l2, n - 1 - tid) * by : 0.f;
     wt[tid] = w;
-    if (HALF) wp[tid] = w != 0.f ? __builtin_ldexpf(by / kEven, decay_exponent(l2, n - 1 - tid)) : 0.f;
+    if (HALF) wp[tid] = w != 0.f ? __builtin_ldexpf(by * kFirst, decay_exponent(l2, n - 1 - tid)) : 0.f;
   }
   __syncthreads();
   const int li = lane & 31, hh = lane >> 5;
@@ -445,21 +446,18 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
 #pragma unroll
       for (int i = 0; i < 8; ++i) range[w].add(v[w][u][i]);
   }
-  constexpr float scale[2] = {1.f, MODE == 0 ? kDown : 1.f};
+  // (fragment f's parts are of the values times scale, those of one part are asked for FLT_MIN alone)
+  constexpr float scale[2] = {1.f, MODE == 0 ? kDown : 1.f}, scale1[2] = {1.f, 1.f / (kEven * kFirst)};
+  constexpr float few = HALF ? __FLT_MIN__ / scale1[1] : kSmall / scale[1];
   bool bad = !(range[0].hi < kSplits) || !(range[1].hi < kSplits);
-  if (range[0].lo < kSmall || range[1].lo < kSmall / scale[1]) {
+  if (range[0].lo < kSmall || range[1].lo < few) {
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
       for (int u = 0; u < NQ / 4; ++u)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int f = wave + 4 * u, j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
-          bad |= below(v[w][u][i], f < XQ ? kSmall / scale[w] : __FLT_MIN__);
-          // (a key of which nothing is left beside its weight)
-          if (MODE == 1 && w == 1)
-            bad |= v[1][u][i] == 0.f && wt[j] != 0.f && ks[j * LS + 32 * (f >> 1) + li] != 0.f;
-        }
+        for (int i = 0; i < 8; ++i)
+          bad |= below(v[w][u][i], wave + 4 * u < XQ ? kSmall / scale[w] : __FLT_MIN__ / scale1[w]);
   }
   bad = __syncthreads_or(bad);
   if (!live) return;
@@ -470,7 +468,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
       bf16x8 part[3];
       float e[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) e[i] = v[w][u][i] * scale[w];
+      for (int i = 0; i < 8; ++i) e[i] = v[w][u][i] * (wave + 4 * u < XQ ? scale[w] : scale1[w]);
       split8(e, part[0], part[1], part[2]);
       if (__builtin_expect(bad, 0)) {      // as they are, in two halves
 #pragma unroll
