@@ -403,14 +403,15 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
       }
     }
   }
-  constexpr float kscale = MODE == 1 ? key_scale<N>() : 1.0f;
+  // (keys of one part are needed without it)
+  constexpr float staged = MODE == 1 && !HALF ? key_scale<N>() : 1.0f, kscale = HALF ? key_scale<N>() : 1.0f;
 #pragma unroll
   for (int u = 0; u < RN; ++u) {
     const int i = i0 + u * RS;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b4 = a;
     if (i < n) {
       a = make_float4(q4[u][0], q4[u][1], q4[u][2], q4[u][3]);
-      b4 = make_float4(k4[u][0], k4[u][1], k4[u][2], k4[u][3]);
+      b4 = make_float4(k4[u][0] * staged, k4[u][1] * staged, k4[u][2] * staged, k4[u][3] * staged);
     }
     *(float4*)(qs + i * LS + d) = a;
     *(float4*)(ks + i * LS + d) = b4;
@@ -439,7 +440,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
     for (int i = 0; i < 8; ++i) {
       const int j = j0 + (i & 3) + 8 * (i >> 2);
       const float k = ks[j * LS + 32 * (f >> 1) + li];
-      v[1][u][i] = MODE == 0 ? k : f < XQ ? k * kscale * wt[j] : k * wp[HALF ? j : 0];
+      v[1][u][i] = MODE == 0 ? k : !HALF || f < XQ ? k * kscale * wt[j] : k * wp[HALF ? j : 0];
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w)
@@ -457,7 +458,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
       for (int u = 0; u < NQ / 4; ++u)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          bad |= below(v[w][u][i], wave + 4 * u < XQ ? kSmall / scale[w] : __FLT_MIN__ / scale1[w]);
+          bad |= below(v[w][u][i], !HALF || wave + 4 * u < XQ ? kSmall / scale[w] : __FLT_MIN__ / scale1[w]);
   }
   bad = __syncthreads_or(bad);
   if (!live) return;
@@ -468,16 +469,16 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
       bf16x8 part[3];
       float e[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) e[i] = v[w][u][i] * (wave + 4 * u < XQ ? scale[w] : scale1[w]);
+      for (int i = 0; i < 8; ++i) e[i] = v[w][u][i] * (!HALF || wave + 4 * u < XQ ? scale[w] : scale1[w]);
       split8(e, part[0], part[1], part[2]);
       if (__builtin_expect(bad, 0)) {      // as they are, in two halves
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           uint32_t bits = __float_as_uint(v[w][u][i]);
           const int f = wave + 4 * u;
-          if (w == 1 && (lift || f >= XQ)) {
+          if (w == 1 && (lift || (HALF && f >= XQ))) {
             const int j = 16 * (f & 1) + 4 * hh + (i & 3) + 8 * (i >> 2);
-            bits = __float_as_uint(ks[j * LS + 32 * (f >> 1) + li] * (f >= XQ ? 1.f : kscale));
+            bits = __float_as_uint(ks[j * LS + 32 * (f >> 1) + li] * (HALF && f >= XQ ? 1.f : kscale));
           }
           part[0][i] = __builtin_bit_cast(bf16, (uint16_t)(bits >> 16));
           part[1][i] = __builtin_bit_cast(bf16, (uint16_t)bits);
@@ -485,7 +486,7 @@ __device__ __forceinline__ void fragments(const ChunkScanParams& p, const int en
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        if (i == 0 || wave + 4 * u < XQ)
+        if (!HALF || i == 0 || wave + 4 * u < XQ)
           ((bf16x8*)buf)[(3 * NQ * w + wave + 4 * u + i * NQ) * 64 + lane] = part[i];
     }
   // q . k with the keys as rows: lane (i, hh) register 4 g + r is q_i . k_(8 g + 4 hh + r), the
@@ -680,13 +681,19 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       o += (s & 3) == 3 ? 5 * step : step;
     }
   };
-  // (the first chunk's are on their way while the state is asked for)
-  values(0);
   auto stage = [&](int c, float4* to) {
     stage_k(c, to);
     stage_scalars(c, to + C0 * 64);
   };
-  if (FULL) stage_q(0); else stage(0, qbuf);
+  // The first chunk's are on their way while the state is asked for.  (Not of a retention in fp32, but with outputs in
+  // segments: its values' parts leave no registers for it.  14 spilled where now 9 do, without outputs 34 and 24; a
+  // prompt of 100 rows, 8 heads x 128 x 128, 34.3 us and 31.9.)
+  constexpr bool kFull32 = MODE == 1 && sizeof(TY) == 4 && !(FULL && SEGM);
+  auto begin = [&] {
+    values(0);
+    if (FULL) stage_q(0); else stage(0, qbuf);
+  };
+  if (!kFull32) begin();
   const float l2 = MODE == 1 ? p.log2_decay[h] : 0.f;
   const bool lift = MODE == 1 && uniform(lifted(l2));
   // retention: decay^k and decay^(k + 1)
@@ -906,10 +913,13 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         float upe[4];      // the same of a key in one part, which takes its own weight's rest besides
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float f = HALF || lift ? tb[max(n - 1 - (8 * g + 4 * hh + r), 0)] : 1.f;
           up[r] = MODE == 0 && !odd ? kUp : 1.f;
-          if (HALF) upe[r] = odd ? key_scale<N>() * (lift ? 1.f : f) : wb[kL - n + 8 * g + 4 * hh + r];
+          if (HALF) {
+            const float f = lift ? 1.f : tb[max(n - 1 - (8 * g + 4 * hh + r), 0)];
+            upe[r] = odd ? key_scale<N>() * f : wb[kL - n + 8 * g + 4 * hh + r];
+          }
           if (lift) {
+            const float f = tb[max(n - 1 - (8 * g + 4 * hh + r), 0)];
             const int e = __builtin_amdgcn_frexp_expf(f);
             xw[4 * g + r] = odd ? xw[4 * g + r] * f : __builtin_ldexpf(xw[4 * g + r], e);
             if (!odd) {
@@ -921,11 +931,11 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const float4 a = joined(kp, 4 * t + g);
-          const float* by = HALF && t >= NT / 2 ? upe : up;
-          S[t] = mfma(a.x * by[0], xw[4 * g], S[t]);
-          S[t] = mfma(a.y * by[1], xw[4 * g + 1], S[t]);
-          S[t] = mfma(a.z * by[2], xw[4 * g + 2], S[t]);
-          S[t] = mfma(a.w * by[3], xw[4 * g + 3], S[t]);
+          const bool one = HALF && t >= NT / 2;
+          S[t] = mfma(a.x * (one ? upe[0] : up[0]), xw[4 * g], S[t]);
+          S[t] = mfma(a.y * (one ? upe[1] : up[1]), xw[4 * g + 1], S[t]);
+          S[t] = mfma(a.z * (one ? upe[2] : up[2]), xw[4 * g + 2], S[t]);
+          S[t] = mfma(a.w * (one ? upe[3] : up[3]), xw[4 * g + 3], S[t]);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1085,7 +1095,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       __builtin_amdgcn_sched_barrier(0);
     }
     if (!kEarlyWeights) fetch_weights(sc, n);
-    dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
+    if (!kFull32) dend = MODE == 0 ? sc[2 * kL - 1] : tb[kL + n - 1];
 #pragma unroll
     for (int s = 0; s < 16; ++s) O[s] = (O[s] + O2[s]) * e;
     __builtin_amdgcn_sched_barrier(0);
@@ -1128,8 +1138,8 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         for (int i = 0; i < 16; ++i) few |= below(S[t][i], kSmall);
     }
     if (__builtin_expect(odd || (XP == 1 && apart) || __any(fin != 0.f || few), 0)) {
-      // an operand that does not split, or is not finite: the fp32 products (queries from memory)
-      const bf16x8* qg = (const bf16x8*)frag_of(c) + fresh(lane);
+      // an operand that does not split, or is not finite: the fp32 products (queries from memory, or still here)
+      const bf16x8* qg = kFull32 ? qp : (const bf16x8*)frag_of(c) + fresh(lane);
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[i] = 0.f;
 #pragma unroll
@@ -1164,6 +1174,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
       }
     }
   };
+  if (kFull32) begin();
   if constexpr (FULL) {
     akap::bf16x4 zb[kNorm ? 4 : 1];
     float4 zf[kNorm ? 4 : 1];
@@ -1214,6 +1225,7 @@ __global__ __launch_bounds__(2 * V * HW, 2) void chunk_walk_kernel(const ChunkSc
         if (c + 1 < chunks) stage_q(c + 1);
       };
       outputs(c, hand_on);
+      if (kFull32) dend = tb[kL + n - 1];
       if (kNorm) {
         float ss = 0.f;
 #pragma unroll
