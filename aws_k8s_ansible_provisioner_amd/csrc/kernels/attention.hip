@@ -898,9 +898,9 @@ __global__ __launch_bounds__(64 * NW * TEAMS, TEAMS > 1 ? 2 : 8 / NW) void paged
   // from there.  (A lane that loads its own columns takes 32 bytes of 32 lines in each of eight
   // instructions.)  Short prompts see few key tiles, and what stands before and behind these is much of the
   // time: of 12.6 thousand rows, 37 prompts, 16 / 8 heads, 40 of 58 us where every workgroup took one tile.
-  // With rows in and out as whole lines and an instruction in six less in the preparation (929 for 1126: its norm a
-  // branch, its weights a lane's own loads) 56 us; the layer with 32 / 8 heads without a q norm 135.6 -> 124.8, 64
-  // prompts of ~115 61.8 -> 55.8, one of 48 12.4 -> 12.0.
+  // With query rows whole, an instruction in six less in the preparation (944 for 1126: its norm a branch, its
+  // weights a lane's own loads) and outputs as lines 56 us; the layer with 32 / 8 heads without a q norm 135.6 ->
+  // 124.8, 64 prompts of ~115 61.8 -> 55.8, one of 48 13.2 -> 12.4.
   bf16x8 qf[8];
   bf16* const q_s = lds + kBuf + w * 32 * kD;
   // The tokens and heads of a lane's part of the wave's rows, every 4th (of the outputs every 8th): the first from
