@@ -28,9 +28,9 @@
 // chunk); the next step's parts are formed between a step's products.  Of the 11200 cycles a chunk takes (8
 // sequences of 64 heads, a wave per SIMD) 5100 issue, 4000 wait to issue, most of them behind products with nothing
 // beside them (the state's own), 2000 wait for LDS, memory and barriers, of which fragments asked for a chunk
-// earlier took none away.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 349 us, 372 on average
+// earlier took none away.  16384 rows of 8 sequences, 64 heads x 128 x 64 states: 351 us, 377 on average
 // under a profiler, where the fp32 products took 409 and the row-by-row scan 1420; 64 sequences of 26 rows
-// 86 -> 65; 8 heads x 128 x 128 (segments) 78 + 34 for the pass before it, and 57 for the fragments: all
+// 86 -> 65; 8 heads x 128 x 128 (segments) 78 + 34 for the pass before it, and 58 for the fragments: all
 // three wait much for memory, and with entries of one part (HALF) 148 MB of fragments are written and 215
 // read, of 215 and 316 where all have three (walks 3 + 4 us more, fragments 67).
 //
